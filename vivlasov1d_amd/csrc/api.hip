@@ -964,7 +964,10 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(dalloc(c, &c->spec, (size_t)c->nmodes * c->fft_rows * Bz), "alloc spectrum");
     if (p->precond == VV_PRECOND_TENSOR_KINETIC)
         VV_CCHECK(dalloc(c, &c->lu64, (size_t)c->nmodes * lu_pivots_per_mode(c->fft_rows) * Bz), "alloc pivots");
-    VV_CCHECK(dalloc(c, &c->pinv, nx * Bz), "alloc pinv");
+    // the FFT form of the Poisson solve reads the context's twiddles, of length fft_n
+    const bool pfft = (nx & (nx - 1)) == 0 && c->fft_n == nx;
+    if (pfft) VV_CCHECK(dalloc(c, &c->plam, nx * Bz), "alloc plam");
+    else VV_CCHECK(dalloc(c, &c->pinv, nx * Bz), "alloc pinv");
     VV_CCHECK(dalloc(c, &c->pwork, (3 * (size_t)nx + 1) * Bz), "alloc Poisson scratch");
     VV_CCHECK(dalloc(c, &c->X, c->N * Bz), "alloc X");
     VV_CCHECK(dalloc(c, &c->rhs, c->N * Bz), "alloc rhs");
@@ -1021,7 +1024,8 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
         tw32[m].y = (float)sinl(ang);
     }
     // mean-free pseudo-inverse of the periodic Laplacian, per instance:
-    // c_m = 1/nx sum_{k>0} cos(2 pi k m/nx) / lambda_k
+    // c_m = 1/nx sum_{k>0} cos(2 pi k m/nx) / lambda_k, or its symbol 1/(nx lambda_k)
+    // where the solve goes through the FFT
     std::vector<long double> ct(nx), lam(nx);
     for (int q = 0; q < nx; ++q)
         ct[q] = cosl(2.0L * 3.141592653589793238462643383279502884L * (long double)q / (long double)nx);
@@ -1035,6 +1039,11 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
             // CFD4 symbol (54 - 64 cos t + 10 cos 2t)/12 = (128 sin^2(t/2) - 20 sin^2 t)/12; CFD2: 4 sin^2(t/2)
             lam[k] = (p->laplace == VV_LAPLACE_CFD4) ? (128.0L * s1 * s1 - 20.0L * s2 * s2) / (12.0L * h2)
                                                      : (4.0L * s1 * s1) / h2;
+        }
+        if (pfft) {
+            pinv[(size_t)b * nx] = 0.0;
+            for (int k = 1; k < nx; ++k) pinv[(size_t)b * nx + k] = (double)(1.0L / (lam[k] * (long double)nx));
+            continue;
         }
         for (int m = 0; m < nx; ++m) {
             long double s = 0.0L;
@@ -1052,7 +1061,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(hipMemcpy(c->eigen, eig.data(), c->nmodes * sizeof(double2), hipMemcpyHostToDevice), "upload");
     VV_CCHECK(hipMemcpy(c->twiddle, tw.data(), nf * sizeof(double2), hipMemcpyHostToDevice), "upload");
     VV_CCHECK(hipMemcpy(c->twiddle32, tw32.data(), nf * sizeof(float2), hipMemcpyHostToDevice), "upload");
-    VV_CCHECK(hipMemcpy(c->pinv, pinv.data(), nx * Bz * sizeof(double), hipMemcpyHostToDevice), "upload");
+    VV_CCHECK(hipMemcpy(pfft ? c->plam : c->pinv, pinv.data(), nx * Bz * sizeof(double), hipMemcpyHostToDevice), "upload");
     // reciprocal LU pivots of the kinetic T_k (fixed for the run)
     if (c->lu64) VV_CCHECK(launch_tridiag_factor(c, c->lu64, nullptr), "pivots");
     // this device's copy of the allocation-free entry point's scratch array
@@ -1092,7 +1101,7 @@ int vv_ctx_destroy(vv_ctx *c)
     (void)hipStreamSynchronize(c->stream);
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     void *bufs[] = {c->inst,   c->active, c->h0,      c->h1p,     c->h1h,  c->h2p,   c->h2h,    c->eigen,
-                    c->gm,     c->g0,     c->gp,      c->twiddle, c->twiddle32, c->spec, c->pinv, c->pwork,
+                    c->gm,     c->g0,     c->gp,      c->twiddle, c->twiddle32, c->spec, c->pinv, c->plam, c->pwork,
                     c->X,      c->rhs,    c->D,       c->basis,   c->basis32, c->R,   c->partial, c->dscalar,
                     c->npart,  c->gs,     c->T2,      c->xs,   c->vgrid, c->tb,     c->fave,    c->db1,
                     c->db2,    c->ex,     c->w64,     c->d64,   c->lu64,   c->lu32};

@@ -1,26 +1,24 @@
 // Moments, the periodic Poisson solve and the invariants.
 //
-//  density_kernel    column partial sums of f over chunks of v-rows
-//                    (n_i = hv * sum_j f_ij, Toolbox.pyx:79-98); coalesced
-//                    along x, one chunk of rows per block row.
-//  poisson_*_kernel  prep (one workgroup): finishes n, forms
-//                    b = -(n - mean n) q (PETScPoissonSolver.pyx:58-74);
-//                    conv: solves A phi = b by the mean-free circulant inverse
-//                    (the periodic CFD4/CFD2 matrix is circulant; its
-//                    pseudo-inverse's first row is precomputed on the host);
-//                    post (one workgroup): h1 = phi - mean phi
+//  column_kernel     column sums over v-rows of f (n_i = hv * sum_j f_ij,
+//                    Toolbox.pyx:79-98) or of v f and v^2 f (u_i, e_i, the
+//                    output moments, Toolbox.pyx:103-148); one chunk of rows
+//                    per block row.
+//  poisson_kernel    one workgroup per instance: finishes n, forms
+//                    b = -(n - mean n) q (PETScPoissonSolver.pyx:58-74),
+//                    solves A phi = b by the mean-free inverse of the periodic
+//                    (circulant) CFD4/CFD2 matrix, then h1 = phi - mean phi
 //                    (Toolbox.pyx:38-74) and the Poisson residual norm
 //                    ||A phi + (n - mean n) q|| of run_base.py:631-637.
-//  velocity_moments_kernel
-//                    u_i = hv sum_j v_j f_ij and e_i = hv sum_j v_j^2 f_ij
-//                    (Toolbox.pyx:103-148), the output moments: one thread
-//                    per column, rows in order, as the reference's loop.
+//  poisson_prep / conv / post_kernel
+//                    the same in three launches, the convolution spread over
+//                    the chip, for long x-grids that are no power of two.
 //  invariants_kernel mass, L2, kinetic / potential energy over f, plus the
 //                    field energy over phi (distribution_function.pyx:130-199,
 //                    hamiltonian.pyx:67-100, potential.pyx:48-59).
 //
-// In a batched context instance b is blockIdx.y (blockIdx.z for the density
-// partials); its fields start at b * N, its x-vectors at b * nx.
+// In a batched context instance b is blockIdx.y (blockIdx.z for the column
+// sums); its fields start at b * N, its x-vectors at b * nx.
 #include "vv1d_internal.h"
 
 namespace vv {
@@ -30,38 +28,89 @@ constexpr int NT = 256;
 constexpr int PT = 1024;     // threads of the single-workgroup Poisson kernel
 constexpr int DCH = kDensityChunks;   // row chunks of the density reduction
 
-__global__ __launch_bounds__(NT) void density_kernel(const double *__restrict__ f, int nx, int nv,
-                                                     double *__restrict__ npart)
+// Column sums over v-rows.  A workgroup owns 64 columns (one per lane, 512-byte
+// row segments) and a chunk of the rows, dealt to its 16 wavefronts in turn;
+// eight loads per lane are in flight.  MOM 0: sum_j f into out0; MOM 1:
+// sum_j v_j f into out0 and sum_j v_j^2 f into out1.  Partial sums go to
+// out[chunk][i]; with one chunk they are the sums, and scale (hv, else 1) is
+// applied here.  HBM-bound for large grids, one memory latency for small ones.
+// One thread per column (four workgroups at nx = 1000) took 429 us for both
+// velocity moments of 1000 x 2001; density took 10.3 us at 1024 x 2048 with
+// one wavefront per 64 columns and 32 rows.
+constexpr int CW = 16;
+template <int MOM>
+__global__ __launch_bounds__(64 * CW) void column_kernel(const double *__restrict__ f, const double *__restrict__ v,
+                                                         int nx, int nv, int rows, int64_t ostride, double scale,
+                                                         double *__restrict__ out0, double *__restrict__ out1)
 {
+    __shared__ double red[MOM + 1][CW][64];
     f += (size_t)blockIdx.z * nx * nv;
-    npart += (size_t)blockIdx.z * DCH * nx;
-    const int i = blockIdx.x * NT + threadIdx.x;
-    if (i >= nx) return;
-    const int rows = (nv + DCH - 1) / DCH;
-    const int j0 = blockIdx.y * rows;
-    const int j1 = min(nv, j0 + rows);
-    double s = 0.0;
-    for (int j = j0; j < j1; ++j) s += f[(size_t)j * nx + i];
-    npart[(size_t)blockIdx.y * nx + i] = s;
+    out0 += blockIdx.z * ostride + (size_t)blockIdx.y * nx;
+    if (MOM) out1 += blockIdx.z * ostride + (size_t)blockIdx.y * nx;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    const int j0 = blockIdx.y * rows, j1 = min(nv, j0 + rows);
+    double s = 0.0, t = 0.0;
+    if (i < nx) {
+        const double *fp = f + i;
+        for (int j = j0 + w; j < j1; j += 8 * CW) {
+            double x[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int r = j + q * CW;
+                const double y = fp[(size_t)(r < j1 ? r : j0) * nx];
+                x[q] = r < j1 ? y : 0.0;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                if (MOM) {
+                    const int r = j + q * CW;
+                    const double vv = v[r < j1 ? r : j0];
+                    s += vv * x[q];
+                    t += (vv * vv) * x[q];          // v2 = v**2 (Grid), then v2_j * f_ij
+                } else {
+                    s += x[q];
+                }
+            }
+        }
+    }
+    red[0][w][lane] = s;
+    if (MOM) red[MOM][w][lane] = t;
+    __syncthreads();
+    if (w <= MOM && i < nx) {
+        double a = red[w][0][lane];
+#pragma unroll
+        for (int q = 1; q < CW; ++q) a += red[w][q][lane];
+        (w == 0 ? out0 : out1)[i] = a * scale;
+    }
 }
 
-__global__ __launch_bounds__(NT) void velocity_moments_kernel(const double *__restrict__ f,
-                                                              const double *__restrict__ v, int nx, int nv,
-                                                              double hv, double *__restrict__ u, double *__restrict__ e)
+// the chunks' partial sums of x-vectors part0 (and part1, when out1), times scale
+__global__ __launch_bounds__(NT) void column_finish_kernel(const double *__restrict__ part0,
+                                                           const double *__restrict__ part1, int nch, int nx,
+                                                           int64_t pstride, double scale, double *__restrict__ out0,
+                                                           double *__restrict__ out1)
 {
-    f += (size_t)blockIdx.y * nx * nv;
-    u += (size_t)blockIdx.y * nx;
-    e += (size_t)blockIdx.y * nx;
     const int i = blockIdx.x * NT + threadIdx.x;
     if (i >= nx) return;
-    double su = 0.0, se = 0.0;
-    for (int j = 0; j < nv; ++j) {
-        const double fv = f[(size_t)j * nx + i];
-        su += v[j] * fv;
-        se += (v[j] * v[j]) * fv;          // v2 = v**2 (Grid), then v2_j * f_ij
-    }
-    u[i] = su * hv;
-    e[i] = se * hv;
+    const double *p = blockIdx.z ? part1 : part0;
+    double *out = (blockIdx.z ? out1 : out0) + (size_t)blockIdx.y * nx;
+    p += blockIdx.y * pstride;
+    double s = 0.0;
+    for (int ch = 0; ch < nch; ++ch) s += p[(size_t)ch * nx + i];
+    out[i] = s * scale;
+}
+
+// Chunks of rows of the column sums (<= kDensityChunks / 2, so the two velocity
+// moments fit the density's scratch; a function of nv alone, so that a batched
+// instance sums as it would alone).  Up to 512 rows one chunk: 32 rows a
+// wavefront, and no finish launch (velocity moments of 100 x 200: 43.5 us
+// before); beyond, 128 rows a chunk, 256 workgroups at 1024 x 2048.
+int column_chunks(int nv)
+{
+    if (nv <= 512) return 1;
+    const int n = (nv + 127) / 128;
+    return n < kDensityChunks / 2 ? n : kDensityChunks / 2;
 }
 
 __device__ double block_sum_big(double v, double *red)
@@ -82,11 +131,14 @@ __device__ double block_sum_big(double v, double *red)
 
 struct PoiArgs {
     int nx, laplace, from_part;
+    int nch, logn;         // density partials per column; log2 nx (FFT form)
     double hv, charge;
     const InstConst *inst;
     const double *npart;   // density partials (from_part = 1)
     const double *n_in;    // density (from_part = 0)
-    const double *pinv;
+    const double *pinv;    // first row of the mean-free circulant inverse
+    const double *plam;    // FFT form: inverse symbol over nx, 0 for the mean
+    const double2 *tw;     // FFT form: exp(-2 pi i m / nx)
     double *work;          // 3*nx + 1 scratch: b | phi | n | mean n
     double *n_out, *phi, *h1, *pres;
     int pres_stride;       // doubles between the instances' residual norms in pres
@@ -94,7 +146,8 @@ struct PoiArgs {
 
 // A x for the periodic CFD4 / CFD2 stencils, in the reference's order
 // (PETScPoissonCFD4.pyx:78, PETScPoissonCFD2.pyx:78).
-__device__ __forceinline__ double lap(const double *x, int i, int nx, int laplace, double hx2_inv)
+template <typename X>
+__device__ __forceinline__ double lap(const X &x, int i, int nx, int laplace, double hx2_inv)
 {
     const int im2 = i >= 2 ? i - 2 : i - 2 + nx, im1 = i >= 1 ? i - 1 : i - 1 + nx;
     const int ip1 = i + 1 < nx ? i + 1 : i + 1 - nx, ip2 = i + 2 < nx ? i + 2 : i + 2 - nx;
@@ -110,7 +163,8 @@ __device__ __forceinline__ void poi_instance(PoiArgs &a)
     const size_t b = blockIdx.y, nx = a.nx;
     if (a.npart) a.npart += b * DCH * nx;
     if (a.n_in) a.n_in += b * nx;
-    a.pinv += b * nx;
+    if (a.pinv) a.pinv += b * nx;
+    if (a.plam) a.plam += b * nx;
     a.work += b * (3 * nx + 1);
     if (a.n_out) a.n_out += b * nx;
     if (a.phi) a.phi += b * nx;
@@ -118,33 +172,253 @@ __device__ __forceinline__ void poi_instance(PoiArgs &a)
     if (a.pres) a.pres += b * a.pres_stride;
 }
 
+// In-place complex FFT of length n = 2^logn (8 .. 4 PT) in LDS by the whole
+// workgroup: radix-4 Stockham stages, one butterfly a thread, and a radix-2
+// stage for odd logn (two butterflies a thread at most); the next stage's
+// twiddles are loaded while the current one runs.  INV: unnormalised inverse.
+template <bool INV>
+__device__ void line_fft(double2 *buf, int n, int logn, const double2 *__restrict__ tw)
+{
+    const int nq = n >> 2, ns = logn >> 1;
+    const int t = threadIdx.x;
+    const bool on = t < nq;
+    double2 w[3] = {{1.0, 0.0}, {1.0, 0.0}, {1.0, 0.0}};
+    for (int s = 0; s < ns; ++s) {
+        const int Ns = 1 << (2 * s);
+        const int k = t & (Ns - 1);
+        double2 v[4], wn[3] = {{1.0, 0.0}, {1.0, 0.0}, {1.0, 0.0}};
+        if (on) {
+            if (s + 1 < ns) {
+                const int st = (t & (4 * Ns - 1)) << (logn - 4 - 2 * s);
+#pragma unroll
+                for (int r = 0; r < 3; ++r) wn[r] = tw[(r + 1) * st];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = buf[t + r * nq];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                const double wy = INV ? -w[r].y : w[r].y;
+                const double2 x = v[r + 1];
+                v[r + 1].x = x.x * w[r].x - x.y * wy;
+                v[r + 1].y = x.x * wy + x.y * w[r].x;
+            }
+        }
+        __syncthreads();
+        if (on) {
+            const double2 a0{v[0].x + v[2].x, v[0].y + v[2].y}, a1{v[0].x - v[2].x, v[0].y - v[2].y};
+            const double2 a2{v[1].x + v[3].x, v[1].y + v[3].y}, d{v[1].x - v[3].x, v[1].y - v[3].y};
+            const double2 a3 = INV ? double2{-d.y, d.x} : double2{d.y, -d.x};
+            double2 *o = buf + ((t - k) << 2) + k;
+            o[0] = double2{a0.x + a2.x, a0.y + a2.y};
+            o[Ns] = double2{a1.x + a3.x, a1.y + a3.y};
+            o[2 * Ns] = double2{a0.x - a2.x, a0.y - a2.y};
+            o[3 * Ns] = double2{a1.x - a3.x, a1.y - a3.y};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 3; ++r) w[r] = wn[r];
+    }
+    if (logn & 1) {                      // sub-transforms of n/2: outputs j, j + n/2
+        const int nh = n >> 1;
+        double2 lo[2], hi[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int j = t + q * PT;
+            if (j < nh) {
+                const double2 x0 = buf[j], x1 = buf[j + nh], c = tw[j];
+                const double cy = INV ? -c.y : c.y;
+                const double2 m{x1.x * c.x - x1.y * cy, x1.x * cy + x1.y * c.x};
+                lo[q] = double2{x0.x + m.x, x0.y + m.y};
+                hi[q] = double2{x0.x - m.x, x0.y - m.y};
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int j = t + q * PT;
+            if (j < nh) {
+                buf[j] = lo[q];
+                buf[j + nh] = hi[q];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// n_i of the thread's columns i = t + q PT from the density partials, or as
+// given; `on` marks the columns that exist.  Grids of up to PT/2 columns
+// deal the chunks to PT / span threads a column (span: the columns padded to
+// a power of two), whose sums are added in order.
+__device__ __forceinline__ void poi_density(const PoiArgs &a, double (&n)[kMaxNx / PT], double *red)
+{
+    const int nx = a.nx, t = threadIdx.x;
+    if (a.from_part && a.nch > 1 && 2 * nx <= PT) {
+        int span = 64;
+        while (span < nx) span <<= 1;
+        const int g = t / span, i = t & (span - 1), G = PT / span;
+        double s = 0.0;
+        if (i < nx)
+            for (int ch = g; ch < a.nch; ch += G) s += a.npart[(size_t)ch * nx + i];
+        red[t] = s;
+        __syncthreads();
+        n[0] = 0.0;
+        if (t < nx) {
+            double v = red[t];
+            for (int q = 1; q < G; ++q) v += red[q * span + t];
+            n[0] = v * a.hv;
+        }
+        __syncthreads();
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < kMaxNx / PT; ++q) {
+        const int i = t + q * PT;
+        n[q] = 0.0;
+        if (i >= nx) continue;
+        if (!a.from_part) {
+            n[q] = a.n_in[i];
+            continue;
+        }
+        double s = 0.0;
+        for (int c0 = 0; c0 < a.nch; c0 += 8) {
+            double v[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) v[c] = c0 + c < a.nch ? a.npart[(size_t)(c0 + c) * nx + i] : 0.0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) s += v[c];
+        }
+        n[q] = s * a.hv;
+    }
+}
+
+struct ReX {                             // real parts of a complex line
+    const double2 *p;
+    __device__ __forceinline__ double operator[](int i) const { return p[i].x; }
+};
+
+// The whole Poisson pipeline of an instance in one workgroup.  FFT: nx a power
+// of two whose twiddles the context holds; phi = F^-1 (b^ / lambda), two
+// in-LDS transforms.  Otherwise (nx <= kPoissonOne): the convolution with the
+// first row of the circulant inverse, dealt to PT / span threads an output.
+// Latency-bound (barriers, LDS passes); what it saves is two dependent
+// launches and the pass over `work`: prep + conv + post took 13.0 + 11.2 +
+// 4.3 us at nx = 1024 and 6.1 + 2.7 + 3.3 us at nx = 64.
+constexpr int kPoissonOne = 320;
+template <bool FFT>
+__global__ __launch_bounds__(PT) void poisson_kernel(PoiArgs a)
+{
+    extern __shared__ double2 pline[];
+    __shared__ double red[PT];
+    __shared__ double rs[PT / 64 + 1];
+    poi_instance(a);
+    const double hx2_inv = a.inst[blockIdx.y].hx2_inv;
+    const int nx = a.nx, t = threadIdx.x;
+    constexpr int Q = kMaxNx / PT;
+    double n[Q];
+    poi_density(a, n, red);
+    double part = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) part += n[q];            // columns past nx hold 0
+    const double nmean = block_sum_big(part, rs) / nx;
+    double *sb = reinterpret_cast<double *>(pline), *sc = sb + nx;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = t + q * PT;
+        if (i >= nx) continue;
+        if (a.n_out) a.n_out[i] = n[q];
+        const double b = -(n[q] - nmean) * a.charge;
+        if (FFT) {
+            pline[i] = double2{b, 0.0};
+        } else {
+            sb[i] = b;
+            sc[i] = a.pinv[i];
+        }
+    }
+    __syncthreads();
+    if (FFT) {
+        line_fft<false>(pline, nx, a.logn, a.tw);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = t + q * PT;
+            if (i < nx) {
+                const double l = a.plam[i];
+                pline[i] = double2{pline[i].x * l, pline[i].y * l};
+            }
+        }
+        __syncthreads();
+        line_fft<true>(pline, nx, a.logn, a.tw);
+    } else {
+        int span = 64;
+        while (span < nx) span <<= 1;
+        const int G = PT / span, g = t / span, i = t & (span - 1);
+        const int len = (nx + G - 1) / G, m0 = g * len, m1 = m0 + len < nx ? m0 + len : nx;
+        double s0 = 0.0, s1 = 0.0;
+        if (i < nx) {
+            int d = i - m0;                              // (i - m) mod nx, kept in [0, nx)
+            d = d < 0 ? d + nx : d;
+            for (int m = m0; m < m1; m += 2) {
+                s0 += sc[m] * sb[d];
+                d = d == 0 ? nx - 1 : d - 1;
+                if (m + 1 < m1) s1 += sc[m + 1] * sb[d];
+                d = d == 0 ? nx - 1 : d - 1;
+            }
+        }
+        red[t] = s0 + s1;
+        __syncthreads();
+        if (t < nx) {
+            double s = red[t];
+            for (int q = 1; q < G; ++q) s += red[q * span + t];
+            sb[t] = s;                                   // phi takes b's place
+        }
+        __syncthreads();
+    }
+    part = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = t + q * PT;
+        if (i < nx) part += FFT ? pline[i].x : sb[i];
+    }
+    const double phiave = block_sum_big(part, rs) / nx;
+    part = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = t + q * PT;
+        if (i >= nx) continue;
+        const double p = FFT ? pline[i].x : sb[i];
+        if (a.phi) a.phi[i] = p;
+        if (a.h1) a.h1[i] = p - phiave;
+        const double l = FFT ? lap(ReX{pline}, i, nx, a.laplace, hx2_inv) : lap(sb, i, nx, a.laplace, hx2_inv);
+        const double r = l + (n[q] - nmean) * a.charge;
+        part += r * r;
+    }
+    if (a.pres == nullptr) return;                       // uniform over the block
+    const double rr = block_sum_big(part, rs);
+    if (t == 0) *a.pres = sqrt(rr);
+}
+
 // one workgroup: n (from the density partials), mean n, b = -(n - mean n) q
 __global__ __launch_bounds__(PT) void poisson_prep_kernel(PoiArgs a)
 {
-    __shared__ double red[PT / 64 + 1];
+    __shared__ double red[PT];
+    __shared__ double rs[PT / 64 + 1];
     poi_instance(a);
     const int nx = a.nx;
     double *b = a.work, *wn = a.work + 2 * nx;
+    constexpr int Q = kMaxNx / PT;
+    double n[Q];
+    poi_density(a, n, red);
     double part = 0.0;
-    for (int i = threadIdx.x; i < nx; i += PT) {
-        double n;
-        if (a.from_part) {
-            double v[DCH];
 #pragma unroll
-            for (int ch = 0; ch < DCH; ++ch) v[ch] = a.npart[(size_t)ch * nx + i];
-            double s = 0.0;
+    for (int q = 0; q < Q; ++q) part += n[q];
+    const double nmean = block_sum_big(part, rs) / nx;
 #pragma unroll
-            for (int ch = 0; ch < DCH; ++ch) s += v[ch];
-            n = s * a.hv;
-        } else {
-            n = a.n_in[i];
-        }
-        wn[i] = n;
-        if (a.n_out) a.n_out[i] = n;
-        part += n;
+    for (int q = 0; q < Q; ++q) {
+        const int i = threadIdx.x + q * PT;
+        if (i >= nx) continue;
+        wn[i] = n[q];
+        if (a.n_out) a.n_out[i] = n[q];
+        b[i] = -(n[q] - nmean) * a.charge;
     }
-    const double nmean = block_sum_big(part, red) / nx;
-    for (int i = threadIdx.x; i < nx; i += PT) b[i] = -(wn[i] - nmean) * a.charge;
     if (threadIdx.x == 0) a.work[3 * nx] = nmean;
 }
 
@@ -259,18 +533,6 @@ __global__ __launch_bounds__(PT) void pot_to_ham_kernel(const double *phi, doubl
     for (int i = threadIdx.x; i < nx; i += PT) h1[i] = phi[i] - ave;
 }
 
-__global__ __launch_bounds__(NT) void density_finish_kernel(const double *npart, int nch, int nx, double hv,
-                                                            double *n)
-{
-    npart += (size_t)blockIdx.y * DCH * nx;
-    n += (size_t)blockIdx.y * nx;
-    const int i = blockIdx.x * NT + threadIdx.x;
-    if (i >= nx) return;
-    double s = 0.0;
-    for (int ch = 0; ch < nch; ++ch) s += npart[(size_t)ch * nx + i];
-    n[i] = s * hv;
-}
-
 struct InvArgs {
     const double *f, *h0, *h1, *h2, *phi;
     int nx, nv;
@@ -292,24 +554,35 @@ __device__ __forceinline__ void inv_instance(InvArgs &a)
     a.out += b * 6;
 }
 
+// Partial sums per workgroup.  On the periodic x-axis each cell average of
+// the mass, (f_ij + f_i+1,j + f_i,j+1 + f_i+1,j+1) over rows j < nv - 1, counts
+// every f of rows 0..nv-2 twice and of rows 1..nv-1 twice, so one read of f
+// serves all five sums (HBM-bound: 8 N bytes).  Column and row advance with the
+// grid stride instead of being divided out.  16.1 us at 1000 x 2001 with the
+// four neighbours read and a 64-bit division a point.
 __global__ __launch_bounds__(NT) void invariants_kernel(InvArgs a)
 {
     inv_instance(a);
     __shared__ double red[5][NT / 64];
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    const int64_t N = (int64_t)a.nx * a.nv;
-    for (int64_t e = (int64_t)blockIdx.x * NT + threadIdx.x; e < N; e += (int64_t)gridDim.x * NT) {
-        const int j = (int)(e / a.nx);
-        const int i = (int)(e - (int64_t)j * a.nx);
+    const unsigned nx = a.nx, nv = a.nv, N = nx * nv;
+    const unsigned stride = gridDim.x * NT, dj = stride / nx, di = stride - dj * nx;
+    unsigned e = blockIdx.x * NT + threadIdx.x;
+    unsigned j = e / nx, i = e - j * nx;
+    for (; e < N; e += stride) {
         const double fv = a.f[e];
-        if (j < a.nv - 1) {
-            const int ip = (i + 1 == a.nx) ? 0 : i + 1;
-            s[0] += (fv + a.f[(size_t)j * a.nx + ip] + a.f[(size_t)(j + 1) * a.nx + ip] + a.f[e + a.nx]);
-            s[1] += fv * fv;
-        }
+        const double w = (j < nv - 1 ? 2.0 : 0.0) + (j > 0 ? 2.0 : 0.0);
+        s[0] += w * fv;
+        s[1] += j < nv - 1 ? fv * fv : 0.0;
         s[2] += fv * a.h0[j];
         s[3] += fv * a.h1[i];
         s[4] += fv * a.h2[i];
+        j += dj;
+        i += di;
+        if (i >= nx) {
+            i -= nx;
+            ++j;
+        }
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int q = 0; q < 5; ++q) {
@@ -325,73 +598,116 @@ __global__ __launch_bounds__(NT) void invariants_kernel(InvArgs a)
     }
 }
 
-// one workgroup: sums the per-block partials (fixed order) and the field energy
+// one workgroup: sums the per-block partials and the field energy, thread
+// shares first, then over the wavefronts (fixed order).  The sums by one thread
+// (256 partials and nx potential differences in a row) took 68 us at nx = 1000.
 __global__ __launch_bounds__(NT) void invariants_finish_kernel(InvArgs a, int nb)
 {
-    __shared__ double red[5][NT];
+    __shared__ double red[6][NT / 64];
     inv_instance(a);
     const double hx = a.inst[blockIdx.y].hx;
-    double t5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    double t6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     for (int b = threadIdx.x; b < nb; b += NT)
-        for (int q = 0; q < 5; ++q) t5[q] += a.partial[(size_t)b * 5 + q];
-    for (int q = 0; q < 5; ++q) red[q][threadIdx.x] = t5[q];
+        for (int q = 0; q < 5; ++q) t6[q] += a.partial[(size_t)b * 5 + q];
+    for (int i = threadIdx.x; i < a.nx; i += NT) {
+        const double d = a.phi[i + 1 < a.nx ? i + 1 : 0] - a.phi[i];
+        t6[5] += d * d;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int q = 0; q < 6; ++q) {
+        double v = t6[q];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+        if (lane == 0) red[q][wave] = v;
+    }
     __syncthreads();
     if (threadIdx.x != 0) return;
-    double t[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int b = 0; b < NT; ++b)
-        for (int q = 0; q < 5; ++q) t[q] += red[q][b];
+    double t[6];
+    for (int q = 0; q < 6; ++q) {
+        t[q] = red[q][0];
+        for (int w = 1; w < NT / 64; ++w) t[q] += red[q][w];
+    }
     const double hxhv = hx * a.hv;
     const double mass = t[0] * 0.25 * hx * a.hv;
     const double l2 = hxhv * t[1];
     const double ekin = t[2] * hx * a.hv;
     const double epot = (t[3] + t[4]) * hx * a.hv;
-    double ef = 0.0;
-    for (int i = 0; i < a.nx; ++i) {
-        const double d = a.phi[(i + 1) % a.nx] - a.phi[i];
-        ef += d * d;
-    }
     a.out[0] = mass;
     a.out[1] = l2;
     a.out[2] = ekin + 0.5 * epot;
     a.out[3] = ekin;
     a.out[4] = epot;
-    a.out[5] = 0.5 * a.charge * ef / hx;
+    a.out[5] = 0.5 * a.charge * t[5] / hx;
+}
+
+}  // namespace
+
+namespace {
+
+template <int MOM>
+void column_launch(vv_ctx *c, const double *f, int64_t ostride, double scale, double *out0, double *out1)
+{
+    const int nx = c->p.nx, nv = c->p.nv, nch = column_chunks(nv);
+    const int rows = (nv + nch - 1) / nch;
+    hipLaunchKernelGGL(column_kernel<MOM>, dim3((nx + 63) / 64, nch, c->B), dim3(64 * CW), 0, c->stream, f, c->vgrid,
+                       nx, nv, rows, ostride, scale, out0, out1);
+}
+
+void column_finish(vv_ctx *c, const double *part1, double *out0, double *out1)
+{
+    const int nx = c->p.nx;
+    hipLaunchKernelGGL(column_finish_kernel, dim3((nx + NT - 1) / NT, c->B, out1 != nullptr ? 2 : 1), dim3(NT), 0,
+                       c->stream, c->npart, part1, column_chunks(c->p.nv), nx, (int64_t)DCH * nx, c->p.hv, out0,
+                       out1);
 }
 
 }  // namespace
 
 hipError_t launch_density_partial(vv_ctx *c, const double *f, double *npart)
 {
-    dim3 grid((c->p.nx + NT - 1) / NT, DCH, c->B);
-    hipLaunchKernelGGL(density_kernel, grid, dim3(NT), 0, c->stream, f, c->p.nx, c->p.nv,
-                       npart != nullptr ? npart : c->npart);
+    column_launch<0>(c, f, (int64_t)DCH * c->p.nx, 1.0, npart != nullptr ? npart : c->npart, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_density(vv_ctx *c, const double *f, double *n)
 {
-    hipError_t e = launch_density_partial(c, f, nullptr);
+    if (column_chunks(c->p.nv) == 1) {
+        column_launch<0>(c, f, c->p.nx, c->p.hv, n, nullptr);
+        return hipGetLastError();
+    }
+    const hipError_t e = launch_density_partial(c, f, nullptr);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(density_finish_kernel, dim3((c->p.nx + NT - 1) / NT, c->B), dim3(NT), 0, c->stream, c->npart,
-                       DCH,
-                       c->p.nx, c->p.hv, n);
+    column_finish(c, nullptr, n, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_velocity_moments(vv_ctx *c, const double *f, double *u, double *e)
 {
-    hipLaunchKernelGGL(velocity_moments_kernel, dim3((c->p.nx + NT - 1) / NT, c->B), dim3(NT), 0, c->stream, f,
-                       c->vgrid, c->p.nx, c->p.nv, c->p.hv, u, e);
+    if (column_chunks(c->p.nv) == 1) {
+        column_launch<1>(c, f, c->p.nx, c->p.hv, u, e);
+        return hipGetLastError();
+    }
+    double *part1 = c->npart + (size_t)(DCH / 2) * c->p.nx;
+    column_launch<1>(c, f, (int64_t)DCH * c->p.nx, 1.0, c->npart, part1);
+    column_finish(c, part1, u, e);
     return hipGetLastError();
 }
 
 hipError_t launch_poisson(vv_ctx *c, const double *n_in, double *n_out, double *phi, double *h1, double *pres,
                           int from_part, const double *npart, double *work, int pres_stride)
 {
-    PoiArgs a{c->p.nx, c->p.laplace, from_part, c->p.hv, c->p.charge, c->inst,
-              from_part ? (npart != nullptr ? npart : c->npart) : nullptr, n_in, c->pinv,
-              work != nullptr ? work : c->pwork, n_out, phi, h1, pres, pres_stride};
     const int nx = c->p.nx;
+    PoiArgs a{nx, c->p.laplace, from_part, column_chunks(c->p.nv), 0, c->p.hv, c->p.charge, c->inst,
+              from_part ? (npart != nullptr ? npart : c->npart) : nullptr, n_in, c->pinv, c->plam, c->twiddle,
+              work != nullptr ? work : c->pwork, n_out, phi, h1, pres, pres_stride};
+    if (c->plam != nullptr) {
+        while ((1 << a.logn) < nx) ++a.logn;
+        hipLaunchKernelGGL(poisson_kernel<true>, dim3(1, c->B), dim3(PT), nx * sizeof(double2), c->stream, a);
+        return hipGetLastError();
+    }
+    if (nx <= kPoissonOne) {
+        hipLaunchKernelGGL(poisson_kernel<false>, dim3(1, c->B), dim3(PT), 2 * nx * sizeof(double), c->stream, a);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(poisson_prep_kernel, dim3(1, c->B), dim3(PT), 0, c->stream, a);
     hipLaunchKernelGGL(poisson_conv_kernel, dim3((nx + CONV_OUT - 1) / CONV_OUT, c->B), dim3(NT),
                        2 * nx * sizeof(double), c->stream, a);

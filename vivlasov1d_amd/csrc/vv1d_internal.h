@@ -17,7 +17,7 @@ constexpr int kMaxRestart = 64;     // GMRES restart limit (basis of restart+1 v
 constexpr int kMaxNx = 4096;        // largest x size
 constexpr int kMaxNv = 8192;
 constexpr int kReduceBlocks = 512;  // fixed block count of N-sized reductions
-constexpr int kDensityChunks = 64;  // row chunks of the density partial sums (DCH x nx per instance)
+constexpr int kDensityChunks = 64;  // rows of nx partial sums kept per instance for the column sums
 
 // Host-visible part of the GMRES state; copied to pinned host memory after
 // each chunk of iterations.
@@ -98,7 +98,8 @@ struct vv_ctx {
     double2 *lu64;
     float2 *lu32;
     // Poisson
-    double *pinv;       // first row of the mean-free circulant inverse (nx per instance)
+    double *pinv;       // first row of the mean-free circulant inverse (nx per instance); null with plam
+    double *plam;       // nx a power of two: the inverse symbol over nx (nx per instance), for the FFT form
     double *pwork;      // Poisson scratch (3*nx + 1 per instance)
     // work vectors (N)
     double *X;          // bracket / residual output before P^-1
