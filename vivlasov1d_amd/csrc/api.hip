@@ -405,6 +405,10 @@ int arnoldi_step(vv_ctx *c, int it)
     double *v = c->basis + (size_t)it * vs;
     double *w = c->basis + (size_t)(it + 1) * vs;
     const double F = b_field(c), S = b_spec(c);
+    // the fused J v + rFFT takes the previous step's Hessenberg update along;
+    // every other first kernel of a step waits for it
+    const bool fuse_jv = c->op_mode == 0 && c->p.precond != VV_PRECOND_NONE && jac_rfft_rows(c) && !diss_on(c);
+    if (!fuse_jv) VV_CHECK(launch_update(c), "Hessenberg update");
     if (c->op_mode != 0) {
         if (int r = linear_apply(c, v, &c->gs->scale[it], c->op_fbar, c->X, c->ht_inv, -0.5, 0.5, true)) return r;
         if (int r = apply_pc(c, c->X, w, done)) return r;
@@ -416,7 +420,7 @@ int arnoldi_step(vv_ctx *c, int it)
     } else if (const int rows = irfft_mdot_rows(c, false)) {
         // P^-1 J v with the irFFT and the CGS dots of w in one launch; J v
         // and the rFFT in one launch too where no dissipation term is added
-        if (jac_rfft_rows(c) && !diss_on(c)) {
+        if (fuse_jv) {
             VV_PLAUNCH(P_JAC_RFFT, F + S, it, launch_jac_rfft(c, v, &c->gs->scale[it], c->spec, done), "jac_rfft");
         } else {
             VV_PLAUNCH(P_JAC, 2 * F, it, launch_jacobian(c, v, &c->gs->scale[it], c->X), "jacobian");
@@ -427,7 +431,7 @@ int arnoldi_step(vv_ctx *c, int it)
         VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_irfft_mdot(c, c->spec, it, done), "irfft_mdot");
         VV_PLAUNCH(P_MAXPY, F * (it + 3), it, launch_maxpy_norm(c, it, rows), "maxpy_norm");
         return VV_OK;
-    } else if (jac_rfft_rows(c) && !diss_on(c)) {
+    } else if (fuse_jv) {
         // the kinetic P^-1 J v with J v fused into the rFFT; irFFT and dots apart
         VV_PLAUNCH(P_JAC_RFFT, F + S, it, launch_jac_rfft(c, v, &c->gs->scale[it], c->spec, done), "jac_rfft");
         VV_PLAUNCH(P_TRI, 2 * S, it, launch_tridiag_k(c, c->spec, done), "tridiag");
@@ -496,6 +500,7 @@ int arnoldi_step32(vv_ctx *c, int it)
     // dissipation term is added
     const bool fuse_ju = rows && jac_rfft_rows(c) && !diss_on(c);
     if (!fuse_ju) {
+        VV_CHECK(launch_update(c), "Hessenberg update");
         VV_PLAUNCH(P_JAC32, 2 * F, it, launch_jacobian32(c, v, &c->gs->scale[it], ju), "jacobian32");
     }
     if (diss_on(c)) {
@@ -527,15 +532,6 @@ int arnoldi_step32(vv_ctx *c, int it)
     return VV_OK;
 }
 
-GmresStatus *status_slot(vv_ctx *c, int slot) { return c->host_status + (size_t)slot * c->B; }
-
-bool all_done(const GmresStatus *s, int B)
-{
-    for (int b = 0; b < B; ++b)
-        if (!s[b].done) return false;
-    return true;
-}
-
 int max_it_of(const GmresStatus *s, int B)
 {
     int m = 0;
@@ -543,57 +539,81 @@ int max_it_of(const GmresStatus *s, int B)
     return m;
 }
 
-// the device statuses into host slot `slot` by a kernel writing the mapped
-// pinned memory (no copy-engine dispatch)
-int copy_status(vv_ctx *c, int slot)
+// the device statuses into host memory by a kernel writing the mapped pinned
+// buffer (no copy-engine dispatch)
+int copy_status(vv_ctx *c)
 {
     hipLaunchKernelGGL(status_to_host_kernel, dim3((c->B + 255) / 256), dim3(256), 0, c->stream, c->gs,
-                       c->host_status_dev + (size_t)slot * c->B, c->B);
+                       c->host_status_dev, c->B);
     VV_CHECK(hipGetLastError(), "status copy");
     return VV_OK;
 }
 
-// Arnoldi steps of one GMRES cycle, polling the device status every two
-// steps (the status copy of step k is read while steps k+1, k+2 run); returns
-// once the cycle has finished on the device for every instance, with the
-// statuses in host slot 0.  Steps enqueued past the end of an instance's
-// cycle return at once on the device.  build: x += V y is enqueued before
-// the final drain (FP64 x, from the FP32 basis when fp32); update: then
+// Waits for the B reports of slot `slot` numbered seq (a kernel enqueued before
+// stores them); *done: every instance's cycle has ended.  The stream is looked
+// at now and then, so an error on the device ends the wait.
+int wait_report(vv_ctx *c, int slot, uint32_t seq, bool *done)
+{
+    const uint32_t *w = c->host_poll + (size_t)slot * c->B;
+    auto seen = [&]() {
+        *done = true;
+        for (int b = 0; b < c->B; ++b) {
+            const uint32_t v = __atomic_load_n(&w[b], __ATOMIC_RELAXED);
+            if ((v >> 1) != seq) return false;
+            if (!(v & 1)) *done = false;
+        }
+        return true;
+    };
+    for (uint32_t spin = 1; !seen(); ++spin) {
+        if ((spin & 0xffff) != 0) continue;
+        const hipError_t e = hipStreamQuery(c->stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return hipfail(c, e, "report");
+        if (!seen()) return fail(c, VV_ERR_HIP, "the device did not report the end of an Arnoldi step");
+        break;
+    }
+    return VV_OK;
+}
+
+// Arnoldi steps of one GMRES cycle.  The end of step k - 1 is reported by the
+// first kernel of step k (or the update launched before it), while step k's
+// other kernels still run, so the host enqueues step k + 1 only when step k - 1
+// has not ended the cycle and the queue never drains: one step, whose later
+// kernels return at once, is enqueued in vain (an event after every second
+// step left two to three).  Returns once the cycle has finished on the device
+// for every instance, with the statuses in host memory.  build: x += V y is
+// enqueued before the final drain (FP64 x, from the FP32 basis when fp32); update: then
 // f -= x for instances whose solve converged (SNESSolve_KSPONLY's step), so
 // one drain ends the solve.
 int run_cycle(vv_ctx *c, bool fp32, double *build = nullptr, double *update = nullptr)
 {
     const int max_k = c->p.restart;
-    const int chunk = 2;
     const size_t prof_from = c->prof ? prof_of(c)->recs.size() : 0;
-    int it = 0, pend = -1, slot = 0;
     bool stop = false;
-    while (it < max_k && !stop) {
-        const int end = it + chunk < max_k ? it + chunk : max_k;
-        for (; it < end; ++it) {
-            // the chunk's last Hessenberg update stores the statuses into the
-            // host slot itself (no copy dispatch between Arnoldi steps)
-            if (it == end - 1) c->status_out = c->host_status_dev + (size_t)slot * c->B;
-            int r = fp32 ? arnoldi_step32(c, it) : arnoldi_step(c, it);
-            c->status_out = nullptr;
-            if (r) return r;
+    c->pend_it = -1;
+    for (int it = 0; it < max_k; ++it) {
+        if (it >= 2) {
+            if (int r = wait_report(c, it & 1, c->report_seq, &stop)) return r;
+            if (stop) break;
         }
-        VV_CHECK(hipEventRecord(c->ev[slot], c->stream), "event");
-        if (pend >= 0) {
-            VV_CHECK(hipEventSynchronize(c->ev[pend]), "event sync");
-            if (all_done(status_slot(c, pend), c->B)) stop = true;
+        if (it >= 1) {
+            c->report_out = c->host_poll_dev + (size_t)((it - 1) & 1) * c->B;
+            c->report_seq = c->report_seq >= 0x7fffffffu ? 1 : c->report_seq + 1;
         }
-        pend = slot;
-        slot ^= 1;
+        const int r = fp32 ? arnoldi_step32(c, it) : arnoldi_step(c, it);
+        c->report_out = nullptr;
+        if (r) return r;
     }
+    if (stop) c->pend_it = -1;         // the last step ran past every instance's end
+    else VV_CHECK(launch_update(c), "Hessenberg update");
     if (build) {
         if (fp32) VV_CHECK(launch_build_solution32(c, build), "build solution");
         else VV_CHECK(launch_build_solution(c, build), "build solution");
         if (update) VV_CHECK(launch_axpy_cond(c, -1.0, build, update), "update");
     }
-    if (int r = copy_status(c, 0)) return r;
+    if (int r = copy_status(c)) return r;
     VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
-    prof_mark_idle(c, prof_from, max_it_of(status_slot(c, 0), c->B));
+    prof_mark_idle(c, prof_from, max_it_of(c->host_status, c->B));
     return VV_OK;
 }
 
@@ -608,7 +628,7 @@ int cycle_start_from(vv_ctx *c, const double *b)
 void fill_results(vv_ctx *c, vv_ksp_result *res)
 {
     if (!res) return;
-    const GmresStatus *st = status_slot(c, 0);
+    const GmresStatus *st = c->host_status;
     for (int b = 0; b < c->B; ++b) {
         res[b].its = st[b].its;
         res[b].reason = st[b].reason;
@@ -623,7 +643,7 @@ void fill_results(vv_ctx *c, vv_ksp_result *res)
 int restart_cycles(vv_ctx *c, const double *b, double *x)
 {
     for (;;) {
-        const GmresStatus *st = status_slot(c, 0);
+        const GmresStatus *st = c->host_status;
         bool more = false;
         for (int q = 0; q < c->B; ++q)
             if (st[q].active && st[q].reason == 0) more = true;
@@ -678,8 +698,10 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
             if ((le = launch_zero(c, c->D, c->N * c->B)) != hipSuccess) break;
             if ((le = launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it)) != hipSuccess) break;
             if ((r = cycle_start_from(c, c->rhs))) break;
+            c->pend_it = -1;
             for (int it = 0; it < c->p.restart && r == VV_OK; ++it) r = arnoldi_step(c, it);
             if (r) break;
+            if ((le = launch_update(c)) != hipSuccess) break;
             le = launch_build_solution(c, c->D);
         } while (0);
         hipGraph_t g = nullptr;
@@ -704,7 +726,7 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
         c->graph_kp[3] = (double)kp->max_it;
     }
     VV_CHECK(hipGraphLaunch(c->graph_exec, c->stream), "graph launch");
-    if (int r = copy_status(c, 0)) return r;
+    if (int r = copy_status(c)) return r;
     VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
     return VV_OK;
 }
@@ -725,7 +747,7 @@ int snes_impl(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp, v
         // the drain (a no-op unless the cycle converged; a restart leaves it
         // to the update below)
         if (int r = run_cycle(c, false, c->D, c->B == 1 ? f : nullptr)) return r;
-        if (c->B == 1 && status_slot(c, 0)[0].reason != 0) {
+        if (c->B == 1 && c->host_status[0].reason != 0) {
             fill_results(c, res);
             return VV_OK;
         }
@@ -771,7 +793,7 @@ int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_par
         VV_CHECK(launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it), "gmres init");
         VV_CHECK(launch_start32(c, b), "cycle start");
         if (int r = run_cycle(c, true, x)) return r;
-        const GmresStatus st = status_slot(c, 0)[0];
+        const GmresStatus st = c->host_status[0];
         if (st.reason != 0) {
             fill_results(c, res);
             if (cycles) *cycles = st.it > 0 ? 1 : 0;
@@ -818,7 +840,7 @@ int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_par
         VV_CHECK(launch_gmres_init(c, rt, 0.0, 1.0e300, kp->max_it - its), "gmres init");
         VV_CHECK(launch_start32(c, rsrc), "cycle start");
         if (int r = run_cycle(c, true, x)) return r;
-        its += status_slot(c, 0)[0].it;
+        its += c->host_status[0].it;
         ++rounds;
         // true FP64 residual r = b - P^-1 J x
         VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian(c, x, nullptr, c->X), "jacobian");
@@ -896,6 +918,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     c->p.hx = hxs[0];
     c->B = B;
     c->fuse = true;
+    c->pend_it = -1;
     c->stream = reinterpret_cast<hipStream_t>(stream);
     const int nx = p->nx, nv = p->nv;
     c->N = (int64_t)nx * nv;
@@ -977,10 +1000,13 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(dalloc(c, &c->dscalar, ds_count(B)), "alloc scalars");
     VV_CCHECK(dalloc(c, &c->npart, (size_t)64 * nx * Bz), "alloc density partials");
     VV_CCHECK(dalloc(c, &c->gs, Bz), "alloc gmres state");
-    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_status), 2 * Bz * sizeof(GmresStatus)),
+    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_status), Bz * sizeof(GmresStatus)),
               "pinned status");
     VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_status_dev), c->host_status, 0),
               "pinned status device address");
+    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_poll), 2 * Bz * sizeof(uint32_t)), "pinned reports");
+    VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_poll_dev), c->host_poll, 0),
+              "pinned reports device address");
     VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_scalars), ds_count(B) * sizeof(double)),
               "pinned scalars");
     VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_scalars_dev), c->host_scalars, 0),
@@ -988,8 +1014,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_active), Bz * sizeof(int32_t)), "pinned mask");
     VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_active_dev), c->host_active, 0),
               "pinned mask device address");
-    VV_CCHECK(hipEventCreateWithFlags(&c->ev[0], hipEventDisableTiming), "event");
-    VV_CCHECK(hipEventCreateWithFlags(&c->ev[1], hipEventDisableTiming), "event");
+    std::memset(c->host_poll, 0, 2 * Bz * sizeof(uint32_t));
     VV_CCHECK(hipMemset(c->gs, 0, Bz * sizeof(GmresState)), "zero gmres state");
     VV_CCHECK(hipMemset(c->partial, 0, (size_t)c->part_stride * Bz * sizeof(double)), "zero partials");
     VV_CCHECK(hipMemset(c->h1p, 0, nx * Bz * sizeof(double)), "zero h1p");
@@ -1110,8 +1135,7 @@ int vv_ctx_destroy(vv_ctx *c)
     if (c->host_status) (void)hipHostFree(c->host_status);
     if (c->host_scalars) (void)hipHostFree(c->host_scalars);
     if (c->host_active) (void)hipHostFree(c->host_active);
-    if (c->ev[0]) (void)hipEventDestroy(c->ev[0]);
-    if (c->ev[1]) (void)hipEventDestroy(c->ev[1]);
+    if (c->host_poll) (void)hipHostFree(c->host_poll);
     Prof *pr = prof_of(c);
     if (pr) {
         for (auto &r : pr->recs) {
@@ -1271,6 +1295,7 @@ int vv_autotune(vv_ctx *c, int32_t *fft_rows, int32_t *cgs_ept)
                 VV_CHECK(launch_gmres_init(c, 1e-300, 0.0, 1e300, 1 << 30), "gmres init");
                 VV_CHECK(launch_mdot(c, col), "mdot");
                 VV_CHECK(launch_maxpy_norm(c, col), "maxpy");
+                VV_CHECK(launch_update(c), "Hessenberg update");
                 return VV_OK;
             };
             if ((rc = timed(body, 5, &ms))) break;

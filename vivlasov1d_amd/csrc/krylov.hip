@@ -22,30 +22,13 @@
 // partials before the finish, so no device-scope fence (an L2 write-back on
 // this GPU) is needed inside the streaming kernels.
 #include "cgs_vec.h"
+#include "gmres_dev.h"
 
 namespace vv {
 namespace {
 
 constexpr int NT = kCgsNT;
 constexpr int NW = kCgsNW;
-
-// Sum over the block, returned in every thread (fixed tree).
-__device__ __forceinline__ double block_sum_all(double v, double *red)
-{
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < NW; ++w) s += red[w];
-        red[NW] = s;
-    }
-    __syncthreads();
-    const double s = red[NW];
-    __syncthreads();
-    return s;
-}
 
 // Sum of part[0..nb) by the whole block (thread t adds t, t+NT, ...).
 __device__ __forceinline__ double final_sum_1(const double *part, int nb, double *red)
@@ -87,14 +70,6 @@ __device__ void final_sum_cols(const double *part, int nb, int ncols, double *ou
         out[threadIdx.x] = s;
     }
     __syncthreads();
-}
-
-__device__ __forceinline__ int ksp_test(const GmresState *g, double res)
-{
-    if (!isfinite(res)) return VV_KSP_DIVERGED_NANORINF;
-    if (res <= g->ttol) return res < g->atol ? VV_KSP_CONVERGED_ATOL : VV_KSP_CONVERGED_RTOL;
-    if (res >= g->dtol * g->st.rnorm0) return VV_KSP_DIVERGED_DTOL;
-    return 0;
 }
 
 // Instance b of a batched context is blockIdx.y in every kernel below.
@@ -353,98 +328,8 @@ __global__ __launch_bounds__(NT) void maxpy_norm_kernel(CgsArgs<S> a, int it)
     if (threadIdx.x == 0) a.part[a.noff + blockIdx.x] = s;
 }
 
-// VecNormalize of V_{it+1} from the maxpy partials, then
-// KSPGMRESUpdateHessenberg (rotations, happy breakdown, residual estimate)
-// and the convergence test; sets done when the cycle ends.  The Hessenberg
-// column and the previous rotations are staged in LDS by the whole block
-// (loads in flight together with the norm's partials), so the sequential
-// rotation chain of thread 0 reads LDS, not dependent global loads.
-// hout (optional, pinned host memory mapped for the device): the instance's
-// status is also stored there, so the host polls it without a copy.
-__device__ __forceinline__ void put_status(GmresStatus *hout, const GmresStatus &st)
-{
-    // per-field vector stores by one lane
-    hout->it = st.it;
-    hout->its = st.its;
-    hout->reason = st.reason;
-    hout->done = st.done;
-    hout->active = st.active;
-    hout->res = st.res;
-    hout->rnorm0 = st.rnorm0;
-}
-
-__global__ __launch_bounds__(NT) void gmres_update_kernel(const double *part, int nb, int64_t pstride, int it,
-                                                          GmresState *g, GmresStatus *hout)
-{
-    g += blockIdx.y;
-    part += blockIdx.y * pstride;
-    if (hout) hout += blockIdx.y;
-    // every load of the block is issued before the early-exit test waits on
-    // the flag's (reading the state of a finished cycle is harmless)
-    const int32_t done = g->st.done;
-    __shared__ double red[NW + 1];
-    __shared__ double s_h[kMaxRestart + 2], s_c[kMaxRestart], s_s[kMaxRestart];
-    double *hh = g->hh + (size_t)it * (kMaxRestart + 1);
-    const double h_t = threadIdx.x <= it ? hh[threadIdx.x] : 0.0;
-    const double c_t = threadIdx.x < it ? g->cc[threadIdx.x] : 0.0;
-    const double s_t = threadIdx.x < it ? g->ss[threadIdx.x] : 0.0;
-    const double grs_it = g->grs[it];
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nb; b += NT) acc += part[b];
-    if (done) {                        // uniform over the block, before any barrier
-        if (hout && threadIdx.x == 0) put_status(hout, g->st);
-        return;
-    }
-    if (threadIdx.x <= it) s_h[threadIdx.x] = h_t;
-    if (threadIdx.x < it) {
-        s_c[threadIdx.x] = c_t;
-        s_s[threadIdx.x] = s_t;
-    }
-    const double tot = block_sum_all(acc, red);        // barriers: the LDS stores above are visible
-    if (threadIdx.x != 0) return;
-    const double tt = sqrt(tot);
-    s_h[it + 1] = tt;
-    g->scale[it + 1] = tt != 0.0 ? 1.0 / tt : 1.0;
-    // happy breakdown
-    double hapbnd = fabs(tt / grs_it);
-    if (hapbnd > g->haptol) hapbnd = g->haptol;
-    const bool hapend = tt < hapbnd;
-    // apply the previous rotations to the new column
-    for (int q = 1; q <= it; ++q) {
-        const double t0 = s_h[q - 1];
-        s_h[q - 1] = s_c[q - 1] * t0 + s_s[q - 1] * s_h[q];
-        s_h[q] = s_c[q - 1] * s_h[q] - s_s[q - 1] * t0;
-    }
-    double res;
-    int reason = 0;
-    if (!hapend) {
-        const double d = sqrt(s_h[it] * s_h[it] + s_h[it + 1] * s_h[it + 1]);
-        if (d == 0.0) {
-            reason = VV_KSP_DIVERGED_BREAKDOWN;
-            res = g->st.res;
-        } else {
-            const double cc = s_h[it] / d, ss = s_h[it + 1] / d;
-            g->cc[it] = cc;
-            g->ss[it] = ss;
-            g->grs[it + 1] = -(ss * grs_it);
-            g->grs[it] = cc * grs_it;
-            s_h[it] = cc * s_h[it] + ss * s_h[it + 1];
-            res = fabs(-(ss * grs_it));
-        }
-    } else {
-        res = 0.0;
-    }
-    for (int q = 0; q <= it + 1; ++q) hh[q] = s_h[q];
-    g->st.it = it + 1;
-    g->st.its += 1;
-    g->st.res = res;
-    if (reason == 0) reason = ksp_test(g, res);
-    if (hapend && reason == 0) reason = VV_KSP_DIVERGED_BREAKDOWN;
-    if (reason == 0 && g->st.its >= g->max_it) reason = VV_KSP_DIVERGED_ITS;
-    g->st.reason = reason;
-    if (reason != 0 || g->st.it >= g->max_k || g->st.its >= g->max_it) g->st.done = 1;
-    if (hout) put_status(hout, g->st);
-}
+// The end of an Arnoldi step in a launch of its own (gmres_dev.h).
+__global__ __launch_bounds__(NT) void gmres_update_kernel(HessArgs a) { hess_update(a); }
 
 // KSPGMRESBuildSoln: back substitution with the rotated Hessenberg matrix;
 // the coefficients go to coef[0..it).  The triangle is staged in LDS first.
@@ -719,11 +604,9 @@ hipError_t mdot_t(vv_ctx *c, const S *basis, int col)
 template <typename S>
 hipError_t maxpy_norm_t(vv_ctx *c, const S *basis, int it, int dot_rows)
 {
-    hipError_t e = cgs_dispatch(c, basis, 1, it, nullptr, dot_rows);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(gmres_update_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, c->partial + norm_partial_offset(c),
-                       cgs_blocks_v(c, c->N / V16<S>::L), c->part_stride, it, c->gs, c->status_out);
-    return hipGetLastError();
+    c->pend_it = it;
+    c->pend_nb = cgs_blocks_v(c, c->N / V16<S>::L);
+    return cgs_dispatch(c, basis, 1, it, nullptr, dot_rows);
 }
 
 template <typename S>
@@ -740,6 +623,24 @@ hipError_t launch_maxpy_norm(vv_ctx *c, int it, int dot_rows)
 {
     return maxpy_norm_t<double>(c, c->basis, it, dot_rows);
 }
+
+HessArgs take_update(vv_ctx *c)
+{
+    const HessArgs a{c->partial + norm_partial_offset(c), c->part_stride, c->pend_it >= 0 ? c->pend_nb : 0,
+                     c->pend_it, c->gs, c->report_out, c->report_seq};
+    c->pend_it = -1;
+    c->report_out = nullptr;
+    return a;
+}
+
+hipError_t launch_update(vv_ctx *c)
+{
+    const HessArgs a = take_update(c);
+    if (a.nb == 0) return hipSuccess;
+    hipLaunchKernelGGL(gmres_update_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_build_solution(vv_ctx *c, double *x) { return build_solution_t<double>(c, c->basis, x); }
 hipError_t launch_mdot32(vv_ctx *c, int col) { return mdot_t<float>(c, c->basis32, col); }
 hipError_t launch_maxpy_norm32(vv_ctx *c, int it, int dot_rows)

@@ -19,8 +19,8 @@ constexpr int kMaxNv = 8192;
 constexpr int kReduceBlocks = 512;  // fixed block count of N-sized reductions
 constexpr int kDensityChunks = 64;  // rows of nx partial sums kept per instance for the column sums
 
-// Host-visible part of the GMRES state; copied to pinned host memory after
-// each chunk of iterations.
+// Host-visible part of the GMRES state; copied to pinned host memory at the end
+// of a cycle.
 struct GmresStatus {
     int32_t it;        // iterations in the current cycle
     int32_t its;       // total iterations
@@ -56,6 +56,19 @@ struct GmresState {
     int32_t max_k;
     int32_t first;                   // first cycle: sets rnorm0 and ttol
     int32_t pad;
+};
+
+// The Hessenberg update of Arnoldi step `it` (gmres_dev.h): its norm partials
+// (instance b at part + b pstride, nb of them; nb = 0: no update is due), the
+// states, and where the host polls for the report (one word per instance;
+// null: nobody does) and its number.
+struct HessArgs {
+    const double *part;
+    int64_t pstride;
+    int nb, it;
+    GmresState *g;
+    uint32_t *hout;
+    uint32_t seq;
 };
 
 }  // namespace vv
@@ -116,14 +129,17 @@ struct vv_ctx {
     double *dscalar;    // device scalars, 16 per instance
     double *npart;      // density partial sums, 64 nx per instance
     vv::GmresState *gs;             // B states
-    vv::GmresStatus *host_status;   // pinned, 2 slots of B statuses
+    vv::GmresStatus *host_status;   // pinned, B statuses
     vv::GmresStatus *host_status_dev;   // the same memory as the device addresses it
-    vv::GmresStatus *status_out;    // set for one launch: the Hessenberg update also stores the statuses there
+    uint32_t *host_poll;            // pinned, 2 slots of B words: reports of the Hessenberg updates
+    uint32_t *host_poll_dev;        // the same memory as the device addresses it
+    uint32_t *report_out;           // set for one launch: where the Hessenberg update reports
+    uint32_t report_seq;            // number of the last report asked for (below 2^31)
+    int pend_it, pend_nb;           // Arnoldi step whose Hessenberg update is due (-1: none), its norm partials
     double *host_scalars;           // pinned staging of device scalars
     double *host_scalars_dev;       // the same memory as the device addresses it
     int32_t *host_active;           // pinned staging of the instance mask
     int32_t *host_active_dev;       // the same memory as the device addresses it
-    hipEvent_t ev[2];
     // profiling (per-kernel HIP event pairs)
     int prof;           // bit k set: time kernel kind k
     void *prof_state;
@@ -236,9 +252,13 @@ hipError_t launch_norm_start(vv_ctx *c);                  // cycle start on basi
 int cgs_blocks_max(int64_t N);                            // partial rows the CGS kernels may use
 int cgs_ept(const vv_ctx *c, int64_t nvv);              // 16-byte vectors per thread of a CGS launch
 hipError_t launch_mdot(vv_ctx *c, int col);               // CGS dots of basis[col+1] vs 0..col
-// CGS update of basis[it+1] + Givens; dot_rows: partial rows of the dots
-// launch before it (0: launch_mdot's grid)
+// CGS update of basis[it+1]; dot_rows: partial rows of the dots launch before
+// it (0: launch_mdot's grid).  The step's Hessenberg update is then due: the
+// next step's fused first kernel takes it along (take_update), anything else
+// runs it first (launch_update; nothing when none is due)
 hipError_t launch_maxpy_norm(vv_ctx *c, int it, int dot_rows = 0);
+HessArgs take_update(vv_ctx *c);
+hipError_t launch_update(vv_ctx *c);
 hipError_t launch_build_solution(vv_ctx *c, double *x);  // x += V y
 hipError_t launch_start32(vv_ctx *c, const double *r);    // FP32 cycle start: V_0 = (float) r
 hipError_t launch_mdot32(vv_ctx *c, int col);
