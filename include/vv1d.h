@@ -139,7 +139,10 @@ int vv_autotune(vv_ctx *ctx, int32_t *fft_rows, int32_t *cgs_ept);
  * P^-1 J v and the CGS dots of the new vector in one launch, and where
  * besides nx >= 256 and no dissipation term is set, J v and its rFFT in one
  * launch (J v is not stored).  Results are identical either way (up to the
- * sign of exact zeros); 0 runs the separate kernels (for timing). */
+ * sign of exact zeros).  At the other x-lengths up to 2048 both launches work
+ * on blocks of whole rows, whose dots are summed in another order than the
+ * separate launch's (equal to rounding).  0 runs the separate kernels (for
+ * timing). */
 int vv_set_fusion(vv_ctx *ctx, int enable);
 
 /* Context lifetime and stream plumbing.  vv_ctx_destroy frees what the

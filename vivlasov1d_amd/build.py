@@ -27,6 +27,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=" + ARCH,
 UNITS = {
     "bracket.hip": ["-ffp-contract=off"],
     "spectral.hip": ["-ffp-contract=fast-honor-pragmas"],
+    "rows.hip": ["-ffp-contract=fast-honor-pragmas"],
     "krylov.hip": ["-ffp-contract=off"],
     "moments.hip": ["-ffp-contract=off"],
     "dissipation.hip": ["-ffp-contract=off"],

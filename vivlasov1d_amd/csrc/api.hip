@@ -390,6 +390,64 @@ int no_diss(vv_ctx *c, const char *what)
     return fail(c, VV_ERR_UNSUPPORTED, std::string(what) + " does not take a dissipation term");
 }
 
+// The spectrum of J u (u times its optional device scale) in one launch: the
+// strip kernel (nx = 256, 512, 1024), or the row blocks for every other length
+// up to kRowsNx and for a collision term.  fwd_fused: whether there is such a
+// launch for the context.
+bool fwd_fused(const vv_ctx *c)
+{
+    if (c->op_mode != 0 || c->p.precond != VV_PRECOND_TENSOR_KINETIC) return false;
+    if (!diss_on(c) && jac_rfft_rows(c)) return true;
+    return rows_apply(c) && (!diss_on(c) || diss_coll(c));
+}
+
+int fwd_jac(vv_ctx *c, const double *u, const double *uscale, const int32_t *done, int it)
+{
+    const double F = b_field(c), S = b_spec(c);
+    if (!diss_on(c) && jac_rfft_rows(c)) {
+        VV_PLAUNCH(P_JAC_RFFT, F + S, it, launch_jac_rfft(c, u, uscale, c->spec, done), "jac_rfft");
+        return VV_OK;
+    }
+    CollTerm ct;
+    bool coll = false;
+    if (diss_coll(c)) {
+        if (int r = need_moments(c)) return r;
+        coll = collision_term(c, c->mom[0], c->mom[1], c->mom[3], 0.5, &ct);
+    }
+    VV_PLAUNCH(P_JAC_RFFT, F + S, it, launch_row_jac(c, u, uscale, coll ? &ct : nullptr, c->spec, done), "row J u");
+    return VV_OK;
+}
+
+// y = P^-1 F(f)
+int pc_residual(vv_ctx *c, const double *f, const double *fh, double *y)
+{
+    if (!rows_apply(c) || diss_on(c)) {
+        VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, c->X), "residual");
+        if (int r = diss_function(c, f, fh, c->X)) return r;
+        return precond(c, c->X, y, nullptr);
+    }
+    const double F = b_field(c), S = b_spec(c);
+    VV_PLAUNCH(P_RES, 2 * F + S, -1, launch_row_res(c, f, fh, c->spec), "row F(f)");
+    VV_PLAUNCH(P_TRI, 2 * S, -1, launch_tridiag_k(c, c->spec, nullptr), "tridiag");
+    VV_PLAUNCH(P_IRFFT, S + F, -1, launch_irfft(c, c->spec, y, nullptr), "irfft");
+    return VV_OK;
+}
+
+// y = P^-1 J u
+int pc_jacobian(vv_ctx *c, const double *u, double *y)
+{
+    const double F = b_field(c), S = b_spec(c);
+    if (!fwd_fused(c)) {
+        VV_PLAUNCH(P_JAC, 2 * F, -1, launch_jacobian(c, u, nullptr, c->X), "jacobian");
+        if (int r = diss_jacobian(c, u, nullptr, c->X, nullptr)) return r;
+        return precond(c, c->X, y, nullptr);
+    }
+    if (int r = fwd_jac(c, u, nullptr, nullptr, -1)) return r;
+    VV_PLAUNCH(P_TRI, 2 * S, -1, launch_tridiag_k(c, c->spec, nullptr), "tridiag");
+    VV_PLAUNCH(P_IRFFT, S + F, -1, launch_irfft(c, c->spec, y, nullptr), "irfft");
+    return VV_OK;
+}
+
 // the preconditioner of the GMRES cycle: P^-1, or P^-T for the adjoint
 int apply_pc(vv_ctx *c, const double *x, double *y, const int32_t *done)
 {
@@ -407,8 +465,13 @@ int arnoldi_step(vv_ctx *c, int it)
     const double F = b_field(c), S = b_spec(c);
     // the fused J v + rFFT takes the previous step's Hessenberg update along;
     // every other first kernel of a step waits for it
-    const bool fuse_jv = c->op_mode == 0 && c->p.precond != VV_PRECOND_NONE && jac_rfft_rows(c) && !diss_on(c);
+    const bool fuse_jv = fwd_fused(c);
     if (!fuse_jv) VV_CHECK(launch_update(c), "Hessenberg update");
+    // the irFFT and the CGS dots of w in one launch: the slice kernel, or row blocks
+    // (not at the strip kernel's lengths, where fused and separate launches are
+    // bit-identical)
+    const int rows = c->op_mode == 0 ? irfft_mdot_rows(c, false) : 0;
+    const bool blocks = c->op_mode == 0 && !rows && rows_apply(c) && !jac_rfft_rows(c);
     if (c->op_mode != 0) {
         if (int r = linear_apply(c, v, &c->gs->scale[it], c->op_fbar, c->X, c->ht_inv, -0.5, 0.5, true)) return r;
         if (int r = apply_pc(c, c->X, w, done)) return r;
@@ -417,25 +480,26 @@ int arnoldi_step(vv_ctx *c, int it)
         // goes straight into the next basis vector
         VV_PLAUNCH(P_JAC, 2 * F, it, launch_jacobian(c, v, &c->gs->scale[it], w), "jacobian");
         if (int r = diss_jacobian(c, v, &c->gs->scale[it], w, done)) return r;
-    } else if (const int rows = irfft_mdot_rows(c, false)) {
-        // P^-1 J v with the irFFT and the CGS dots of w in one launch; J v
-        // and the rFFT in one launch too where no dissipation term is added
+    } else if (fuse_jv || rows || blocks) {
         if (fuse_jv) {
-            VV_PLAUNCH(P_JAC_RFFT, F + S, it, launch_jac_rfft(c, v, &c->gs->scale[it], c->spec, done), "jac_rfft");
+            if (int r = fwd_jac(c, v, &c->gs->scale[it], done, it)) return r;
         } else {
             VV_PLAUNCH(P_JAC, 2 * F, it, launch_jacobian(c, v, &c->gs->scale[it], c->X), "jacobian");
             if (int r = diss_jacobian(c, v, &c->gs->scale[it], c->X, done)) return r;
             VV_PLAUNCH(P_RFFT, F + S, it, launch_rfft(c, c->X, c->spec, done), "rfft");
         }
         VV_PLAUNCH(P_TRI, 2 * S, it, launch_tridiag_k(c, c->spec, done), "tridiag");
-        VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_irfft_mdot(c, c->spec, it, done), "irfft_mdot");
-        VV_PLAUNCH(P_MAXPY, F * (it + 3), it, launch_maxpy_norm(c, it, rows), "maxpy_norm");
+        if (rows) {
+            VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_irfft_mdot(c, c->spec, it, done), "irfft_mdot");
+        } else if (blocks) {
+            VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_row_inv(c, c->spec, it, done), "row irfft + dots");
+        } else {
+            VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft(c, c->spec, w, done), "irfft");
+            VV_PLAUNCH(P_MDOT, F * (it + 2), it, launch_mdot(c, it), "mdot");
+        }
+        VV_PLAUNCH(P_MAXPY, F * (it + 3), it,
+                   launch_maxpy_norm(c, it, rows ? rows : (blocks ? row_inv_blocks(c) : 0)), "maxpy_norm");
         return VV_OK;
-    } else if (fuse_jv) {
-        // the kinetic P^-1 J v with J v fused into the rFFT; irFFT and dots apart
-        VV_PLAUNCH(P_JAC_RFFT, F + S, it, launch_jac_rfft(c, v, &c->gs->scale[it], c->spec, done), "jac_rfft");
-        VV_PLAUNCH(P_TRI, 2 * S, it, launch_tridiag_k(c, c->spec, done), "tridiag");
-        VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft(c, c->spec, w, done), "irfft");
     } else {
         VV_PLAUNCH(P_JAC, 2 * F, it, launch_jacobian(c, v, &c->gs->scale[it], c->X), "jacobian");
         if (int r = diss_jacobian(c, v, &c->gs->scale[it], c->X, done)) return r;
@@ -495,10 +559,13 @@ int arnoldi_step32(vv_ctx *c, int it)
     float *X = reinterpret_cast<float *>(c->X);
     const double F = 4.0 * (double)c->N * c->B;
     float *ju = c->p.precond == VV_PRECOND_NONE ? w : X;
-    const int rows = c->p.precond != VV_PRECOND_NONE ? irfft_mdot_rows(c, true) : 0;
+    int rows = c->p.precond != VV_PRECOND_NONE ? irfft_mdot_rows(c, true) : 0;
+    const bool blocks = !rows && rows_apply(c) && !jac_rfft_rows(c);
+    if (blocks) rows = row_inv_blocks(c);
     // J u and its rFFT in one launch where the fused kernels apply and no
     // dissipation term is added
-    const bool fuse_ju = rows && jac_rfft_rows(c) && !diss_on(c);
+    const bool strips = jac_rfft_rows(c) > 0;
+    const bool fuse_ju = rows && (strips || rows_apply(c)) && !diss_on(c);
     if (!fuse_ju) {
         VV_CHECK(launch_update(c), "Hessenberg update");
         VV_PLAUNCH(P_JAC32, 2 * F, it, launch_jacobian32(c, v, &c->gs->scale[it], ju), "jacobian32");
@@ -516,12 +583,16 @@ int arnoldi_step32(vv_ctx *c, int it)
         float2 *spec = reinterpret_cast<float2 *>(c->spec);
         const double S = 0.5 * b_spec(c);
         if (fuse_ju) {
-            VV_PLAUNCH(P_JAC_RFFT32, F + S, it, launch_jac_rfft32(c, v, &c->gs->scale[it], spec, done), "jac_rfft32");
+            VV_PLAUNCH(P_JAC_RFFT32, F + S, it,
+                       strips ? launch_jac_rfft32(c, v, &c->gs->scale[it], spec, done)
+                              : launch_row_jac32(c, v, &c->gs->scale[it], spec, done), "jac_rfft32");
         } else {
             VV_PLAUNCH(P_RFFT32, F + S, it, launch_rfft32(c, X, spec, done), "rfft32");
         }
         VV_PLAUNCH(P_TRI32, 2 * S, it, launch_tridiag32(c, spec, done), "tridiag32");
-        VV_PLAUNCH(P_IRFFT_MDOT32, S + F * (it + 2), it, launch_irfft_mdot32(c, spec, it, done), "irfft_mdot32");
+        VV_PLAUNCH(P_IRFFT_MDOT32, S + F * (it + 2), it,
+                   blocks ? launch_row_inv32(c, spec, it, done) : launch_irfft_mdot32(c, spec, it, done),
+                   "irfft_mdot32");
         VV_PLAUNCH(P_MAXPY32, F * (it + 3), it, launch_maxpy_norm32(c, it, rows), "maxpy_norm32");
         return VV_OK;
     }
@@ -693,8 +764,7 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
         int r = VV_OK;
         hipError_t le = hipSuccess;
         do {
-            if ((le = launch_residual(c, f, fh, c->X)) != hipSuccess) break;
-            if ((r = precond(c, c->X, c->rhs, nullptr))) break;
+            if ((r = pc_residual(c, f, fh, c->rhs))) break;
             if ((le = launch_zero(c, c->D, c->N * c->B)) != hipSuccess) break;
             if ((le = launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it)) != hipSuccess) break;
             if ((r = cycle_start_from(c, c->rhs))) break;
@@ -737,9 +807,7 @@ int snes_impl(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp, v
         if (int r = no_diss(c, "graph replay")) return r;
         if (int r = snes_graph(c, f, fh, kp)) return r;
     } else {
-        VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, c->X), "residual");
-        if (int r = diss_function(c, f, fh, c->X)) return r;
-        if (int r = precond(c, c->X, c->rhs, nullptr)) return r;
+        if (int r = pc_residual(c, f, fh, c->rhs)) return r;
         VV_CHECK(launch_zero(c, c->D, c->N * c->B), "zero x");
         VV_CHECK(launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it), "gmres init");
         if (int r = cycle_start_from(c, c->rhs)) return r;
@@ -929,6 +997,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     c->nmodes = c->fft_n / 2 + 1;
     c->logn = 0;
     while ((1 << c->logn) < c->fft_n) ++c->logn;
+    if ((c->fft_n & (c->fft_n - 1)) != 0 && c->fft_n <= kRowsNx) c->dft = make_dft_plan(c->fft_n);
     c->coef_stride = pot ? nx : 0;
     c->cf_lo = pot ? 1.0 : 0.5;     // PotentialFast.pyx:250-252 / KineticFast.pyx:258-260
     c->cf_mid = pot ? 2.0 : 1.0;
@@ -966,6 +1035,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     const int nfb = fft_blocks(c), ncb = cgs_blocks_max(c->N);
     int nrows = (nfb > kReduceBlocks ? nfb : kReduceBlocks);
     if (ncb > nrows) nrows = ncb;
+    if ((c->fft_rows + 1) / 2 > nrows) nrows = (c->fft_rows + 1) / 2;   // row blocks of two rows
     c->part_stride = (int64_t)nrows * (kMaxRestart + 2);
     const size_t Bz = (size_t)B;
     VV_CCHECK(dalloc(c, &c->inst, Bz), "alloc instance constants");
@@ -1378,18 +1448,14 @@ int vv_function(vv_ctx *c, const double *f, const double *fh, double *y)
 {
     if (int r = check_ctx(c)) return r;
     if (!f || !fh || !y) return fail(c, VV_ERR_INVALID, "null field");
-    VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, c->X), "residual");
-    if (int r = diss_function(c, f, fh, c->X)) return r;
-    return precond(c, c->X, y, nullptr);
+    return pc_residual(c, f, fh, y);
 }
 
 int vv_jacobian(vv_ctx *c, const double *u, double *y)
 {
     if (int r = check_ctx(c)) return r;
     if (!u || !y) return fail(c, VV_ERR_INVALID, "null field");
-    VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian(c, u, nullptr, c->X), "jacobian");
-    if (int r = diss_jacobian(c, u, nullptr, c->X, nullptr)) return r;
-    return precond(c, c->X, y, nullptr);
+    return pc_jacobian(c, u, y);
 }
 
 int vv_function_norm(vv_ctx *c, const double *f, const double *fh, double *y, double *out)

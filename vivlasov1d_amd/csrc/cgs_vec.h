@@ -66,13 +66,20 @@ struct CgsArgs {
     int nbd;           // maxpy: rows of dot partials (the mdot grid)
 };
 
+// Vectors per group: 16 loads in flight a lane with 8 or 4 vectors of 16 bytes
+// a thread, 8 vectors at once below (a small grid's step is a chain of memory
+// latencies: by pairs, k/2 of them at Arnoldi step k).
+template <int EPT> constexpr int cgs_group() { return EPT >= 8 ? 2 : EPT == 4 ? 4 : 8; }
+
+// G vectors from v0 on, of which the first `have` exist (the others are zero)
 template <int EPT, int G, typename S>
-__device__ __forceinline__ void load_group(const S *basis, int64_t vstride, int v0, int64_t e0, int64_t nvv,
-                                           typename V16<S>::type (&x)[G][EPT])
+__device__ __forceinline__ void load_group(const S *basis, int64_t vstride, int v0, int have, int64_t e0,
+                                           int64_t nvv, typename V16<S>::type (&x)[G][EPT])
 {
     using V = typename V16<S>::type;
 #pragma unroll
     for (int gg = 0; gg < G; ++gg) {
+        if (gg >= have) break;             // uniform over the launch
         const V *Vp = reinterpret_cast<const V *>(basis + (size_t)(v0 + gg) * vstride);
 #pragma unroll
         for (int q = 0; q < EPT; ++q) {

@@ -108,12 +108,23 @@ hipError_t launch_narrow_add(vv_ctx *c, float *y, const double *d)
     return hipGetLastError();
 }
 
+// The collision operator with its factors, - factor * coll_freq * coll_drag *
+// hv_inv * 0.5 and - factor * coll_freq * coll_diff * hv2_inv, left to right
+// (CollisionOperator.pyx:80-81); false: it adds nothing (:87).
+bool collision_term(vv_ctx *c, const double *n, const double *U, const double *a, double factor, CollTerm *t)
+{
+    const double nu = c->coll_freq;
+    if (nu == 0. || factor == 0. || c->p.nv <= 4) return false;
+    *t = CollTerm{n, U, a, -factor * nu * c->coll_drag * c->hv_inv * 0.5, -factor * nu * c->coll_diff * c->hv2_inv,
+                  c->diss_kind == VV_DISSIPATION_COLLE ? 1 : 0};
+    return true;
+}
+
 hipError_t launch_collision(vv_ctx *c, const double *f, const double *fscale, double *y, const double *n,
                             const double *U, const double *a, double factor, const int32_t *done)
 {
-    const double nu = c->coll_freq;
-    if (nu == 0. || factor == 0.) return hipSuccess;       // CollisionOperator.pyx:87
-    if (c->p.nv <= 4) return hipSuccess;
+    CollTerm ct;
+    if (!collision_term(c, n, U, a, factor, &ct)) return hipSuccess;
     CollArgs p{};
     p.f = f;
     p.fscale = fscale;
@@ -124,10 +135,8 @@ hipError_t launch_collision(vv_ctx *c, const double *f, const double *fscale, do
     p.a = a;
     p.nx = c->p.nx;
     p.nv = c->p.nv;
-    // - factor * coll_freq * coll_drag * hv_inv * 0.5 and
-    // - factor * coll_freq * coll_diff * hv2_inv, left to right (:80-81)
-    p.drag_fac = -factor * nu * c->coll_drag * c->hv_inv * 0.5;
-    p.diff_fac = -factor * nu * c->coll_diff * c->hv2_inv;
+    p.drag_fac = ct.drag_fac;
+    p.diff_fac = ct.diff_fac;
     p.done = done;
     dim3 grid((p.nx + NT - 1) / NT, p.nv - 4), block(NT);
     if (c->diss_kind == VV_DISSIPATION_COLLE) launch_timed(c, collision_kernel<true>, grid, block, 0, p);

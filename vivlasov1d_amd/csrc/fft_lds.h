@@ -74,55 +74,26 @@ __device__ __forceinline__ C twiddle(const C *__restrict__ tw, int m)
     return INV ? cmk<C>(t.x, -t.y) : t;
 }
 
-constexpr int MAXS = 6;     // radix-4 stages of the longest transform (MAXE = 4^6)
-
-// Twiddles of one thread's butterflies, loaded once before a transform of
-// length n <= 4 NT.  There every butterfly the thread owns, in any transform
-// of the block and any stage, has the index j = threadIdx.x mod n/4 (mod n/2
-// in the radix-2 stage of odd logn, where n <= 2 NT), so 3 twiddles per stage
-// cover them; their loads are in flight with the tile's own loads instead of
-// being waited on after every barrier of the transform.
-// n = 1024 runs the plan 4 x 8 x 8 x 4 (see lds_fft1024): its 17 twiddles
-// take the same registers, flat index i (always a compile-time index) at
-// w[i / 3][i % 3] for i < 15, then w2 and w8 (0..6 and 7..13 for the radix-8
-// stages with sub-transforms of 4 and 32, 14..16 for the last radix-4 stage;
-// the last row of w, used only by n = 4096, stays out of it).
+// Twiddles of the n = 1024 plan 4 x 8 x 8 x 4 (see lds_fft1024), loaded once by
+// each thread before the transform: every butterfly it owns, in any transform
+// of the block and any stage, has the index j = threadIdx.x mod n/4 (n/8), so
+// 17 of them cover it; their loads are in flight with the tile's own instead of
+// being waited on after every barrier.  w: 0..6 and 7..13 for the radix-8 stages
+// with sub-transforms of 4 and 32, 14..16 for the last radix-4 stage.
 constexpr int N8 = 1024;
 template <bool INV, typename C>
 struct FftTw {
-    C w[MAXS][3];
-    C w2, w8;
-    // P8: the n = 1024 plan's twiddles (n must be 1024), else the radix-4 ones
-    template <bool P8 = false>
-    __device__ __forceinline__ void load(const C *__restrict__ tw, int n, int logn)
+    C w[17];
+    __device__ __forceinline__ void load(const C *__restrict__ tw)
     {
-        if (P8) {
-            const int t = threadIdx.x, ka = t & 3, kb = t & 31, kc = t & 255;
+        const int t = threadIdx.x, ka = t & 3, kb = t & 31, kc = t & 255;
 #pragma unroll
-            for (int r = 1; r < 8; ++r) {
-                w[(r - 1) / 3][(r - 1) % 3] = twiddle<INV>(tw, r * ka * 32);
-                w[(6 + r) / 3][(6 + r) % 3] = twiddle<INV>(tw, r * kb * 4);
-            }
-            w[4][2] = twiddle<INV>(tw, kc);
-            w2 = twiddle<INV>(tw, 2 * kc);
-            w8 = twiddle<INV>(tw, 3 * kc);
-            return;
+        for (int r = 1; r < 8; ++r) {
+            w[r - 1] = twiddle<INV>(tw, r * ka * 32);
+            w[6 + r] = twiddle<INV>(tw, r * kb * 4);
         }
-        const int ns = logn >> 1;
-        const int j = threadIdx.x & ((n >> 2) - 1);
 #pragma unroll
-        for (int s = 0; s < MAXS; ++s) {
-            if (s < ns) {
-                const int st = (j & ((1 << (2 * s)) - 1)) << (logn - 2 - 2 * s);
-                w[s][0] = twiddle<INV>(tw, st);
-                w[s][1] = twiddle<INV>(tw, 2 * st);
-                w[s][2] = twiddle<INV>(tw, 3 * st);
-            }
-        }
-        if (logn & 1) {
-            const int jj = threadIdx.x & ((n >> 1) - 1);
-            w2 = twiddle<INV>(tw, (jj & ((1 << (2 * ns)) - 1)) << (logn - 1 - 2 * ns));
-        }
+        for (int r = 1; r < 4; ++r) w[13 + r] = twiddle<INV>(tw, r * kc);
     }
 };
 
@@ -194,7 +165,7 @@ __device__ __forceinline__ void stage8_1024(C *buf, int nb, const FftTw<INV, C> 
 #pragma unroll
             for (int r = 0; r < 8; ++r) v[q][r] = src[j + r * nq];
 #pragma unroll
-            for (int r = 1; r < 8; ++r) v[q][r] = cmul(v[q][r], pt.w[(OFF + r - 1) / 3][(OFF + r - 1) % 3]);
+            for (int r = 1; r < 8; ++r) v[q][r] = cmul(v[q][r], pt.w[OFF + r - 1]);
             dft8<INV>(v[q]);
             dst[q] = b * N8 + ((j - k) << 3) + k;
         }
@@ -257,9 +228,9 @@ __device__ __forceinline__ void lds_fft1024(C *buf, int nb, const FftTw<INV, C> 
             const C *src = buf + b * N8;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[q][r] = src[j + r * nq];
-            v[q][1] = cmul(v[q][1], pt.w[4][2]);
-            v[q][2] = cmul(v[q][2], pt.w2);
-            v[q][3] = cmul(v[q][3], pt.w8);
+            v[q][1] = cmul(v[q][1], pt.w[14]);
+            v[q][2] = cmul(v[q][2], pt.w[15]);
+            v[q][3] = cmul(v[q][3], pt.w[16]);
             dft4<INV>(v[q][0], v[q][1], v[q][2], v[q][3]);
             dst[q] = b * N8 + j;
         }
@@ -274,115 +245,95 @@ __device__ __forceinline__ void lds_fft1024(C *buf, int nb, const FftTw<INV, C> 
     __syncthreads();
 }
 
-// Batched in-LDS Stockham FFT of `nb` transforms of length n = 2^logn stored
-// back to back in buf.  Forward uses exp(-2 pi i m/n), inverse the conjugate
-// (unnormalised).  Each stage loads every butterfly of the thread into
-// registers, synchronises, then stores, so one buffer suffices.  C is
-// double2 (FP64 path) or float2 (FP32 preconditioner of the mixed solver).
-// PRE: twiddles from pt (n <= 4 NT), else from the global table tw.  P8:
-// n = 1024 by the 4 x 8 x 8 x 4 plan (pt loaded with load<true>).
-// s0: first radix-4 stage to run (1 when the caller did stage 0 in
-// registers); the last stage's outputs go to `last`.
-// Inlined so that buf is known to be LDS (ds_read/ds_write, not flat
-// accesses); index arithmetic by shifts (n is a power of two).
-template <bool INV, bool PRE, bool P8 = false, typename C, typename Sink>
-__device__ __forceinline__ void lds_fft(C *buf, int n, int logn, int nb, const C *__restrict__ tw,
-                                        const FftTw<INV, C> &pt, int s0, const Sink &last)
+// One Stockham stage of radix RAD (4 or 8) on nb transforms of length 2^logn:
+// sub-transforms of length Ns = 2^l combined; butterfly j of a transform takes
+// elements j + r n/RAD, twiddled by W_n^(r k n/(RAD Ns)), k = j mod Ns, and
+// stores output m at RAD (j - k) + k + m Ns.  Every butterfly of the thread (Q
+// at most) is loaded before the barrier and stored after it, so one buffer
+// suffices; the final stage's outputs go to `last`.
+template <int RAD, bool INV, int Q, typename C, typename Sink>
+__device__ __forceinline__ void fft_stage(C *buf, int logn, int nb, int l, const C *tw, bool fin, const Sink &last)
 {
-    if (P8) {                              // n = 1024, twiddles loaded for the plan
-        lds_fft1024<INV>(buf, nb, pt, s0, last);
-        return;
+    constexpr int LR = RAD == 8 ? 3 : 2;
+    const int lq = logn - LR, nq = 1 << lq, Ns = 1 << l, sh = lq - l, total = nb << lq;
+    C v[Q][RAD];
+    int dst[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int bq = threadIdx.x + q * NT;
+        dst[q] = -1;
+        if (bq < total) {
+            const int b = bq >> lq, j = bq & (nq - 1), k = j & (Ns - 1);
+            const C *src = buf + (b << logn) + j;
+#pragma unroll
+            for (int r = 0; r < RAD; ++r) v[q][r] = src[r << lq];
+            if (l > 0) {
+#pragma unroll
+                for (int r = 1; r < RAD; ++r) v[q][r] = cmul(v[q][r], twiddle<INV>(tw, (r * k) << sh));
+            }
+            if constexpr (RAD == 8) dft8<INV>(v[q]);
+            else dft4<INV>(v[q][0], v[q][1], v[q][2], v[q][3]);
+            dst[q] = (b << logn) + ((j - k) << LR) + k;
+        }
     }
-    const int nq = n >> 2, lq = logn - 2, ns = logn >> 1;
-    const int total4 = nb * nq;
+    __syncthreads();
 #pragma unroll
-    for (int s = 0; s < MAXS; ++s) {
-        if (s >= ns) break;                // uniform over the block
-        if (s < s0) continue;
-        const int Ns = 1 << (2 * s);
-        C v[MAXE / 4 / NT][4];
-        int dst[MAXE / 4 / NT];
+    for (int q = 0; q < Q; ++q) {
+        if (dst[q] >= 0) {
 #pragma unroll
-        for (int q = 0; q < MAXE / 4 / NT; ++q) {
-            const int t = threadIdx.x + q * NT;
-            dst[q] = -1;
-            if (t < total4) {
-                const int b = t >> lq;
-                const int j = t & (nq - 1);
-                const int k = j & (Ns - 1);
-                const C *src = buf + (b << logn);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[q][r] = src[j + r * nq];
-                if (PRE) {
-                    v[q][1] = cmul(v[q][1], pt.w[s][0]);
-                    v[q][2] = cmul(v[q][2], pt.w[s][1]);
-                    v[q][3] = cmul(v[q][3], pt.w[s][2]);
-                } else {
-                    const int st = k << (lq - 2 * s);
-                    v[q][1] = cmul(v[q][1], twiddle<INV>(tw, st));
-                    v[q][2] = cmul(v[q][2], twiddle<INV>(tw, 2 * st));
-                    v[q][3] = cmul(v[q][3], twiddle<INV>(tw, 3 * st));
-                }
-                const C a0 = cadd(v[q][0], v[q][2]);
-                const C a1 = csub(v[q][0], v[q][2]);
-                const C a2 = cadd(v[q][1], v[q][3]);
-                const C d = csub(v[q][1], v[q][3]);
-                // forward: (v1 - v3) * (-i); inverse: (v1 - v3) * (+i)
-                const C a3 = INV ? cmk<C>(-d.y, d.x) : cmk<C>(d.y, -d.x);
-                v[q][0] = cadd(a0, a2);
-                v[q][1] = cadd(a1, a3);
-                v[q][2] = csub(a0, a2);
-                v[q][3] = csub(a1, a3);
-                dst[q] = (b << logn) + ((j - k) << 2) + k;
+            for (int m = 0; m < RAD; ++m) {
+                if (fin) last(dst[q] + (m << l), v[q][m]);
+                else buf[dst[q] + (m << l)] = v[q][m];
             }
         }
-        __syncthreads();
-        const bool fin = (s == ns - 1) && !(logn & 1);
-#pragma unroll
-        for (int q = 0; q < MAXE / 4 / NT; ++q) {
-            if (dst[q] >= 0) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (fin) last(dst[q] + r * Ns, v[q][r]);
-                    else buf[dst[q] + r * Ns] = v[q][r];
-                }
-            }
-        }
-        __syncthreads();
     }
-    if (logn & 1) {
-        const int Ns = 1 << (2 * ns);
-        const int nh = n >> 1;
-        const int total = nb * nh;
-        C v[MAXE / 2 / NT][2];
-        int dst[MAXE / 2 / NT];
-#pragma unroll
-        for (int q = 0; q < MAXE / 2 / NT; ++q) {
-            const int t = threadIdx.x + q * NT;
-            dst[q] = -1;
-            if (t < total) {
-                const int b = t >> (logn - 1);
-                const int j = t & (nh - 1);
-                const int k = j & (Ns - 1);
-                const C *src = buf + (b << logn);
-                const C x0 = src[j];
-                const C w = PRE ? pt.w2 : twiddle<INV>(tw, k << (logn - 1 - 2 * ns));
-                const C x1 = cmul(src[j + nh], w);
-                v[q][0] = cadd(x0, x1);
-                v[q][1] = csub(x0, x1);
-                dst[q] = (b << logn) + ((j - k) << 1) + k;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < MAXE / 2 / NT; ++q) {
-            if (dst[q] >= 0) {
-                last(dst[q], v[q][0]);
-                last(dst[q] + Ns, v[q][1]);
-            }
-        }
-        __syncthreads();
+    __syncthreads();
+}
+
+// radix-4 stages a transform of length 2^logn begins with (the rest are of
+// radix 8): 64 = 8 x 8, 128 = 4 x 4 x 8, 256 = 4 x 8 x 8, 512 = 8 x 8 x 8,
+// 2048 = 4 x 8 x 8 x 8, 4096 = 8 x 8 x 8 x 8
+__host__ __device__ __forceinline__ int fft_lead4(int logn)
+{
+    const int b = logn % 3;
+    return b == 0 ? 0 : b == 1 ? 2 : 1;
+}
+// log2 of the first stage's radix (which kernels may run in registers)
+__host__ __device__ __forceinline__ int fft_first(int logn) { return fft_lead4(logn) ? 2 : 3; }
+
+// Batched in-LDS Stockham FFT of `nb` transforms of length n = 2^logn stored
+// back to back in buf, at most EB * 1024 elements.  Forward uses
+// exp(-2 pi i m/n), inverse the conjugate (unnormalised).  C is double2 (FP64
+// path) or float2 (FP32 preconditioner of the mixed solver).  tw: the table of
+// exp(-2 pi i m/n), a copy in LDS for the short lengths.  P8: n = 1024 by the
+// 4 x 8 x 8 x 4 plan (pt loaded).  l0: log2 of the sub-transforms already done
+// (the caller ran the first stage in registers); the last stage's outputs go
+// to `last`.  The stages are a loop, not unrolled: the code of a transform
+// stays a few KB (unrolled by stage and butterfly it was 25-40 KB, and a small
+// grid's kernels, each on a few CUs for a few microseconds, fetched it all).
+// Inlined so that buf is known to be LDS (ds_read/ds_write, not flat accesses).
+template <bool INV, bool P8, int EB, typename C, typename Sink>
+__device__ __forceinline__ void lds_fft(C *buf, int logn, int nb, const C *tw, const FftTw<INV, C> &pt, int l0,
+                                        const Sink &last)
+{
+    if constexpr (P8) {                    // n = 1024, twiddles loaded for the plan
+        lds_fft1024<INV>(buf, nb, pt, l0 ? 1 : 0, last);
+    } else {
+        const int l4 = 2 * fft_lead4(logn);
+        int l = l0;
+        for (; l < l4; l += 2) fft_stage<4, INV, EB, C>(buf, logn, nb, l, tw, l + 2 == logn, last);
+        for (; l < logn; l += 3) fft_stage<8, INV, (EB + 1) / 2, C>(buf, logn, nb, l, tw, l + 3 == logn, last);
     }
+}
+
+// the twiddle table (or, TWL, its copy in LDS at stw, written by the block;
+// read only after a barrier)
+template <bool TWL, typename C>
+__device__ __forceinline__ const C *tw_table(const C *__restrict__ tw, C *stw, int n)
+{
+    if constexpr (!TWL) return tw;
+    for (int m = threadIdx.x; m < n; m += NT) stw[m] = tw[m];
+    return stw;
 }
 
 // Instance b of a batched context is blockIdx.y: real fields at b * N,
@@ -421,6 +372,23 @@ __device__ __forceinline__ void store_real_spectrum(const C *buf, int nx, int R,
         else out = cmk<C>((zk.y + zm.y) * half, (zm.x - zk.x) * half);
         spec[(size_t)k * nv + j0 + r] = out;
     }
+}
+
+// what J u of a row block needs besides u
+struct JacRows {
+    const double *uscale;                       // optional device scale of u (GMRES state)
+    const double *h0, *h1p, *h1h, *h2p, *h2h;   // 1D factors of H_ave
+    const InstConst *inst;
+    double ht_inv, factor;
+};
+
+// H_ave from its factors in the tile's type: FP64 as is, FP32 relative to
+// href (formed in FP64, rounded once), as the bracket kernel stages it
+template <typename T>
+__device__ __forceinline__ T have_rel(double h0, const double (&x)[4], double href)
+{
+    if constexpr (sizeof(T) == 8) return compose_have(h0, x[0], x[1], x[2], x[3]);
+    else return (T)(compose_have(h0, x[0], x[1], x[2], x[3]) - href);
 }
 
 }  // namespace

@@ -11,7 +11,8 @@
 // Bandwidth layout of the CGS kernels (mdot, maxpy + norm, solution update):
 // one thread owns EPT double2 elements (coalesced, NT apart) of every vector;
 // vectors are streamed in groups of two whose 2*EPT loads are issued back to
-// back, so each wavefront keeps 16 x 16 B in flight per lane.  The grid
+// back, so each wavefront keeps 16 x 16 B in flight per lane (in groups of
+// eight with 1 or 2 elements).  The grid
 // covers N exactly once (no grid-stride loop), EPT in {1,2,4,8} chosen so the
 // launch has >= 256 workgroups.
 //
@@ -199,27 +200,19 @@ __global__ __launch_bounds__(NT) void mdot_kernel(CgsArgs<S> a, int col)
         w[q] = (e < nvv) ? W[e] : V{};
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int v = 0;
-    for (; v + 2 <= nvec; v += 2) {
-        V x[2][EPT];
-        load_group<EPT, 2, S>(a.basis, a.vstride, v, e0, nvv, x);
+    constexpr int G = cgs_group<EPT>();
+    for (int v = 0; v < nvec; v += G) {
+        V x[G][EPT];
+        load_group<EPT, G, S>(a.basis, a.vstride, v, nvec - v, e0, nvv, x);
 #pragma unroll
-        for (int gg = 0; gg < 2; ++gg) {
+        for (int gg = 0; gg < G; ++gg) {
+            if (v + gg >= nvec) break;
             const double sv = s_scale[v + gg];
             double acc = dot_slice<EPT, S>(w, x[gg], sv);
             if (TAIL && et >= 0) acc = __builtin_fma(wt, (double)a.basis[(size_t)(v + gg) * a.vstride + et] * sv, acc);
             acc = wave_sum(acc);
             if (lane == 0) red[wave][v + gg] = acc;
         }
-    }
-    if (v < nvec) {
-        V x[1][EPT];
-        load_group<EPT, 1, S>(a.basis, a.vstride, v, e0, nvv, x);
-        const double sv = s_scale[v];
-        double acc = dot_slice<EPT, S>(w, x[0], sv);
-        if (TAIL && et >= 0) acc = __builtin_fma(wt, (double)a.basis[(size_t)v * a.vstride + et] * sv, acc);
-        acc = wave_sum(acc);
-        if (lane == 0) red[wave][v] = acc;
     }
     __syncthreads();
     if (threadIdx.x < PV) {
@@ -277,12 +270,13 @@ __global__ __launch_bounds__(NT) void maxpy_norm_kernel(CgsArgs<S> a, int it)
 #pragma unroll
         for (int l = 0; l < L; ++l) w[q][l] = vget(wl[q], l);
     }
-    int j = 0;
-    for (; j + 2 <= nvec; j += 2) {
-        V x[2][EPT];
-        load_group<EPT, 2, S>(a.basis, a.vstride, j, e0, nvv, x);
+    constexpr int G = cgs_group<EPT>();
+    for (int j = 0; j < nvec; j += G) {
+        V x[G][EPT];
+        load_group<EPT, G, S>(a.basis, a.vstride, j, nvec - j, e0, nvv, x);
 #pragma unroll
-        for (int gg = 0; gg < 2; ++gg) {
+        for (int gg = 0; gg < G; ++gg) {
+            if (j + gg >= nvec) break;
             const double sj = s_scale[j + gg], cj = s_coef[j + gg];
 #pragma unroll
             for (int q = 0; q < EPT; ++q) {
@@ -291,17 +285,6 @@ __global__ __launch_bounds__(NT) void maxpy_norm_kernel(CgsArgs<S> a, int it)
             }
             if (TAIL && et >= 0) wt = wt + cj * ((double)a.basis[(size_t)(j + gg) * a.vstride + et] * sj);
         }
-    }
-    if (j < nvec) {
-        V x[1][EPT];
-        load_group<EPT, 1, S>(a.basis, a.vstride, j, e0, nvv, x);
-        const double sj = s_scale[j], cj = s_coef[j];
-#pragma unroll
-        for (int q = 0; q < EPT; ++q) {
-#pragma unroll
-            for (int l = 0; l < L; ++l) w[q][l] = w[q][l] + cj * (vget(x[0][q], l) * sj);
-        }
-        if (TAIL && et >= 0) wt = wt + cj * ((double)a.basis[(size_t)j * a.vstride + et] * sj);
     }
     double acc = 0.0;
     if (TAIL && et >= 0) {
@@ -396,12 +379,13 @@ __global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, CgsA
     for (int q = 0; q < EPT; ++q)
 #pragma unroll
         for (int l = 0; l < L; ++l) t[q][l] = 0.0;
-    int j = 0;
-    for (; j + 2 <= n; j += 2) {
-        V v[2][EPT];
-        load_group<EPT, 2, S>(a.basis, a.vstride, j, e0, nvv, v);
+    constexpr int G = cgs_group<EPT>();
+    for (int j = 0; j < n; j += G) {
+        V v[G][EPT];
+        load_group<EPT, G, S>(a.basis, a.vstride, j, n - j, e0, nvv, v);
 #pragma unroll
-        for (int gg = 0; gg < 2; ++gg) {
+        for (int gg = 0; gg < G; ++gg) {
+            if (j + gg >= n) break;
             const double sj = s_scale[j + gg], cj = s_coef[j + gg];
 #pragma unroll
             for (int q = 0; q < EPT; ++q) {
@@ -410,17 +394,6 @@ __global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, CgsA
             }
             if (TAIL && et >= 0) tt = tt + cj * ((double)a.basis[(size_t)(j + gg) * a.vstride + et] * sj);
         }
-    }
-    if (j < n) {
-        V v[1][EPT];
-        load_group<EPT, 1, S>(a.basis, a.vstride, j, e0, nvv, v);
-        const double sj = s_scale[j], cj = s_coef[j];
-#pragma unroll
-        for (int q = 0; q < EPT; ++q) {
-#pragma unroll
-            for (int l = 0; l < L; ++l) t[q][l] = t[q][l] + cj * (vget(v[0][q], l) * sj);
-        }
-        if (TAIL && et >= 0) tt = tt + cj * ((double)a.basis[(size_t)j * a.vstride + et] * sj);
     }
     if (TAIL && et >= 0) x[et] = x[et] + tt;
     double2 *X = reinterpret_cast<double2 *>(x);

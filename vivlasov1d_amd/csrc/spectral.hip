@@ -34,9 +34,16 @@
 namespace vv {
 namespace {
 
-// PRE (nx <= 4 NT): the thread's twiddles are loaded with its tile; P8:
-// nx = 1024 by the radix-8 plan.
-template <typename T, bool PRE, bool P8>
+// Transform variants of the kernels below: VP8 nx = 1024 by the radix-8 plan
+// with preloaded twiddles; VTWL shorter powers of two, twiddles copied to LDS;
+// VLONG longer ones, twiddles from the table.
+enum { VTWL = 0, VP8 = 1, VLONG = 2 };
+
+// LF: log2 of the first stage's radix (fft_first), which runs in registers:
+// butterfly (p, j) of complex row p (real rows 2p, 2p+1) takes z_p[j + m nx/2^LF],
+// exactly the elements the thread loads (coalesced along j); its twiddles are
+// 1.  Every global load of the thread is issued before anything waits.
+template <typename T, int V, int LF>
 __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restrict__ x, cx_t<T> *__restrict__ spec)
 {
     using C = cx_t<T>;
@@ -50,48 +57,44 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
     // XCD-aware row-block order: the mode-major segments of neighbouring row
     // blocks share L2 lines, so they are kept on one XCD
     const int j0 = xcd_tile(blockIdx.x, gridDim.x) * R;
-    // Stage 0 of the FFT runs in registers: butterfly (p, j) of complex row p
-    // (real rows 2p, 2p+1) takes z_p[j + m nx/4], m = 0..3, exactly the
-    // elements the thread loads (coalesced along j); its twiddles are 1.
-    // Every global load of the thread is issued before anything waits.
-    constexpr int QB = MAXE / 4 / NT;    // butterflies per thread
-    const int nq = nx >> 2, lq = a.logn - 2;
-    const int total4 = (R >> 1) * nq;
-    T xr[QB][4], xi[QB][4];
+    constexpr int RAD = 1 << LF, QB = MAXE / RAD / NT;    // butterflies per thread
+    const int lq = a.logn - LF, nq = 1 << lq;
+    const int total = (R >> 1) * nq;
+    T xr[QB][RAD], xi[QB][RAD];
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
         const int bq = threadIdx.x + q * NT;
         const int p = bq >> lq, j = bq & (nq - 1);
-        const bool ok = bq < total4;
+        const bool ok = bq < total;
         const bool r0 = ok && j0 + 2 * p < a.nv, r1 = ok && j0 + 2 * p + 1 < a.nv;
         const T *x0 = x + (size_t)(j0 + 2 * p) * nx + j;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
+        for (int m = 0; m < RAD; ++m) {
             xr[q][m] = r0 ? x0[m * nq] : T(0);
             xi[q][m] = r1 ? x0[nx + m * nq] : T(0);
         }
     }
     FftTw<false, C> pt;
-    if (PRE) pt.template load<P8>(a.tw, nx, a.logn);
+    if (V == VP8) pt.load(a.tw);
+    const C *tw = tw_table<V == VTWL>(a.tw, buf + (size_t)(R >> 1) * nx, nx);
     if (dflag) return;                 // uniform over the block, before any barrier
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
         const int bq = threadIdx.x + q * NT;
-        if (bq < total4) {
+        if (bq < total) {
             const int p = bq >> lq, j = bq & (nq - 1);
-            const C v0 = cmk<C>(xr[q][0], xi[q][0]), v1 = cmk<C>(xr[q][1], xi[q][1]);
-            const C v2 = cmk<C>(xr[q][2], xi[q][2]), v3 = cmk<C>(xr[q][3], xi[q][3]);
-            const C a0 = cadd(v0, v2), a1 = csub(v0, v2), a2 = cadd(v1, v3), d = csub(v1, v3);
-            const C a3 = cmk<C>(d.y, -d.x);             // (v1 - v3) * (-i)
-            C *z = buf + (p << a.logn) + (j << 2);      // stage 0 outputs: 4j + r
-            z[0] = cadd(a0, a2);
-            z[1] = cadd(a1, a3);
-            z[2] = csub(a0, a2);
-            z[3] = csub(a1, a3);
+            C v[RAD];
+#pragma unroll
+            for (int m = 0; m < RAD; ++m) v[m] = cmk<C>(xr[q][m], xi[q][m]);
+            if constexpr (LF == 3) dft8<false>(v);
+            else dft4<false>(v[0], v[1], v[2], v[3]);
+            C *z = buf + (p << a.logn) + (j << LF);     // first stage's outputs: RAD j + m
+#pragma unroll
+            for (int m = 0; m < RAD; ++m) z[m] = v[m];
         }
     }
     __syncthreads();
-    lds_fft<false, PRE, P8>(buf, nx, a.logn, R >> 1, a.tw, pt, 1, LdsSink<C>{buf});
+    lds_fft<false, V == VP8, 4>(buf, a.logn, R >> 1, tw, pt, LF, LdsSink<C>{buf});
     store_real_spectrum(buf, nx, R, j0, a.nv, spec);
 }
 
@@ -112,13 +115,6 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
 // arithmetic, bit for bit).  nx = NT, 2 NT: the rows go to the FFT buffer and
 // the transform starts from LDS (its unit twiddles can change only the sign
 // of an exact zero).  R in 2, 4, 8.
-struct JacRows {
-    const double *uscale;                       // optional device scale of u (GMRES state)
-    const double *h0, *h1p, *h1h, *h2p, *h2h;   // 1D factors of H_ave
-    const InstConst *inst;
-    double ht_inv, factor;
-};
-
 template <int R, typename T>
 struct JacStrip {
     T u[R + 4];          // own column, rows j0-2 .. j0+R+1 (0 outside the grid)
@@ -156,15 +152,6 @@ __device__ __forceinline__ void jac_strip_load(const T *__restrict__ u, const Ja
         g.ex[2] = jr.h2p[xo + gi];
         g.ex[3] = jr.h2h[xo + gi];
     }
-}
-
-// H_ave from its factors in the tile's type: FP64 as is, FP32 relative to
-// href (formed in FP64, rounded once), as the bracket kernel stages it
-template <typename T>
-__device__ __forceinline__ T have_rel(double h0, const double (&x)[4], double href)
-{
-    if constexpr (sizeof(T) == 8) return compose_have(h0, x[0], x[1], x[2], x[3]);
-    else return (T)(compose_have(h0, x[0], x[1], x[2], x[3]) - href);
 }
 
 // Thread t's column of the staged strip down the R output rows (tile rows
@@ -221,6 +208,9 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
     T *sH = sF + RH * SP;
     const int nv = a.nv, t = threadIdx.x;
     const int j0 = xcd_tile((int)blockIdx.x - extra, (int)gridDim.x - extra) * R;
+    // nx = NT, 2 NT: the twiddles' copy lies behind the strips and the FFT buffer
+    constexpr size_t kStrip = 2 * (size_t)RH * SP * sizeof(T), kLines = (size_t)(R >> 1) * nx * sizeof(C);
+    const C *tw = tw_table<NS != 4>(a.tw, reinterpret_cast<C *>(lds_raw + (kStrip > kLines ? kStrip : kLines)), nx);
     __shared__ double red[kGdNW + 1];
     const double nshare = extra ? norm_share(hs.part + b * hs.pstride, hs.nb) : 0.0;
     // FP32: H_ave - href, href = h0 at the centre row of the bracket kernel's
@@ -266,7 +256,7 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
     }
     // twiddles in flight during the first stage (not held through the walks)
     FftTw<false, C> pt;
-    pt.template load<NS == 4>(a.tw, nx, a.logn);
+    if (NS == 4) pt.load(a.tw);
     if (NS == 4) {
         // stage 0 of the transform in registers, as rfft_kernel: butterfly
         // (p, t) of complex row p (real rows 2p, 2p+1) takes columns t + m NT
@@ -290,7 +280,7 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
             for (int p = 0; p < (R >> 1); ++p) buf[p * nx + s * NT + t] = cmk<C>(res[s][2 * p], res[s][2 * p + 1]);
     }
     __syncthreads();
-    lds_fft<false, true, NS == 4>(buf, nx, a.logn, R >> 1, a.tw, pt, NS == 4 ? 1 : 0, LdsSink<C>{buf});
+    lds_fft<false, NS == 4, 4>(buf, a.logn, R >> 1, tw, pt, NS == 4 ? 2 : 0, LdsSink<C>{buf});
     store_real_spectrum(buf, nx, R, j0, nv, spec);
 }
 
@@ -320,7 +310,7 @@ struct IrfftSink {
     }
 };
 
-template <typename T, bool PRE, bool P8>
+template <typename T, int V>
 __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *__restrict__ spec, T *__restrict__ y)
 {
     using C = cx_t<T>;
@@ -347,7 +337,8 @@ __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *
         vb[q] = load_or_zero(spec, (int64_t)k * a.nv + ja + 1, idx < total && ja + 1 < a.nv);
     }
     FftTw<true, C> pt;
-    if (PRE) pt.template load<P8>(a.tw, nx, a.logn);
+    if (V == VP8) pt.load(a.tw);
+    const C *tw = tw_table<V == VTWL>(a.tw, buf + (size_t)npair * nx, nx);
     if (dflag) return;                 // uniform over the block, before any barrier
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -367,7 +358,7 @@ __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *
     }
     __syncthreads();
     // the last stage's outputs (natural order) go straight to the output rows
-    lds_fft<true, PRE, P8>(buf, nx, a.logn, npair, a.tw, pt, 0, IrfftSink<T>{y, j0, nx, a.logn, a.nv});
+    lds_fft<true, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, IrfftSink<T>{y, j0, nx, a.logn, a.nv});
 }
 
 // Real rows of the irFFT left in the workgroup's LDS buffer itself, natural
@@ -419,7 +410,8 @@ __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t
     const int npair = R >> 1;
     const int nvec = col + 1;
     const int total = (nh + 1) * npair;
-    constexpr int PER = (MAXE / 2 + 64 + NT - 1) / NT;
+    // the slice's points; mode pairs (nx/2 + 1) R/2 <= PTS/4 + PTS/16 (nx >= 8)
+    constexpr int PTS = NT * EPT * V16<T>::L, PER = (5 * PTS / 16 + NT - 1) / NT;
     C va[PER], vb[PER];
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -431,21 +423,15 @@ __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t
     }
     const double sc = (int)threadIdx.x < nvec ? gs->scale[threadIdx.x] : 0.0;
     FftTw<true, C> pt;
-    pt.template load<P8>(a.tw, nx, a.logn);
+    if (P8) pt.load(a.tw);
+    const C *tw = tw_table<!P8>(a.tw, buf + (size_t)npair * nx, nx);
     if (dflag) return;                 // uniform over the block, before any barrier
-    // the first pair of basis vectors is in flight while the FFT stages run
+    // the first group of basis vectors is in flight while the FFT stages run
     const int64_t nvv = g.N / V16<T>::L;
     const int64_t e0 = (int64_t)slice * NT * EPT + threadIdx.x;
-    V x[2][EPT];
-#pragma unroll
-    for (int gg = 0; gg < 2; ++gg) {
-        const V *Vp = reinterpret_cast<const V *>(basis + (size_t)gg * g.vstride);
-#pragma unroll
-        for (int q = 0; q < EPT; ++q) {
-            const int64_t e = e0 + (int64_t)q * NT;
-            x[gg][q] = (gg < nvec && e < nvv) ? Vp[e] : V{};
-        }
-    }
+    constexpr int G = cgs_group<EPT>();
+    V x[G][EPT];
+    load_group<EPT, G, T>(basis, g.vstride, 0, nvec, e0, nvv, x);
     if ((int)threadIdx.x < PV) s_scale[threadIdx.x] = sc;
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -465,7 +451,7 @@ __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t
     }
     __syncthreads();
     T *wr = reinterpret_cast<T *>(buf);
-    lds_fft<true, true, P8>(buf, nx, a.logn, npair, a.tw, pt, 0, RealRowsSink<T>{wr, nx, a.logn});
+    lds_fft<true, P8, (PTS / 2 + 1023) / 1024>(buf, a.logn, npair, tw, pt, 0, RealRowsSink<T>{wr, nx, a.logn});
 
     // w of the slice: to the basis, and into registers for the dots
     const V *wl = reinterpret_cast<const V *>(wr);
@@ -477,27 +463,15 @@ __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t
         W[e0 + (int64_t)q * NT] = w[q];
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int v = 0;
-    for (; v + 2 <= nvec; v += 2) {
-        if (v > 0) load_group<EPT, 2, T>(basis, g.vstride, v, e0, nvv, x);
+    for (int v = 0; v < nvec; v += G) {
+        if (v > 0) load_group<EPT, G, T>(basis, g.vstride, v, nvec - v, e0, nvv, x);
 #pragma unroll
-        for (int gg = 0; gg < 2; ++gg) {
+        for (int gg = 0; gg < G; ++gg) {
+            if (v + gg >= nvec) break;
             double acc = dot_slice<EPT, T>(w, x[gg], s_scale[v + gg]);
             acc = wave_sum(acc);
             if (lane == 0) red[wave][v + gg] = acc;
         }
-    }
-    if (v < nvec) {
-        V y[1][EPT];
-        if (v > 0) {
-            load_group<EPT, 1, T>(basis, g.vstride, v, e0, nvv, y);
-        } else {
-#pragma unroll
-            for (int q = 0; q < EPT; ++q) y[0][q] = x[0][q];
-        }
-        double acc = dot_slice<EPT, T>(w, y[0], s_scale[v]);
-        acc = wave_sum(acc);
-        if (lane == 0) red[wave][v] = acc;
     }
     __syncthreads();
     if (threadIdx.x < PV) {
@@ -1056,6 +1030,19 @@ FftArgs<T> dft_args(vv_ctx *c, const cx_t<T> *tw, const int32_t *done, bool *twl
     return FftArgs<T>{n, 0, c->fft_rows, R, c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
 }
 
+// LDS of an FFT kernel: the packed rows, and the twiddles' copy below 1024
+template <typename T>
+size_t fft_lds(const FftArgs<T> &a)
+{
+    return ((size_t)(a.rows >> 1) * a.nx + (a.nx < N8 ? a.nx : 0)) * sizeof(cx_t<T>);
+}
+
+// the row-block transforms of lengths with a plan
+hipError_t row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done) { return launch_row_rfft(c, x, spec, done); }
+hipError_t row_rfft(vv_ctx *c, const float *x, float2 *spec, const int32_t *done) { return launch_row_rfft32(c, x, spec, done); }
+hipError_t row_irfft(vv_ctx *c, const double2 *spec, double *y, const int32_t *done) { return launch_row_irfft(c, spec, y, done); }
+hipError_t row_irfft(vv_ctx *c, const float2 *spec, float *y, const int32_t *done) { return launch_row_irfft32(c, spec, y, done); }
+
 template <typename T>
 hipError_t rdft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done)
 {
@@ -1083,15 +1070,19 @@ hipError_t irdft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, cons
 template <typename T>
 hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done)
 {
+    if (c->dft.n) return row_rfft(c, x, spec, done);
     if (c->fft_n & (c->fft_n - 1)) return rdft_t<T>(c, tw, x, spec, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
                  (int64_t)sizeof(GmresState), tw, done};
     const int nb = (a.nv + a.rows - 1) / a.rows;
-    const size_t lds = (size_t)(a.rows >> 1) * a.nx * sizeof(cx_t<T>);
-    if (a.nx == N8) launch_timed(c, rfft_kernel<T, true, true>, dim3(nb, c->B), dim3(NT), (uint32_t)lds, a, x, spec);
-    else if (a.nx <= 4 * NT)
-        launch_timed(c, rfft_kernel<T, true, false>, dim3(nb, c->B), dim3(NT), (uint32_t)lds, a, x, spec);
-    else launch_timed(c, rfft_kernel<T, false, false>, dim3(nb, c->B), dim3(NT), (uint32_t)lds, a, x, spec);
+    const uint32_t lds = (uint32_t)fft_lds<T>(a);
+    const dim3 grid(nb, c->B), block(NT);
+    const bool first8 = fft_first(a.logn) == 3;
+    if (a.nx == N8) launch_timed(c, rfft_kernel<T, VP8, 2>, grid, block, lds, a, x, spec);
+    else if (a.nx < N8 && first8) launch_timed(c, rfft_kernel<T, VTWL, 3>, grid, block, lds, a, x, spec);
+    else if (a.nx < N8) launch_timed(c, rfft_kernel<T, VTWL, 2>, grid, block, lds, a, x, spec);
+    else if (first8) launch_timed(c, rfft_kernel<T, VLONG, 3>, grid, block, lds, a, x, spec);
+    else launch_timed(c, rfft_kernel<T, VLONG, 2>, grid, block, lds, a, x, spec);
     return hipGetLastError();
 }
 
@@ -1102,8 +1093,9 @@ void jac_rfft_launch(vv_ctx *c, const FftArgs<T> &a, const JacRows &jr, const T 
     const size_t strip = 2 * (size_t)(R + 4) * (NT + 4) * sizeof(T);
     const HessArgs hs = take_update(c);
     const dim3 grid((a.nv + R - 1) / R + (hs.nb > 0 ? 1 : 0), c->B);
-    launch_timed(c, jac_rfft_kernel<KIND, R, NS, T>, grid, dim3(NT), (uint32_t)(fft > strip ? fft : strip), a, jr, hs,
-                 u, spec);
+    const size_t tws = NS != 4 ? a.nx * sizeof(cx_t<T>) : 0;
+    launch_timed(c, jac_rfft_kernel<KIND, R, NS, T>, grid, dim3(NT), (uint32_t)((fft > strip ? fft : strip) + tws), a,
+                 jr, hs, u, spec);
 }
 
 template <int KIND, int R, typename T>
@@ -1143,15 +1135,17 @@ hipError_t jac_rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *u, const double *us
 template <typename T>
 hipError_t irfft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, const int32_t *done)
 {
+    // the row blocks store pairs: a y that is not aligned for them takes the direct DFT
+    if (c->dft.n && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0) return row_irfft(c, spec, y, done);
     if (c->fft_n & (c->fft_n - 1)) return irdft_t<T>(c, tw, spec, y, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
                  (int64_t)sizeof(GmresState), tw, done};
     const int nb = (a.nv + a.rows - 1) / a.rows;
-    const size_t lds = (size_t)(a.rows >> 1) * a.nx * sizeof(cx_t<T>);
-    if (a.nx == N8) launch_timed(c, irfft_kernel<T, true, true>, dim3(nb, c->B), dim3(NT), (uint32_t)lds, a, spec, y);
-    else if (a.nx <= 4 * NT)
-        launch_timed(c, irfft_kernel<T, true, false>, dim3(nb, c->B), dim3(NT), (uint32_t)lds, a, spec, y);
-    else launch_timed(c, irfft_kernel<T, false, false>, dim3(nb, c->B), dim3(NT), (uint32_t)lds, a, spec, y);
+    const uint32_t lds = (uint32_t)fft_lds<T>(a);
+    const dim3 grid(nb, c->B), block(NT);
+    if (a.nx == N8) launch_timed(c, irfft_kernel<T, VP8>, grid, block, lds, a, spec, y);
+    else if (a.nx < N8) launch_timed(c, irfft_kernel<T, VTWL>, grid, block, lds, a, spec, y);
+    else launch_timed(c, irfft_kernel<T, VLONG>, grid, block, lds, a, spec, y);
     return hipGetLastError();
 }
 
@@ -1194,7 +1188,7 @@ hipError_t irfft_mdot_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, const
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
                  (int64_t)sizeof(GmresState), tw, done};
     const int nb = a.nv / a.rows;
-    const size_t lds = (size_t)(a.rows >> 1) * a.nx * sizeof(cx_t<T>);
+    const size_t lds = fft_lds<T>(a);
     const CgsArgs<T> g{basis, c->N, c->vs, c->partial, c->part_stride, c->gs, 0, nb};
     const dim3 grid(nb, c->B);
     switch (ept) {
@@ -1276,6 +1270,8 @@ int lu_rows(int nv)
 }
 
 int lu_pivots_per_mode(int nv) { return NT * lu_rows(nv); }
+
+int fft_rows_of(const vv_ctx *c) { return fft_rows(c); }
 
 int fft_blocks(vv_ctx *c)
 {

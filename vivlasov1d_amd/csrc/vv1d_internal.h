@@ -71,6 +71,25 @@ struct HessArgs {
     uint32_t seq;
 };
 
+// Plan of the mixed-radix line transform (rows.hip): stage s has radix r[s]
+// after sub-transforms of length ns[s]; nr = n / r, step = n / (ns r); mn, mnr,
+// mns: reciprocals of n, nr, ns for division by multiplication.
+constexpr int kDftStages = 11;
+struct DftPlan {
+    int n, stages;
+    int r[kDftStages], ns[kDftStages], nr[kDftStages], step[kDftStages];
+    uint32_t mn, mnr[kDftStages], mns[kDftStages];
+};
+
+// The collision operator a Jacobian-vector product adds (dissipation.hip).
+struct CollTerm {
+    const double *n, *U, *a;   // x-vectors
+    double drag_fac, diff_fac;
+    int e;                     // collE
+};
+
+constexpr int kRowsNx = 2048;   // longest x of the row-block kernels (rows.hip)
+
 }  // namespace vv
 
 struct vv_ctx {
@@ -91,6 +110,7 @@ struct vv_ctx {
     int nmodes;         // fft_n/2 + 1
     int logn;           // log2(fft_n) when fft_n is a power of two (FFT kernels); else a direct DFT
     int fft_n, fft_rows;
+    vv::DftPlan dft;    // fft_n no power of two and <= kRowsNx: the line transform's plan (else n = 0)
     int64_t coef_stride;        // instance stride of gm/g0/gp (0: shared)
     double cf_lo, cf_mid, cf_hi;  // band constants: kinetic 0.5/1.0/0.5, potential 1.0/2.0/1.0
     double *tb;                 // potential: the transposed field (B N doubles)
@@ -214,8 +234,27 @@ hipError_t launch_rk18_stage4(vv_ctx *c, const double *x, const double *t1, cons
                               double s, double *out);
 hipError_t launch_rk4_end(vv_ctx *c, bool three_eighths, double *x, const double *t1, const double *t2,
                           const double *t3, const double *t4, double s);
+bool collision_term(vv_ctx *c, const double *n, const double *U, const double *a, double factor, CollTerm *t);
+// rows.hip: row blocks of the kinetic form for any nx <= kRowsNx (rows_apply);
+// J u (with the previous step's Hessenberg update, and the collision term when
+// given) or F(f) formed and transformed in one launch, and the irFFT into
+// basis[col+1] with its CGS dots in row_inv_blocks partial rows
+DftPlan make_dft_plan(int n);
+bool rows_apply(const vv_ctx *c);
+int row_inv_blocks(const vv_ctx *c);
+hipError_t launch_row_jac(vv_ctx *c, const double *u, const double *uscale, const CollTerm *coll, double2 *spec,
+                          const int32_t *done);
+hipError_t launch_row_jac32(vv_ctx *c, const float *u, const double *uscale, float2 *spec, const int32_t *done);
+hipError_t launch_row_res(vv_ctx *c, const double *f, const double *fh, double2 *spec);
+hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done);
+hipError_t launch_row_rfft32(vv_ctx *c, const float *x, float2 *spec, const int32_t *done);
+hipError_t launch_row_irfft(vv_ctx *c, const double2 *spec, double *y, const int32_t *done);
+hipError_t launch_row_irfft32(vv_ctx *c, const float2 *spec, float *y, const int32_t *done);
+hipError_t launch_row_inv(vv_ctx *c, const double2 *spec, int col, const int32_t *done);
+hipError_t launch_row_inv32(vv_ctx *c, const float2 *spec, int col, const int32_t *done);
 // spectral.hip
 int fft_blocks(vv_ctx *c);
+int fft_rows_of(const vv_ctx *c);
 hipError_t launch_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done);
 // J u (u times its optional device scale) and its rFFT in one launch, the
 // Jacobian never stored; jac_rfft_rows: the rows per workgroup where the
