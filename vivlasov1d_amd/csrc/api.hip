@@ -28,12 +28,11 @@ const char *kProfNames[P_NKINDS] = {"jacobian",   "residual", "rfft",      "trid
                                     "irfft32",    "mdot32",   "maxpy_norm32", "irfft_mdot", "irfft_mdot32",
                                     "jac_rfft",   "jac_rfft32"};
 
-// device scalar regions (doubles): per-instance norms | Poisson residuals
-// (16 apart) | invariants (6 per instance)
-inline double *ds_norms(vv_ctx *c) { return c->dscalar; }
-inline double *ds_pres(vv_ctx *c) { return c->dscalar + c->B; }
-inline double *ds_inv(vv_ctx *c) { return c->dscalar + 17 * (size_t)c->B; }
-inline size_t ds_count(int B) { return 24 * (size_t)B + 16; }
+// device scalars: the Poisson residuals of the last moments, 16 doubles apart;
+// host scalars: up to 6 per instance
+inline double *ds_pres(vv_ctx *c) { return c->dscalar; }
+inline size_t ds_count(int B) { return 16 * (size_t)B; }
+inline size_t hs_count(int B) { return 16 * (size_t)B + 16; }
 
 struct ProfRec {
     int kind;
@@ -132,27 +131,11 @@ hipError_t dalloc(vv_ctx *c, T **p, size_t count)
     return e;
 }
 
-// count doubles from device memory into the mapped pinned staging buffer
-__global__ void scalars_to_host_kernel(const double *__restrict__ src, double *dst, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
-}
-
-// the statuses of the B instances into a mapped pinned slot, one lane per
-// instance (per-field stores)
-__global__ void status_to_host_kernel(const GmresState *__restrict__ g, GmresStatus *dst, int B)
+// the instances' Poisson residuals into mapped pinned memory
+__global__ void pres_to_host_kernel(const double *__restrict__ src, double *dst, int B)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const GmresStatus st = g[b].st;
-    dst[b].it = st.it;
-    dst[b].its = st.its;
-    dst[b].reason = st.reason;
-    dst[b].done = st.done;
-    dst[b].active = st.active;
-    dst[b].res = st.res;
-    dst[b].rnorm0 = st.rnorm0;
+    if (b < B) dst[b] = src[16 * (size_t)b];
 }
 
 // the instance mask from its mapped pinned staging into device memory
@@ -176,15 +159,11 @@ __global__ void factors_copy_kernel(FactorCopy a)
         if (i < a.n[q]) a.dst[q][i] = a.src[q][i];
 }
 
-// count doubles from device to host: a small kernel writes them into the
-// mapped pinned buffer (no copy-engine dispatch and its host-side set-up),
-// then the stream is drained
-int read_scalars(vv_ctx *c, const double *dev, size_t count, double *out)
+// count doubles of the mapped pinned buffer, into which the kernels that form
+// scalars for the host write them (no copy, no launch for it), once the stream
+// is drained
+int read_host(vv_ctx *c, size_t count, double *out)
 {
-    const int n = (int)count;
-    hipLaunchKernelGGL(scalars_to_host_kernel, dim3((n + 255) / 256), dim3(256), 0, c->stream, dev,
-                       c->host_scalars_dev, n);
-    VV_CHECK(hipGetLastError(), "copy scalars");
     VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
     for (size_t q = 0; q < count; ++q) out[q] = c->host_scalars[q];
     return VV_OK;
@@ -433,6 +412,38 @@ int pc_residual(vv_ctx *c, const double *f, const double *fh, double *y)
     return VV_OK;
 }
 
+// V_0 = P^-1 F(f) and its norm partials, a solve's start: the irFFT writes V_0
+// where a fused form applies, else it is copied from rhs
+int residual_start(vv_ctx *c, const double *f, const double *fh)
+{
+    const int slices = c->p.precond != VV_PRECOND_NONE ? irfft_mdot_rows(c, false) : 0;
+    const bool blocks = !slices && rows_apply(c) && !jac_rfft_rows(c);
+    if (!slices && !blocks) {
+        if (int r = pc_residual(c, f, fh, c->rhs)) return r;
+        VV_CHECK(launch_start(c, c->rhs, true), "cycle start");
+        return VV_OK;
+    }
+    const double F = b_field(c), S = b_spec(c);
+    if (!rows_apply(c) || diss_on(c)) {
+        VV_PLAUNCH(P_RES, 3 * F, -1, launch_residual(c, f, fh, c->X), "residual");
+        if (int r = diss_function(c, f, fh, c->X)) return r;
+        VV_PLAUNCH(P_RFFT, F + S, -1, launch_rfft(c, c->X, c->spec, nullptr), "rfft");
+    } else {
+        VV_PLAUNCH(P_RES, 2 * F + S, -1, launch_row_res(c, f, fh, c->spec), "row F(f)");
+    }
+    VV_PLAUNCH(P_TRI, 2 * S, -1, launch_tridiag_k(c, c->spec, nullptr), "tridiag");
+    VV_PLAUNCH(P_IRFFT, S + F, -1, slices ? launch_irfft_start(c, c->spec) : launch_row_inv_start(c, c->spec), "irfft");
+    c->pend_it = -1;
+    c->pend_nb = slices ? slices : row_inv_blocks(c);
+    c->pend_start = 2;
+    return VV_OK;
+}
+
+void set_start(vv_ctx *c, double rtol, double atol, double dtol, int max_it)
+{
+    c->start = SolveStart{c->active, rtol, atol, dtol, max_it, c->p.restart};
+}
+
 // y = P^-1 J u
 int pc_jacobian(vv_ctx *c, const double *u, double *y)
 {
@@ -610,16 +621,6 @@ int max_it_of(const GmresStatus *s, int B)
     return m;
 }
 
-// the device statuses into host memory by a kernel writing the mapped pinned
-// buffer (no copy-engine dispatch)
-int copy_status(vv_ctx *c)
-{
-    hipLaunchKernelGGL(status_to_host_kernel, dim3((c->B + 255) / 256), dim3(256), 0, c->stream, c->gs,
-                       c->host_status_dev, c->B);
-    VV_CHECK(hipGetLastError(), "status copy");
-    return VV_OK;
-}
-
 // Waits for the B reports of slot `slot` numbered seq (a kernel enqueued before
 // stores them); *done: every instance's cycle has ended.  The stream is looked
 // at now and then, so an error on the device ends the wait.
@@ -652,16 +653,16 @@ int wait_report(vv_ctx *c, int slot, uint32_t seq, bool *done)
 // has not ended the cycle and the queue never drains: one step, whose later
 // kernels return at once, is enqueued in vain (an event after every second
 // step left two to three).  Returns once the cycle has finished on the device
-// for every instance, with the statuses in host memory.  build: x += V y is
-// enqueued before the final drain (FP64 x, from the FP32 basis when fp32); update: then
-// f -= x for instances whose solve converged (SNESSolve_KSPONLY's step), so
-// one drain ends the solve.
-int run_cycle(vv_ctx *c, bool fp32, double *build = nullptr, double *update = nullptr)
+// for every instance, with the statuses in host memory.  The solution is
+// enqueued before the final drain: x = V y (store, a solve's first cycle) or x
+// += V y (FP64 x, from the FP32 basis when fp32); update (one instance): f -=
+// V y instead where the solve converged (SNESSolve_KSPONLY's step), so one
+// drain ends the solve.
+int run_cycle(vv_ctx *c, bool fp32, double *x, bool store, double *update = nullptr)
 {
     const int max_k = c->p.restart;
     const size_t prof_from = c->prof ? prof_of(c)->recs.size() : 0;
     bool stop = false;
-    c->pend_it = -1;
     for (int it = 0; it < max_k; ++it) {
         if (it >= 2) {
             if (int r = wait_report(c, it & 1, c->report_seq, &stop)) return r;
@@ -677,22 +678,10 @@ int run_cycle(vv_ctx *c, bool fp32, double *build = nullptr, double *update = nu
     }
     if (stop) c->pend_it = -1;         // the last step ran past every instance's end
     else VV_CHECK(launch_update(c), "Hessenberg update");
-    if (build) {
-        if (fp32) VV_CHECK(launch_build_solution32(c, build), "build solution");
-        else VV_CHECK(launch_build_solution(c, build), "build solution");
-        if (update) VV_CHECK(launch_axpy_cond(c, -1.0, build, update), "update");
-    }
-    if (int r = copy_status(c)) return r;
+    VV_CHECK(fp32 ? launch_build_solution32(c, x, update, store, c->host_status_dev)
+                  : launch_build_solution(c, x, update, store, c->host_status_dev), "build solution");
     VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
     prof_mark_idle(c, prof_from, max_it_of(c->host_status, c->B));
-    return VV_OK;
-}
-
-// V_0 = b (per instance) and the cycle start
-int cycle_start_from(vv_ctx *c, const double *b)
-{
-    VV_CHECK(launch_copy(c, b, c->basis, c->N * c->B), "copy b");
-    VV_CHECK(launch_norm_start(c), "cycle start");
     return VV_OK;
 }
 
@@ -711,14 +700,17 @@ void fill_results(vv_ctx *c, vv_ksp_result *res)
 // Cycles after the first: while some instance still iterates, restart from
 // r = b - (P^-1 J) x (KSPInitialResidual) and run another cycle.  Instances
 // that finished stay done (their cycle start keeps done set).
+bool more_cycles(vv_ctx *c)
+{
+    const GmresStatus *st = c->host_status;
+    for (int q = 0; q < c->B; ++q)
+        if (st[q].active && st[q].reason == 0) return true;
+    return false;
+}
+
 int restart_cycles(vv_ctx *c, const double *b, double *x)
 {
-    for (;;) {
-        const GmresStatus *st = c->host_status;
-        bool more = false;
-        for (int q = 0; q < c->B; ++q)
-            if (st[q].active && st[q].reason == 0) more = true;
-        if (!more) return VV_OK;
+    while (more_cycles(c)) {
         if (c->op_mode != 0) {
             if (int r = linear_apply(c, x, nullptr, c->op_fbar, c->X, c->ht_inv, -0.5, 0.5, true)) return r;
         } else {
@@ -726,26 +718,25 @@ int restart_cycles(vv_ctx *c, const double *b, double *x)
             if (int r = diss_jacobian(c, x, nullptr, c->X, nullptr)) return r;
         }
         if (int r = apply_pc(c, c->X, c->basis, nullptr)) return r;
-        VV_CHECK(launch_residual_restart(c, b, c->basis), "restart residual");
-        VV_CHECK(launch_norm_start(c), "cycle start");
-        if (int r = run_cycle(c, false, x)) return r;
+        VV_CHECK(launch_restart(c, b), "restart residual");
+        if (int r = run_cycle(c, false, x, false)) return r;
     }
+    return VV_OK;
 }
 
 int ksp_solve_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_params *kp, vv_ksp_result *res)
 {
-    VV_CHECK(launch_zero(c, x, c->N * c->B), "zero x");
-    VV_CHECK(launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it), "gmres init");
-    if (int r = cycle_start_from(c, b)) return r;
-    if (int r = run_cycle(c, false, x)) return r;
+    set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
+    VV_CHECK(launch_start(c, b, true), "cycle start");
+    if (int r = run_cycle(c, false, x, true)) return r;
     if (int r = restart_cycles(c, b, x)) return r;
     fill_results(c, res);
     return VV_OK;
 }
 
 // The first GMRES cycle of SNESSolve_KSPONLY as one captured graph:
-// b = P^-1 F(f); x = 0; GMRES init; V_0 = b; cycle start; `restart` Arnoldi
-// steps (steps past an instance's convergence return at once); x += V y.
+// V_0 = P^-1 F(f); cycle start; `restart` Arnoldi steps (steps past an
+// instance's convergence return at once); x = V y and the statuses.
 // The graph is kept per (f, fh) pair and replayed while they stay the same;
 // the KSP tolerances are kernel arguments, so a change re-captures too.
 int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
@@ -764,15 +755,12 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
         int r = VV_OK;
         hipError_t le = hipSuccess;
         do {
-            if ((r = pc_residual(c, f, fh, c->rhs))) break;
-            if ((le = launch_zero(c, c->D, c->N * c->B)) != hipSuccess) break;
-            if ((le = launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it)) != hipSuccess) break;
-            if ((r = cycle_start_from(c, c->rhs))) break;
-            c->pend_it = -1;
+            set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
+            if ((r = residual_start(c, f, fh))) break;
             for (int it = 0; it < c->p.restart && r == VV_OK; ++it) r = arnoldi_step(c, it);
             if (r) break;
             if ((le = launch_update(c)) != hipSuccess) break;
-            le = launch_build_solution(c, c->D);
+            le = launch_build_solution(c, c->D, nullptr, true, c->host_status_dev);
         } while (0);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(c->stream, &g);
@@ -796,7 +784,6 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
         c->graph_kp[3] = (double)kp->max_it;
     }
     VV_CHECK(hipGraphLaunch(c->graph_exec, c->stream), "graph launch");
-    if (int r = copy_status(c)) return r;
     VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
     return VV_OK;
 }
@@ -807,19 +794,20 @@ int snes_impl(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp, v
         if (int r = no_diss(c, "graph replay")) return r;
         if (int r = snes_graph(c, f, fh, kp)) return r;
     } else {
-        if (int r = pc_residual(c, f, fh, c->rhs)) return r;
-        VV_CHECK(launch_zero(c, c->D, c->N * c->B), "zero x");
-        VV_CHECK(launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it), "gmres init");
-        if (int r = cycle_start_from(c, c->rhs)) return r;
-        // one instance: the step f -= D is enqueued with the solution before
-        // the drain (a no-op unless the cycle converged; a restart leaves it
-        // to the update below)
-        if (int r = run_cycle(c, false, c->D, c->B == 1 ? f : nullptr)) return r;
+        set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
+        if (int r = residual_start(c, f, fh)) return r;
+        // one instance: the step is enqueued with the solution before the drain
+        // (a cycle that ends without a reason leaves it to the update below)
+        if (int r = run_cycle(c, false, c->D, true, c->B == 1 ? f : nullptr)) return r;
         if (c->B == 1 && c->host_status[0].reason != 0) {
             fill_results(c, res);
             return VV_OK;
         }
     }
+    // the right-hand side of the restarts, formed again (the first cycle's V_0
+    // was it, and f is still as it was)
+    if (more_cycles(c))
+        if (int r = pc_residual(c, f, fh, c->rhs)) return r;
     if (int r = restart_cycles(c, c->rhs, c->D)) return r;
     // SNESSolve_KSPONLY takes the step unless the linear solve diverged
     VV_CHECK(launch_axpy_cond(c, -1.0, c->D, f), "update");
@@ -846,21 +834,32 @@ int ensure_mixed(vv_ctx *c)
 // r = b - P^-1 J x, solution x and stopping test are FP64.  The stopping test
 // is the reference's (||r|| <= max(rtol ||b||, atol)) applied to the true
 // FP64 preconditioned residual; every cycle restarts from that residual.
+// update: the solution is taken off this field where the solve converged (x
+// need not be formed then).
 int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_params *kp, const vv_mixed_params *mp,
-                         vv_ksp_result *res, int32_t *cycles)
+                         vv_ksp_result *res, int32_t *cycles, double *update = nullptr)
 {
     if (c->B != 1) return fail(c, VV_ERR_UNSUPPORTED, "the mixed-precision solve takes one instance");
     if (int r = ensure_mixed(c)) return r;
     const int64_t N = c->N;
-    VV_CHECK(launch_zero(c, x, N), "zero x");
     double rnorm0 = 0.0, rnorm = 0.0;
     const double *rsrc = b;
     int its = 0, rounds = 0, reason = 0;
+    // r = b - P^-1 J x into c->R and its norm
+    auto true_residual = [&]() -> int {
+        VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian(c, x, nullptr, c->X), "jacobian");
+        if (int r = diss_jacobian(c, x, nullptr, c->X, nullptr)) return r;
+        if (int r = precond(c, c->X, c->R, nullptr)) return r;
+        VV_CHECK(launch_rsub(c, b, c->R), "residual");
+        VV_CHECK(launch_norm2(c, c->R, N, c->host_scalars_dev), "norm");
+        rsrc = c->R;
+        return read_host(c, 1, &rnorm);
+    };
     if (!mp->fp64_check) {
         // one FP32 cycle with the KSP's own tolerances; its reason stands
-        VV_CHECK(launch_gmres_init(c, kp->rtol, kp->atol, kp->dtol, kp->max_it), "gmres init");
-        VV_CHECK(launch_start32(c, b), "cycle start");
-        if (int r = run_cycle(c, true, x)) return r;
+        set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
+        VV_CHECK(launch_start32(c, b, true), "cycle start");
+        if (int r = run_cycle(c, true, x, true, update)) return r;
         const GmresStatus st = c->host_status[0];
         if (st.reason != 0) {
             fill_results(c, res);
@@ -871,16 +870,10 @@ int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_par
         its = st.it;
         rounds = 1;
         rnorm0 = st.rnorm0;
-        VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian(c, x, nullptr, c->X), "jacobian");
-        if (int r = diss_jacobian(c, x, nullptr, c->X, nullptr)) return r;
-        if (int r = precond(c, c->X, c->R, nullptr)) return r;
-        VV_CHECK(launch_residual_restart(c, b, c->R), "residual");
-        VV_CHECK(launch_norm2(c, c->R, N, ds_norms(c)), "norm");
-        if (int r = read_scalars(c, ds_norms(c), 1, &rnorm)) return r;
-        rsrc = c->R;
+        if (int r = true_residual()) return r;
     } else {
-        VV_CHECK(launch_norm2(c, b, N, ds_norms(c)), "norm");
-        if (int r = read_scalars(c, ds_norms(c), 1, &rnorm0)) return r;
+        VV_CHECK(launch_norm2(c, b, N, c->host_scalars_dev), "norm");
+        if (int r = read_host(c, 1, &rnorm0)) return r;
         rnorm = rnorm0;
     }
     const double ttol = std::fmax(kp->rtol * rnorm0, kp->atol);
@@ -905,20 +898,15 @@ int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_par
         // reduction of inner_rtol, or less when less already meets the target
         double rt = 0.5 * ttol / rnorm;
         if (rt < mp->inner_rtol) rt = mp->inner_rtol;
-        VV_CHECK(launch_gmres_init(c, rt, 0.0, 1.0e300, kp->max_it - its), "gmres init");
-        VV_CHECK(launch_start32(c, rsrc), "cycle start");
-        if (int r = run_cycle(c, true, x)) return r;
+        set_start(c, rt, 0.0, 1.0e300, kp->max_it - its);
+        VV_CHECK(launch_start32(c, rsrc, true), "cycle start");
+        if (int r = run_cycle(c, true, x, rounds == 0)) return r;
         its += c->host_status[0].it;
         ++rounds;
-        // true FP64 residual r = b - P^-1 J x
-        VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian(c, x, nullptr, c->X), "jacobian");
-        if (int r = diss_jacobian(c, x, nullptr, c->X, nullptr)) return r;
-        if (int r = precond(c, c->X, c->R, nullptr)) return r;
-        VV_CHECK(launch_residual_restart(c, b, c->R), "residual");
-        VV_CHECK(launch_norm2(c, c->R, N, ds_norms(c)), "norm");
-        if (int r = read_scalars(c, ds_norms(c), 1, &rnorm)) return r;
-        rsrc = c->R;
+        if (int r = true_residual()) return r;
     }
+    if (rounds == 0) VV_CHECK(launch_zero(c, x, N), "zero x");
+    if (update && reason > 0) VV_CHECK(launch_axpy(c, -1.0, x, update, N), "update");
     if (res) {
         res->its = its;
         res->reason = reason;
@@ -1035,6 +1023,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     const int nfb = fft_blocks(c), ncb = cgs_blocks_max(c->N);
     int nrows = (nfb > kReduceBlocks ? nfb : kReduceBlocks);
     if (ncb > nrows) nrows = ncb;
+    if (br_tiles(nx, nv) > nrows) nrows = br_tiles(nx, nv);             // the residual's norm partials
     if ((c->fft_rows + 1) / 2 > nrows) nrows = (c->fft_rows + 1) / 2;   // row blocks of two rows
     c->part_stride = (int64_t)nrows * (kMaxRestart + 2);
     const size_t Bz = (size_t)B;
@@ -1077,7 +1066,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_poll), 2 * Bz * sizeof(uint32_t)), "pinned reports");
     VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_poll_dev), c->host_poll, 0),
               "pinned reports device address");
-    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_scalars), ds_count(B) * sizeof(double)),
+    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_scalars), hs_count(B) * sizeof(double)),
               "pinned scalars");
     VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_scalars_dev), c->host_scalars, 0),
               "pinned scalars device address");
@@ -1458,15 +1447,26 @@ int vv_jacobian(vv_ctx *c, const double *u, double *y)
     return pc_jacobian(c, u, y);
 }
 
+namespace {
+// y = F(f), its norms (and the Poisson residuals pres) on their way to the host
+// scalars; without a dissipation term the residual kernel sums its own squares
+int residual_and_norms(vv_ctx *c, const double *f, const double *fh, double *y, const double *pres)
+{
+    const bool own = !diss_on(c);
+    VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, y, own ? c->partial : nullptr), "residual");
+    if (int r = diss_function(c, f, fh, y)) return r;
+    VV_CHECK(launch_norms(c, own ? nullptr : y, residual_blocks(c), pres, c->host_scalars_dev), "norm");
+    return VV_OK;
+}
+}  // namespace
+
 int vv_function_norm(vv_ctx *c, const double *f, const double *fh, double *y, double *out)
 {
     if (int r = check_ctx(c)) return r;
     if (!f || !fh || !y || !out) return fail(c, VV_ERR_INVALID, "null argument");
     if (y == f || y == fh) return fail(c, VV_ERR_INVALID, "function_norm: y must not alias f or fh");
-    VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, y), "residual");
-    if (int r = diss_function(c, f, fh, y)) return r;
-    VV_CHECK(launch_norms(c, y, ds_norms(c)), "norm");
-    return read_scalars(c, ds_norms(c), (size_t)c->B, out);
+    if (int r = residual_and_norms(c, f, fh, y, nullptr)) return r;
+    return read_host(c, (size_t)c->B, out);
 }
 
 int vv_batched_timestep(vv_ctx *c, const vv_batch_fields *s, const vv_ksp_params *kp, double snes_atol,
@@ -1554,16 +1554,12 @@ int vv_residual_norms(vv_ctx *c, const double *f, const double *fh, double *y, d
     if (int r = check_ctx(c)) return r;
     if (!f || !fh || !y || !fnorm || !pnorm) return fail(c, VV_ERR_INVALID, "null argument");
     if (y == f || y == fh) return fail(c, VV_ERR_INVALID, "residual_norms: y must not alias f or fh");
-    VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, y), "residual");
-    if (int r = diss_function(c, f, fh, y)) return r;
-    VV_CHECK(launch_norms(c, y, ds_norms(c)), "norm");
-    // ds_norms (B values) is followed by the Poisson residuals ds_pres (stride 16)
+    if (int r = residual_and_norms(c, f, fh, y, ds_pres(c))) return r;
     const size_t B = (size_t)c->B;
-    std::vector<double> tmp(B + 16 * B);
-    if (int r = read_scalars(c, ds_norms(c), B + 16 * (B - 1) + 1, tmp.data())) return r;
+    VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
     for (size_t b = 0; b < B; ++b) {
-        fnorm[b] = tmp[b];
-        pnorm[b] = tmp[B + 16 * b];
+        fnorm[b] = c->host_scalars[b];
+        pnorm[b] = c->host_scalars[B + b];
     }
     return VV_OK;
 }
@@ -1788,10 +1784,10 @@ int vv_moments(vv_ctx *c, const double *f, double *n, double *phi, double *h1, d
     VV_CHECK(launch_density_partial(c, f, nullptr), "density");
     VV_CHECK(launch_poisson(c, nullptr, n, phi, h1, ds_pres(c), 1), "poisson");
     if (!pnorm) return VV_OK;
-    std::vector<double> tmp(16 * (size_t)c->B);
-    if (int r = read_scalars(c, ds_pres(c), 16 * (size_t)(c->B - 1) + 1, tmp.data())) return r;
-    for (int b = 0; b < c->B; ++b) pnorm[b] = tmp[16 * (size_t)b];
-    return VV_OK;
+    hipLaunchKernelGGL(pres_to_host_kernel, dim3((c->B + 255) / 256), dim3(256), 0, c->stream, ds_pres(c),
+                       c->host_scalars_dev, c->B);
+    VV_CHECK(hipGetLastError(), "copy scalars");
+    return read_host(c, (size_t)c->B, pnorm);
 }
 
 int vv_moments_noalloc(vv_ctx *c, const double *f, double *n, double *phi, double *h1, double *pnorm)
@@ -1815,16 +1811,16 @@ int vv_norm2(vv_ctx *c, const double *x, int64_t len, double *out)
 {
     if (int r = check_ctx(c)) return r;
     if (!x || !out || len < 0) return fail(c, VV_ERR_INVALID, "bad argument");
-    VV_CHECK(launch_norm2(c, x, len, ds_norms(c)), "norm");
-    return read_scalars(c, ds_norms(c), 1, out);
+    VV_CHECK(launch_norm2(c, x, len, c->host_scalars_dev), "norm");
+    return read_host(c, 1, out);
 }
 
 int vv_dot(vv_ctx *c, const double *x, const double *y, int64_t len, double *out)
 {
     if (int r = check_ctx(c)) return r;
     if (!x || !y || !out || len < 0) return fail(c, VV_ERR_INVALID, "bad argument");
-    VV_CHECK(launch_dot(c, x, y, len, ds_norms(c)), "dot");
-    return read_scalars(c, ds_norms(c), 1, out);
+    VV_CHECK(launch_dot(c, x, y, len, c->host_scalars_dev), "dot");
+    return read_host(c, 1, out);
 }
 
 int vv_axpy(vv_ctx *c, double alpha, const double *x, double *y, int64_t len)
@@ -1873,9 +1869,8 @@ int vv_snes_ksponly_mixed(vv_ctx *c, double *f, const double *fh, const vv_ksp_p
     if (c->B != 1) return fail(c, VV_ERR_UNSUPPORTED, "the mixed-precision solve takes one instance");
     if (int r = vv_function(c, f, fh, c->rhs)) return r;
     vv_ksp_result kr{};
-    if (int r = ksp_solve_mixed_impl(c, c->rhs, c->D, kp, mp, &kr, cycles)) return r;
     // SNESSolve_KSPONLY takes the step unless the linear solve diverged
-    if (kr.reason > 0) VV_CHECK(launch_axpy(c, -1.0, c->D, f, c->N), "update");
+    if (int r = ksp_solve_mixed_impl(c, c->rhs, c->D, kp, mp, &kr, cycles, f)) return r;
     if (res) *res = kr;
     return VV_OK;
 }
@@ -1961,8 +1956,8 @@ int vv_invariants(vv_ctx *c, const double *f, const double *h0, const double *h1
 {
     if (int r = check_ctx(c)) return r;
     if (!f || !h0 || !h1 || !h2 || !phi || !out) return fail(c, VV_ERR_INVALID, "null argument");
-    VV_CHECK(launch_invariants(c, f, h0, h1, h2, phi, ds_inv(c)), "invariants");
-    return read_scalars(c, ds_inv(c), 6 * (size_t)c->B, out);
+    VV_CHECK(launch_invariants(c, f, h0, h1, h2, phi, c->host_scalars_dev), "invariants");
+    return read_host(c, 6 * (size_t)c->B, out);
 }
 
 int vv_profile_enable(vv_ctx *c, int enable)

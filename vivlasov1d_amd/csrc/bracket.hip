@@ -62,6 +62,8 @@ struct BrArgs {
     double ht_inv, factor, alpha;
     const int32_t *done;   // optional early-exit flag (GMRES cycle finished)
     int64_t gstride;
+    double *part;          // residual: per-workgroup sums of y^2 (null: none), pstride apart per instance
+    int64_t pstride;
     int store;             // accumulate mode: y = 0 + factor {x, H} (the reference's
                            // Vec.set(0.) followed by PoissonBracket.function)
 };
@@ -193,8 +195,9 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int i = i0 + lane;
-    if (i >= nx) return;
+    if (MODE != MODE_RESIDUAL && i >= nx) return;
     const int cx = lane + 2;
+    double sq = 0.0;
     const T ht_inv = (T)a.ht_inv, af1 = (T)a.inst[b].af1, af2 = (T)a.inst[b].af2, factor = (T)a.factor;
 
     // Each lane walks down its column with the stencil values of F and H in
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     for (int q = 0; q < ROWS_PER_WAVE; ++q) {
         const int rr = rr0 + q;
         const int j = j0 + rr;
-        if (j < nv) {
+        if (j < nv && (MODE != MODE_RESIDUAL || i < nx)) {
             const size_t o = (size_t)j * nx + i;
             T base;
             if (MODE == MODE_RESIDUAL) {
@@ -224,9 +227,22 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
             if (MODE == MODE_TRANSPOSED || (j >= 2 && j < nv - 2))
                 out = arakawa_add<KIND>(win, base, factor, af1, af2);
             yout[o] = out;
+            if (MODE == MODE_RESIDUAL) sq += (double)out * (double)out;
         }
         // move the window one row down (rows stay inside the staged tile)
         if (q + 1 < ROWS_PER_WAVE) win.advance(rF, rH, rr + 3, cx);
+    }
+    // the residual's norm without another pass over it (6.8 us at 1024 x 2048)
+    if (MODE == MODE_RESIDUAL && a.part != nullptr) {
+        __shared__ double red[NT / 64];
+        for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off);
+        if (lane == 0) red[wave] = sq;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s = 0.0;
+            for (int w = 0; w < NT / 64; ++w) s += red[w];
+            a.part[b * a.pstride + blockIdx.x] = s;
+        }
     }
 }
 
@@ -268,12 +284,16 @@ BrArgs<T> base_args(vv_ctx *c)
 
 }  // namespace
 
-hipError_t launch_residual(vv_ctx *c, const double *f, const double *fh, double *y)
+int residual_blocks(const vv_ctx *c) { return br_tiles(c->p.nx, c->p.nv); }
+
+hipError_t launch_residual(vv_ctx *c, const double *f, const double *fh, double *y, double *part)
 {
     BrArgs<double> a = base_args<double>(c);
     a.f = f;
     a.fh = fh;
     a.y = y;
+    a.part = part;
+    a.pstride = c->part_stride;
     a.factor = 1.0;                 // B(Fave, H, 1.0)  (PETScNLVlasovMP.pyx:55)
     return launch_mode<MODE_RESIDUAL>(c, a);
 }

@@ -65,6 +65,63 @@ __device__ __forceinline__ void report(uint32_t *hout, uint32_t seq, bool done)
     __hip_atomic_store(hout, 2 * seq + (done ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Start of a cycle on V_0 with ||V_0||^2 = tot (KSPGMRESCycle entry:
+// VecNormalize(VV(0)), zero-residual and convergence tests), by one thread.
+__device__ __forceinline__ void cycle_start(const HessArgs &a, GmresState *g, double tot)
+{
+#pragma clang fp contract(off)
+    if (a.start == 2) {
+        const int32_t act = a.init.active != nullptr ? a.init.active[blockIdx.y] : 1;
+        g->st.its = 0;
+        g->st.reason = 0;
+        g->st.active = act;
+        g->st.res = 0.0;
+        g->st.rnorm0 = 0.0;
+        g->rtol = a.init.rtol;
+        g->atol = a.init.atol;
+        g->dtol = a.init.dtol;
+        g->haptol = 1.0e-30;     // PETSc gmres->haptol
+        g->max_it = a.init.max_it;
+        g->max_k = a.init.max_k;
+    }
+    g->st.it = 0;
+    // an instance that is not solving, or whose solve has ended, stays done
+    if (!g->st.active || g->st.reason != 0) {
+        g->st.done = 1;
+        return;
+    }
+    const double nrm = sqrt(tot);
+    g->st.done = 0;
+    g->scale[0] = scale_of(tot);
+    g->grs[0] = nrm;
+    g->st.res = nrm;
+    if (nrm == 0.0) {
+        g->st.reason = VV_KSP_CONVERGED_ATOL;
+        g->st.done = 1;
+        return;
+    }
+    if (a.start == 2) {
+        g->st.rnorm0 = nrm;
+        g->ttol = fmax(a.init.rtol * nrm, a.init.atol);
+    }
+    const int rsn = ksp_test(g, nrm);
+    if (rsn != 0) {
+        g->st.reason = rsn;
+        g->st.done = 1;
+    }
+}
+
+// Whether a kernel that carries the update or start `a` has nothing to do for
+// its instance: done as of the step before; at a start the flag is stale, and
+// the instances that take part count.
+__device__ __forceinline__ bool hess_skip(const HessArgs &a)
+{
+    const GmresState *g = a.g + blockIdx.y;
+    if (a.start == 2) return a.init.active != nullptr && a.init.active[blockIdx.y] == 0;
+    if (a.start == 1) return !g->st.active || g->st.reason != 0;
+    return g->st.done != 0;
+}
+
 // VecNormalize of V_{it+1} from the maxpy partials, then
 // KSPGMRESUpdateHessenberg (rotations, happy breakdown, residual estimate)
 // and the convergence test of instance blockIdx.y; sets done when the cycle
@@ -78,6 +135,12 @@ __device__ __forceinline__ void hess_update(const HessArgs &a)
     GmresState *g = a.g + blockIdx.y;
     const double *part = a.part + blockIdx.y * a.pstride;
     uint32_t *hout = a.hout != nullptr ? a.hout + blockIdx.y : nullptr;
+    if (a.start) {
+        __shared__ double sred[kGdNW + 1];
+        const double tot = block_sum_all(norm_share(part, a.nb), sred);
+        if (threadIdx.x == 0) cycle_start(a, g, tot);
+        return;
+    }
     const int it = a.it;
     // every load of the block is issued before the early-exit test waits on
     // the flag's (reading the state of a finished cycle is harmless)

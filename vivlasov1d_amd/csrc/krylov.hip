@@ -93,7 +93,6 @@ __global__ void gmres_init_kernel(GmresState *g, const int32_t *active, double r
     g->haptol = 1.0e-30;     // PETSc gmres->haptol
     g->max_it = max_it;
     g->max_k = max_k;
-    g->first = 1;
 }
 
 // Per-block partial sums of x*y over len elements (x == y: sum of squares).
@@ -114,53 +113,24 @@ __global__ __launch_bounds__(NT) void dot_partial_kernel(const double *__restric
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-// mode 0: *out = sqrt(sum) (VecNorm); mode 2: *out = sum (VecDot);
-// mode 1: GMRES cycle start on V_0 with sum = ||V_0||^2.
-__global__ __launch_bounds__(NT) void reduce_finish_kernel(const double *partial, int nb, int64_t pstride,
-                                                           GmresState *g, double *out, int mode)
+// *out = sqrt(sum) (VecNorm) or the sum (VecDot)
+__global__ __launch_bounds__(NT) void reduce_finish_kernel(const double *partial, int nb, double *out, int root)
 {
     __shared__ double red[NW + 1];
-    partial += blockIdx.y * pstride;
-    g += blockIdx.y;
-    if (out != nullptr) out += blockIdx.y;
     const double tot = final_sum_1(partial, nb, red);
+    if (threadIdx.x == 0) *out = root ? sqrt(tot) : tot;
+}
+
+// the norms of the B instances' fields from nb partials each, and their Poisson
+// residuals, into host memory
+__global__ __launch_bounds__(NT) void norms_finish_kernel(const double *partial, int nb, int64_t pstride,
+                                                          const double *pres, double *host)
+{
+    __shared__ double red[NW + 1];
+    const double tot = final_sum_1(partial + blockIdx.y * pstride, nb, red);
     if (threadIdx.x != 0) return;
-    if (mode == 2) {
-        *out = tot;
-        return;
-    }
-    const double nrm = sqrt(tot);
-    if (mode == 0) {
-        *out = nrm;
-        return;
-    }
-    // an instance that is not solving, or whose solve has ended, stays done
-    if (!g->st.active || g->st.reason != 0) {
-        g->st.it = 0;
-        g->st.done = 1;
-        return;
-    }
-    // KSPGMRESCycle entry: VecNormalize(VV(0)), zero-residual and convergence tests
-    g->st.it = 0;
-    g->st.done = 0;
-    g->scale[0] = nrm != 0.0 ? 1.0 / nrm : 1.0;
-    g->grs[0] = nrm;
-    g->st.res = nrm;
-    if (nrm == 0.0) {
-        g->st.reason = VV_KSP_CONVERGED_ATOL;
-        g->st.done = 1;
-        return;
-    }
-    if (g->first) {
-        g->st.rnorm0 = nrm;
-        g->ttol = fmax(g->rtol * nrm, g->atol);
-        g->first = 0;
-    }
-    const int rsn = ksp_test(g, nrm);
-    if (rsn != 0) {
-        g->st.reason = rsn;
-        g->st.done = 1;
-    }
+    host[blockIdx.y] = sqrt(tot);
+    if (pres != nullptr) host[gridDim.y + blockIdx.y] = pres[16 * (size_t)blockIdx.y];
 }
 
 // TAIL: N is not a multiple of the vector width L (odd grids such as 9 x 9;
@@ -311,78 +281,90 @@ __global__ __launch_bounds__(NT) void maxpy_norm_kernel(CgsArgs<S> a, int it)
     if (threadIdx.x == 0) a.part[a.noff + blockIdx.x] = s;
 }
 
-// The end of an Arnoldi step in a launch of its own (gmres_dev.h).
+// The end of an Arnoldi step, or the start of a cycle, in a launch of its own
+// (gmres_dev.h).
 __global__ __launch_bounds__(NT) void gmres_update_kernel(HessArgs a) { hess_update(a); }
 
-// KSPGMRESBuildSoln: back substitution with the rotated Hessenberg matrix;
-// the coefficients go to coef[0..it).  The triangle is staged in LDS first.
-__global__ __launch_bounds__(NT) void backsolve_kernel(GmresState *g)
-{
-    g += blockIdx.y;
-    __shared__ double sh[kMaxRestart][kMaxRestart];
-    __shared__ double sg[kMaxRestart];
-    __shared__ double y[kMaxRestart];     // in LDS: a runtime-indexed register array would live in scratch
-    const int n = g->st.it;
-    if (n <= 0) return;
-    for (int idx = threadIdx.x; idx < n * n; idx += NT) {
-        const int col = idx / n, r = idx - col * n;
-        sh[r][col] = g->hh[(size_t)col * (kMaxRestart + 1) + r];
-    }
-    if (threadIdx.x < n) sg[threadIdx.x] = g->grs[threadIdx.x];
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    const int k = n - 1;
-    if (sh[k][k] != 0.0) {
-        y[k] = sg[k] / sh[k][k];
-    } else {
-        g->st.reason = VV_KSP_DIVERGED_BREAKDOWN;
-        y[k] = 0.0;
-    }
-    for (int ii = 1; ii <= k; ++ii) {
-        const int kk = k - ii;
-        double tt = sg[kk];
-        for (int j = kk + 1; j <= k; ++j) tt = tt - sh[kk][j] * y[j];
-        if (sh[kk][kk] == 0.0) {
-            g->st.reason = VV_KSP_DIVERGED_BREAKDOWN;
-            y[kk] = 0.0;
-        } else {
-            y[kk] = tt / sh[kk][kk];
-        }
-    }
-    for (int j = 0; j <= k; ++j) g->coef[j] = y[j];
-}
-
-// x += sum_j coef_j v_j  (VEC_TEMP = 0 + sum_j nrs_j v_j; x = x + VEC_TEMP);
-// x is FP64 for either basis type.
+// KSPGMRESBuildSoln, and what follows it, in one launch: y from the rotated
+// (triangular) Hessenberg matrix, then x = V y (store) or x += V y
+// (VEC_TEMP = 0 + sum_j nrs_j v_j; x = x + VEC_TEMP; x is FP64 for either
+// basis type).  With f (one instance): f -= V y in place of the store where the
+// solve converged (SNESSolve_KSPONLY's step); a cycle that ended without a
+// reason stores x for the restarts.  hout: workgroup 0 also stores the
+// instance's final status there.
+// Every workgroup solves the triangle itself, in its first wavefront, while the
+// first group of basis vectors is on its way: lane r holds row r's right-hand
+// side, and each unknown found is taken off the rows above (n steps of one
+// division and one FMA; by one thread in a launch of its own it was n^2 / 2
+// dependent LDS reads, 8.5 us at n = 21 and 15 at 30).  With zeroing x, its
+// read-back and f -= x in their own launches the end of a solve took 8.5 +
+// 39.4 + 11.8 us at 1024 x 2048 and its start 6.5 more.
 template <int EPT, typename S, bool TAIL>
-__global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, CgsArgs<S> a)
+__global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, double *__restrict__ f, int store,
+                                                    CgsArgs<S> a, GmresStatus *hout)
 {
     using V = typename V16<S>::type;
     constexpr int L = V16<S>::L;
-    const GmresState *g = a.g + blockIdx.y;
+    GmresState *g = a.g + blockIdx.y;
     a.basis += blockIdx.y * a.N;
     x += blockIdx.y * a.N;
     const int n = g->st.it;
-    if (n <= 0) return;
+    int reason = g->st.reason;
     __shared__ double s_coef[kMaxRestart + 1], s_scale[kMaxRestart + 1];
-    if (threadIdx.x < n) {
-        s_coef[threadIdx.x] = g->coef[threadIdx.x];
-        s_scale[threadIdx.x] = g->scale[threadIdx.x];
+    __shared__ double sh[kMaxRestart * kMaxRestart];        // column j at j n
+    __shared__ int s_sing;
+    const int t = threadIdx.x;
+    const int64_t nvv = a.N / L;
+    const int64_t e0 = (int64_t)blockIdx.x * NT * EPT + t;
+    constexpr int G = cgs_group<EPT>();
+    V v[G][EPT];
+    load_group<EPT, G, S>(a.basis, a.vstride, 0, n, e0, nvv, v);
+    for (int idx = t; idx < n * n; idx += NT) {
+        const int col = idx / n, r = idx - col * n;
+        sh[idx] = g->hh[(size_t)col * (kMaxRestart + 1) + r];
+    }
+    double rhs = t < n ? g->grs[t] : 0.0;
+    if (t < n) s_scale[t] = g->scale[t];
+    if (t == 0) s_sing = 0;
+    __syncthreads();
+    if (t < 64) {
+        double coef = 0.0;
+        for (int k = n - 1; k >= 0; --k) {
+            const double d = sh[k * n + k], h = t < k ? sh[k * n + t] : 0.0;
+            const double y = d != 0.0 ? __shfl(rhs, k) / d : 0.0;
+            if (d == 0.0 && t == 0) s_sing = 1;
+            if (t == k) coef = y;
+            rhs = rhs - h * y;
+        }
+        if (t < n) s_coef[t] = coef;
     }
     __syncthreads();
-    const int64_t nvv = a.N / L;
-    const int64_t e0 = (int64_t)blockIdx.x * NT * EPT + threadIdx.x;
+    if (s_sing) {
+        reason = VV_KSP_DIVERGED_BREAKDOWN;
+        if (blockIdx.x == 0 && t == 0) g->st.reason = reason;
+    }
+    if (hout != nullptr && blockIdx.x == 0 && t == 0) {
+        // per-field stores by one lane
+        GmresStatus *ho = hout + blockIdx.y;
+        ho->it = n;
+        ho->its = g->st.its;
+        ho->reason = reason;
+        ho->done = g->st.done;
+        ho->active = g->st.active;
+        ho->res = g->st.res;
+        ho->rnorm0 = g->st.rnorm0;
+    }
+    const bool step = f != nullptr && reason > 0;
+    if (n <= 0 && (!store || f != nullptr) && reason != 0) return;
     const int64_t et = tail_element<S, TAIL>(a.N, nvv);
     double tt = 0.0;
-    double t[EPT][L];
+    double acc[EPT][L];
 #pragma unroll
     for (int q = 0; q < EPT; ++q)
 #pragma unroll
-        for (int l = 0; l < L; ++l) t[q][l] = 0.0;
-    constexpr int G = cgs_group<EPT>();
+        for (int l = 0; l < L; ++l) acc[q][l] = 0.0;
     for (int j = 0; j < n; j += G) {
-        V v[G][EPT];
-        load_group<EPT, G, S>(a.basis, a.vstride, j, n - j, e0, nvv, v);
+        if (j > 0) load_group<EPT, G, S>(a.basis, a.vstride, j, n - j, e0, nvv, v);
 #pragma unroll
         for (int gg = 0; gg < G; ++gg) {
             if (j + gg >= n) break;
@@ -390,46 +372,64 @@ __global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, CgsA
 #pragma unroll
             for (int q = 0; q < EPT; ++q) {
 #pragma unroll
-                for (int l = 0; l < L; ++l) t[q][l] = t[q][l] + cj * (vget(v[gg][q], l) * sj);
+                for (int l = 0; l < L; ++l) acc[q][l] = acc[q][l] + cj * (vget(v[gg][q], l) * sj);
             }
             if (TAIL && et >= 0) tt = tt + cj * ((double)a.basis[(size_t)(j + gg) * a.vstride + et] * sj);
         }
     }
-    if (TAIL && et >= 0) x[et] = x[et] + tt;
-    double2 *X = reinterpret_cast<double2 *>(x);
+    // out = base + sign * acc
+    double *out = step ? f : x;
+    const double sign = step ? -1.0 : 1.0;
+    const bool add = step || !store;
+    if (TAIL && et >= 0) out[et] = (add ? out[et] : 0.0) + sign * tt;
+    // x, f: FP64, pairs where both are 16-byte aligned
+    const bool pairs = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
 #pragma unroll
     for (int q = 0; q < EPT; ++q) {
         const int64_t e = e0 + (int64_t)q * NT;
         if (e < nvv) {
 #pragma unroll
             for (int h = 0; h < L / 2; ++h) {
-                double2 xv = X[e * (L / 2) + h];
-                xv.x = xv.x + t[q][2 * h];
-                xv.y = xv.y + t[q][2 * h + 1];
-                X[e * (L / 2) + h] = xv;
+                double *o = out + e * L + 2 * h;
+                double2 xv{0.0, 0.0};
+                if (pairs) {
+                    if (add) xv = *reinterpret_cast<const double2 *>(o);
+                } else if (add) {
+                    xv.x = o[0];
+                    xv.y = o[1];
+                }
+                xv.x = xv.x + sign * acc[q][2 * h];
+                xv.y = xv.y + sign * acc[q][2 * h + 1];
+                if (pairs) {
+                    *reinterpret_cast<double2 *>(o) = xv;
+                } else {
+                    o[0] = xv.x;
+                    o[1] = xv.y;
+                }
             }
         }
     }
 }
 
-// Cycle start of the FP32 GMRES cycle: V_0 = (float) r and per-block partial
-// sums of the squares of the rounded values.
-__global__ __launch_bounds__(NT) void cvt_partial_kernel(const double *__restrict__ r, float *__restrict__ v0,
-                                                         int64_t len, int64_t bstride, double *partial,
-                                                         int64_t pstride)
+// V_0 of a cycle with the partial sums of its squares: MODE 0 V_0 = b (FP64),
+// 1 V_0 = (float) r with ||r|| of the FP64 right-hand side, 2 V_0 = b - V_0
+// (KSPInitialResidual after a restart: r = b - A x).
+template <int MODE, typename S>
+__global__ __launch_bounds__(NT) void start_kernel(const double *__restrict__ b, S *v0, int64_t len, double *partial,
+                                                   int64_t pstride)
 {
     __shared__ double red[NW + 1];
-    r += blockIdx.y * len;
-    v0 += blockIdx.y * bstride;
-    partial += blockIdx.y * pstride;
+    b += blockIdx.y * len;
+    v0 += blockIdx.y * len;
     double acc = 0.0;
     for (int64_t e = (int64_t)blockIdx.x * NT + threadIdx.x; e < len; e += (int64_t)gridDim.x * NT) {
-        const double d = r[e];
-        v0[e] = (float)d;
-        acc += d * d;          // ||r|| of the FP64 right-hand side
+        double d = b[e];
+        if (MODE == 2) d = d + (-1.0) * (double)v0[e];
+        v0[e] = (S)d;
+        acc += d * d;
     }
     const double s = block_sum_all(acc, red);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
+    if (threadIdx.x == 0) partial[blockIdx.y * pstride + blockIdx.x] = s;
 }
 
 // y = y + alpha*x (VecAXPY).  mode 1: only when the GMRES reason is positive
@@ -444,8 +444,7 @@ __global__ __launch_bounds__(NT) void axpy_kernel(double alpha, const double *__
         y[e] = y[e] + alpha * x[e];
 }
 
-// y = b - y   (KSPInitialResidual after a restart: r = b - A x); instance
-// blockIdx.y at b + blockIdx.y len, y + blockIdx.y ystride
+// y = b - y; instance blockIdx.y at b + blockIdx.y len, y + blockIdx.y ystride
 __global__ __launch_bounds__(NT) void rsub_kernel(const double *__restrict__ b, double *y, int64_t len,
                                                   int64_t ystride)
 {
@@ -517,20 +516,12 @@ hipError_t launch_gmres_init(vv_ctx *c, double rtol, double atol, double dtol, i
     return hipGetLastError();
 }
 
-hipError_t launch_norm_start(vv_ctx *c)
-{
-    const int nb = grid_for(c->N);
-    hipLaunchKernelGGL(dot_partial_kernel, dim3(nb, c->B), dim3(NT), 0, c->stream, c->basis, c->basis, c->N, c->N,
-                       c->partial, c->part_stride);
-    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, c->partial, nb, c->part_stride,
-                       c->gs, (double *)nullptr, 1);
-    return hipGetLastError();
-}
+double *norm_partials(vv_ctx *c) { return c->partial + norm_partial_offset(c); }
 
 namespace {
 
 template <int E, typename S, bool TAIL>
-void cgs_launch(vv_ctx *c, const S *basis, int which, int arg, double *x, int dot_rows)
+void cgs_launch(vv_ctx *c, const S *basis, int which, int arg, double *x, int dot_rows, double *f, GmresStatus *hout)
 {
     const int nb = cgs_blocks_v(c, c->N / V16<S>::L);
     CgsArgs<S> a{basis, c->N, c->vs, c->partial, c->part_stride, c->gs, norm_partial_offset(c),
@@ -543,26 +534,28 @@ void cgs_launch(vv_ctx *c, const S *basis, int which, int arg, double *x, int do
         if (c->p.restart < 32) launch_timed(c, maxpy_norm_kernel<E, 32, S, TAIL>, grid, block, 0, a, arg);
         else launch_timed(c, maxpy_norm_kernel<E, 64, S, TAIL>, grid, block, 0, a, arg);
     } else {
-        launch_timed(c, update_kernel<E, S, TAIL>, grid, block, 0, x, a);
+        launch_timed(c, update_kernel<E, S, TAIL>, grid, block, 0, x, f, arg, a, hout);
     }
 }
 
 template <typename S, bool TAIL>
-void cgs_dispatch_e(vv_ctx *c, const S *basis, int which, int arg, double *x, int dot_rows)
+void cgs_dispatch_e(vv_ctx *c, const S *basis, int which, int arg, double *x, int dot_rows, double *f,
+                    GmresStatus *hout)
 {
     switch (cgs_ept_v(c, c->N / V16<S>::L)) {
-    case 8: cgs_launch<8, S, TAIL>(c, basis, which, arg, x, dot_rows); break;
-    case 4: cgs_launch<4, S, TAIL>(c, basis, which, arg, x, dot_rows); break;
-    case 2: cgs_launch<2, S, TAIL>(c, basis, which, arg, x, dot_rows); break;
-    default: cgs_launch<1, S, TAIL>(c, basis, which, arg, x, dot_rows); break;
+    case 8: cgs_launch<8, S, TAIL>(c, basis, which, arg, x, dot_rows, f, hout); break;
+    case 4: cgs_launch<4, S, TAIL>(c, basis, which, arg, x, dot_rows, f, hout); break;
+    case 2: cgs_launch<2, S, TAIL>(c, basis, which, arg, x, dot_rows, f, hout); break;
+    default: cgs_launch<1, S, TAIL>(c, basis, which, arg, x, dot_rows, f, hout); break;
     }
 }
 
 template <typename S>
-hipError_t cgs_dispatch(vv_ctx *c, const S *basis, int which, int arg, double *x, int dot_rows = 0)
+hipError_t cgs_dispatch(vv_ctx *c, const S *basis, int which, int arg, double *x, int dot_rows = 0,
+                        double *f = nullptr, GmresStatus *hout = nullptr)
 {
-    if (c->N % V16<S>::L) cgs_dispatch_e<S, true>(c, basis, which, arg, x, dot_rows);
-    else cgs_dispatch_e<S, false>(c, basis, which, arg, x, dot_rows);
+    if (c->N % V16<S>::L) cgs_dispatch_e<S, true>(c, basis, which, arg, x, dot_rows, f, hout);
+    else cgs_dispatch_e<S, false>(c, basis, which, arg, x, dot_rows, f, hout);
     return hipGetLastError();
 }
 
@@ -582,13 +575,6 @@ hipError_t maxpy_norm_t(vv_ctx *c, const S *basis, int it, int dot_rows)
     return cgs_dispatch(c, basis, 1, it, nullptr, dot_rows);
 }
 
-template <typename S>
-hipError_t build_solution_t(vv_ctx *c, const S *basis, double *x)
-{
-    hipLaunchKernelGGL(backsolve_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, c->gs);
-    return cgs_dispatch(c, basis, 2, 0, x);
-}
-
 }  // namespace
 
 hipError_t launch_mdot(vv_ctx *c, int col) { return mdot_t<double>(c, c->basis, col); }
@@ -599,9 +585,11 @@ hipError_t launch_maxpy_norm(vv_ctx *c, int it, int dot_rows)
 
 HessArgs take_update(vv_ctx *c)
 {
-    const HessArgs a{c->partial + norm_partial_offset(c), c->part_stride, c->pend_it >= 0 ? c->pend_nb : 0,
-                     c->pend_it, c->gs, c->report_out, c->report_seq};
+    const bool due = c->pend_it >= 0 || c->pend_start;
+    const HessArgs a{norm_partials(c), c->part_stride, due ? c->pend_nb : 0, c->pend_it, c->gs,
+                     c->pend_start ? nullptr : c->report_out, c->report_seq, c->pend_start, c->start};
     c->pend_it = -1;
+    c->pend_start = 0;
     c->report_out = nullptr;
     return a;
 }
@@ -614,37 +602,69 @@ hipError_t launch_update(vv_ctx *c)
     return hipGetLastError();
 }
 
-hipError_t launch_build_solution(vv_ctx *c, double *x) { return build_solution_t<double>(c, c->basis, x); }
+hipError_t launch_build_solution(vv_ctx *c, double *x, double *f, bool store, GmresStatus *hout)
+{
+    return cgs_dispatch(c, c->basis, 2, store ? 1 : 0, x, 0, f, hout);
+}
 hipError_t launch_mdot32(vv_ctx *c, int col) { return mdot_t<float>(c, c->basis32, col); }
 hipError_t launch_maxpy_norm32(vv_ctx *c, int it, int dot_rows)
 {
     return maxpy_norm_t<float>(c, c->basis32, it, dot_rows);
 }
-hipError_t launch_build_solution32(vv_ctx *c, double *x) { return build_solution_t<float>(c, c->basis32, x); }
-
-hipError_t launch_start32(vv_ctx *c, const double *r)
+hipError_t launch_build_solution32(vv_ctx *c, double *x, double *f, bool store, GmresStatus *hout)
 {
-    const int nb = grid_for(c->N);
-    hipLaunchKernelGGL(cvt_partial_kernel, dim3(nb, c->B), dim3(NT), 0, c->stream, r, c->basis32, c->N, c->N,
-                       c->partial, c->part_stride);
-    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, c->partial, nb, c->part_stride,
-                       c->gs, (double *)nullptr, 1);
-    return hipGetLastError();
+    return cgs_dispatch(c, c->basis32, 2, store ? 1 : 0, x, 0, f, hout);
 }
 
-hipError_t launch_residual_restart(vv_ctx *c, const double *b, double *y)
+namespace {
+hipError_t start_due(vv_ctx *c, int nb, bool first)
+{
+    c->pend_it = -1;
+    c->pend_nb = nb;
+    c->pend_start = first ? 2 : 1;
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_start(vv_ctx *c, const double *b, bool first)
+{
+    const int nb = grid_for(c->N);
+    hipLaunchKernelGGL((start_kernel<0, double>), dim3(nb, c->B), dim3(NT), 0, c->stream, b, c->basis, c->N,
+                       norm_partials(c), c->part_stride);
+    return start_due(c, nb, first);
+}
+
+hipError_t launch_start32(vv_ctx *c, const double *r, bool first)
+{
+    const int nb = grid_for(c->N);
+    hipLaunchKernelGGL((start_kernel<1, float>), dim3(nb, c->B), dim3(NT), 0, c->stream, r, c->basis32, c->N,
+                       norm_partials(c), c->part_stride);
+    return start_due(c, nb, first);
+}
+
+hipError_t launch_restart(vv_ctx *c, const double *b)
+{
+    const int nb = grid_for(c->N);
+    hipLaunchKernelGGL((start_kernel<2, double>), dim3(nb, c->B), dim3(NT), 0, c->stream, b, c->basis, c->N,
+                       norm_partials(c), c->part_stride);
+    return start_due(c, nb, false);
+}
+
+hipError_t launch_rsub(vv_ctx *c, const double *b, double *y)
 {
     hipLaunchKernelGGL(rsub_kernel, dim3(grid_for(c->N), c->B), dim3(NT), 0, c->stream, b, y, c->N, c->N);
     return hipGetLastError();
 }
 
-hipError_t launch_norms(vv_ctx *c, const double *x, double *out_dev)
+hipError_t launch_norms(vv_ctx *c, const double *x, int nb, const double *pres, double *host)
 {
-    const int nb = grid_for(c->N);
-    hipLaunchKernelGGL(dot_partial_kernel, dim3(nb, c->B), dim3(NT), 0, c->stream, x, x, c->N, c->N, c->partial,
-                       c->part_stride);
-    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, c->partial, nb, c->part_stride,
-                       c->gs, out_dev, 0);
+    if (x != nullptr) {
+        nb = grid_for(c->N);
+        hipLaunchKernelGGL(dot_partial_kernel, dim3(nb, c->B), dim3(NT), 0, c->stream, x, x, c->N, c->N, c->partial,
+                           c->part_stride);
+    }
+    hipLaunchKernelGGL(norms_finish_kernel, dim3(1, c->B), dim3(NT), 0, c->stream, c->partial, nb, c->part_stride,
+                       pres, host);
     return hipGetLastError();
 }
 
@@ -653,8 +673,7 @@ hipError_t launch_norm2(vv_ctx *c, const double *x, int64_t n, double *out_dev)
     const int nb = grid_for(n);
     hipLaunchKernelGGL(dot_partial_kernel, dim3(nb), dim3(NT), 0, c->stream, x, x, n, (int64_t)0, c->partial,
                        c->part_stride);
-    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1), dim3(NT), 0, c->stream, c->partial, nb, c->part_stride, c->gs,
-                       out_dev, 0);
+    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1), dim3(NT), 0, c->stream, c->partial, nb, out_dev, 1);
     return hipGetLastError();
 }
 
@@ -663,8 +682,7 @@ hipError_t launch_dot(vv_ctx *c, const double *x, const double *y, int64_t n, do
     const int nb = grid_for(n);
     hipLaunchKernelGGL(dot_partial_kernel, dim3(nb), dim3(NT), 0, c->stream, x, y, n, (int64_t)0, c->partial,
                        c->part_stride);
-    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1), dim3(NT), 0, c->stream, c->partial, nb, c->part_stride, c->gs,
-                       out_dev, 2);
+    hipLaunchKernelGGL(reduce_finish_kernel, dim3(1), dim3(NT), 0, c->stream, c->partial, nb, out_dev, 0);
     return hipGetLastError();
 }
 

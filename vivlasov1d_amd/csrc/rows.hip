@@ -222,7 +222,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
         hess_update(hs);
         return;
     }
-    const int32_t dflag = cycle_done(a.done, a.gstride);
+    const int32_t dflag = extra ? hess_skip(hs) : cycle_done(a.done, a.gstride);
     if (gridDim.y > 1 && dflag) return;   // batched: a finished instance skips its loads
     const int b = blockIdx.y, t = threadIdx.x;
     const int nx = a.nx, nv = a.nv, RW = g.RW, RH = RW + 4, W = g.W, SP = W + 4;
@@ -425,7 +425,7 @@ __device__ __forceinline__ typename V2<T>::type load_pair(const T *p, int v, int
 
 // irFFT of the workgroup's RI rows into w = V_{col+1}, and the dots of w with
 // v_0 .. v_col from LDS, partials per block as irfft_mdot_kernel's; col = -1:
-// into y, no dots.  RI is even, so a block starts on an even element and is
+// into y, with the block's sum of squares at part[block] when part is given.  RI is even, so a block starts on an even element and is
 // read in pairs (thread t the pairs t + 256 q, q < EPT); the last block may be
 // short, and odd.  Replaces irFFT + mdot: 4.9 + 3.3 us at 64 x 128 and 9.3 +
 // 4.6 us at 201 x 401 with a launch between.
@@ -518,8 +518,25 @@ __global__ __launch_bounds__(NT) void row_inv_kernel(FftArgs<T> a, const cx_t<T>
         if (2 * v + 1 < cnt) reinterpret_cast<V *>(W)[v] = w[q];
         else if (2 * v < cnt) W[2 * v] = w[q].x;
     }
-    if (nvec == 0) return;
     const int lane = t & 63, wave = t >> 6;
+    if (nvec == 0) {
+        if (g.part == nullptr) return;
+        double acc = 0.0;
+#pragma unroll
+        for (int q = 0; q < EPT; ++q) {
+            acc = __builtin_fma((double)w[q].x, (double)w[q].x, acc);
+            acc = __builtin_fma((double)w[q].y, (double)w[q].y, acc);
+        }
+        acc = wave_sum(acc);
+        if (lane == 0) red[wave][0] = acc;
+        __syncthreads();
+        if (t == 0) {
+            double s = 0.0;
+            for (int wv = 0; wv < kCgsNW; ++wv) s += red[wv][0];
+            (g.part + bi * g.pstride)[blk] = s;
+        }
+        return;
+    }
     for (int v = 0; v < nvec; v += G) {
         if (v > 0) load_vectors(v);
 #pragma unroll
@@ -646,7 +663,7 @@ void inv_launch(vv_ctx *c, const FftArgs<T> &a, const cx_t<T> *spec, const CgsAr
 }
 
 template <typename T>
-hipError_t row_inv_t(vv_ctx *c, const T *basis, const cx_t<T> *spec, int col, T *y, const int32_t *done)
+hipError_t row_inv_t(vv_ctx *c, const T *basis, const cx_t<T> *spec, int col, T *y, double *part, const int32_t *done)
 {
     const int RI = inv_rows(c);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, RI, c->N, spec_stride(c), (int64_t)sizeof(GmresState),
@@ -654,7 +671,7 @@ hipError_t row_inv_t(vv_ctx *c, const T *basis, const cx_t<T> *spec, int col, T 
     const int nb = (a.nv + RI - 1) / RI;
     const bool dft = fft_kind(a.nx) == kDft;
     const size_t lds = (size_t)(RI >> 1) * a.nx * sizeof(cx_t<T>) * (dft ? 2 : 1) + (size_t)a.nx * sizeof(cx_t<T>);
-    const CgsArgs<T> g{basis, c->N, c->vs, c->partial, c->part_stride, c->gs, 0, nb};
+    const CgsArgs<T> g{basis, c->N, c->vs, part, c->part_stride, c->gs, 0, nb};
     const int pitch = c->p.restart < 32 ? 32 : 64;
     const dim3 grid(nb, c->B);
     const int pts = RI * a.nx;
@@ -737,22 +754,27 @@ hipError_t launch_row_rfft32(vv_ctx *c, const float *x, float2 *spec, const int3
 
 hipError_t launch_row_irfft(vv_ctx *c, const double2 *spec, double *y, const int32_t *done)
 {
-    return row_inv_t<double>(c, nullptr, spec, -1, y, done);
+    return row_inv_t<double>(c, nullptr, spec, -1, y, nullptr, done);
 }
 
 hipError_t launch_row_irfft32(vv_ctx *c, const float2 *spec, float *y, const int32_t *done)
 {
-    return row_inv_t<float>(c, nullptr, spec, -1, y, done);
+    return row_inv_t<float>(c, nullptr, spec, -1, y, nullptr, done);
+}
+
+hipError_t launch_row_inv_start(vv_ctx *c, const double2 *spec)
+{
+    return row_inv_t<double>(c, nullptr, spec, -1, c->basis, norm_partials(c), nullptr);
 }
 
 hipError_t launch_row_inv(vv_ctx *c, const double2 *spec, int col, const int32_t *done)
 {
-    return row_inv_t<double>(c, c->basis, spec, col, nullptr, done);
+    return row_inv_t<double>(c, c->basis, spec, col, nullptr, c->partial, done);
 }
 
 hipError_t launch_row_inv32(vv_ctx *c, const float2 *spec, int col, const int32_t *done)
 {
-    return row_inv_t<float>(c, c->basis32, spec, col, nullptr, done);
+    return row_inv_t<float>(c, c->basis32, spec, col, nullptr, c->partial, done);
 }
 
 // Radices of a length that is no power of two: the divisors' product that

@@ -194,7 +194,7 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
     }
     static_assert(NT == kJrSW, "a strip is one column per thread");
     constexpr int RH = R + 4, SP = NT + 4, nx = NS * NT;
-    const int32_t dflag = cycle_done(a.done, a.gstride);
+    const int32_t dflag = extra ? hess_skip(hs) : cycle_done(a.done, a.gstride);
     if (gridDim.y > 1 && dflag) return;   // batched: a finished instance skips its loads
     const int b = blockIdx.y;
     u += b * a.N;
@@ -388,7 +388,10 @@ struct RealRowsSink {
 // bit-identical to irfft_kernel followed by mdot_kernel.  What the fusion
 // saves: the second read of w, one launch, and the wait for the first basis
 // vectors, whose loads are in flight while the FFT stages run.
-template <typename T, int EPT, int PV, bool P8>
+// START (col = -1): the irFFT into V_0 = P^-1 F and its norm partials, at
+// part[slice]: a solve's first vector without the copy and the norm pass (8.4 +
+// 6.7 us at 1024 x 2048).
+template <typename T, int EPT, int PV, bool P8, bool START>
 __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t<T> *__restrict__ spec,
                                                         CgsArgs<T> g, int col)
 {
@@ -463,6 +466,22 @@ __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t
         W[e0 + (int64_t)q * NT] = w[q];
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if constexpr (START) {
+        double acc = 0.0;
+#pragma unroll
+        for (int q = 0; q < EPT; ++q)
+#pragma unroll
+            for (int l = 0; l < V16<T>::L; ++l) acc = __builtin_fma(vget(w[q], l), vget(w[q], l), acc);
+        acc = wave_sum(acc);
+        if (lane == 0) red[wave][0] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s = 0.0;
+            for (int wv = 0; wv < kCgsNW; ++wv) s += red[wv][0];
+            part[slice] = s;
+        }
+        return;
+    }
     for (int v = 0; v < nvec; v += G) {
         if (v > 0) load_group<EPT, G, T>(basis, g.vstride, v, nvec - v, e0, nvv, x);
 #pragma unroll
@@ -1171,12 +1190,20 @@ void irfft_mdot_launch(vv_ctx *c, const FftArgs<T> &a, dim3 grid, size_t lds, co
                        const CgsArgs<T> &g, int col)
 {
     const bool p8 = a.nx == N8;
+    const uint32_t l = (uint32_t)lds;
+    if constexpr (sizeof(T) == 8) {
+        if (col < 0) {
+            if (p8) launch_timed(c, irfft_mdot_kernel<T, EPT, 32, true, true>, grid, dim3(NT), l, a, spec, g, col);
+            else launch_timed(c, irfft_mdot_kernel<T, EPT, 32, false, true>, grid, dim3(NT), l, a, spec, g, col);
+            return;
+        }
+    }
     if (c->p.restart < 32) {
-        if (p8) launch_timed(c, irfft_mdot_kernel<T, EPT, 32, true>, grid, dim3(NT), (uint32_t)lds, a, spec, g, col);
-        else launch_timed(c, irfft_mdot_kernel<T, EPT, 32, false>, grid, dim3(NT), (uint32_t)lds, a, spec, g, col);
+        if (p8) launch_timed(c, irfft_mdot_kernel<T, EPT, 32, true, false>, grid, dim3(NT), l, a, spec, g, col);
+        else launch_timed(c, irfft_mdot_kernel<T, EPT, 32, false, false>, grid, dim3(NT), l, a, spec, g, col);
     } else {
-        if (p8) launch_timed(c, irfft_mdot_kernel<T, EPT, 64, true>, grid, dim3(NT), (uint32_t)lds, a, spec, g, col);
-        else launch_timed(c, irfft_mdot_kernel<T, EPT, 64, false>, grid, dim3(NT), (uint32_t)lds, a, spec, g, col);
+        if (p8) launch_timed(c, irfft_mdot_kernel<T, EPT, 64, true, false>, grid, dim3(NT), l, a, spec, g, col);
+        else launch_timed(c, irfft_mdot_kernel<T, EPT, 64, false, false>, grid, dim3(NT), l, a, spec, g, col);
     }
 }
 
@@ -1189,7 +1216,7 @@ hipError_t irfft_mdot_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, const
                  (int64_t)sizeof(GmresState), tw, done};
     const int nb = a.nv / a.rows;
     const size_t lds = fft_lds<T>(a);
-    const CgsArgs<T> g{basis, c->N, c->vs, c->partial, c->part_stride, c->gs, 0, nb};
+    const CgsArgs<T> g{basis, c->N, c->vs, col < 0 ? norm_partials(c) : c->partial, c->part_stride, c->gs, 0, nb};
     const dim3 grid(nb, c->B);
     switch (ept) {
     case 8: irfft_mdot_launch<T, 8>(c, a, grid, lds, spec, g, col); break;
@@ -1323,6 +1350,11 @@ int irfft_mdot_rows(const vv_ctx *c, bool fp32)
 hipError_t launch_irfft_mdot(vv_ctx *c, const double2 *spec, int col, const int32_t *done)
 {
     return irfft_mdot_t<double>(c, c->twiddle, spec, c->basis, col, done);
+}
+
+hipError_t launch_irfft_start(vv_ctx *c, const double2 *spec)
+{
+    return irfft_mdot_t<double>(c, c->twiddle, spec, c->basis, -1, nullptr);
 }
 
 hipError_t launch_irfft_mdot32(vv_ctx *c, const float2 *spec, int col, const int32_t *done)

@@ -54,11 +54,19 @@ struct GmresState {
     double ttol, rtol, atol, dtol, haptol;
     int32_t max_it;
     int32_t max_k;
-    int32_t first;                   // first cycle: sets rnorm0 and ttol
-    int32_t pad;
 };
 
-// The Hessenberg update of Arnoldi step `it` (gmres_dev.h): its norm partials
+// Tolerances and limits a solve starts with, and which instances take part
+// (null: all).
+struct SolveStart {
+    const int32_t *active;
+    double rtol, atol, dtol;
+    int32_t max_it, max_k;
+};
+
+// The Hessenberg update of Arnoldi step `it` (gmres_dev.h), or, with start, the
+// start of a cycle on V_0 (1: a restart; 2: the first of a solve, whose state
+// `init` fills): its norm partials
 // (instance b at part + b pstride, nb of them; nb = 0: no update is due), the
 // states, and where the host polls for the report (one word per instance;
 // null: nobody does) and its number.
@@ -69,6 +77,8 @@ struct HessArgs {
     GmresState *g;
     uint32_t *hout;
     uint32_t seq;
+    int start;
+    SolveStart init;
 };
 
 // Plan of the mixed-radix line transform (rows.hip): stage s has radix r[s]
@@ -156,6 +166,8 @@ struct vv_ctx {
     uint32_t *report_out;           // set for one launch: where the Hessenberg update reports
     uint32_t report_seq;            // number of the last report asked for (below 2^31)
     int pend_it, pend_nb;           // Arnoldi step whose Hessenberg update is due (-1: none), its norm partials
+    int pend_start;                 // a cycle start is due instead (HessArgs::start; 0: none)
+    vv::SolveStart start;           // what a first cycle starts with
     double *host_scalars;           // pinned staging of device scalars
     double *host_scalars_dev;       // the same memory as the device addresses it
     int32_t *host_active;           // pinned staging of the instance mask
@@ -203,7 +215,9 @@ namespace vv {
 
 // ---- launchers -------------------------------------------------------------
 // bracket.hip
-hipError_t launch_residual(vv_ctx *c, const double *f, const double *fh, double *y);
+// part: per-workgroup sums of y^2 (residual_blocks of them, instances part_stride apart) when not null
+hipError_t launch_residual(vv_ctx *c, const double *f, const double *fh, double *y, double *part = nullptr);
+int residual_blocks(const vv_ctx *c);
 hipError_t launch_jacobian(vv_ctx *c, const double *u, const double *uscale, double *y);
 hipError_t launch_bracket_add(vv_ctx *c, const double *x, double *y, double factor);
 hipError_t launch_jacobian32(vv_ctx *c, const float *u, const double *uscale, float *y);
@@ -250,6 +264,8 @@ hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int3
 hipError_t launch_row_rfft32(vv_ctx *c, const float *x, float2 *spec, const int32_t *done);
 hipError_t launch_row_irfft(vv_ctx *c, const double2 *spec, double *y, const int32_t *done);
 hipError_t launch_row_irfft32(vv_ctx *c, const float2 *spec, float *y, const int32_t *done);
+// the irFFT into V_0 with its norm partials (row_inv_blocks of them)
+hipError_t launch_row_inv_start(vv_ctx *c, const double2 *spec);
 hipError_t launch_row_inv(vv_ctx *c, const double2 *spec, int col, const int32_t *done);
 hipError_t launch_row_inv32(vv_ctx *c, const float2 *spec, int col, const int32_t *done);
 // spectral.hip
@@ -278,6 +294,7 @@ int irfft_mdot_rows(const vv_ctx *c, bool fp32);
 int lu_rows(int nv);
 int lu_pivots_per_mode(int nv);
 hipError_t launch_irfft_mdot(vv_ctx *c, const double2 *spec, int col, const int32_t *done);
+hipError_t launch_irfft_start(vv_ctx *c, const double2 *spec);   // into V_0, with its norm partials per slice
 hipError_t launch_irfft_mdot32(vv_ctx *c, const float2 *spec, int col, const int32_t *done);
 // potential preconditioner: field (nv rows of nx) <-> transposed (nx rows of nv)
 // reciprocal LU pivots of the kinetic T_k into rp64 (FP64) and / or rp32 (rounded)
@@ -287,7 +304,13 @@ hipError_t launch_transpose32(vv_ctx *c, const float *in, float *out, bool back,
 hipError_t launch_potential_bands(vv_ctx *c, const double *phi);
 // krylov.hip
 hipError_t launch_gmres_init(vv_ctx *c, double rtol, double atol, double dtol, int max_it);
-hipError_t launch_norm_start(vv_ctx *c);                  // cycle start on basis[0]
+// V_0 for a cycle start, with its norm partials: copied from b, rounded from r,
+// or in place; the start is then due as a Hessenberg update is (take_update).
+// A first cycle starts with c->start.
+double *norm_partials(vv_ctx *c);                         // where they go (instances part_stride apart)
+hipError_t launch_start(vv_ctx *c, const double *b, bool first);        // V_0 = b
+hipError_t launch_start32(vv_ctx *c, const double *r, bool first);      // V_0 = (float) r
+hipError_t launch_restart(vv_ctx *c, const double *b);    // V_0 = b - V_0
 int cgs_blocks_max(int64_t N);                            // partial rows the CGS kernels may use
 int cgs_ept(const vv_ctx *c, int64_t nvv);              // 16-byte vectors per thread of a CGS launch
 hipError_t launch_mdot(vv_ctx *c, int col);               // CGS dots of basis[col+1] vs 0..col
@@ -298,13 +321,17 @@ hipError_t launch_mdot(vv_ctx *c, int col);               // CGS dots of basis[c
 hipError_t launch_maxpy_norm(vv_ctx *c, int it, int dot_rows = 0);
 HessArgs take_update(vv_ctx *c);
 hipError_t launch_update(vv_ctx *c);
-hipError_t launch_build_solution(vv_ctx *c, double *x);  // x += V y
-hipError_t launch_start32(vv_ctx *c, const double *r);    // FP32 cycle start: V_0 = (float) r
+// x (FP64) = V y (store) or x += V y, y from the triangular system; with f:
+// f -= V y instead of the store where the solve converged; hout: the statuses
+// to host memory
+hipError_t launch_build_solution(vv_ctx *c, double *x, double *f, bool store, GmresStatus *hout);
 hipError_t launch_mdot32(vv_ctx *c, int col);
 hipError_t launch_maxpy_norm32(vv_ctx *c, int it, int dot_rows = 0);
-hipError_t launch_build_solution32(vv_ctx *c, double *x);  // x (FP64) += V y (FP32 basis)
-hipError_t launch_residual_restart(vv_ctx *c, const double *b, double *y);  // y = b - y (B fields)
-hipError_t launch_norms(vv_ctx *c, const double *x, double *out_dev);       // ||x_b|| of the B fields
+hipError_t launch_build_solution32(vv_ctx *c, double *x, double *f, bool store, GmresStatus *hout);
+hipError_t launch_rsub(vv_ctx *c, const double *b, double *y);   // y = b - y (B fields)
+// ||x_b|| of the B fields (x null: from nb partials already in c->partial) to
+// host[b], and pres[16 b] to host[B + b] when pres is given
+hipError_t launch_norms(vv_ctx *c, const double *x, int nb, const double *pres, double *host);
 hipError_t launch_norm2(vv_ctx *c, const double *x, int64_t n, double *out_dev);
 hipError_t launch_dot(vv_ctx *c, const double *x, const double *y, int64_t n, double *out_dev);
 hipError_t launch_axpy(vv_ctx *c, double alpha, const double *x, double *y, int64_t n);
