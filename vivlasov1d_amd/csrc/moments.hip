@@ -252,6 +252,8 @@ __device__ void line_fft(double2 *buf, int n, int logn, const double2 *__restric
 __device__ __forceinline__ void poi_density(const PoiArgs &a, double (&n)[kMaxNx / PT], double *red)
 {
     const int nx = a.nx, t = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < kMaxNx / PT; ++q) n[q] = 0.0;        // columns past nx count as 0
     if (a.from_part && a.nch > 1 && 2 * nx <= PT) {
         int span = 64;
         while (span < nx) span <<= 1;
@@ -261,7 +263,6 @@ __device__ __forceinline__ void poi_density(const PoiArgs &a, double (&n)[kMaxNx
             for (int ch = g; ch < a.nch; ch += G) s += a.npart[(size_t)ch * nx + i];
         red[t] = s;
         __syncthreads();
-        n[0] = 0.0;
         if (t < nx) {
             double v = red[t];
             for (int q = 1; q < G; ++q) v += red[q * span + t];
@@ -273,7 +274,6 @@ __device__ __forceinline__ void poi_density(const PoiArgs &a, double (&n)[kMaxNx
 #pragma unroll
     for (int q = 0; q < kMaxNx / PT; ++q) {
         const int i = t + q * PT;
-        n[q] = 0.0;
         if (i >= nx) continue;
         if (!a.from_part) {
             n[q] = a.n_in[i];
