@@ -200,20 +200,24 @@ int pc_apply(vv_ctx *c, const double *x, double *y, const int32_t *done, int it,
 {
     const double F = b_field(c), S = b_spec(c);
     const bool pot = c->tb != nullptr;
-    const double *src = x;
-    double *dst = y;
-    if (pot) {
-        VV_CHECK(launch_transpose(c, x, c->tb, false, done), "transpose");
-        src = dst = c->tb;
+    const bool cin = pot && potential_cols(c, x), cout = pot && potential_cols(c, y);
+    if (cin) {
+        VV_PLAUNCH(P_RFFT, F + S, it, launch_rfft_cols(c, x, c->spec, done), "rfft");
+    } else {
+        if (pot) VV_CHECK(launch_transpose(c, x, c->tb, false, done), "transpose");
+        VV_PLAUNCH(P_RFFT, F + S, it, launch_rfft(c, pot ? c->tb : x, c->spec, done), "rfft");
     }
-    VV_PLAUNCH(P_RFFT, F + S, it, launch_rfft(c, src, c->spec, done), "rfft");
     if (tr) {
         VV_CHECK(launch_tridiag_t(c, c->spec, done), "tridiag (transposed)");
     } else {
         VV_PLAUNCH(P_TRI, 2 * S, it, launch_tridiag_k(c, c->spec, done), "tridiag");
     }
-    VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft(c, c->spec, dst, done), "irfft");
-    if (pot) VV_CHECK(launch_transpose(c, c->tb, y, true, done), "transpose");
+    if (cout) {
+        VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft_cols(c, c->spec, y, done), "irfft");
+    } else {
+        VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft(c, c->spec, pot ? c->tb : y, done), "irfft");
+        if (pot) VV_CHECK(launch_transpose(c, c->tb, y, true, done), "transpose");
+    }
     return VV_OK;
 }
 
@@ -269,17 +273,30 @@ int h1_of(vv_ctx *c, const double *g)
 // with h1[g] (x-only) broadcast over the rows.  linear_apply forms
 //   forward:    y = alpha u + beta R {u, H} + gamma R {f_bar, h1[u]}
 //   transposed: y = alpha u + beta {u~, H} + gamma h1[{u~, f_bar}]
+
+// y = alpha u + beta {u~, H} and h1[{u~, f_bar}] into xs_h1 (the coupling's
+// x-only field, not added yet); with uscale the due Hessenberg update goes along
+int transposed_parts(vv_ctx *c, const double *u, const double *uscale, const double *fbar, double *y, double alpha,
+                     double beta)
+{
+    VV_CHECK(launch_bracket_pair(c, u, uscale, fbar, y, alpha, beta, c->T2, c->N), "bracket (transposed)");
+    VV_CHECK(launch_poisson(c, nullptr, nullptr, nullptr, xs_h1(c), nullptr, 1, c->T2, nullptr, 16,
+                            band_rows(c->p.nv), c->N), "poisson");
+    return VV_OK;
+}
+
 int linear_apply(vv_ctx *c, const double *u, const double *uscale, const double *fbar, double *y, double alpha,
                  double beta, double gamma, bool transposed)
 {
     if (int r = ensure_linear(c)) return r;
     const double *h1 = xs_h1(c);
     if (transposed) {
-        VV_CHECK(launch_bracket_t(c, u, uscale, nullptr, nullptr, y, alpha, beta), "bracket (transposed)");
         if (fbar && gamma != 0.0) {
-            VV_CHECK(launch_bracket_t(c, u, uscale, fbar, nullptr, c->T2, 0.0, 1.0), "coupling bracket");
-            if (int r = h1_of(c, c->T2)) return r;
+            if (int r = transposed_parts(c, u, uscale, fbar, y, alpha, beta)) return r;
             VV_CHECK(launch_xadd(c, y, h1, gamma), "coupling");
+        } else {
+            VV_CHECK(launch_update(c), "Hessenberg update");
+            VV_CHECK(launch_bracket_t(c, u, uscale, nullptr, nullptr, y, alpha, beta), "bracket (transposed)");
         }
     } else {
         if (uscale) return fail(c, VV_ERR_INVALID, "internal: scaled input of the forward linearisation");
@@ -466,6 +483,12 @@ int apply_pc(vv_ctx *c, const double *x, double *y, const int32_t *done)
     return precond(c, x, y, done);
 }
 
+// whether the rFFT takes an x-only field along (not the direct DFT of long odd lengths)
+bool add_fused(const vv_ctx *c)
+{
+    return c->tb == nullptr && ((c->fft_n & (c->fft_n - 1)) == 0 || c->dft.n > 0);
+}
+
 // one Arnoldi step of GMRES on P^-1 J: V_{it+1} from V_it (every instance)
 int arnoldi_step(vv_ctx *c, int it)
 {
@@ -477,12 +500,34 @@ int arnoldi_step(vv_ctx *c, int it)
     // the fused J v + rFFT takes the previous step's Hessenberg update along;
     // every other first kernel of a step waits for it
     const bool fuse_jv = fwd_fused(c);
-    if (!fuse_jv) VV_CHECK(launch_update(c), "Hessenberg update");
+    if (!fuse_jv && c->op_mode == 0) VV_CHECK(launch_update(c), "Hessenberg update");
     // the irFFT and the CGS dots of w in one launch: the slice kernel, or row blocks
     // (not at the strip kernel's lengths, where fused and separate launches are
     // bit-identical)
-    const int rows = c->op_mode == 0 ? irfft_mdot_rows(c, false) : 0;
-    const bool blocks = c->op_mode == 0 && !rows && rows_apply(c) && !jac_rfft_rows(c);
+    const bool kinetic = c->p.precond == VV_PRECOND_TENSOR_KINETIC;
+    const int rows = kinetic ? irfft_mdot_rows(c, false) : 0;
+    const bool blocks = kinetic && !rows && rows_apply(c) && !jac_rfft_rows(c);
+    // w and its dots from the spectrum, then the CGS update
+    auto finish = [&]() -> int {
+        if (rows) {
+            VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_irfft_mdot(c, c->spec, it, done), "irfft_mdot");
+        } else if (blocks) {
+            VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_row_inv(c, c->spec, it, done), "row irfft + dots");
+        } else {
+            VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft(c, c->spec, w, done), "irfft");
+            VV_PLAUNCH(P_MDOT, F * (it + 2), it, launch_mdot(c, it), "mdot");
+        }
+        VV_PLAUNCH(P_MAXPY, F * (it + 3), it,
+                   launch_maxpy_norm(c, it, rows ? rows : (blocks ? row_inv_blocks(c) : 0)), "maxpy_norm");
+        return VV_OK;
+    };
+    if (c->op_mode != 0 && kinetic && c->op_fbar != nullptr && add_fused(c)) {
+        // P^-T A^T v: the coupling's x-only field is added as the rows are transformed
+        if (int r = transposed_parts(c, v, &c->gs->scale[it], c->op_fbar, c->X, c->ht_inv, -0.5)) return r;
+        VV_PLAUNCH(P_RFFT, F + S, it, launch_rfft(c, c->X, c->spec, done, xs_h1(c), 0.5), "rfft");
+        VV_CHECK(launch_tridiag_t(c, c->spec, done), "tridiag (transposed)");
+        return finish();
+    }
     if (c->op_mode != 0) {
         if (int r = linear_apply(c, v, &c->gs->scale[it], c->op_fbar, c->X, c->ht_inv, -0.5, 0.5, true)) return r;
         if (int r = apply_pc(c, c->X, w, done)) return r;
@@ -500,17 +545,7 @@ int arnoldi_step(vv_ctx *c, int it)
             VV_PLAUNCH(P_RFFT, F + S, it, launch_rfft(c, c->X, c->spec, done), "rfft");
         }
         VV_PLAUNCH(P_TRI, 2 * S, it, launch_tridiag_k(c, c->spec, done), "tridiag");
-        if (rows) {
-            VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_irfft_mdot(c, c->spec, it, done), "irfft_mdot");
-        } else if (blocks) {
-            VV_PLAUNCH(P_IRFFT_MDOT, S + F * (it + 2), it, launch_row_inv(c, c->spec, it, done), "row irfft + dots");
-        } else {
-            VV_PLAUNCH(P_IRFFT, S + F, it, launch_irfft(c, c->spec, w, done), "irfft");
-            VV_PLAUNCH(P_MDOT, F * (it + 2), it, launch_mdot(c, it), "mdot");
-        }
-        VV_PLAUNCH(P_MAXPY, F * (it + 3), it,
-                   launch_maxpy_norm(c, it, rows ? rows : (blocks ? row_inv_blocks(c) : 0)), "maxpy_norm");
-        return VV_OK;
+        return finish();
     } else {
         VV_PLAUNCH(P_JAC, 2 * F, it, launch_jacobian(c, v, &c->gs->scale[it], c->X), "jacobian");
         if (int r = diss_jacobian(c, v, &c->gs->scale[it], c->X, done)) return r;
@@ -541,16 +576,20 @@ int pc_apply32(vv_ctx *c, const float *x, float *y, const int32_t *done, int it)
     const double F = 4.0 * (double)c->N * c->B, S = 0.5 * b_spec(c);
     const bool pot = c->tb != nullptr;
     float *tb = reinterpret_cast<float *>(c->tb);
-    const float *src = x;
-    float *dst = y;
-    if (pot) {
-        VV_CHECK(launch_transpose32(c, x, tb, false, done), "transpose32");
-        src = dst = tb;
+    const bool cin = pot && potential_cols32(c, x), cout = pot && potential_cols32(c, y);
+    if (cin) {
+        VV_PLAUNCH(P_RFFT32, F + S, it, launch_rfft_cols32(c, x, spec, done), "rfft32");
+    } else {
+        if (pot) VV_CHECK(launch_transpose32(c, x, tb, false, done), "transpose32");
+        VV_PLAUNCH(P_RFFT32, F + S, it, launch_rfft32(c, pot ? tb : x, spec, done), "rfft32");
     }
-    VV_PLAUNCH(P_RFFT32, F + S, it, launch_rfft32(c, src, spec, done), "rfft32");
     VV_PLAUNCH(P_TRI32, 2 * S, it, launch_tridiag32(c, spec, done), "tridiag32");
-    VV_PLAUNCH(P_IRFFT32, S + F, it, launch_irfft32(c, spec, dst, done), "irfft32");
-    if (pot) VV_CHECK(launch_transpose32(c, tb, y, true, done), "transpose32");
+    if (cout) {
+        VV_PLAUNCH(P_IRFFT32, S + F, it, launch_irfft_cols32(c, spec, y, done), "irfft32");
+    } else {
+        VV_PLAUNCH(P_IRFFT32, S + F, it, launch_irfft32(c, spec, pot ? tb : y, done), "irfft32");
+        if (pot) VV_CHECK(launch_transpose32(c, tb, y, true, done), "transpose32");
+    }
     return VV_OK;
 }
 
@@ -1059,20 +1098,20 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(dalloc(c, &c->dscalar, ds_count(B)), "alloc scalars");
     VV_CCHECK(dalloc(c, &c->npart, (size_t)64 * nx * Bz), "alloc density partials");
     VV_CCHECK(dalloc(c, &c->gs, Bz), "alloc gmres state");
-    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_status), Bz * sizeof(GmresStatus)),
-              "pinned status");
-    VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_status_dev), c->host_status, 0),
-              "pinned status device address");
-    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_poll), 2 * Bz * sizeof(uint32_t)), "pinned reports");
-    VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_poll_dev), c->host_poll, 0),
-              "pinned reports device address");
-    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_scalars), hs_count(B) * sizeof(double)),
-              "pinned scalars");
-    VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_scalars_dev), c->host_scalars, 0),
-              "pinned scalars device address");
-    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&c->host_active), Bz * sizeof(int32_t)), "pinned mask");
-    VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&c->host_active_dev), c->host_active, 0),
-              "pinned mask device address");
+    // one pinned block: statuses | scalars | reports | instance mask
+    const size_t pin_sc = Bz * sizeof(GmresStatus), pin_rp = pin_sc + hs_count(B) * sizeof(double);
+    const size_t pin_ac = pin_rp + 2 * Bz * sizeof(uint32_t), pin_n = pin_ac + Bz * sizeof(int32_t);
+    char *pin = nullptr, *pin_dev = nullptr;
+    VV_CCHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), pin_n), "pinned block");
+    c->host_status = reinterpret_cast<GmresStatus *>(pin);
+    VV_CCHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&pin_dev), pin, 0), "pinned block device address");
+    c->host_status_dev = reinterpret_cast<GmresStatus *>(pin_dev);
+    c->host_scalars = reinterpret_cast<double *>(pin + pin_sc);
+    c->host_scalars_dev = reinterpret_cast<double *>(pin_dev + pin_sc);
+    c->host_poll = reinterpret_cast<uint32_t *>(pin + pin_rp);
+    c->host_poll_dev = reinterpret_cast<uint32_t *>(pin_dev + pin_rp);
+    c->host_active = reinterpret_cast<int32_t *>(pin + pin_ac);
+    c->host_active_dev = reinterpret_cast<int32_t *>(pin_dev + pin_ac);
     std::memset(c->host_poll, 0, 2 * Bz * sizeof(uint32_t));
     VV_CCHECK(hipMemset(c->gs, 0, Bz * sizeof(GmresState)), "zero gmres state");
     VV_CCHECK(hipMemset(c->partial, 0, (size_t)c->part_stride * Bz * sizeof(double)), "zero partials");
@@ -1191,10 +1230,7 @@ int vv_ctx_destroy(vv_ctx *c)
                     c->db2,    c->ex,     c->w64,     c->d64,   c->lu64,   c->lu32};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
-    if (c->host_status) (void)hipHostFree(c->host_status);
-    if (c->host_scalars) (void)hipHostFree(c->host_scalars);
-    if (c->host_active) (void)hipHostFree(c->host_active);
-    if (c->host_poll) (void)hipHostFree(c->host_poll);
+    if (c->host_status) (void)hipHostFree(c->host_status);     // the whole pinned block
     Prof *pr = prof_of(c);
     if (pr) {
         for (auto &r : pr->recs) {

@@ -21,6 +21,7 @@
 // window.
 
 #include "arakawa.h"
+#include "gmres_dev.h"
 #include "vv1d_internal.h"
 
 namespace vv {
@@ -246,6 +247,119 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     }
 }
 
+// The transposed linearisation's two brackets in one launch: with u~ = u (times
+// its scale) on rows 2..nv-3 and 0 elsewhere,
+//   y = alpha u + factor {u~, H_ave} on all rows,  csum = sum_j {u~, g}_ij
+// by 16-row bands (tile row t at csum[t nx + i], instances cstride apart): the
+// coupling term needs only the column sums of its bracket (g = f_bar in a.h2d),
+// so that field is neither stored nor read back.  u~ is staged once for both;
+// three 20 x 68 tiles (33 KB of LDS).  hs: the previous step's Hessenberg
+// update or the cycle's start, as in the fused J u + rFFT.  At 256 x 512 it
+// replaces two bracket launches (5.2 us each), the density (3.7 us) and the
+// update (3.6 us).
+template <int KIND>
+__global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, HessArgs hs, double *csum,
+                                                          int64_t cstride)
+{
+    const int extra = hs.nb > 0 ? 1 : 0;
+    if (extra && blockIdx.x == 0) {
+        hess_update(hs);
+        return;
+    }
+    const int b = blockIdx.y;
+    __shared__ double sF[HY][HX], sH[HY][HX], sG[HY][HX];
+    __shared__ double sX[4][HX], sV[HY];
+    __shared__ double red[kGdNW + 1];
+    const int nx = a.nx, nv = a.nv;
+    const BrTile tile = br_tile((int)blockIdx.x - extra, nx, nv);
+    const size_t fo = (size_t)b * a.N, xo = (size_t)b * nx;
+    const double *__restrict__ fin = a.f + fo;
+    const double *__restrict__ gin = a.h2d + fo;
+    const int32_t dflag = extra ? hess_skip(hs)
+                          : a.done != nullptr
+                              ? *reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(a.done) + b * a.gstride)
+                              : 0;
+    if (gridDim.y > 1 && dflag) return;
+    const double nshare = extra ? norm_share(hs.part + b * hs.pstride, hs.nb) : 0.0;
+    double us = a.uscale != nullptr && !extra
+                    ? *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a.uscale) + b * a.gstride)
+                    : 1.0;
+    double xf[4] = {0.0, 0.0, 0.0, 0.0}, vf = 0.0;
+    if (threadIdx.x < HX) {
+        const size_t gi = xo + br_halo_column(tile, (int)threadIdx.x, nx);
+        xf[0] = a.h1p[gi];
+        xf[1] = a.h1h[gi];
+        xf[2] = a.h2p[gi];
+        xf[3] = a.h2h[gi];
+    } else if (threadIdx.x < HX + HY) {
+        const int gj = br_halo_row(tile, (int)threadIdx.x - HX, nv);
+        if (gj >= 0) vf = a.h0[gj];
+    }
+    constexpr int NQ = (HY * HX + NT - 1) / NT;
+    double fa[NQ], ga[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int idx = threadIdx.x + q * NT;
+        fa[q] = ga[q] = 0.0;
+        if (idx < HY * HX) {
+            const int r = idx / HX;
+            const int64_t o = br_halo_offset(tile, r, idx - r * HX, nx, nv);
+            if (o >= 0) {
+                fa[q] = fin[o];
+                ga[q] = gin[o];
+            }
+        }
+    }
+    if (dflag) return;                 // uniform over the block, before any barrier
+    if (extra) us = scale_of(block_sum_all(nshare, red));
+    if (threadIdx.x < HX) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) sX[m][threadIdx.x] = xf[m];
+    } else if (threadIdx.x < HX + HY) {
+        sV[threadIdx.x - HX] = vf;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int idx = threadIdx.x + q * NT;
+        if (idx < HY * HX) {
+            const int r = idx / HX, c = idx - r * HX;
+            const int gj = br_halo_row(tile, r, nv);
+            sF[r][c] = (gj >= 2 && gj < nv - 2) ? fa[q] * us : 0.0;
+            sH[r][c] = gj >= 0 ? compose_have(sV[r], sX[0][c], sX[1][c], sX[2][c], sX[3][c]) : 0.0;
+            sG[r][c] = ga[q];
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = tile.i0 + lane, cx = lane + 2, rr0 = wave * ROWS_PER_WAVE;
+    const double af1 = a.inst[b].af1, af2 = a.inst[b].af2;
+    const TileRd<double, HX> rF{&sF[0][0]}, rH{&sH[0][0]}, rG{&sG[0][0]};
+    double *__restrict__ yout = a.y + fo;
+    double cs = 0.0;
+    ArakawaWin<double> wh, wg;
+    wh.load(rF, rH, rr0 + 2, cx);
+    wg.load(rF, rG, rr0 + 2, cx);
+#pragma unroll
+    for (int q = 0; q < ROWS_PER_WAVE; ++q) {
+        const int j = tile.j0 + rr0 + q;
+        if (j < nv && i < nx) {
+            const size_t o = (size_t)j * nx + i;
+            yout[o] = arakawa_add<KIND>(wh, a.alpha * (fin[o] * us), a.factor, af1, af2);
+            cs += arakawa_add<KIND>(wg, 0.0, 1.0, af1, af2);
+        }
+        if (q + 1 < ROWS_PER_WAVE) {
+            wh.advance(rF, rH, rr0 + q + 3, cx);
+            wg.advance(rF, rG, rr0 + q + 3, cx);
+        }
+    }
+    __syncthreads();                   // the tiles are read: sX takes the waves' sums
+    sX[wave][lane] = cs;
+    __syncthreads();
+    if (wave == 0 && i < nx)
+        csum[b * cstride + (size_t)(tile.j0 / TY) * nx + i] = ((sX[0][lane] + sX[1][lane]) + sX[2][lane]) + sX[3][lane];
+}
+
 template <int MODE, typename T>
 hipError_t launch_mode(vv_ctx *c, BrArgs<T> a)
 {
@@ -331,6 +445,30 @@ hipError_t launch_bracket_t(vv_ctx *c, const double *u, const double *uscale, co
     a.factor = factor;
     a.done = uscale != nullptr ? &c->gs->st.done : nullptr;
     return launch_mode<MODE_TRANSPOSED>(c, a);
+}
+
+int band_rows(int nv) { return (nv + TY - 1) / TY; }
+
+hipError_t launch_bracket_pair(vv_ctx *c, const double *u, const double *uscale, const double *g, double *y,
+                               double alpha, double factor, double *csum, int64_t cstride)
+{
+    BrArgs<double> a = base_args<double>(c);
+    a.f = u;
+    a.uscale = uscale;
+    a.h2d = g;
+    a.y = y;
+    a.alpha = alpha;
+    a.factor = factor;
+    a.done = uscale != nullptr ? &c->gs->st.done : nullptr;
+    HessArgs hs{};
+    if (uscale != nullptr) hs = take_update(c);
+    const dim3 grid(br_tiles(c->p.nx, c->p.nv) + (hs.nb > 0 ? 1 : 0), c->B), block(NT);
+    switch (c->p.bracket) {
+    case VV_BRACKET_J1: launch_timed(c, bracket_pair_kernel<VV_BRACKET_J1>, grid, block, 0, a, hs, csum, cstride); break;
+    case VV_BRACKET_J2: launch_timed(c, bracket_pair_kernel<VV_BRACKET_J2>, grid, block, 0, a, hs, csum, cstride); break;
+    default: launch_timed(c, bracket_pair_kernel<VV_BRACKET_J4>, grid, block, 0, a, hs, csum, cstride); break;
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_bracket_gen(vv_ctx *c, const double *x, const double *h2d, const double *hxv, double *y,

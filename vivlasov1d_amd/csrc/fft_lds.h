@@ -26,6 +26,7 @@ template <typename C> __device__ __forceinline__ C cmul(C a, C b)
     return cmk<C>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 template <typename C> __device__ __forceinline__ C cneg(C a) { return cmk<C>(-a.x, -a.y); }
+template <typename C> __device__ __forceinline__ C cconj(C a) { return cmk<C>(a.x, -a.y); }
 // 1/d for the complex divisions of the tridiagonal solve: the hardware
 // reciprocal estimate refined by two Newton steps r <- r (2 - d r) instead of
 // the IEEE division sequence.  The dependent chain of the Thomas sweep is
@@ -344,6 +345,8 @@ struct FftArgs {
     int64_t N, S, gstride;
     const cx_t<T> *tw;
     const int32_t *done;
+    const T *add;               // rfft: x-only field added to every row, gamma add (null: none), nx per instance
+    T gamma;
 };
 
 __device__ __forceinline__ int32_t cycle_done(const int32_t *done, int64_t gstride)

@@ -132,6 +132,7 @@ __device__ double block_sum_big(double v, double *red)
 struct PoiArgs {
     int nx, laplace, from_part;
     int nch, logn;         // density partials per column; log2 nx (FFT form)
+    int64_t npstride;      // instance stride of npart
     double hv, charge;
     const InstConst *inst;
     const double *npart;   // density partials (from_part = 1)
@@ -161,7 +162,7 @@ __device__ __forceinline__ double lap(const X &x, int i, int nx, int laplace, do
 __device__ __forceinline__ void poi_instance(PoiArgs &a)
 {
     const size_t b = blockIdx.y, nx = a.nx;
-    if (a.npart) a.npart += b * DCH * nx;
+    if (a.npart) a.npart += b * a.npstride;
     if (a.n_in) a.n_in += b * nx;
     if (a.pinv) a.pinv += b * nx;
     if (a.plam) a.plam += b * nx;
@@ -693,10 +694,12 @@ hipError_t launch_velocity_moments(vv_ctx *c, const double *f, double *u, double
 }
 
 hipError_t launch_poisson(vv_ctx *c, const double *n_in, double *n_out, double *phi, double *h1, double *pres,
-                          int from_part, const double *npart, double *work, int pres_stride)
+                          int from_part, const double *npart, double *work, int pres_stride, int nch,
+                          int64_t npstride)
 {
     const int nx = c->p.nx;
-    PoiArgs a{nx, c->p.laplace, from_part, column_chunks(c->p.nv), 0, c->p.hv, c->p.charge, c->inst,
+    PoiArgs a{nx, c->p.laplace, from_part, nch > 0 ? nch : column_chunks(c->p.nv), 0,
+              nch > 0 ? npstride : (int64_t)DCH * nx, c->p.hv, c->p.charge, c->inst,
               from_part ? (npart != nullptr ? npart : c->npart) : nullptr, n_in, c->pinv, c->plam, c->twiddle,
               work != nullptr ? work : c->pwork, n_out, phi, h1, pres, pres_stride};
     if (c->plam != nullptr) {

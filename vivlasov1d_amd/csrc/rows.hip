@@ -242,7 +242,8 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
         const uint32_t mnx = 0xffffffffu / (uint32_t)nx + 1;
         for (int idx = t; idx < RW * nx; idx += NT) {
             const int r = div_by(idx, mnx), i = idx - r * nx;
-            const T v = j0 + r < nv ? u[(size_t)(j0 + r) * nx + i] : T(0);
+            T v = j0 + r < nv ? u[(size_t)(j0 + r) * nx + i] : T(0);
+            if (a.add != nullptr && j0 + r < nv) v += a.gamma * a.add[xo + i];
             T *z = reinterpret_cast<T *>(buf + (r >> 1) * nx + i);
             z[r & 1] = v;
         }
@@ -625,13 +626,14 @@ void fwd_launch(vv_ctx *c, const FftArgs<T> &a, const RowGeom &g, const RowFwd<T
 }
 
 template <int MODE, typename T>
-hipError_t row_fwd_t(vv_ctx *c, RowFwd<T> p, cx_t<T> *spec, const int32_t *done)
+hipError_t row_fwd_t(vv_ctx *c, RowFwd<T> p, cx_t<T> *spec, const int32_t *done, const T *add = nullptr,
+                     T gamma = T(0))
 {
     int R;
     size_t lds;
     const RowGeom g = row_geom<T>(c, MODE, &R, &lds);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, g.RW, c->N, spec_stride(c), (int64_t)sizeof(GmresState),
-                 twiddles<T>(c), done};
+                 twiddles<T>(c), done, add, gamma};
     HessArgs hs{};
     if (MODE == F_JAC) hs = take_update(c);
     const dim3 grid((a.nv + g.RW - 1) / g.RW + (hs.nb > 0 ? 1 : 0), c->B);
@@ -738,11 +740,12 @@ hipError_t launch_row_res(vv_ctx *c, const double *f, const double *fh, double2 
 }
 
 // rows as they are (lengths with a DFT plan); y of the inverse 16-byte aligned
-hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done)
+hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add,
+                           double gamma)
 {
     RowFwd<double> p{};
     p.u = x;
-    return row_fwd_t<F_PLAIN, double>(c, p, spec, done);
+    return row_fwd_t<F_PLAIN, double>(c, p, spec, done, add, gamma);
 }
 
 hipError_t launch_row_rfft32(vv_ctx *c, const float *x, float2 *spec, const int32_t *done)

@@ -73,6 +73,15 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
             xr[q][m] = r0 ? x0[m * nq] : T(0);
             xi[q][m] = r1 ? x0[nx + m * nq] : T(0);
         }
+        if (a.add != nullptr) {
+            const T *ad = a.add + (size_t)blockIdx.y * nx + j;
+#pragma unroll
+            for (int m = 0; m < RAD; ++m) {
+                const T w = a.gamma * ad[m * nq];
+                xr[q][m] += r0 ? w : T(0);
+                xi[q][m] += r1 ? w : T(0);
+            }
+        }
     }
     FftTw<false, C> pt;
     if (V == VP8) pt.load(a.tw);
@@ -294,6 +303,66 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 4 ? 3 :
     jac_rfft_body<KIND, R, NS>(a, jr, hs, u, spec);
 }
 
+// The potential form's rFFT along v straight from the field (nv rows of nx):
+// a workgroup takes R consecutive x (R, nx even), whose lines run down the
+// columns.  The packed complex line p, (x = i0 + 2p, i0 + 2p + 1), is 16 bytes
+// a row of the field as it lies there, so it is loaded as such; the lines of a
+// 128-byte segment belong to neighbouring workgroups of one XCD, which find it
+// in its L2.  The spectrum goes out x-contiguous per mode, as rfft_kernel's.
+// With the inverse below it replaces a transpose before and after (4.0 us each
+// and a launch at 512 x 1024).
+template <typename T, int V>
+__global__ __launch_bounds__(NT) void rfft_cols_kernel(FftArgs<T> a, const T *__restrict__ x,
+                                                       cx_t<T> *__restrict__ spec)
+{
+    using C = cx_t<T>;
+    const int32_t dflag = cycle_done(a.done, a.gstride);
+    if (gridDim.y > 1 && dflag) return;   // batched: a finished instance skips its loads
+    x += blockIdx.y * a.N;
+    spec += blockIdx.y * a.S;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    C *buf = reinterpret_cast<C *>(lds_raw);
+    const int n = a.nx, nc = a.nv, npair = a.rows >> 1;      // line length, columns, lines
+    const int i0 = xcd_tile(blockIdx.x, gridDim.x) * a.rows;
+    const int total = n * npair;
+    constexpr int QL = MAXE / NT;
+    C z[QL];
+#pragma unroll
+    for (int q = 0; q < QL; ++q) {
+        const int idx = threadIdx.x + q * NT;
+        const int m = idx / npair, i = i0 + 2 * (idx - m * npair);
+        const bool ok = idx < total && i < nc;
+        const C v = *reinterpret_cast<const C *>(x + (ok ? (size_t)m * nc + i : 0));
+        z[q] = ok ? v : cmk<C>(T(0), T(0));
+    }
+    FftTw<false, C> pt;
+    if (V == VP8) pt.load(a.tw);
+    const C *tw = tw_table<V == VTWL>(a.tw, buf + (size_t)npair * n, n);
+    if (dflag) return;                 // uniform over the block, before any barrier
+#pragma unroll
+    for (int q = 0; q < QL; ++q) {
+        const int idx = threadIdx.x + q * NT;
+        const int m = idx / npair;
+        if (idx < total) buf[(idx - m * npair) * n + m] = z[q];
+    }
+    __syncthreads();
+    lds_fft<false, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, LdsSink<C>{buf});
+    store_real_spectrum(buf, n, a.rows, i0, nc, spec);
+}
+
+// the same columns back: line b of the workgroup to x = i0 + 2b, i0 + 2b + 1
+template <typename T>
+struct IrfftColSink {
+    T *y;
+    int i0, n, logn, nc;
+    __device__ __forceinline__ void operator()(int pos, cx_t<T> z) const
+    {
+        const int b = pos >> logn, m = pos & (n - 1), i = i0 + 2 * b;
+        const T inv_n = T(1) / (T)n;
+        if (i < nc) *reinterpret_cast<cx_t<T> *>(y + (size_t)m * nc + i) = cmk<cx_t<T>>(z.x * inv_n, z.y * inv_n);
+    }
+};
+
 // Real rows 2b, 2b+1 of an irFFT workgroup from its complex transform b
 // (backward-normalised by 1/nx, exact: nx is a power of two).
 template <typename T>
@@ -310,7 +379,7 @@ struct IrfftSink {
     }
 };
 
-template <typename T, int V>
+template <typename T, int V, bool COLS>
 __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *__restrict__ spec, T *__restrict__ y)
 {
     using C = cx_t<T>;
@@ -358,7 +427,8 @@ __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *
     }
     __syncthreads();
     // the last stage's outputs (natural order) go straight to the output rows
-    lds_fft<true, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, IrfftSink<T>{y, j0, nx, a.logn, a.nv});
+    if constexpr (COLS) lds_fft<true, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, IrfftColSink<T>{y, j0, nx, a.logn, a.nv});
+    else lds_fft<true, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, IrfftSink<T>{y, j0, nx, a.logn, a.nv});
 }
 
 // Real rows of the irFFT left in the workgroup's LDS buffer itself, natural
@@ -783,6 +853,128 @@ __global__ __launch_bounds__(NT) void tridiag_kernel(TriArgs a, cx_t<T> *__restr
     for (int j = threadIdx.x; j < a.nv; j += NT) S[j] = sd[j + j / M];
 }
 
+// The same solve for systems of up to 64 M rows (M <= 8), a wavefront per mode
+// and four modes a workgroup: lane c owns the chunk of M rows, and the reduced
+// system of the 64 chunk-last unknowns is solved by parallel cyclic reduction
+// on shuffles, six steps without a barrier (the workgroup form: eight steps of
+// two barriers and twelve LDS accesses at 512 rows, 12.0 us for the 513 modes
+// of 512 x 1024).  A lane past the end holds identity rows; the couplings of a
+// lane without a neighbour at the step's distance are zero by then, so no step
+// needs a branch.
+template <typename C> __device__ __forceinline__ C shfl_up_cx(C v, int off)
+{
+    return cmk<C>(__shfl_up(v.x, off), __shfl_up(v.y, off));
+}
+template <typename C> __device__ __forceinline__ C shfl_down_cx(C v, int off)
+{
+    return cmk<C>(__shfl_down(v.x, off), __shfl_down(v.y, off));
+}
+
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int M, typename T, bool TR>
+__global__ __launch_bounds__(NT) void tridiag_wave_kernel(TriArgs a, int nmodes, cx_t<T> *__restrict__ spec)
+{
+    using C = cx_t<T>;
+    const int32_t dflag = cycle_done(a.done, a.gstride);
+    if (dflag) return;                    // uniform over the launch's instance
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int k = blockIdx.x * (NT / 64) + wave;
+    if (k >= nmodes) return;              // whole wavefronts; no barrier below
+    a.gm += blockIdx.y * a.cstride;
+    a.g0 += blockIdx.y * a.cstride;
+    a.gp += blockIdx.y * a.cstride;
+    const double af = a.inst[blockIdx.y].afpc;
+    __shared__ C lds[NT / 64][64 * (M + 1)];
+    C *sd = lds[wave];                    // chunk c at c (M + 1)
+    const double2 e = a.eigen[k];
+    C *S = spec + blockIdx.y * a.S + (size_t)k * a.nv;
+    const C zero = cmk<C>(T(0), T(0));
+    double lo[M], mid[M], hi[M];
+    {
+        C v[M];
+#pragma unroll
+        for (int q = 0; q < M; ++q) v[q] = load_or_zero(S, lane + 64 * q, lane + 64 * q < a.nv);
+#pragma unroll
+        for (int q = 0; q < M; ++q) tri_load<TR>(a, lane * M + q, lo[q], mid[q], hi[q]);
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            const int j = lane + 64 * q;
+            sd[j + j / M] = v[q];
+        }
+    }
+    wave_lds_fence();
+    const int ls = lane * (M + 1);
+    C Am[M], Cm[M], Dm[M], ae, be, ce;
+    {
+        // forward sweep: y_j + c'_j y_{j+1} = d'_j - a'_j y_{s-1}
+        C aj, bj, cj;
+        tri_row<TR>(a, af, e, lane * M, lo[0], mid[0], hi[0], aj, bj, cj);
+        C r = crecip(bj);
+        Cm[0] = cmul(cj, r);
+        Dm[0] = cmul(sd[ls], r);
+        Am[0] = cmul(aj, r);
+#pragma unroll
+        for (int q = 1; q < M; ++q) {
+            tri_row<TR>(a, af, e, lane * M + q, lo[q], mid[q], hi[q], aj, bj, cj);
+            if (q < M - 1) {
+                r = crecip(csub(bj, cmul(aj, Cm[q - 1])));
+                Cm[q] = cmul(cj, r);
+                Dm[q] = cmul(csub(sd[ls + q], cmul(aj, Dm[q - 1])), r);
+                Am[q] = cneg(cmul(cmul(aj, Am[q - 1]), r));
+            } else {
+                ae = aj;
+                be = bj;
+                ce = cj;
+            }
+        }
+        // backward sweep over the chunk but its last row: y_j = D_j - A_j y_{s-1} - C_j y_e
+#pragma unroll
+        for (int q = M - 3; q >= 0; --q) {
+            Dm[q] = csub(Dm[q], cmul(Cm[q], Dm[q + 1]));
+            Am[q] = csub(Am[q], cmul(Cm[q], Am[q + 1]));
+            Cm[q] = cneg(cmul(Cm[q], Cm[q + 1]));
+        }
+    }
+    // reduced equation of the chunk in the chunk-last unknowns E:
+    //   al E_{c-1} + bt E_c + gm E_{c+1} = dl  (lane 63's next is its own, times ce = 0)
+    const C na = shfl_down_cx(Am[0], 1), nc = shfl_down_cx(Cm[0], 1), nd = shfl_down_cx(Dm[0], 1);
+    if (lane == 63) ce = zero;
+    C al = cneg(cmul(ae, Am[M - 2]));
+    C bt = csub(csub(be, cmul(ae, Cm[M - 2])), cmul(ce, na));
+    C gm = cneg(cmul(ce, nc));
+    C dl = csub(csub(sd[ls + M - 1], cmul(ae, Dm[M - 2])), cmul(ce, nd));
+#pragma unroll 1
+    for (int st = 1; st < 64; st <<= 1) {
+        const C ri = crecip(bt);
+        const C k1 = cmul(al, shfl_up_cx(ri, st)), k2 = cmul(gm, shfl_down_cx(ri, st));
+        const C ua = shfl_up_cx(al, st), ug = shfl_up_cx(gm, st), ud = shfl_up_cx(dl, st);
+        const C da = shfl_down_cx(al, st), dg = shfl_down_cx(gm, st), dd = shfl_down_cx(dl, st);
+        bt = csub(csub(bt, cmul(ug, k1)), cmul(da, k2));
+        dl = csub(csub(dl, cmul(ud, k1)), cmul(dd, k2));
+        al = cneg(cmul(ua, k1));
+        gm = cneg(cmul(dg, k2));
+        if (lane < 2 * st) al = zero;
+        if (lane + 2 * st > 63) gm = zero;
+    }
+    const C E = cdiv(dl, bt);             // y at the chunk's last row
+    C Ep = shfl_up_cx(E, 1);
+    if (lane == 0) Ep = zero;
+#pragma unroll
+    for (int q = 0; q < M - 1; ++q) sd[ls + q] = csub(csub(Dm[q], cmul(Am[q], Ep)), cmul(Cm[q], E));
+    sd[ls + M - 1] = E;
+    wave_lds_fence();
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        const int j = lane + 64 * q;
+        if (j < a.nv) S[j] = sd[j + j / M];
+    }
+}
+
 // ---- kinetic solve with precomputed pivots ---------------------------------
 // The kinetic T_k do not change during a run, so their LU factors are formed
 // once per context (KineticFast.pyx:88-90 factors once with zgbtrf as well):
@@ -822,22 +1014,17 @@ __global__ __launch_bounds__(NT) void tridiag_factor_kernel(TriArgs a, int nmode
     for (int j = a.nv; j < L; ++j) R[(j % M) * NT + j / M] = cmk<cx_t<T>>(T(0), T(0));
 }
 
-template <typename C> __device__ __forceinline__ C shfl_up_cx(C v, int off)
-{
-    return cmk<C>(__shfl_up(v.x, off), __shfl_up(v.y, off));
-}
-template <typename C> __device__ __forceinline__ C shfl_down_cx(C v, int off)
-{
-    return cmk<C>(__shfl_down(v.x, off), __shfl_down(v.y, off));
-}
-
 // One workgroup per mode (blockIdx.x) and instance (blockIdx.y); thread t
 // owns the chunk of M rows [t M, t M + M).  The spectrum row and its pivots
 // are staged in LDS (coalesced loads).  Across chunks the recurrences are
 // affine maps y_out = A + B y_in, composed by a scan over the wavefront's
 // lanes (shuffles) and over the 4 wavefronts (one LDS exchange), first
 // forward, then backward; no thread waits on a division.
-template <int M, typename T>
+// TR: T_k^H x = d from the same pivots, U^H y = d then L^H x = y:
+//   y_j = conj(rp_j) (d_j - conj(c_{j-1}) y_{j-1}),  x_j = y_j - conj(a_{j+1} rp_j) x_{j+1}
+// (cyclic reduction with divisions took 7.7 us at 256 x 512, the forward solve
+// 5.5).
+template <int M, typename T, bool TR>
 __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T> *__restrict__ rp,
                                                         cx_t<T> *__restrict__ spec)
 {
@@ -885,12 +1072,37 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
         tri_load<false>(a, s + q, lo, mid, hi);
         tri_row<false>(a, af, e, s + q, lo, mid, hi, av[q], bj, cv[q]);
     }
+    C cprev = zero, anext = zero;                 // TR: c of row s - 1, a of row s + M
+    if constexpr (TR) {
+        double lo, mid, hi;
+        C u, v;
+        if (s > 0) {
+            tri_load<false>(a, s - 1, lo, mid, hi);
+            tri_row<false>(a, af, e, s - 1, lo, mid, hi, u, v, cprev);
+        }
+        tri_load<false>(a, s + M, lo, mid, hi);
+        tri_row<false>(a, af, e, s + M, lo, mid, hi, anext, u, v);
+    }
+    // the recurrences' coefficients: y_j = w_j d_j - m_j y_{j-1} (w = 1 but for TR),
+    // x_j = z_j y_j - n_j x_{j+1} (z = 1 for TR)
+    auto mcoef = [&](int q) {
+        if constexpr (TR) return cmul(cconj(rpv[q]), cconj(q > 0 ? cv[q > 0 ? q - 1 : 0] : cprev));
+        else return cmul(av[q], q > 0 ? rpv[q > 0 ? q - 1 : 0] : rprev);
+    };
+    auto ncoef = [&](int q) {
+        if constexpr (TR) return cconj(cmul(q < M - 1 ? av[q < M - 1 ? q + 1 : q] : anext, rpv[q]));
+        else return cmul(rpv[q], cv[q]);
+    };
+    auto wd = [&](int q) {
+        if constexpr (TR) return cmul(cconj(rpv[q]), sd[ls + q]);
+        else return sd[ls + q];
+    };
     // forward map of the chunk: y_{s+M-1} = A + B y_{s-1}
-    C A = sd[ls], B = cneg(cmul(av[0], rprev));
+    C A = wd(0), B = cneg(mcoef(0));
 #pragma unroll
     for (int q = 1; q < M; ++q) {
-        const C m = cmul(av[q], rpv[q - 1]);
-        A = csub(sd[ls + q], cmul(m, A));
+        const C m = mcoef(q);
+        A = csub(wd(q), cmul(m, A));
         B = cneg(cmul(m, B));
     }
 #pragma unroll
@@ -914,19 +1126,21 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
     C y = zero;                                   // y at the end of the previous wavefronts' rows
     for (int w = 0; w < wave; ++w) y = cadd(wa[w], cmul(wb[w], y));
     y = cadd(ea, cmul(eb, y));                    // y_{s-1}
-    y = csub(sd[ls], cmul(cmul(av[0], rprev), y));
-    sd[ls] = y;
 #pragma unroll
-    for (int q = 1; q < M; ++q) {
-        y = csub(sd[ls + q], cmul(cmul(av[q], rpv[q - 1]), y));
+    for (int q = 0; q < M; ++q) {
+        y = csub(wd(q), cmul(mcoef(q), y));
         sd[ls + q] = y;
     }
     // backward map of the chunk: x_s = G + D x_{s+M}
-    C G = cmul(rpv[M - 1], sd[ls + M - 1]), D = cneg(cmul(rpv[M - 1], cv[M - 1]));
+    auto zy = [&](int q) {
+        if constexpr (TR) return sd[ls + q];
+        else return cmul(rpv[q], sd[ls + q]);
+    };
+    C G = zy(M - 1), D = cneg(ncoef(M - 1));
 #pragma unroll
     for (int q = M - 2; q >= 0; --q) {
-        const C rc = cmul(rpv[q], cv[q]);
-        G = csub(cmul(rpv[q], sd[ls + q]), cmul(rc, G));
+        const C rc = ncoef(q);
+        G = csub(zy(q), cmul(rc, G));
         D = cneg(cmul(rc, D));
     }
 #pragma unroll
@@ -953,7 +1167,8 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
     x = cadd(xa, cmul(xb, x));                    // x_{s+M}
 #pragma unroll
     for (int q = M - 1; q >= 0; --q) {
-        x = cmul(rpv[q], csub(sd[ls + q], cmul(cv[q], x)));
+        if constexpr (TR) x = csub(sd[ls + q], cmul(ncoef(q), x));
+        else x = cmul(rpv[q], csub(sd[ls + q], cmul(cv[q], x)));
         sd[ls + q] = x;
     }
     __syncthreads();
@@ -1057,8 +1272,14 @@ size_t fft_lds(const FftArgs<T> &a)
 }
 
 // the row-block transforms of lengths with a plan
-hipError_t row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done) { return launch_row_rfft(c, x, spec, done); }
-hipError_t row_rfft(vv_ctx *c, const float *x, float2 *spec, const int32_t *done) { return launch_row_rfft32(c, x, spec, done); }
+hipError_t row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add, double gamma)
+{
+    return launch_row_rfft(c, x, spec, done, add, gamma);
+}
+hipError_t row_rfft(vv_ctx *c, const float *x, float2 *spec, const int32_t *done, const float *, float)
+{
+    return launch_row_rfft32(c, x, spec, done);
+}
 hipError_t row_irfft(vv_ctx *c, const double2 *spec, double *y, const int32_t *done) { return launch_row_irfft(c, spec, y, done); }
 hipError_t row_irfft(vv_ctx *c, const float2 *spec, float *y, const int32_t *done) { return launch_row_irfft32(c, spec, y, done); }
 
@@ -1087,12 +1308,13 @@ hipError_t irdft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, cons
 }
 
 template <typename T>
-hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done)
+hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done,
+                  const T *add = nullptr, T gamma = T(0))
 {
-    if (c->dft.n) return row_rfft(c, x, spec, done);
-    if (c->fft_n & (c->fft_n - 1)) return rdft_t<T>(c, tw, x, spec, done);
+    if (c->dft.n) return row_rfft(c, x, spec, done, add, gamma);
+    if (c->fft_n & (c->fft_n - 1)) return add != nullptr ? hipErrorInvalidValue : rdft_t<T>(c, tw, x, spec, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
-                 (int64_t)sizeof(GmresState), tw, done};
+                 (int64_t)sizeof(GmresState), tw, done, add, gamma};
     const int nb = (a.nv + a.rows - 1) / a.rows;
     const uint32_t lds = (uint32_t)fft_lds<T>(a);
     const dim3 grid(nb, c->B), block(NT);
@@ -1162,9 +1384,42 @@ hipError_t irfft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, cons
     const int nb = (a.nv + a.rows - 1) / a.rows;
     const uint32_t lds = (uint32_t)fft_lds<T>(a);
     const dim3 grid(nb, c->B), block(NT);
-    if (a.nx == N8) launch_timed(c, irfft_kernel<T, VP8>, grid, block, lds, a, spec, y);
-    else if (a.nx < N8) launch_timed(c, irfft_kernel<T, VTWL>, grid, block, lds, a, spec, y);
-    else launch_timed(c, irfft_kernel<T, VLONG>, grid, block, lds, a, spec, y);
+    if (a.nx == N8) launch_timed(c, irfft_kernel<T, VP8, false>, grid, block, lds, a, spec, y);
+    else if (a.nx < N8) launch_timed(c, irfft_kernel<T, VTWL, false>, grid, block, lds, a, spec, y);
+    else launch_timed(c, irfft_kernel<T, VLONG, false>, grid, block, lds, a, spec, y);
+    return hipGetLastError();
+}
+
+// The potential form's transforms on the field's columns: lines of a power of
+// two, pairs of columns aligned in every row.
+template <typename T>
+bool cols_apply(const vv_ctx *c, const T *f)
+{
+    return c->tb != nullptr && c->dft.n == 0 && (c->fft_n & (c->fft_n - 1)) == 0 && (c->fft_rows & 1) == 0 &&
+           (reinterpret_cast<uintptr_t>(f) & (2 * sizeof(T) - 1)) == 0;
+}
+
+template <typename T>
+hipError_t rfft_cols_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done)
+{
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
+    const uint32_t lds = (uint32_t)fft_lds<T>(a);
+    const dim3 grid((a.nv + a.rows - 1) / a.rows, c->B), block(NT);
+    if (a.nx == N8) launch_timed(c, rfft_cols_kernel<T, VP8>, grid, block, lds, a, x, spec);
+    else if (a.nx < N8) launch_timed(c, rfft_cols_kernel<T, VTWL>, grid, block, lds, a, x, spec);
+    else launch_timed(c, rfft_cols_kernel<T, VLONG>, grid, block, lds, a, x, spec);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t irfft_cols_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, const int32_t *done)
+{
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
+    const uint32_t lds = (uint32_t)fft_lds<T>(a);
+    const dim3 grid((a.nv + a.rows - 1) / a.rows, c->B), block(NT);
+    if (a.nx == N8) launch_timed(c, irfft_kernel<T, VP8, true>, grid, block, lds, a, spec, y);
+    else if (a.nx < N8) launch_timed(c, irfft_kernel<T, VTWL, true>, grid, block, lds, a, spec, y);
+    else launch_timed(c, irfft_kernel<T, VLONG, true>, grid, block, lds, a, spec, y);
     return hipGetLastError();
 }
 
@@ -1228,27 +1483,12 @@ hipError_t irfft_mdot_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, const
     return hipGetLastError();
 }
 
-void tridiag_shape(int nv, int *P, int *M)
-{
-    if (nv <= 512) {
-        *M = 2;
-        int p = 1;
-        while (p * 2 < nv) p <<= 1;          // P = next power of two >= nv/2
-        *P = p;
-    } else {
-        *P = 256;
-        int m = (nv + 255) / 256;
-        *M = m <= 4 ? 4 : (m <= 8 ? 8 : 16);
-    }
-}
-
-
 template <typename T>
 const cx_t<T> *lu_factors(const vv_ctx *c);
 template <> const double2 *lu_factors<double>(const vv_ctx *c) { return c->lu64; }
 template <> const float2 *lu_factors<float>(const vv_ctx *c) { return c->lu32; }
 
-template <typename T>
+template <typename T, bool TR>
 hipError_t tridiag_lu_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 {
     TriArgs a{c->fft_rows, NT, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
@@ -1258,27 +1498,38 @@ hipError_t tridiag_lu_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
     const cx_t<T> *rp = lu_factors<T>(c);
     dim3 grid(c->nmodes, c->B), block(NT);
     switch (M) {
-    case 1: launch_timed(c, tridiag_lu_kernel<1, T>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    case 2: launch_timed(c, tridiag_lu_kernel<2, T>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    case 4: launch_timed(c, tridiag_lu_kernel<4, T>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    case 8: launch_timed(c, tridiag_lu_kernel<8, T>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    default: launch_timed(c, tridiag_lu_kernel<16, T>, grid, block, (uint32_t)lds, a, rp, spec); break;
+    case 1: launch_timed(c, tridiag_lu_kernel<1, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
+    case 2: launch_timed(c, tridiag_lu_kernel<2, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
+    case 4: launch_timed(c, tridiag_lu_kernel<4, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
+    case 8: launch_timed(c, tridiag_lu_kernel<8, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
+    default: launch_timed(c, tridiag_lu_kernel<16, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
     }
+    return hipGetLastError();
+}
+
+template <typename T, bool TR>
+hipError_t tridiag_wave_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
+{
+    TriArgs a{c->fft_rows, 64, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
+              c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, done};
+    const dim3 grid((c->nmodes + NT / 64 - 1) / (NT / 64), c->B), block(NT);
+    if (c->fft_rows <= 128) launch_timed(c, tridiag_wave_kernel<2, T, TR>, grid, block, 0, a, c->nmodes, spec);
+    else if (c->fft_rows <= 256) launch_timed(c, tridiag_wave_kernel<4, T, TR>, grid, block, 0, a, c->nmodes, spec);
+    else launch_timed(c, tridiag_wave_kernel<8, T, TR>, grid, block, 0, a, c->nmodes, spec);
     return hipGetLastError();
 }
 
 template <typename T, bool TR = false>
 hipError_t tridiag_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 {
-    if (!TR && lu_factors<T>(c) != nullptr) return tridiag_lu_t<T>(c, spec, done);
-    int P, M;
-    tridiag_shape(c->fft_rows, &P, &M);
+    if (lu_factors<T>(c) != nullptr) return tridiag_lu_t<T, TR>(c, spec, done);
+    if (c->fft_rows <= 512) return tridiag_wave_t<T, TR>(c, spec, done);
+    const int P = 256, m = (c->fft_rows + 255) / 256, M = m <= 4 ? 4 : (m <= 8 ? 8 : 16);
     TriArgs a{c->fft_rows, P, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, done};
     const size_t lds = (size_t)P * (M + 1) * sizeof(cx_t<T>);
     dim3 grid(c->nmodes, c->B), block(NT);
     switch (M) {
-    case 2: launch_timed(c, tridiag_kernel<2, T, TR>, grid, block, (uint32_t)lds, a, spec); break;
     case 4: launch_timed(c, tridiag_kernel<4, T, TR>, grid, block, (uint32_t)lds, a, spec); break;
     case 8: launch_timed(c, tridiag_kernel<8, T, TR>, grid, block, (uint32_t)lds, a, spec); break;
     default: launch_timed(c, tridiag_kernel<16, T, TR>, grid, block, (uint32_t)lds, a, spec); break;
@@ -1306,9 +1557,9 @@ int fft_blocks(vv_ctx *c)
     return (c->fft_rows + R - 1) / R;
 }
 
-hipError_t launch_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done)
+hipError_t launch_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add, double gamma)
 {
-    return rfft_t<double>(c, c->twiddle, x, spec, done);
+    return rfft_t<double>(c, c->twiddle, x, spec, done, add, gamma);
 }
 
 // Rows per workgroup of the fused J u + rFFT (its own choice: the spectrum's
@@ -1406,6 +1657,25 @@ hipError_t launch_transpose(vv_ctx *c, const double *in, double *out, bool back,
 hipError_t launch_transpose32(vv_ctx *c, const float *in, float *out, bool back, const int32_t *done)
 {
     return transpose_t<float>(c, in, out, back, done);
+}
+
+bool potential_cols(const vv_ctx *c, const double *f) { return cols_apply<double>(c, f); }
+bool potential_cols32(const vv_ctx *c, const float *f) { return cols_apply<float>(c, f); }
+hipError_t launch_rfft_cols(vv_ctx *c, const double *x, double2 *spec, const int32_t *done)
+{
+    return rfft_cols_t<double>(c, c->twiddle, x, spec, done);
+}
+hipError_t launch_irfft_cols(vv_ctx *c, const double2 *spec, double *y, const int32_t *done)
+{
+    return irfft_cols_t<double>(c, c->twiddle, spec, y, done);
+}
+hipError_t launch_rfft_cols32(vv_ctx *c, const float *x, float2 *spec, const int32_t *done)
+{
+    return rfft_cols_t<float>(c, c->twiddle32, x, spec, done);
+}
+hipError_t launch_irfft_cols32(vv_ctx *c, const float2 *spec, float *y, const int32_t *done)
+{
+    return irfft_cols_t<float>(c, c->twiddle32, spec, y, done);
 }
 
 hipError_t launch_potential_bands(vv_ctx *c, const double *phi)

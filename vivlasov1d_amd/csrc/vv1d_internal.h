@@ -227,6 +227,11 @@ hipError_t launch_narrow_add(vv_ctx *c, float *y, const double *d);           //
 // H = h2d (2D) or hxv (x only) when given, else H_ave
 hipError_t launch_bracket_t(vv_ctx *c, const double *u, const double *uscale, const double *h2d, const double *hxv,
                             double *y, double alpha, double factor);
+// y = alpha u + factor {u~, H_ave} on all rows and the column sums of {u~, g} over
+// band_rows(nv) bands of rows; takes the due Hessenberg update when uscale is given
+int band_rows(int nv);
+hipError_t launch_bracket_pair(vv_ctx *c, const double *u, const double *uscale, const double *g, double *y,
+                               double alpha, double factor, double *csum, int64_t cstride);
 // y += factor {x, H} on rows 2..nv-3, H = h2d / hxv / H_ave as above
 hipError_t launch_bracket_gen(vv_ctx *c, const double *x, const double *h2d, const double *hxv, double *y,
                               double factor);
@@ -260,7 +265,8 @@ hipError_t launch_row_jac(vv_ctx *c, const double *u, const double *uscale, cons
                           const int32_t *done);
 hipError_t launch_row_jac32(vv_ctx *c, const float *u, const double *uscale, float2 *spec, const int32_t *done);
 hipError_t launch_row_res(vv_ctx *c, const double *f, const double *fh, double2 *spec);
-hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done);
+hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add,
+                           double gamma);
 hipError_t launch_row_rfft32(vv_ctx *c, const float *x, float2 *spec, const int32_t *done);
 hipError_t launch_row_irfft(vv_ctx *c, const double2 *spec, double *y, const int32_t *done);
 hipError_t launch_row_irfft32(vv_ctx *c, const float2 *spec, float *y, const int32_t *done);
@@ -271,7 +277,9 @@ hipError_t launch_row_inv32(vv_ctx *c, const float2 *spec, int col, const int32_
 // spectral.hip
 int fft_blocks(vv_ctx *c);
 int fft_rows_of(const vv_ctx *c);
-hipError_t launch_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done);
+// (rows x + gamma add with an x-only field `add`, B nx)
+hipError_t launch_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add = nullptr,
+                       double gamma = 0.0);
 // J u (u times its optional device scale) and its rFFT in one launch, the
 // Jacobian never stored; jac_rfft_rows: the rows per workgroup where the
 // fused kernel applies to the context (the kinetic form with a power-of-two
@@ -301,6 +309,14 @@ hipError_t launch_irfft_mdot32(vv_ctx *c, const float2 *spec, int col, const int
 hipError_t launch_tridiag_factor(vv_ctx *c, double2 *rp64, float2 *rp32);
 hipError_t launch_transpose(vv_ctx *c, const double *in, double *out, bool back, const int32_t *done);
 hipError_t launch_transpose32(vv_ctx *c, const float *in, float *out, bool back, const int32_t *done);
+// the potential form's transforms straight on the field's columns, where they
+// apply to the field f (its alignment; an even nx, nv a power of two)
+bool potential_cols(const vv_ctx *c, const double *f);
+bool potential_cols32(const vv_ctx *c, const float *f);
+hipError_t launch_rfft_cols(vv_ctx *c, const double *x, double2 *spec, const int32_t *done);
+hipError_t launch_irfft_cols(vv_ctx *c, const double2 *spec, double *y, const int32_t *done);
+hipError_t launch_rfft_cols32(vv_ctx *c, const float *x, float2 *spec, const int32_t *done);
+hipError_t launch_irfft_cols32(vv_ctx *c, const float2 *spec, float *y, const int32_t *done);
 hipError_t launch_potential_bands(vv_ctx *c, const double *phi);
 // krylov.hip
 hipError_t launch_gmres_init(vv_ctx *c, double rtol, double atol, double dtol, int max_it);
@@ -346,11 +362,12 @@ hipError_t launch_density_partial(vv_ctx *c, const double *f, double *npart);
 hipError_t launch_density(vv_ctx *c, const double *f, double *n);
 hipError_t launch_velocity_moments(vv_ctx *c, const double *f, double *u, double *e);
 // Poisson pipeline; npart / work (3 nx + 1 per instance) default to the
-// context's buffers when null; the residual norm of instance b goes to
+// context's buffers when null (nch partials a column, npstride apart per
+// instance, when given); the residual norm of instance b goes to
 // pres[b * pres_stride]
 hipError_t launch_poisson(vv_ctx *c, const double *n_in, double *n_out, double *phi, double *h1, double *pres,
                           int from_part, const double *npart = nullptr, double *work = nullptr,
-                          int pres_stride = 16);
+                          int pres_stride = 16, int nch = 0, int64_t npstride = 0);
 hipError_t launch_poisson_mult(vv_ctx *c, const double *x, const double *n, double *y);
 hipError_t launch_pot_to_ham(vv_ctx *c, const double *phi, double *h1);
 hipError_t launch_invariants(vv_ctx *c, const double *f, const double *h0, const double *h1,
