@@ -236,7 +236,7 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     // the residual's norm without another pass over it (6.8 us at 1024 x 2048)
     if (MODE == MODE_RESIDUAL && a.part != nullptr) {
         __shared__ double red[NT / 64];
-        for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off);
+        sq = wave_sum(sq);
         if (lane == 0) red[wave] = sq;
         __syncthreads();
         if (threadIdx.x == 0) {

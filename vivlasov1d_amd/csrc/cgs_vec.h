@@ -6,12 +6,13 @@
 // the slice of NT*EPT 16-byte vectors starting at s*NT*EPT, thread t the
 // vectors t + q*NT (q < EPT) of it.  The dot of a slice is accumulated per
 // thread in (q, lane-element) order without contraction, reduced over the
-// wavefront by shuffles and over the NT/64 wavefronts in a fixed order, so a
+// wavefront (wave_ops.h) and over the NT/64 wavefronts in a fixed order, so a
 // kernel that forms the same slice's w by other means (the fused irFFT)
 // produces bit-identical partials.
 #pragma once
 
 #include "vv1d_internal.h"
+#include "wave_ops.h"
 
 namespace vv {
 namespace {
@@ -87,12 +88,6 @@ __device__ __forceinline__ void load_group(const S *basis, int64_t vstride, int 
             x[gg][q] = (e < nvv) ? Vp[e] : V{};
         }
     }
-}
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    return v;   // lane 0
 }
 
 // sum_q sum_l w[q]_l (x[q]_l sv): one thread's share of <w, sv V> over a

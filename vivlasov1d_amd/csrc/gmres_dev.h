@@ -8,6 +8,7 @@
 #pragma once
 
 #include "vv1d_internal.h"
+#include "wave_ops.h"
 
 namespace vv {
 namespace {
@@ -18,17 +19,12 @@ constexpr int kGdNW = kGdNT / 64;
 // Sum over the block, returned in every thread (fixed tree).
 __device__ __forceinline__ double block_sum_all(double v, double *red)
 {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) red[wave] = v;
+    const double ws = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ws;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < kGdNW; ++w) s += red[w];
-        red[kGdNW] = s;
-    }
-    __syncthreads();
-    const double s = red[kGdNW];
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < kGdNW; ++w) s += red[w];
     __syncthreads();
     return s;
 }

@@ -19,12 +19,12 @@
 //
 // In a batched context instance b is blockIdx.y (blockIdx.z for the column
 // sums); its fields start at b * N, its x-vectors at b * nx.
+#include "fft_lds.h"
 #include "vv1d_internal.h"
 
 namespace vv {
 namespace {
 
-constexpr int NT = 256;
 constexpr int PT = 1024;     // threads of the single-workgroup Poisson kernel
 constexpr int DCH = kDensityChunks;   // row chunks of the density reduction
 
@@ -103,30 +103,28 @@ __global__ __launch_bounds__(NT) void column_finish_kernel(const double *__restr
 
 // Chunks of rows of the column sums (<= kDensityChunks / 2, so the two velocity
 // moments fit the density's scratch; a function of nv alone, so that a batched
-// instance sums as it would alone).  Up to 512 rows one chunk: 32 rows a
-// wavefront, and no finish launch (velocity moments of 100 x 200: 43.5 us
-// before); beyond, 128 rows a chunk, 256 workgroups at 1024 x 2048.
+// instance sums as it would alone): 128 rows a chunk, one round of eight loads
+// a lane and 256 workgroups at 1024 x 2048.
 int column_chunks(int nv)
 {
-    if (nv <= 512) return 1;
     const int n = (nv + 127) / 128;
     return n < kDensityChunks / 2 ? n : kDensityChunks / 2;
 }
+// Where the sums themselves are wanted, up to 512 rows go in one chunk: 32 rows
+// a wavefront, and no finish launch (velocity moments of 100 x 200: 43.5 us
+// before).
+int sum_chunks(int nv) { return nv <= 512 ? 1 : column_chunks(nv); }
 
-__device__ double block_sum_big(double v, double *red)
+__device__ __forceinline__ double block_sum_big(double v, double *red)
 {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const double ws = wave_sum(v);
+    __syncthreads();                   // the sum before is read
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ws;
     __syncthreads();
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < PT / 64; ++w) s += red[w];
-        red[PT / 64] = s;
-    }
-    __syncthreads();
-    return red[PT / 64];    // valid in every thread
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < PT / 64; ++w) s += red[w];
+    return s;                          // valid in every thread
 }
 
 struct PoiArgs {
@@ -173,79 +171,6 @@ __device__ __forceinline__ void poi_instance(PoiArgs &a)
     if (a.pres) a.pres += b * a.pres_stride;
 }
 
-// In-place complex FFT of length n = 2^logn (8 .. 4 PT) in LDS by the whole
-// workgroup: radix-4 Stockham stages, one butterfly a thread, and a radix-2
-// stage for odd logn (two butterflies a thread at most); the next stage's
-// twiddles are loaded while the current one runs.  INV: unnormalised inverse.
-template <bool INV>
-__device__ void line_fft(double2 *buf, int n, int logn, const double2 *__restrict__ tw)
-{
-    const int nq = n >> 2, ns = logn >> 1;
-    const int t = threadIdx.x;
-    const bool on = t < nq;
-    double2 w[3] = {{1.0, 0.0}, {1.0, 0.0}, {1.0, 0.0}};
-    for (int s = 0; s < ns; ++s) {
-        const int Ns = 1 << (2 * s);
-        const int k = t & (Ns - 1);
-        double2 v[4], wn[3] = {{1.0, 0.0}, {1.0, 0.0}, {1.0, 0.0}};
-        if (on) {
-            if (s + 1 < ns) {
-                const int st = (t & (4 * Ns - 1)) << (logn - 4 - 2 * s);
-#pragma unroll
-                for (int r = 0; r < 3; ++r) wn[r] = tw[(r + 1) * st];
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = buf[t + r * nq];
-#pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                const double wy = INV ? -w[r].y : w[r].y;
-                const double2 x = v[r + 1];
-                v[r + 1].x = x.x * w[r].x - x.y * wy;
-                v[r + 1].y = x.x * wy + x.y * w[r].x;
-            }
-        }
-        __syncthreads();
-        if (on) {
-            const double2 a0{v[0].x + v[2].x, v[0].y + v[2].y}, a1{v[0].x - v[2].x, v[0].y - v[2].y};
-            const double2 a2{v[1].x + v[3].x, v[1].y + v[3].y}, d{v[1].x - v[3].x, v[1].y - v[3].y};
-            const double2 a3 = INV ? double2{-d.y, d.x} : double2{d.y, -d.x};
-            double2 *o = buf + ((t - k) << 2) + k;
-            o[0] = double2{a0.x + a2.x, a0.y + a2.y};
-            o[Ns] = double2{a1.x + a3.x, a1.y + a3.y};
-            o[2 * Ns] = double2{a0.x - a2.x, a0.y - a2.y};
-            o[3 * Ns] = double2{a1.x - a3.x, a1.y - a3.y};
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 3; ++r) w[r] = wn[r];
-    }
-    if (logn & 1) {                      // sub-transforms of n/2: outputs j, j + n/2
-        const int nh = n >> 1;
-        double2 lo[2], hi[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int j = t + q * PT;
-            if (j < nh) {
-                const double2 x0 = buf[j], x1 = buf[j + nh], c = tw[j];
-                const double cy = INV ? -c.y : c.y;
-                const double2 m{x1.x * c.x - x1.y * cy, x1.x * cy + x1.y * c.x};
-                lo[q] = double2{x0.x + m.x, x0.y + m.y};
-                hi[q] = double2{x0.x - m.x, x0.y - m.y};
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int j = t + q * PT;
-            if (j < nh) {
-                buf[j] = lo[q];
-                buf[j + nh] = hi[q];
-            }
-        }
-        __syncthreads();
-    }
-}
-
 // n_i of the thread's columns i = t + q PT from the density partials, or as
 // given; `on` marks the columns that exist.  Grids of up to PT/2 columns
 // deal the chunks to PT / span threads a column (span: the columns padded to
@@ -260,8 +185,15 @@ __device__ __forceinline__ void poi_density(const PoiArgs &a, double (&n)[kMaxNx
         while (span < nx) span <<= 1;
         const int g = t / span, i = t & (span - 1), G = PT / span;
         double s = 0.0;
-        if (i < nx)
-            for (int ch = g; ch < a.nch; ch += G) s += a.npart[(size_t)ch * nx + i];
+        if (i < nx) {
+            for (int c0 = g; c0 < a.nch; c0 += 8 * G) {      // eight loads in flight
+                double v[8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c) v[c] = c0 + c * G < a.nch ? a.npart[(size_t)(c0 + c * G) * nx + i] : 0.0;
+#pragma unroll
+                for (int c = 0; c < 8; ++c) s += v[c];
+            }
+        }
         red[t] = s;
         __syncthreads();
         if (t < nx) {
@@ -305,6 +237,7 @@ struct ReX {                             // real parts of a complex line
 // launches and the pass over `work`: prep + conv + post took 13.0 + 11.2 +
 // 4.3 us at nx = 1024 and 6.1 + 2.7 + 3.3 us at nx = 64.
 constexpr int kPoissonOne = 320;
+constexpr int kPoissonTw = 2048;
 template <bool FFT>
 __global__ __launch_bounds__(PT) void poisson_kernel(PoiArgs a)
 {
@@ -315,6 +248,18 @@ __global__ __launch_bounds__(PT) void poisson_kernel(PoiArgs a)
     const double hx2_inv = a.inst[blockIdx.y].hx2_inv;
     const int nx = a.nx, t = threadIdx.x;
     constexpr int Q = kMaxNx / PT;
+    // the symbol and (up to 2048 points) the twiddles' LDS copy, in flight with n
+    double lam[Q];
+    const double2 *tw = a.tw;
+    if (FFT) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) lam[q] = t + q * PT < nx ? a.plam[t + q * PT] : 0.0;
+        if (nx <= kPoissonTw) {
+            double2 *stw = pline + nx;
+            for (int m = t; m < nx; m += PT) stw[m] = a.tw[m];
+            tw = stw;
+        }
+    }
     double n[Q];
     poi_density(a, n, red);
     double part = 0.0;
@@ -337,17 +282,15 @@ __global__ __launch_bounds__(PT) void poisson_kernel(PoiArgs a)
     }
     __syncthreads();
     if (FFT) {
-        line_fft<false>(pline, nx, a.logn, a.tw);
+        // at most one butterfly a thread: nx / 4 <= PT
+        lds_fft<false, false, 1>(pline, a.logn, 1, tw, FftTw<false, double2>{}, 0, LdsSink<double2>{pline});
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int i = t + q * PT;
-            if (i < nx) {
-                const double l = a.plam[i];
-                pline[i] = double2{pline[i].x * l, pline[i].y * l};
-            }
+            if (i < nx) pline[i] = double2{pline[i].x * lam[q], pline[i].y * lam[q]};
         }
         __syncthreads();
-        line_fft<true>(pline, nx, a.logn, a.tw);
+        lds_fft<true, false, 1>(pline, a.logn, 1, tw, FftTw<true, double2>{}, 0, LdsSink<double2>{pline});
     } else {
         int span = 64;
         while (span < nx) span <<= 1;
@@ -587,8 +530,7 @@ __global__ __launch_bounds__(NT) void invariants_kernel(InvArgs a)
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int q = 0; q < 5; ++q) {
-        double v = s[q];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+        const double v = wave_sum(s[q]);
         if (lane == 0) red[q][wave] = v;
     }
     __syncthreads();
@@ -616,8 +558,7 @@ __global__ __launch_bounds__(NT) void invariants_finish_kernel(InvArgs a, int nb
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int q = 0; q < 6; ++q) {
-        double v = t6[q];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+        const double v = wave_sum(t6[q]);
         if (lane == 0) red[q][wave] = v;
     }
     __syncthreads();
@@ -645,9 +586,9 @@ __global__ __launch_bounds__(NT) void invariants_finish_kernel(InvArgs a, int nb
 namespace {
 
 template <int MOM>
-void column_launch(vv_ctx *c, const double *f, int64_t ostride, double scale, double *out0, double *out1)
+void column_launch(vv_ctx *c, const double *f, int nch, int64_t ostride, double scale, double *out0, double *out1)
 {
-    const int nx = c->p.nx, nv = c->p.nv, nch = column_chunks(nv);
+    const int nx = c->p.nx, nv = c->p.nv;
     const int rows = (nv + nch - 1) / nch;
     hipLaunchKernelGGL(column_kernel<MOM>, dim3((nx + 63) / 64, nch, c->B), dim3(64 * CW), 0, c->stream, f, c->vgrid,
                        nx, nv, rows, ostride, scale, out0, out1);
@@ -665,14 +606,14 @@ void column_finish(vv_ctx *c, const double *part1, double *out0, double *out1)
 
 hipError_t launch_density_partial(vv_ctx *c, const double *f, double *npart)
 {
-    column_launch<0>(c, f, (int64_t)DCH * c->p.nx, 1.0, npart != nullptr ? npart : c->npart, nullptr);
+    column_launch<0>(c, f, column_chunks(c->p.nv), (int64_t)DCH * c->p.nx, 1.0, npart != nullptr ? npart : c->npart, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_density(vv_ctx *c, const double *f, double *n)
 {
-    if (column_chunks(c->p.nv) == 1) {
-        column_launch<0>(c, f, c->p.nx, c->p.hv, n, nullptr);
+    if (sum_chunks(c->p.nv) == 1) {
+        column_launch<0>(c, f, 1, c->p.nx, c->p.hv, n, nullptr);
         return hipGetLastError();
     }
     const hipError_t e = launch_density_partial(c, f, nullptr);
@@ -683,12 +624,12 @@ hipError_t launch_density(vv_ctx *c, const double *f, double *n)
 
 hipError_t launch_velocity_moments(vv_ctx *c, const double *f, double *u, double *e)
 {
-    if (column_chunks(c->p.nv) == 1) {
-        column_launch<1>(c, f, c->p.nx, c->p.hv, u, e);
+    if (sum_chunks(c->p.nv) == 1) {
+        column_launch<1>(c, f, 1, c->p.nx, c->p.hv, u, e);
         return hipGetLastError();
     }
     double *part1 = c->npart + (size_t)(DCH / 2) * c->p.nx;
-    column_launch<1>(c, f, (int64_t)DCH * c->p.nx, 1.0, c->npart, part1);
+    column_launch<1>(c, f, column_chunks(c->p.nv), (int64_t)DCH * c->p.nx, 1.0, c->npart, part1);
     column_finish(c, part1, u, e);
     return hipGetLastError();
 }
@@ -704,7 +645,8 @@ hipError_t launch_poisson(vv_ctx *c, const double *n_in, double *n_out, double *
               work != nullptr ? work : c->pwork, n_out, phi, h1, pres, pres_stride};
     if (c->plam != nullptr) {
         while ((1 << a.logn) < nx) ++a.logn;
-        hipLaunchKernelGGL(poisson_kernel<true>, dim3(1, c->B), dim3(PT), nx * sizeof(double2), c->stream, a);
+        hipLaunchKernelGGL(poisson_kernel<true>, dim3(1, c->B), dim3(PT),
+                           (nx <= kPoissonTw ? 2 : 1) * nx * sizeof(double2), c->stream, a);
         return hipGetLastError();
     }
     if (nx <= kPoissonOne) {

@@ -869,6 +869,14 @@ template <typename C> __device__ __forceinline__ C shfl_down_cx(C v, int off)
 {
     return cmk<C>(__shfl_down(v.x, off), __shfl_down(v.y, off));
 }
+template <int CTRL, int ROWS = 0xf, typename C> __device__ __forceinline__ C dpp_cx(C v)
+{
+    return cmk<C>(dpp_move<CTRL, ROWS>(v.x), dpp_move<CTRL, ROWS>(v.y));
+}
+template <typename C> __device__ __forceinline__ C lane_cx(C v, int lane)
+{
+    return cmk<C>(read_lane(v.x, lane), read_lane(v.y, lane));
+}
 
 __device__ __forceinline__ void wave_lds_fence()
 {
@@ -1014,11 +1022,78 @@ __global__ __launch_bounds__(NT) void tridiag_factor_kernel(TriArgs a, int nmode
     for (int j = a.nv; j < L; ++j) R[(j % M) * NT + j / M] = cmk<cx_t<T>>(T(0), T(0));
 }
 
+// The affine maps y -> A + B y of a wavefront's lanes composed: (ea, eb) the map
+// of the lanes before this one (REV: after it) applied to the value entering
+// the wavefront, and (ta, tb) that of all 64 lanes, in every lane.  Rows of 16 by DPP, then the four rows'
+// maps, which every lane reads and composes itself: ~350 cycles where six steps
+// of four-double shuffles took ~900.
+template <bool REV, typename C>
+__device__ __forceinline__ void affine_scan(C A, C B, int lane, C &ea, C &eb, C &ta, C &tb)
+{
+    using R = typename C::value_type;
+    const C zero = cmk<C>(R(0), R(0)), one = cmk<C>(R(1), R(0));
+    const int r = lane & 15, row = lane >> 4;
+    constexpr int DIR = REV ? kDppShl : kDppShr;
+    const int pos = REV ? 15 - r : r;              // lanes of the row that come before
+    {
+        const C pa = dpp_cx<DIR + 1>(A), pb = dpp_cx<DIR + 1>(B);
+        if (pos >= 1) {
+            A = cadd(A, cmul(B, pa));
+            B = cmul(B, pb);
+        }
+    }
+    {
+        const C pa = dpp_cx<DIR + 2>(A), pb = dpp_cx<DIR + 2>(B);
+        if (pos >= 2) {
+            A = cadd(A, cmul(B, pa));
+            B = cmul(B, pb);
+        }
+    }
+    {
+        const C pa = dpp_cx<DIR + 4>(A), pb = dpp_cx<DIR + 4>(B);
+        if (pos >= 4) {
+            A = cadd(A, cmul(B, pa));
+            B = cmul(B, pb);
+        }
+    }
+    {
+        const C pa = dpp_cx<DIR + 8>(A), pb = dpp_cx<DIR + 8>(B);
+        if (pos >= 8) {
+            A = cadd(A, cmul(B, pa));
+            B = cmul(B, pb);
+        }
+    }
+    ea = dpp_cx<DIR + 1>(A);
+    eb = dpp_cx<DIR + 1>(B);
+    if (pos == 0) {
+        ea = zero;
+        eb = one;
+    }
+    // rows in the order the recurrence meets them: last lane of each holds its map
+    C pa = zero, pb = one;                         // of the rows before this lane's
+    ta = zero;
+    tb = one;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int rr = REV ? 3 - q : q;
+        if (row == rr) {
+            pa = ta;
+            pb = tb;
+        }
+        const int last = REV ? 16 * rr : 16 * rr + 15;
+        const C ra = lane_cx(A, last), rb = lane_cx(B, last);
+        ta = cadd(ra, cmul(rb, ta));
+        tb = cmul(rb, tb);
+    }
+    ea = cadd(ea, cmul(eb, pa));
+    eb = cmul(eb, pb);
+}
+
 // One workgroup per mode (blockIdx.x) and instance (blockIdx.y); thread t
 // owns the chunk of M rows [t M, t M + M).  The spectrum row and its pivots
 // are staged in LDS (coalesced loads).  Across chunks the recurrences are
 // affine maps y_out = A + B y_in, composed by a scan over the wavefront's
-// lanes (shuffles) and over the 4 wavefronts (one LDS exchange), first
+// lanes (affine_scan) and over the 4 wavefronts (one LDS exchange), first
 // forward, then backward; no thread waits on a division.
 // TR: T_k^H x = d from the same pivots, U^H y = d then L^H x = y:
 //   y_j = conj(rp_j) (d_j - conj(c_{j-1}) y_{j-1}),  x_j = y_j - conj(a_{j+1} rp_j) x_{j+1}
@@ -1105,22 +1180,11 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
         A = csub(wd(q), cmul(m, A));
         B = cneg(cmul(m, B));
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {     // inclusive scan, earlier lanes first
-        const C pa = shfl_up_cx(A, off), pb = shfl_up_cx(B, off);
-        if (lane >= off) {
-            A = cadd(A, cmul(B, pa));
-            B = cmul(B, pb);
-        }
-    }
-    if (lane == 63) {
-        wa[wave] = A;
-        wb[wave] = B;
-    }
-    C ea = shfl_up_cx(A, 1), eb = shfl_up_cx(B, 1);   // lanes 0 .. lane-1
+    C ea, eb, ta, tb;                             // maps of lanes 0 .. lane-1, of the wavefront
+    affine_scan<false>(A, B, lane, ea, eb, ta, tb);
     if (lane == 0) {
-        ea = zero;
-        eb = one;
+        wa[wave] = ta;
+        wb[wave] = tb;
     }
     __syncthreads();
     C y = zero;                                   // y at the end of the previous wavefronts' rows
@@ -1143,23 +1207,12 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
         G = csub(zy(q), cmul(rc, G));
         D = cneg(cmul(rc, D));
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {     // inclusive scan, later lanes first
-        const C na = shfl_down_cx(G, off), nb = shfl_down_cx(D, off);
-        if (lane + off < 64) {
-            G = cadd(G, cmul(D, na));
-            D = cmul(D, nb);
-        }
-    }
+    C xa, xb;                                     // maps of lanes lane+1 .. 63
+    affine_scan<true>(G, D, lane, xa, xb, ta, tb);
     __syncthreads();                              // every thread has read wa / wb
     if (lane == 0) {
-        wa[wave] = G;
-        wb[wave] = D;
-    }
-    C xa = shfl_down_cx(G, 1), xb = shfl_down_cx(D, 1);   // lanes lane+1 .. 63
-    if (lane == 63) {
-        xa = zero;
-        xb = one;
+        wa[wave] = ta;
+        wb[wave] = tb;
     }
     __syncthreads();
     C x = zero;                                   // x at the first row of the next wavefronts
