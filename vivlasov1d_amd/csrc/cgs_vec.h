@@ -81,7 +81,7 @@ __device__ __forceinline__ void load_group(const S *basis, int64_t vstride, int 
 #pragma unroll
     for (int gg = 0; gg < G; ++gg) {
         if (gg >= have) break;             // uniform over the launch
-        const V *Vp = reinterpret_cast<const V *>(basis + (size_t)(v0 + gg) * vstride);
+        const V *Vp = reinterpret_cast<const V *>(basis + (int64_t)(v0 + gg) * vstride);
 #pragma unroll
         for (int q = 0; q < EPT; ++q) {
             const int64_t e = e0 + (int64_t)q * kCgsNT;
