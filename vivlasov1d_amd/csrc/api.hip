@@ -1083,8 +1083,11 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(dalloc(c, &c->twiddle, c->fft_n), "alloc twiddle");
     VV_CCHECK(dalloc(c, &c->twiddle32, c->fft_n), "alloc twiddle32");
     VV_CCHECK(dalloc(c, &c->spec, (size_t)c->nmodes * c->fft_rows * Bz), "alloc spectrum");
-    if (p->precond == VV_PRECOND_TENSOR_KINETIC)
+    if (p->precond == VV_PRECOND_TENSOR_KINETIC) {
         VV_CCHECK(dalloc(c, &c->lu64, (size_t)c->nmodes * lu_pivots_per_mode(c->fft_rows) * Bz), "alloc pivots");
+        VV_CCHECK(dalloc(c, &c->lu_gm, lu_pivots_per_mode(c->fft_rows)), "alloc band factors");
+        VV_CCHECK(dalloc(c, &c->lu_gp, lu_pivots_per_mode(c->fft_rows)), "alloc band factors");
+    }
     // the FFT form of the Poisson solve reads the context's twiddles, of length fft_n
     const bool pfft = (nx & (nx - 1)) == 0 && c->fft_n == nx;
     if (pfft) VV_CCHECK(dalloc(c, &c->plam, nx * Bz), "alloc plam");
@@ -1180,6 +1183,18 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(hipMemcpy(c->gm, gm.data(), ncoef * sizeof(double), hipMemcpyHostToDevice), "upload");
     VV_CCHECK(hipMemcpy(c->g0, g0.data(), ncoef * sizeof(double), hipMemcpyHostToDevice), "upload");
     VV_CCHECK(hipMemcpy(c->gp, gp.data(), ncoef * sizeof(double), hipMemcpyHostToDevice), "upload");
+    if (c->lu64) {
+        // in the pivots' order; no sub-diagonal in row 0, no super-diagonal in
+        // row nv - 1, neither in the rows that pad the chunks
+        const int L = lu_pivots_per_mode(nv), M = lu_rows(nv), TN = L / M;
+        std::vector<double> lo(L, 0.0), hi(L, 0.0);
+        for (int j = 0; j < nv; ++j) {
+            if (j > 0) lo[(j % M) * TN + j / M] = gm[j];
+            if (j < nv - 1) hi[(j % M) * TN + j / M] = gp[j];
+        }
+        VV_CCHECK(hipMemcpy(c->lu_gm, lo.data(), L * sizeof(double), hipMemcpyHostToDevice), "upload");
+        VV_CCHECK(hipMemcpy(c->lu_gp, hi.data(), L * sizeof(double), hipMemcpyHostToDevice), "upload");
+    }
     VV_CCHECK(hipMemcpy(c->vgrid, p->v, nv * sizeof(double), hipMemcpyHostToDevice), "upload");
     VV_CCHECK(hipMemcpy(c->eigen, eig.data(), c->nmodes * sizeof(double2), hipMemcpyHostToDevice), "upload");
     VV_CCHECK(hipMemcpy(c->twiddle, tw.data(), nf * sizeof(double2), hipMemcpyHostToDevice), "upload");
@@ -1227,7 +1242,8 @@ int vv_ctx_destroy(vv_ctx *c)
                     c->gm,     c->g0,     c->gp,      c->twiddle, c->twiddle32, c->spec, c->pinv, c->plam, c->pwork,
                     c->X,      c->rhs,    c->D,       c->basis,   c->basis32, c->R,   c->partial, c->dscalar,
                     c->npart,  c->gs,     c->T2,      c->xs,   c->vgrid, c->tb,     c->fave,    c->db1,
-                    c->db2,    c->ex,     c->w64,     c->d64,   c->lu64,   c->lu32};
+                    c->db2,    c->ex,     c->w64,     c->d64,   c->lu64,   c->lu32,
+                    c->lu_gm,  c->lu_gp};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (c->host_status) (void)hipHostFree(c->host_status);     // the whole pinned block

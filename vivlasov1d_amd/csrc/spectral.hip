@@ -995,7 +995,7 @@ __global__ __launch_bounds__(NT) void tridiag_wave_kernel(TriArgs a, int nmodes,
 //   backward  x_j = rp_j (y_j - c_j x_{j+1}),
 // a_j and c_j being rebuilt from e_k and the per-row factors as in tri_row.
 template <typename T>
-__global__ __launch_bounds__(NT) void tridiag_factor_kernel(TriArgs a, int nmodes, int M, cx_t<T> *__restrict__ rp)
+__global__ __launch_bounds__(NT) void tridiag_factor_kernel(TriArgs a, int nmodes, int TN, int M, cx_t<T> *__restrict__ rp)
 {
     const int k = blockIdx.x * NT + threadIdx.x;
     if (k >= nmodes) return;
@@ -1004,7 +1004,7 @@ __global__ __launch_bounds__(NT) void tridiag_factor_kernel(TriArgs a, int nmode
     // chunk-interleaved: the pivot of row j = t M + q at q NT + t, so that the
     // solve's thread t, which owns rows t M .. t M + M - 1, loads them
     // coalesced; rows nv .. NT M - 1 hold zero
-    const int L = NT * M;
+    const int L = TN * M;
     cx_t<T> *R = rp + ((size_t)blockIdx.y * nmodes + k) * L;
     double lo, mid, hi;
     double2 aj, bj, cj;
@@ -1017,9 +1017,9 @@ __global__ __launch_bounds__(NT) void tridiag_factor_kernel(TriArgs a, int nmode
         tri_load<false>(a, j, lo, mid, hi);
         tri_row<false>(a, af, e, j, lo, mid, hi, aj, bj, cj);
         r = crecip(csub(bj, cmul(cmul(aj, r), cprev)));
-        R[(j % M) * NT + j / M] = cmk<cx_t<T>>((T)r.x, (T)r.y);
+        R[(j % M) * TN + j / M] = cmk<cx_t<T>>((T)r.x, (T)r.y);
     }
-    for (int j = a.nv; j < L; ++j) R[(j % M) * NT + j / M] = cmk<cx_t<T>>(T(0), T(0));
+    for (int j = a.nv; j < L; ++j) R[(j % M) * TN + j / M] = cmk<cx_t<T>>(T(0), T(0));
 }
 
 // The affine maps y -> A + B y of a wavefront's lanes composed: (ea, eb) the map
@@ -1089,19 +1089,28 @@ __device__ __forceinline__ void affine_scan(C A, C B, int lane, C &ea, C &eb, C 
     eb = cmul(eb, pb);
 }
 
-// One workgroup per mode (blockIdx.x) and instance (blockIdx.y); thread t
-// owns the chunk of M rows [t M, t M + M).  The spectrum row and its pivots
-// are staged in LDS (coalesced loads).  Across chunks the recurrences are
-// affine maps y_out = A + B y_in, composed by a scan over the wavefront's
-// lanes (affine_scan) and over the 4 wavefronts (one LDS exchange), first
-// forward, then backward; no thread waits on a division.
+// One workgroup of TN threads per mode (blockIdx.x) and instance (blockIdx.y);
+// thread t owns the chunk of M rows [t M, t M + M), in registers.  The
+// spectrum row turns from coalesced to chunks and back in each wavefront's own
+// part of LDS; the pivots and the band factors lie in chunk-interleaved order
+// (read in row order, the factors' 8 M-byte strides took 64 lines a load: 73 us
+// at 2048 x 4096 where it is 42 now, 17.2 and 14.0 at 1024 x 2048).  Across
+// chunks the recurrences are affine maps y_out = A + B y_in, composed by a scan
+// over the wavefront's lanes (affine_scan) and over the wavefronts (one LDS
+// exchange), first forward, then backward; no thread waits on a division.
+// Bound by memory and by its phases, which the two or three workgroups of a CU
+// go through nearly together: 50 MB in 14 us at 1024 x 2048, 201 MB in 42 at
+// 2048 x 4096.
+// M = 16: the backward sweep's factors are loaded after the forward scan, so
+// the kernel keeps 256 registers and two workgroups a CU (111 us with spills, 54
+// with one workgroup).
 // TR: T_k^H x = d from the same pivots, U^H y = d then L^H x = y:
 //   y_j = conj(rp_j) (d_j - conj(c_{j-1}) y_{j-1}),  x_j = y_j - conj(a_{j+1} rp_j) x_{j+1}
 // (cyclic reduction with divisions took 7.7 us at 256 x 512, the forward solve
-// 5.5).
-template <int M, typename T, bool TR>
-__global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T> *__restrict__ rp,
-                                                        cx_t<T> *__restrict__ spec)
+// 5.1).
+template <int TN, int M, typename T, bool TR>
+__global__ __launch_bounds__(TN) __attribute__((amdgpu_waves_per_eu(2))) void tridiag_lu_kernel(
+    TriArgs a, const cx_t<T> *__restrict__ rp, cx_t<T> *__restrict__ spec)
 {
     using C = cx_t<T>;
     const int32_t dflag = cycle_done(a.done, a.gstride);
@@ -1110,76 +1119,83 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
     const double af = a.inst[blockIdx.y].afpc;
     const double2 e = a.eigen[k];
     C *S = spec + blockIdx.y * a.S + (size_t)k * a.nv;
-    // pivots in the chunk-interleaved order of tridiag_factor_kernel: thread
-    // t's rows t M + q at q NT + t, loaded coalesced straight into registers
-    const C *Rg = rp + ((size_t)blockIdx.y * gridDim.x + k) * (NT * M);
+    // pivots and band factors in chunk-interleaved order: thread t's rows
+    // t M + q at q TN + t, loaded coalesced straight into registers
+    const C *Rg = rp + ((size_t)blockIdx.y * gridDim.x + k) * (TN * M);
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    C *sd = reinterpret_cast<C *>(lds_raw);      // NT (M+1): right-hand side, then y, then x
-    __shared__ C wa[NT / 64], wb[NT / 64];
-    const C zero = cmk<C>(T(0), T(0)), one = cmk<C>(T(1), T(0));
+    constexpr int NW = TN / 64;
+    __shared__ C wa[2 * NW], wb[2 * NW];
+    const C zero = cmk<C>(T(0), T(0));
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    C rpv[M];                                     // pivots of rows t M .. t M + M - 1
-    C rprev;                                      // pivot of row t M - 1 (last row of chunk t - 1)
-    {
-        C v[M];
-#pragma unroll
-        for (int q = 0; q < M; ++q) {
-            const int j = t + q * NT;
-            v[q] = load_or_zero(S, j, j < a.nv);
-            rpv[q] = Rg[q * NT + t];
-        }
-        rprev = load_or_zero(Rg, (M - 1) * NT + t - 1, t > 0);
-        if (dflag) return;             // uniform over the block, before any barrier
-#pragma unroll
-        for (int q = 0; q < M; ++q) {
-            const int j = t + q * NT;
-            sd[j + j / M] = v[q];     // one pad slot per chunk
-        }
-    }
-    __syncthreads();
-    const int s = t * M, ls = t * (M + 1);
-    // sub- and super-diagonals of the chunk's rows (rows past nv: identity rows)
-    C av[M], cv[M];
+    // the wavefront's own 64 (M + 1) slots: its right-hand side, then its x
+    C *sd = reinterpret_cast<C *>(lds_raw) + wave * (64 * (M + 1));
+    const int w0 = wave * 64 * M + lane;          // first of the rows lane loads and stores: w0 + 64 q
+    C rpv[M], d[M];                               // pivots of rows t M .. t M + M - 1; d, then y
+    double gf[M], gb[M];                          // factors of the forward and the backward sweeps' diagonals (0: none)
+    C rprev = zero;                               // pivot of row t M - 1 (last row of chunk t - 1)
+    const double *gfw = TR ? a.gp : a.gm, *gbw = TR ? a.gm : a.gp;
+    double gprev = 0.0, gnext = 0.0;              // TR: super-diagonal of row t M - 1, sub-diagonal of row t M + M
 #pragma unroll
     for (int q = 0; q < M; ++q) {
-        double lo, mid, hi;
-        C bj;
-        tri_load<false>(a, s + q, lo, mid, hi);
-        tri_row<false>(a, af, e, s + q, lo, mid, hi, av[q], bj, cv[q]);
+        const int j = w0 + 64 * q;
+        d[q] = load_or_zero(S, j, j < a.nv);
     }
-    C cprev = zero, anext = zero;                 // TR: c of row s - 1, a of row s + M
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        rpv[q] = Rg[q * TN + t];
+        gf[q] = gfw[q * TN + t];
+        if (M < 16) gb[q] = gbw[q * TN + t];
+    }
     if constexpr (TR) {
-        double lo, mid, hi;
-        C u, v;
-        if (s > 0) {
-            tri_load<false>(a, s - 1, lo, mid, hi);
-            tri_row<false>(a, af, e, s - 1, lo, mid, hi, u, v, cprev);
-        }
-        tri_load<false>(a, s + M, lo, mid, hi);
-        tri_row<false>(a, af, e, s + M, lo, mid, hi, anext, u, v);
+        gprev = a.gp[t > 0 ? (M - 1) * TN + t - 1 : TN * M - 1];
+        gnext = a.gm[t < TN - 1 ? t + 1 : 0];   // row 0's is 0
+    } else {
+        rprev = load_or_zero(Rg, (M - 1) * TN + t - 1, t > 0);
     }
+    if (dflag) return;                            // uniform over the block, before any barrier
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        const int j = lane + 64 * q;
+        sd[j + j / M] = d[q];                     // one pad slot per chunk
+    }
+    wave_lds_fence();
+    const int ls = lane * (M + 1);
+#pragma unroll
+    for (int q = 0; q < M; ++q) d[q] = sd[ls + q];
+    const double exl = e.x * a.clo, eyl = e.y * a.clo, exh = e.x * a.chi, eyh = e.y * a.chi;
+    auto sub = [&](double g) { return cmk<C>((T)((exl * g) * af), (T)((eyl * g) * af)); };
+    auto sup = [&](double g) { return cmk<C>((T)((exh * g) * af), (T)((eyh * g) * af)); };
     // the recurrences' coefficients: y_j = w_j d_j - m_j y_{j-1} (w = 1 but for TR),
     // x_j = z_j y_j - n_j x_{j+1} (z = 1 for TR)
     auto mcoef = [&](int q) {
-        if constexpr (TR) return cmul(cconj(rpv[q]), cconj(q > 0 ? cv[q > 0 ? q - 1 : 0] : cprev));
-        else return cmul(av[q], q > 0 ? rpv[q > 0 ? q - 1 : 0] : rprev);
+        if constexpr (TR) return cmul(cconj(rpv[q]), cconj(sup(q > 0 ? gf[q > 0 ? q - 1 : 0] : gprev)));
+        else return cmul(sub(gf[q]), q > 0 ? rpv[q > 0 ? q - 1 : 0] : rprev);
     };
     auto ncoef = [&](int q) {
-        if constexpr (TR) return cconj(cmul(q < M - 1 ? av[q < M - 1 ? q + 1 : q] : anext, rpv[q]));
-        else return cmul(rpv[q], cv[q]);
+        if constexpr (TR) return cconj(cmul(sub(q < M - 1 ? gb[q < M - 1 ? q + 1 : q] : gnext), rpv[q]));
+        else return cmul(rpv[q], sup(gb[q]));
     };
-    auto wd = [&](int q) {
-        if constexpr (TR) return cmul(cconj(rpv[q]), sd[ls + q]);
-        else return sd[ls + q];
+    if constexpr (TR) {
+#pragma unroll
+        for (int q = 0; q < M; ++q) d[q] = cmul(cconj(rpv[q]), d[q]);
+    }
+    // long chunks: the coefficients are formed again for each sweep (the
+    // factors look changed) instead of held, 8 M more registers
+    auto again = [&](double (&g)[M]) {
+        if constexpr (M >= 8) {
+#pragma unroll
+            for (int q = 0; q < M; ++q) asm volatile("" : "+v"(g[q]));
+        }
     };
     // forward map of the chunk: y_{s+M-1} = A + B y_{s-1}
-    C A = wd(0), B = cneg(mcoef(0));
+    C A = d[0], B = cneg(mcoef(0));
 #pragma unroll
     for (int q = 1; q < M; ++q) {
         const C m = mcoef(q);
-        A = csub(wd(q), cmul(m, A));
+        A = csub(d[q], cmul(m, A));
         B = cneg(cmul(m, B));
     }
+    again(gf);
     C ea, eb, ta, tb;                             // maps of lanes 0 .. lane-1, of the wavefront
     affine_scan<false>(A, B, lane, ea, eb, ta, tb);
     if (lane == 0) {
@@ -1190,15 +1206,19 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
     C y = zero;                                   // y at the end of the previous wavefronts' rows
     for (int w = 0; w < wave; ++w) y = cadd(wa[w], cmul(wb[w], y));
     y = cadd(ea, cmul(eb, y));                    // y_{s-1}
+    if constexpr (M >= 16) {                      // on their way during the sweep
+#pragma unroll
+        for (int q = 0; q < M; ++q) gb[q] = gbw[q * TN + t];
+    }
 #pragma unroll
     for (int q = 0; q < M; ++q) {
-        y = csub(wd(q), cmul(mcoef(q), y));
-        sd[ls + q] = y;
+        y = csub(d[q], cmul(mcoef(q), y));
+        d[q] = y;
     }
     // backward map of the chunk: x_s = G + D x_{s+M}
     auto zy = [&](int q) {
-        if constexpr (TR) return sd[ls + q];
-        else return cmul(rpv[q], sd[ls + q]);
+        if constexpr (TR) return d[q];
+        else return cmul(rpv[q], d[q]);
     };
     C G = zy(M - 1), D = cneg(ncoef(M - 1));
 #pragma unroll
@@ -1207,25 +1227,29 @@ __global__ __launch_bounds__(NT) void tridiag_lu_kernel(TriArgs a, const cx_t<T>
         G = csub(zy(q), cmul(rc, G));
         D = cneg(cmul(rc, D));
     }
+    again(gb);
     C xa, xb;                                     // maps of lanes lane+1 .. 63
     affine_scan<true>(G, D, lane, xa, xb, ta, tb);
-    __syncthreads();                              // every thread has read wa / wb
     if (lane == 0) {
-        wa[wave] = ta;
-        wb[wave] = tb;
+        wa[NW + wave] = ta;
+        wb[NW + wave] = tb;
     }
     __syncthreads();
     C x = zero;                                   // x at the first row of the next wavefronts
-    for (int w = NT / 64 - 1; w > wave; --w) x = cadd(wa[w], cmul(wb[w], x));
+    for (int w = NW - 1; w > wave; --w) x = cadd(wa[NW + w], cmul(wb[NW + w], x));
     x = cadd(xa, cmul(xb, x));                    // x_{s+M}
 #pragma unroll
     for (int q = M - 1; q >= 0; --q) {
-        if constexpr (TR) x = csub(sd[ls + q], cmul(ncoef(q), x));
-        else x = cmul(rpv[q], csub(sd[ls + q], cmul(cv[q], x)));
+        if constexpr (TR) x = csub(d[q], cmul(ncoef(q), x));
+        else x = cmul(rpv[q], csub(d[q], cmul(sup(gb[q]), x)));
         sd[ls + q] = x;
     }
-    __syncthreads();
-    for (int j = t; j < a.nv; j += NT) S[j] = sd[j + j / M];
+    wave_lds_fence();
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        const int j = lane + 64 * q;
+        if (w0 + 64 * q < a.nv) S[w0 + 64 * q] = sd[j + j / M];
+    }
 }
 
 // out = in^T for every instance (blockIdx.z): in holds R rows of C, out C
@@ -1544,19 +1568,25 @@ template <> const float2 *lu_factors<float>(const vv_ctx *c) { return c->lu32; }
 template <typename T, bool TR>
 hipError_t tridiag_lu_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 {
-    TriArgs a{c->fft_rows, NT, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
+    TriArgs a{c->fft_rows, NT, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->lu_gm, nullptr, c->lu_gp,
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, done};
-    const int M = lu_rows(c->fft_rows);
-    const size_t lds = (size_t)NT * (M + 1) * sizeof(cx_t<T>);
+    const int TN = lu_threads(c->fft_rows), M = lu_rows(c->fft_rows);
+    const size_t lds = (size_t)TN * (M + 1) * sizeof(cx_t<T>);
     const cx_t<T> *rp = lu_factors<T>(c);
-    dim3 grid(c->nmodes, c->B), block(NT);
-    switch (M) {
-    case 1: launch_timed(c, tridiag_lu_kernel<1, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    case 2: launch_timed(c, tridiag_lu_kernel<2, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    case 4: launch_timed(c, tridiag_lu_kernel<4, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    case 8: launch_timed(c, tridiag_lu_kernel<8, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
-    default: launch_timed(c, tridiag_lu_kernel<16, T, TR>, grid, block, (uint32_t)lds, a, rp, spec); break;
+    dim3 grid(c->nmodes, c->B), block(TN);
+#define VV_TRI(TN_, M_) launch_timed(c, tridiag_lu_kernel<TN_, M_, T, TR>, grid, block, (uint32_t)lds, a, rp, spec)
+    if (TN == 64) {
+        if (M == 1) VV_TRI(64, 1);
+        else VV_TRI(64, 2);
+    } else if (TN == 128) {
+        if (M == 2) VV_TRI(128, 2);
+        else VV_TRI(128, 4);
+    } else {
+        if (M == 4) VV_TRI(256, 4);
+        else if (M == 8) VV_TRI(256, 8);
+        else VV_TRI(256, 16);
     }
+#undef VV_TRI
     return hipGetLastError();
 }
 
@@ -1592,15 +1622,23 @@ hipError_t tridiag_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 
 }  // namespace
 
-// rows per thread of the pivoted solve (NT threads per mode), and the pivots
-// stored per mode (NT x rows per thread, chunk-interleaved)
+// The pivoted solve's threads per mode and rows per thread.  Every wavefront
+// pays for two scans whatever its rows, so short systems take few wavefronts
+// (64 x 128: 4.0 us by one of 2 rows a lane, 4.5 by 256 threads of which half
+// hold no row; 1025 modes of 256 rows: 6.9 by 128 threads, 9.2 by 256; of 512:
+// 10.0 and 11.2), long ones 256 threads (513 modes of 2048 rows: 14.0 us by 256
+// threads of 8 rows, 15.7 by 512 of 4, 16.1 by 128 of 16; 1025 of 4096: 42, 56
+// by 512 of 8).
+int lu_threads(int nv) { return nv <= 128 ? 64 : nv <= 512 ? 128 : NT; }
+
 int lu_rows(int nv)
 {
-    const int m = (nv + NT - 1) / NT;
+    const int m = (nv + lu_threads(nv) - 1) / lu_threads(nv);
     return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : 16;
 }
 
-int lu_pivots_per_mode(int nv) { return NT * lu_rows(nv); }
+// pivots stored per mode (threads x rows per thread, chunk-interleaved)
+int lu_pivots_per_mode(int nv) { return lu_threads(nv) * lu_rows(nv); }
 
 int fft_rows_of(const vv_ctx *c) { return fft_rows(c); }
 
@@ -1697,8 +1735,8 @@ hipError_t launch_tridiag_factor(vv_ctx *c, double2 *rp64, float2 *rp32)
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, nullptr};
     dim3 grid((c->nmodes + NT - 1) / NT, c->B);
     const int M = lu_rows(c->fft_rows);
-    if (rp64) hipLaunchKernelGGL(tridiag_factor_kernel<double>, grid, dim3(NT), 0, c->stream, a, c->nmodes, M, rp64);
-    if (rp32) hipLaunchKernelGGL(tridiag_factor_kernel<float>, grid, dim3(NT), 0, c->stream, a, c->nmodes, M, rp32);
+    if (rp64) hipLaunchKernelGGL(tridiag_factor_kernel<double>, grid, dim3(NT), 0, c->stream, a, c->nmodes, lu_threads(c->fft_rows), M, rp64);
+    if (rp32) hipLaunchKernelGGL(tridiag_factor_kernel<float>, grid, dim3(NT), 0, c->stream, a, c->nmodes, lu_threads(c->fft_rows), M, rp32);
     return hipGetLastError();
 }
 

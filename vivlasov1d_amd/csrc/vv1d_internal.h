@@ -130,6 +130,7 @@ struct vv_ctx {
     double *h0, *h1p, *h1h, *h2p, *h2h;
     // preconditioner data (device)
     double2 *eigen;     // nmodes used (mode k = 0..fft_n/2)
+    double *lu_gm, *lu_gp;  // kinetic gm (0 at row 0) and gp (0 from row nv-1 on) in the pivots' order
     double *gm, *g0, *gp;   // per-row real factors of the bands (kinetic: of v; potential: phi differences per instance)
     double *vgrid;          // v_j (velocity moments)
     double2 *twiddle;   // exp(-2 pi i m / fft_n), m = 0..fft_n-1
@@ -299,6 +300,7 @@ hipError_t launch_irfft32(vv_ctx *c, const float2 *spec, float *y, const int32_t
 int irfft_mdot_rows(const vv_ctx *c, bool fp32);
 // rows per thread of the LU tridiagonal solve, and the pivots it stores per
 // mode (chunk-interleaved, >= nv)
+int lu_threads(int nv);
 int lu_rows(int nv);
 int lu_pivots_per_mode(int nv);
 hipError_t launch_irfft_mdot(vv_ctx *c, const double2 *spec, int col, const int32_t *done);
