@@ -115,9 +115,10 @@ int32_t vv_batch_size(const vv_ctx *ctx);
 int vv_set_active(vv_ctx *ctx, const int32_t *active);
 
 /* Graph replay of vv_snes_ksponly: the residual, P^-1, GMRES set-up and the
- * first `restart` Arnoldi steps are captured once into a HIP graph (per f/fh
- * pair and tolerances) and replayed as one launch per Newton step; Arnoldi
- * steps past an instance's convergence return at once.  Needs a non-null
+ * first `restart` Arnoldi steps are captured once (per f/fh pair and
+ * tolerances) into HIP graphs of a few Arnoldi steps each, replayed one after
+ * the other while some instance iterates; Arnoldi steps past an instance's
+ * convergence return at once.  Needs a non-null
  * stream.  Restart cycles, if any instance needs one, run as ordinary
  * launches. */
 int vv_set_graph(vv_ctx *ctx, int enable);

@@ -8,9 +8,9 @@ this module runs a set of instances with uneven grids together:
   covers all of its instances (instance = second grid dimension);
 * each bucket has its own HIP stream and host thread, so buckets of
   different shapes overlap on the GPU;
-* each Newton (SNES ksponly) step of a bucket is one replay of a captured HIP
-  graph (residual, P^-1, GMRES set-up and a full cycle of Arnoldi steps that
-  return at once past an instance's convergence), when ``graph`` is set;
+* each Newton (SNES ksponly) step of a bucket replays captured HIP graphs
+  (residual, P^-1, GMRES set-up and the Arnoldi steps of a cycle, a few steps a
+  graph, as long as some instance iterates), when ``graph`` is set;
 * launch shapes (FFT rows per workgroup, Gram-Schmidt vectors per thread) are
   chosen per bucket by timing the candidates on the bucket's own buffers
   (``autotune``).

@@ -169,6 +169,16 @@ int read_host(vv_ctx *c, size_t count, double *out)
     return VV_OK;
 }
 
+// The captured cycle, where there is one, is dropped: its kernels' arguments or
+// its stream change.
+void drop_graph(vv_ctx *c)
+{
+    for (hipGraphExec_t &g : c->graph_exec) {
+        if (g) (void)hipGraphExecDestroy(g);
+        g = nullptr;
+    }
+}
+
 int check_ctx(vv_ctx *c)
 {
     if (!c) return fail(nullptr, VV_ERR_INVALID, "null context");
@@ -660,6 +670,10 @@ int max_it_of(const GmresStatus *s, int B)
     return m;
 }
 
+// Reports of run_cycle are numbered from 1, those of the captured cycle's parts
+// from here.
+constexpr uint32_t kGraphSeq = 0x7fffffff - kGraphParts;
+
 // Waits for the B reports of slot `slot` numbered seq (a kernel enqueued before
 // stores them); *done: every instance's cycle has ended.  The stream is looked
 // at now and then, so an error on the device ends the wait.
@@ -709,7 +723,7 @@ int run_cycle(vv_ctx *c, bool fp32, double *x, bool store, double *update = null
         }
         if (it >= 1) {
             c->report_out = c->host_poll_dev + (size_t)((it - 1) & 1) * c->B;
-            c->report_seq = c->report_seq >= 0x7fffffffu ? 1 : c->report_seq + 1;
+            c->report_seq = c->report_seq >= kGraphSeq - 1 ? 1 : c->report_seq + 1;
         }
         const int r = fp32 ? arnoldi_step32(c, it) : arnoldi_step(c, it);
         c->report_out = nullptr;
@@ -773,48 +787,70 @@ int ksp_solve_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_params *k
     return VV_OK;
 }
 
-// The first GMRES cycle of SNESSolve_KSPONLY as one captured graph:
-// V_0 = P^-1 F(f); cycle start; `restart` Arnoldi steps (steps past an
-// instance's convergence return at once); x = V y and the statuses.
-// The graph is kept per (f, fh) pair and replayed while they stay the same;
-// the KSP tolerances are kernel arguments, so a change re-captures too.
+// Part `part` of the captured cycle: V_0 = P^-1 F(f) and the cycle start (part
+// 0), then its Arnoldi steps; the last step's first kernel reports the end of
+// the step before.
+int graph_part(vv_ctx *c, int part, const double *f, const double *fh, const vv_ksp_params *kp)
+{
+    const int it0 = part * kGraphSteps, end = it0 + kGraphSteps, it1 = end < c->p.restart ? end : c->p.restart;
+    VV_CHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "begin capture");
+    c->capturing = true;
+    const uint32_t seq = c->report_seq;
+    int r = VV_OK;
+    c->pend_it = it0 - 1;                 // the part before ended with this update due
+    c->pend_nb = c->graph_nb;
+    if (part == 0) {
+        set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
+        r = residual_start(c, f, fh);
+    }
+    for (int it = it0; it < it1 && r == VV_OK; ++it) {
+        if (it == it1 - 1 && it >= 1) {
+            c->report_out = c->host_poll_dev + (size_t)(part & 1) * c->B;
+            c->report_seq = kGraphSeq + part;
+        }
+        r = arnoldi_step(c, it);
+        c->report_out = nullptr;
+    }
+    hipGraph_t g = nullptr;
+    const hipError_t e = hipStreamEndCapture(c->stream, &g);
+    c->capturing = false;
+    c->report_seq = seq;
+    c->graph_nb = c->pend_nb;
+    c->pend_it = -1;
+    c->pend_start = 0;
+    if (r != VV_OK || e != hipSuccess) {
+        if (g) (void)hipGraphDestroy(g);
+        return r != VV_OK ? r : hipfail(c, e, "graph capture");
+    }
+    const hipError_t ei = hipGraphInstantiate(&c->graph_exec[part], g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (ei != hipSuccess) {
+        c->graph_exec[part] = nullptr;
+        return hipfail(c, ei, "graph instantiate");
+    }
+    return VV_OK;
+}
+
+// The first GMRES cycle of SNESSolve_KSPONLY as captured graphs, kept per (f,
+// fh) pair and replayed while they stay the same; the KSP tolerances are kernel
+// arguments, so a change re-captures too.  The cycle is cut into parts of
+// kGraphSteps steps, each captured when it is first needed: as in run_cycle the
+// host waits for the report of a part's last step, while that step's other
+// kernels still run, and launches the next part only if some instance still
+// iterates.  As one graph of `restart` steps most of the cycle's kernels
+// returned at once (12 of 30 steps needed): a step of 16 x (128 x 256) took 2.70
+// ms, now 2.36, of 64 instances in 16 shapes side by side 34.7, now 32.5.  Parts
+// of 2, 3, 4, 6 and 8 steps: 2.46, 2.27, 2.36, 2.36, 2.47 ms for the former, 3.48,
+// 3.40, 3.35, 3.33, 3.34 for 6 x (256 x 512).
 int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
 {
-    const bool same = c->graph_exec != nullptr && c->graph_f == f && c->graph_fh == fh &&
+    const int parts = (c->p.restart + kGraphSteps - 1) / kGraphSteps;
+    const bool same = c->graph_exec[0] != nullptr && c->graph_f == f && c->graph_fh == fh &&
                       c->graph_kp[0] == kp->rtol && c->graph_kp[1] == kp->atol && c->graph_kp[2] == kp->dtol &&
                       c->graph_kp[3] == (double)kp->max_it;
     if (!same) {
-        if (c->graph_exec) {
-            (void)hipGraphExecDestroy(c->graph_exec);
-            c->graph_exec = nullptr;
-        }
+        drop_graph(c);
         if (c->stream == nullptr) return fail(c, VV_ERR_INVALID, "graph capture needs a non-null stream");
-        VV_CHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "begin capture");
-        c->capturing = true;
-        int r = VV_OK;
-        hipError_t le = hipSuccess;
-        do {
-            set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
-            if ((r = residual_start(c, f, fh))) break;
-            for (int it = 0; it < c->p.restart && r == VV_OK; ++it) r = arnoldi_step(c, it);
-            if (r) break;
-            if ((le = launch_update(c)) != hipSuccess) break;
-            le = launch_build_solution(c, c->D, nullptr, true, c->host_status_dev);
-        } while (0);
-        hipGraph_t g = nullptr;
-        const hipError_t e = hipStreamEndCapture(c->stream, &g);
-        c->capturing = false;
-        if (r != VV_OK || le != hipSuccess || e != hipSuccess) {
-            if (g) (void)hipGraphDestroy(g);
-            if (r != VV_OK) return r;
-            return hipfail(c, le != hipSuccess ? le : e, "graph capture");
-        }
-        const hipError_t ei = hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (ei != hipSuccess) {
-            c->graph_exec = nullptr;
-            return hipfail(c, ei, "graph instantiate");
-        }
         c->graph_f = f;
         c->graph_fh = fh;
         c->graph_kp[0] = kp->rtol;
@@ -822,7 +858,28 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
         c->graph_kp[2] = kp->dtol;
         c->graph_kp[3] = (double)kp->max_it;
     }
-    VV_CHECK(hipGraphLaunch(c->graph_exec, c->stream), "graph launch");
+    // no report of an earlier replay is taken for this one's (the stream is idle
+    // as far as the reports go: every solve ends drained)
+    std::memset(c->host_poll, 0, 2 * (size_t)c->B * sizeof(uint32_t));
+    bool stop = false;
+    for (int p = 0; p < parts && !stop; ++p) {
+        int r = c->graph_exec[p] == nullptr ? graph_part(c, p, f, fh, kp) : VV_OK;
+        if (r == VV_OK) {
+            const hipError_t e = hipGraphLaunch(c->graph_exec[p], c->stream);
+            if (e != hipSuccess) r = hipfail(c, e, "graph launch");
+        }
+        if (r == VV_OK && p + 1 < parts) r = wait_report(c, p & 1, kGraphSeq + p, &stop);
+        if (r != VV_OK) {
+            (void)hipStreamSynchronize(c->stream);   // no part's report may come after this solve
+            return r;
+        }
+    }
+    if (!stop) {
+        c->pend_it = c->p.restart - 1;
+        c->pend_nb = c->graph_nb;
+        VV_CHECK(launch_update(c), "Hessenberg update");
+    }
+    VV_CHECK(launch_build_solution(c, c->D, nullptr, true, c->host_status_dev), "build solution");
     VV_CHECK(hipStreamSynchronize(c->stream), "synchronize");
     return VV_OK;
 }
@@ -1237,7 +1294,7 @@ int vv_ctx_destroy(vv_ctx *c)
 {
     if (!c) return VV_OK;
     (void)hipStreamSynchronize(c->stream);
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
+    drop_graph(c);
     void *bufs[] = {c->inst,   c->active, c->h0,      c->h1p,     c->h1h,  c->h2p,   c->h2h,    c->eigen,
                     c->gm,     c->g0,     c->gp,      c->twiddle, c->twiddle32, c->spec, c->pinv, c->plam, c->pwork,
                     c->X,      c->rhs,    c->D,       c->basis,   c->basis32, c->R,   c->partial, c->dscalar,
@@ -1263,10 +1320,7 @@ int vv_ctx_destroy(vv_ctx *c)
 int vv_set_stream(vv_ctx *c, void *stream)
 {
     if (int r = check_ctx(c)) return r;
-    if (c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
+    drop_graph(c);
     c->stream = reinterpret_cast<hipStream_t>(stream);
     return VV_OK;
 }
@@ -1304,10 +1358,7 @@ int vv_set_graph(vv_ctx *c, int enable)
     if (enable)
         if (int r = no_diss(c, "graph replay")) return r;
     if (enable && c->stream == nullptr) return fail(c, VV_ERR_INVALID, "graph replay needs a non-null stream");
-    if (!enable && c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
+    if (!enable) drop_graph(c);
     c->use_graph = enable != 0;
     return VV_OK;
 }
@@ -1319,10 +1370,7 @@ int vv_set_tuning(vv_ctx *c, int32_t fft_rows, int32_t cgs_ept)
         return fail(c, VV_ERR_INVALID, "fft_rows must be 0 or even, >= 2, with fft_rows * (FFT length) <= 8192");
     if (cgs_ept != 0 && cgs_ept != 1 && cgs_ept != 2 && cgs_ept != 4 && cgs_ept != 8)
         return fail(c, VV_ERR_INVALID, "cgs_ept must be 0, 1, 2, 4 or 8");
-    if (c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
+    drop_graph(c);
     c->tune_fft_rows = fft_rows;
     c->tune_cgs_ept = cgs_ept;
     return VV_OK;
@@ -1331,10 +1379,7 @@ int vv_set_tuning(vv_ctx *c, int32_t fft_rows, int32_t cgs_ept)
 int vv_set_fusion(vv_ctx *c, int enable)
 {
     if (int r = check_ctx(c)) return r;
-    if (c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
+    drop_graph(c);
     c->fuse = enable != 0;
     return VV_OK;
 }
@@ -1356,10 +1401,7 @@ int vv_autotune(vv_ctx *c, int32_t *fft_rows, int32_t *cgs_ept)
     if (int r = check_ctx(c)) return r;
     if (c->p.precond == VV_PRECOND_NONE)
         return fail(c, VV_ERR_UNSUPPORTED, "autotune needs a tensor-product preconditioner");
-    if (c->graph_exec) {
-        (void)hipGraphExecDestroy(c->graph_exec);
-        c->graph_exec = nullptr;
-    }
+    drop_graph(c);
     const int prof = c->prof;
     c->prof = 0;
     hipEvent_t e0, e1;

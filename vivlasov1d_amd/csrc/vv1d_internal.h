@@ -14,6 +14,8 @@
 namespace vv {
 
 constexpr int kMaxRestart = 64;     // GMRES restart limit (basis of restart+1 vectors)
+constexpr int kGraphSteps = 6;      // Arnoldi steps of a part of the captured cycle
+constexpr int kGraphParts = (kMaxRestart + kGraphSteps - 1) / kGraphSteps;
 constexpr int kMaxNx = 4096;        // largest x size
 constexpr int kMaxNv = 8192;
 constexpr int kReduceBlocks = 512;  // fixed block count of N-sized reductions
@@ -165,7 +167,7 @@ struct vv_ctx {
     uint32_t *host_poll;            // pinned, 2 slots of B words: reports of the Hessenberg updates
     uint32_t *host_poll_dev;        // the same memory as the device addresses it
     uint32_t *report_out;           // set for one launch: where the Hessenberg update reports
-    uint32_t report_seq;            // number of the last report asked for (below 2^31)
+    uint32_t report_seq;            // number of the last report asked for (below kGraphSeq)
     int pend_it, pend_nb;           // Arnoldi step whose Hessenberg update is due (-1: none), its norm partials
     int pend_start;                 // a cycle start is due instead (HessArgs::start; 0: none)
     vv::SolveStart start;           // what a first cycle starts with
@@ -191,9 +193,11 @@ struct vv_ctx {
     // kernel fusion (default on): the Arnoldi step's irFFT and CGS dots in
     // one launch where the geometry allows; results are bit-identical
     bool fuse;
-    // captured first GMRES cycle of SNESSolve_KSPONLY (graph replay mode)
+    // captured first GMRES cycle of SNESSolve_KSPONLY (graph replay mode), in
+    // parts of kGraphSteps Arnoldi steps; the norm partials of a step
     bool use_graph, capturing;
-    hipGraphExec_t graph_exec;
+    hipGraphExec_t graph_exec[vv::kGraphParts];
+    int graph_nb;
     const double *graph_f, *graph_fh;
     double graph_kp[4];
     // dissipation term (VV_DISSIPATION_*) and its parameters; moment vectors
