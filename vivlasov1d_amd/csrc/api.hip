@@ -428,7 +428,7 @@ int fwd_jac(vv_ctx *c, const double *u, const double *uscale, const int32_t *don
 int pc_residual(vv_ctx *c, const double *f, const double *fh, double *y)
 {
     if (!rows_apply(c) || diss_on(c)) {
-        VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, c->X), "residual");
+        VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual_sep(c, f, fh, c->X), "residual");
         if (int r = diss_function(c, f, fh, c->X)) return r;
         return precond(c, c->X, y, nullptr);
     }
@@ -452,7 +452,7 @@ int residual_start(vv_ctx *c, const double *f, const double *fh)
     }
     const double F = b_field(c), S = b_spec(c);
     if (!rows_apply(c) || diss_on(c)) {
-        VV_PLAUNCH(P_RES, 3 * F, -1, launch_residual(c, f, fh, c->X), "residual");
+        VV_PLAUNCH(P_RES, 3 * F, -1, launch_residual_sep(c, f, fh, c->X), "residual");
         if (int r = diss_function(c, f, fh, c->X)) return r;
         VV_PLAUNCH(P_RFFT, F + S, -1, launch_rfft(c, c->X, c->spec, nullptr), "rfft");
     } else {
@@ -1498,7 +1498,7 @@ int vv_jacobian_apply(vv_ctx *c, const double *u, double *y)
     if (int r = check_ctx(c)) return r;
     if (!u || !y) return fail(c, VV_ERR_INVALID, "null field");
     if (u == y) return fail(c, VV_ERR_INVALID, "jacobian_apply: u and y must not alias");
-    VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian(c, u, nullptr, y), "jacobian");
+    VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian_plain(c, u, y), "jacobian");
     return diss_jacobian(c, u, nullptr, y, nullptr);
 }
 

@@ -1,13 +1,14 @@
 // The Arakawa J1 / J2 / J4 stencils on one lane's sliding register window,
 // shared by the bracket kernels (bracket.hip) and the Jacobian-vector product
-// fused with the forward rFFT (spectral.hip).
+// fused with the forward rFFT (spectral.hip, rows.hip).
 //
 // Every expression keeps the reference's IEEE operation order
 // (PoissonBracket.pyx:100-113, 221-234, 360-389; C left-to-right) and is
 // evaluated without contraction whatever the including unit's setting (the
-// pragma below; the spectral unit is built with -ffp-contract=fast-honor-
-// pragmas), so both kernels produce the reference's unfused double results
-// bit for bit.
+// pragma below), so the callbacks that return a bracket produce the
+// reference's unfused double results bit for bit.  The solver's own J u and
+// F(f) use the factored form (SepWin), with the products fused explicitly, so
+// every kernel that forms them agrees bit for bit whatever its unit's setting.
 //
 // The window of a lane at column cx, output row cy of a tile (read through
 // a functor of (row, column, column offset)) holds the first argument F and the second
@@ -137,6 +138,121 @@ __device__ __forceinline__ T arakawa_add(const ArakawaWin<T> &w, T base, T facto
 #undef H
 }
 
+// The same stencils where H = h0(v) + phi(x), as H_ave always is: every term is
+// a difference of H, so with the row differences of h0 and the column
+// differences of phi
+//   c1 J1 + c2 J2 = A+ D+ + A0 D0 + A- D- + A2 D2 - (B+ E+ + B0 E0 + B- E- + B2 E2),
+// D+, D0, D- = F(1, b) - F(-1, b) for b = 1, 0, -1, D2 = F(2, 0) - F(-2, 0);
+// E+, E0, E- = F(b, 1) - F(b, -1) for b = 1, 0, -1, E2 = F(0, 2) - F(0, -2);
+// A depends on the row, B on the column:
+//   A+- = c1 v+- + c2 (V + v2+-), A0 = 2 c1 V, A2 = c2 V   (B alike from phi)
+// v+ = h0(1) - h0(0), v- = h0(0) - h0(-1), V = h0(1) - h0(-1), v2+ = h0(2) -
+// h0(0), v2- = h0(0) - h0(-2).  No H in LDS, 5 reads and 17 operations a point
+// instead of 10 and ~75, and closer to exact: the unfactored stencil subtracts
+// values of H rounded at |H|, which costs |H| / (hv dH/dv) ulps.  The solver's
+// J u and P^-1 F use it; the callbacks that return F and J u themselves keep the
+// reference's operation order above.
+__device__ __forceinline__ double phi_ave(double x0, double x1, double x2, double x3)
+{
+#pragma clang fp contract(off)
+    return ((0.5 * x0 + 0.5 * x1) + 0.5 * x2) + 0.5 * x3;
+}
+
+// c1, c2 of factor {F, H}: J1, J2 or J4 = 2 J1 - J2
+__device__ __forceinline__ void sep_weights(int kind, double factor, double af1, double af2, double &c1, double &c2)
+{
+#pragma clang fp contract(off)
+    c1 = kind == VV_BRACKET_J2 ? 0.0 : kind == VV_BRACKET_J4 ? 2.0 * (factor * af1) : factor * af1;
+    c2 = kind == VV_BRACKET_J1 ? 0.0 : kind == VV_BRACKET_J4 ? -(factor * af2) : factor * af2;
+}
+
+// A (or B) from the five values of h0 (or phi) around the centre h
+template <typename T>
+__device__ __forceinline__ void sep_coef(double hmm, double hm, double h, double hp, double hpp, double c1, double c2,
+                                         T (&k)[4])
+{
+#pragma clang fp contract(off)
+    const double W = hp - hm;
+    k[0] = (T)(c1 * (hp - h) + c2 * (W + (hpp - h)));
+    k[1] = (T)(2.0 * (c1 * W));
+    k[2] = (T)(c1 * (h - hm) + c2 * (W + (h - hmm)));
+    k[3] = (T)(c2 * W);
+}
+
+// row j's coefficients from h0 itself (rows past the grid read as 0: they only
+// meet rows whose result is not formed)
+template <typename T>
+__device__ __forceinline__ void sep_row(const double *__restrict__ h0, int j, int nv, double c1, double c2, T *k)
+{
+    double h[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        const int r = j - 2 + q;
+        h[q] = r >= 0 && r < nv ? h0[r] : 0.0;
+    }
+    T a[4];
+    sep_coef(h[0], h[1], h[2], h[3], h[4], c1, c2, a);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) k[q] = a[q];
+}
+
+// The first argument's window alone.
+template <typename T>
+struct SepWin {
+    T f0[5], fm[3], fp[3], fm2, fp2;
+
+    template <typename RF>
+    __device__ __forceinline__ void load(const RF &F, int cy, int cx)
+    {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) f0[k] = F(cy - 2 + k, cx, 0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            fm[k] = F(cy - 1 + k, cx, -1);
+            fp[k] = F(cy - 1 + k, cx, 1);
+        }
+        fm2 = F(cy, cx, -2);
+        fp2 = F(cy, cx, 2);
+    }
+
+    template <typename RF>
+    __device__ __forceinline__ void advance(const RF &F, int cn, int cx)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f0[k] = f0[k + 1];
+        f0[4] = F(cn + 2, cx, 0);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            fm[k] = fm[k + 1];
+            fp[k] = fp[k + 1];
+        }
+        fm[2] = F(cn + 1, cx, -1);
+        fp[2] = F(cn + 1, cx, 1);
+        fm2 = F(cn, cx, -2);
+        fp2 = F(cn, cx, 2);
+    }
+
+    // the weighted bracket at the centre; far: the kind has J2 terms (their
+    // points at distance 2 are not read into a J1 result)
+    __device__ __forceinline__ T bracket(const T *A, const T (&B)[4], bool far) const
+    {
+#pragma clang fp contract(off)
+        T s = A[0] * (fp[2] - fm[2]), t = B[0] * (fp[2] - fp[0]);
+        s = fma_t(A[1], fp[1] - fm[1], s);
+        t = fma_t(B[1], f0[3] - f0[1], t);
+        s = fma_t(A[2], fp[0] - fm[0], s);
+        t = fma_t(B[2], fm[2] - fm[0], t);
+        if (far) {
+            s = fma_t(A[3], fp2 - fm2, s);
+            t = fma_t(B[3], f0[4] - f0[0], t);
+        }
+        return s - t;
+    }
+
+    static __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+    static __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+};
+
 // H_ave at (i, j) from its 1D factors: ((((h0_j + .5 h1p_i) + .5 h1h_i) +
 // .5 h2p_i) + .5 h2h_i), exactly the value the reference's 2D Have vector
 // holds (PETScVlasovSolver.pyx:145-149).
@@ -152,6 +268,14 @@ __device__ __forceinline__ T jacobian_base(T ht_inv, T u)
 {
 #pragma clang fp contract(off)
     return T(0) + ht_inv * u;
+}
+
+// the result times the Krylov vector's scale, rounded on its own
+template <typename T>
+__device__ __forceinline__ T scaled(T f, T s)
+{
+#pragma clang fp contract(off)
+    return f * s;
 }
 
 }  // namespace

@@ -42,9 +42,8 @@ constexpr int ROWS_PER_WAVE = TY / (NT / 64);
 // M^T g = -{R g, H} evaluated on all rows: this mode with factor = -1.
 enum { MODE_RESIDUAL = 0, MODE_JACOBIAN = 1, MODE_ACCUMULATE = 2, MODE_TRANSPOSED = 3 };
 
-// T is the field type: double (bit-exact FP64 path) or float (Jacobian-apply
-// of the FP32 GMRES cycle of the mixed-precision solver; H_ave is composed in
-// FP64 and rounded once, the stencil runs in float).
+// T is the field type: double, or float (bracket_sep_kernel: J u of the FP32
+// GMRES cycle of the mixed-precision solver, coefficients rounded once).
 // Instance b of a batched context is blockIdx.y: its fields start at b * N,
 // its x-factors of H at b * nx, its GMRES state b * gstride bytes after
 // instance 0's (uscale, done), its hx-dependent factors in inst[b].
@@ -69,12 +68,12 @@ struct BrArgs {
                            // Vec.set(0.) followed by PoissonBracket.function)
 };
 
-template <int KIND, int MODE, typename T>
-__global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
+template <int KIND, int MODE>
+__global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<double> a)
 {
     const int b = blockIdx.y;
-    __shared__ T sF[HY][HX];
-    __shared__ T sH[HY][HX];
+    __shared__ double sF[HY][HX];
+    __shared__ double sH[HY][HX];
     __shared__ double sX[4][HX];      // h1p, h1h, h2p, h2h (or the x-only H) of the tile's columns
     __shared__ double sV[HY];         // h0 of the tile's rows
 
@@ -82,10 +81,10 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     const BrTile tile = br_tile(blockIdx.x, nx, nv);
     const int i0 = tile.i0, j0 = tile.j0;
     const size_t fo = (size_t)b * a.N, xo = (size_t)b * nx;
-    const T *__restrict__ fin = a.f + fo;
-    const T *__restrict__ fhin = (MODE == MODE_RESIDUAL) ? a.fh + fo : nullptr;
-    T *__restrict__ yout = a.y + fo;
-    const T half = T(0.5);
+    const double *__restrict__ fin = a.f + fo;
+    const double *__restrict__ fhin = (MODE == MODE_RESIDUAL) ? a.fh + fo : nullptr;
+    double *__restrict__ yout = a.y + fo;
+    const double half = 0.5;
     const bool factors = (a.h2d == nullptr && a.hxv == nullptr);
 
     // Phase 1: every global load of the block is issued before anything waits
@@ -116,13 +115,13 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
         if (factors && gj >= 0) vf = a.h0[gj];
     }
     constexpr int NQ = (HY * HX + NT - 1) / NT;
-    T fa[NQ], fb[NQ];
+    double fa[NQ], fb[NQ];
     double hq[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int idx = threadIdx.x + q * NT;
-        fa[q] = T(0);
-        fb[q] = T(0);
+        fa[q] = 0.0;
+        fb[q] = 0.0;
         hq[q] = 0.0;
         if (idx < HY * HX) {
             const int r = idx / HX;
@@ -148,16 +147,7 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     }
     __syncthreads();
 
-    const T us = (T)usd;
-    // FP32: H_ave enters every Arakawa term only through differences, so the
-    // float tile holds H_ave - h0(j0 + TY/2) (h0 at the centre row of the
-    // tile's 16-row band, 0 past the grid), formed in FP64 and rounded once;
-    // the rounding error is then relative to H's variation over the band
-    // (h0's over its rows plus the x-dependent part), not to |H| (which would
-    // cost ~|H|/(hv dH/dv) ulps on fine v grids).  The offset depends on the
-    // band only, so a kernel that stages other tiles of the same rows (the
-    // fused J u + rFFT) forms the same values.
-    const double href = (sizeof(T) == 4 && factors) ? sV[HY / 2] : 0.0;
+    const double us = usd;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int idx = threadIdx.x + q * NT;
@@ -166,11 +156,11 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
             const int c = idx - r * HX;
             const int gj = br_halo_row(tile, r, nv);
             const bool in = gj >= 0;
-            T fv;
+            double fv;
             if (MODE == MODE_RESIDUAL) {
                 fv = half * fb[q] + half * fa[q];            // Fave (PETScNLVlasovMP.pyx:44-46)
             } else if (MODE == MODE_TRANSPOSED) {
-                fv = (gj >= 2 && gj < nv - 2) ? fa[q] * us : T(0);
+                fv = (gj >= 2 && gj < nv - 2) ? fa[q] * us : 0.0;
             } else if (MODE == MODE_JACOBIAN) {
                 fv = fa[q] * us;                             // == VecScale'd Krylov vector
             } else {
@@ -181,13 +171,11 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
             // outside the grid H is 0: those cells only meet rows whose result
             // is not formed (j < 2 or j >= nv - 2) except in the transposed mode
             if (a.h2d != nullptr) {
-                sH[r][c] = in ? (T)hq[q] : T(0);
+                sH[r][c] = in ? hq[q] : 0.0;
             } else if (a.hxv != nullptr) {
-                sH[r][c] = in ? (T)sX[0][c] : T(0);
-            } else if (sizeof(T) == 8) {
-                sH[r][c] = in ? (T)compose_have(sV[r], sX[0][c], sX[1][c], sX[2][c], sX[3][c]) : T(0);
+                sH[r][c] = in ? sX[0][c] : 0.0;
             } else {
-                sH[r][c] = in ? (T)(compose_have(sV[r], sX[0][c], sX[1][c], sX[2][c], sX[3][c]) - href) : T(0);
+                sH[r][c] = in ? compose_have(sV[r], sX[0][c], sX[1][c], sX[2][c], sX[3][c]) : 0.0;
             }
         }
     }
@@ -199,13 +187,13 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
     if (MODE != MODE_RESIDUAL && i >= nx) return;
     const int cx = lane + 2;
     double sq = 0.0;
-    const T ht_inv = (T)a.ht_inv, af1 = (T)a.inst[b].af1, af2 = (T)a.inst[b].af2, factor = (T)a.factor;
+    const double ht_inv = a.ht_inv, af1 = a.inst[b].af1, af2 = a.inst[b].af2, factor = a.factor;
 
     // Each lane walks down its column with the stencil values of F and H in
     // a sliding register window (arakawa.h).  Same values, same expressions.
     const int rr0 = wave * ROWS_PER_WAVE;
-    const TileRd<T, HX> rF{&sF[0][0]}, rH{&sH[0][0]};
-    ArakawaWin<T> win;
+    const TileRd<double, HX> rF{&sF[0][0]}, rH{&sH[0][0]};
+    ArakawaWin<double> win;
     win.load(rF, rH, rr0 + 2, cx);
 #pragma unroll
     for (int q = 0; q < ROWS_PER_WAVE; ++q) {
@@ -213,18 +201,18 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
         const int j = j0 + rr;
         if (j < nv && (MODE != MODE_RESIDUAL || i < nx)) {
             const size_t o = (size_t)j * nx + i;
-            T base;
+            double base;
             if (MODE == MODE_RESIDUAL) {
-                const T fder = fin[o] - fhin[o];                 // Fder = (0 + F) - Fh
-                base = T(0) + ht_inv * fder;                     // Y = 0; Y += Fder/dt
+                const double fder = fin[o] - fhin[o];                 // Fder = (0 + F) - Fh
+                base = 0.0 + ht_inv * fder;                     // Y = 0; Y += Fder/dt
             } else if (MODE == MODE_JACOBIAN) {
                 base = jacobian_base(ht_inv, win.f0[2]);         // Y = 0; Y += u/dt
             } else if (MODE == MODE_TRANSPOSED) {
-                base = (T)a.alpha * (fin[o] * us);
+                base = a.alpha * (fin[o] * us);
             } else {
-                base = a.store ? T(0) : yout[o];
+                base = a.store ? 0.0 : yout[o];
             }
-            T out = base;
+            double out = base;
             if (MODE == MODE_TRANSPOSED || (j >= 2 && j < nv - 2))
                 out = arakawa_add<KIND>(win, base, factor, af1, af2);
             yout[o] = out;
@@ -244,6 +232,100 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<T> a)
             for (int w = 0; w < NT / 64; ++w) s += red[w];
             a.part[b * a.pstride + blockIdx.x] = s;
         }
+    }
+}
+
+// J u and F(f) inside the solver: the same tiles with the bracket split into row
+// and column coefficients (SepWin, arakawa.h), so one tile in LDS (12 KB: as
+// many wavefronts a CU as there are slots for, against 24 with H beside it) and
+// a quarter of the arithmetic.  F(f) at 1024 x 2048 18.6 us unfactored, 13.9 here;
+// J u at 2048 x 1024 13.7, 9.6.  T is double, or float for the FP32 cycle.
+template <bool FAR, int MODE, typename T>
+__global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
+{
+    const int b = blockIdx.y;
+    __shared__ T sF[HY][HX];
+    __shared__ double sP[HX];                      // x-part of H of the tile's columns
+    __shared__ __align__(16) T sA[TY][4];          // coefficients of its rows
+
+    const int nx = a.nx, nv = a.nv, t = threadIdx.x;
+    const BrTile tile = br_tile(blockIdx.x, nx, nv);
+    const int i0 = tile.i0, j0 = tile.j0;
+    const size_t fo = (size_t)b * a.N, xo = (size_t)b * nx;
+    const T *__restrict__ fin = a.f + fo;
+    const T *__restrict__ fhin = (MODE == MODE_RESIDUAL) ? a.fh + fo : nullptr;
+    T *__restrict__ yout = a.y + fo;
+    const T half = T(0.5);
+    const int32_t dflag =
+        (a.done != nullptr) ? *reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(a.done) + b * a.gstride)
+                            : 0;
+    // batched: a finished instance skips its loads (one instance keeps them
+    // in flight with the flag's)
+    if (gridDim.y > 1 && dflag) return;
+    const double usd = (a.uscale != nullptr)
+                           ? *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a.uscale) + b * a.gstride)
+                           : 1.0;
+    double c1, c2;
+    sep_weights(kind, a.factor, a.inst[b].af1, a.inst[b].af2, c1, c2);
+    constexpr int NQ = (HY * HX + NT - 1) / NT;
+    T fa[NQ], fb[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int idx = t + q * NT;
+        fa[q] = T(0);
+        fb[q] = T(0);
+        if (idx < HY * HX) {
+            const int r = idx / HX;
+            const int64_t o = br_halo_offset(tile, r, idx - r * HX, nx, nv);
+            if (o >= 0) {
+                fa[q] = fin[o];
+                if (MODE == MODE_RESIDUAL) fb[q] = fhin[o];
+            }
+        }
+    }
+    double phi = 0.0;
+    if (t < HX) {
+        const size_t gi = xo + br_halo_column(tile, t, nx);
+        phi = phi_ave(a.h1p[gi], a.h1h[gi], a.h2p[gi], a.h2h[gi]);
+    }
+    T k[4];
+    const bool krow = t >= 128 && t < 128 + TY;
+    if (krow) sep_row(a.h0, j0 + t - 128, nv, c1, c2, k);
+    if (dflag) return;                 // uniform over the block, before any barrier
+    const T us = (T)usd;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int idx = t + q * NT;
+        if (idx < HY * HX) (&sF[0][0])[idx] = MODE == MODE_RESIDUAL ? half * fb[q] + half * fa[q] : fa[q];
+    }
+    if (t < HX) sP[t] = phi;
+    if (krow) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sA[t - 128][q] = k[q];
+    }
+    __syncthreads();
+    const int lane = t & 63, wave = t >> 6;
+    const int i = i0 + lane, cx = lane + 2, rr0 = wave * ROWS_PER_WAVE;
+    if (i >= nx) return;
+    const T ht_inv = (T)a.ht_inv;
+    T B[4];
+    sep_coef(sP[cx - 2], sP[cx - 1], sP[cx], sP[cx + 1], sP[cx + 2], c1, c2, B);
+    const TileRd<T, HX> rF{&sF[0][0]};
+    SepWin<T> win;
+    win.load(rF, rr0 + 2, cx);
+#pragma unroll
+    for (int q = 0; q < ROWS_PER_WAVE; ++q) {
+        const int rr = rr0 + q, j = j0 + rr;
+        if (j < nv) {
+            const size_t o = (size_t)j * nx + i;
+            T out;
+            if (MODE == MODE_RESIDUAL) out = T(0) + ht_inv * (fin[o] - fhin[o]);
+            else out = jacobian_base(ht_inv, win.f0[2]);
+            if (j >= 2 && j < nv - 2) out += win.bracket(sA[rr], B, FAR);
+            if (MODE == MODE_JACOBIAN) out = scaled(out, us);      // J is linear
+            yout[o] = out;
+        }
+        if (q + 1 < ROWS_PER_WAVE) win.advance(rF, rr + 3, cx);
     }
 }
 
@@ -360,21 +442,31 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
         csum[b * cstride + (size_t)(tile.j0 / TY) * nx + i] = ((sX[0][lane] + sX[1][lane]) + sX[2][lane]) + sX[3][lane];
 }
 
-template <int MODE, typename T>
-hipError_t launch_mode(vv_ctx *c, BrArgs<T> a)
+template <int MODE>
+hipError_t launch_mode(vv_ctx *c, const BrArgs<double> &a)
 {
     dim3 grid(br_tiles(c->p.nx, c->p.nv), c->B), block(NT);
     switch (c->p.bracket) {
     case VV_BRACKET_J1:
-        launch_timed(c, bracket_kernel<VV_BRACKET_J1, MODE, T>, grid, block, 0, a);
+        launch_timed(c, bracket_kernel<VV_BRACKET_J1, MODE>, grid, block, 0, a);
         break;
     case VV_BRACKET_J2:
-        launch_timed(c, bracket_kernel<VV_BRACKET_J2, MODE, T>, grid, block, 0, a);
+        launch_timed(c, bracket_kernel<VV_BRACKET_J2, MODE>, grid, block, 0, a);
         break;
     default:
-        launch_timed(c, bracket_kernel<VV_BRACKET_J4, MODE, T>, grid, block, 0, a);
+        launch_timed(c, bracket_kernel<VV_BRACKET_J4, MODE>, grid, block, 0, a);
         break;
     }
+    return hipGetLastError();
+}
+
+template <int MODE, typename T>
+hipError_t launch_sep(vv_ctx *c, BrArgs<T> a)
+{
+    const dim3 grid(br_tiles(c->p.nx, c->p.nv), c->B), block(NT);
+    const int kind = c->p.bracket;
+    if (kind == VV_BRACKET_J1) launch_timed(c, bracket_sep_kernel<false, MODE, T>, grid, block, 0, a, kind);
+    else launch_timed(c, bracket_sep_kernel<true, MODE, T>, grid, block, 0, a, kind);
     return hipGetLastError();
 }
 
@@ -412,15 +504,34 @@ hipError_t launch_residual(vv_ctx *c, const double *f, const double *fh, double 
     return launch_mode<MODE_RESIDUAL>(c, a);
 }
 
+hipError_t launch_residual_sep(vv_ctx *c, const double *f, const double *fh, double *y)
+{
+    BrArgs<double> a = base_args<double>(c);
+    a.f = f;
+    a.fh = fh;
+    a.y = y;
+    a.factor = 1.0;
+    return launch_sep<MODE_RESIDUAL>(c, a);
+}
+
+hipError_t launch_jacobian_plain(vv_ctx *c, const double *u, double *y)
+{
+    BrArgs<double> a = base_args<double>(c);
+    a.f = u;
+    a.y = y;
+    a.factor = 0.5;                 // B(u, H, 0.5)  (PETScNLVlasovMP.pyx:37)
+    return launch_mode<MODE_JACOBIAN>(c, a);
+}
+
 hipError_t launch_jacobian(vv_ctx *c, const double *u, const double *uscale, double *y)
 {
     BrArgs<double> a = base_args<double>(c);
     a.f = u;
     a.uscale = uscale;
     a.y = y;
-    a.factor = 0.5;                 // B(u, H, 0.5)  (PETScNLVlasovMP.pyx:37)
+    a.factor = 0.5;
     a.done = uscale != nullptr ? &c->gs->st.done : nullptr;
-    return launch_mode<MODE_JACOBIAN>(c, a);
+    return launch_sep<MODE_JACOBIAN>(c, a);
 }
 
 hipError_t launch_bracket_add(vv_ctx *c, const double *x, double *y, double factor)
@@ -505,7 +616,7 @@ hipError_t launch_jacobian32(vv_ctx *c, const float *u, const double *uscale, fl
     a.y = y;
     a.factor = 0.5;
     a.done = uscale != nullptr ? &c->gs->st.done : nullptr;
-    return launch_mode<MODE_JACOBIAN>(c, a);
+    return launch_sep<MODE_JACOBIAN>(c, a);
 }
 
 }  // namespace vv

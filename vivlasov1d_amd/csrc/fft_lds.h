@@ -385,14 +385,5 @@ struct JacRows {
     double ht_inv, factor;
 };
 
-// H_ave from its factors in the tile's type: FP64 as is, FP32 relative to
-// href (formed in FP64, rounded once), as the bracket kernel stages it
-template <typename T>
-__device__ __forceinline__ T have_rel(double h0, const double (&x)[4], double href)
-{
-    if constexpr (sizeof(T) == 8) return compose_have(h0, x[0], x[1], x[2], x[3]);
-    else return (T)(compose_have(h0, x[0], x[1], x[2], x[3]) - href);
-}
-
 }  // namespace
 }  // namespace vv

@@ -130,8 +130,7 @@ enum { F_JAC = 0, F_RES = 1, F_PLAIN = 2 };
 
 // Row-block geometry: strips of W columns (all of x when nx <= 256, else 256),
 // NS of them; G groups of R rows side by side in the workgroup when a row is
-// shorter than the workgroup; RW = G R rows, at most 16 (the FP32 H_ave offset
-// is taken per 16-row band).
+// shorter than the workgroup; RW = G R rows, at most 16.
 struct RowGeom {
     int W, G, NS, RW;
     uint32_t mW, mSP;      // reciprocals of W and W + 4 (div_by)
@@ -157,14 +156,6 @@ struct PitchRd {                   // cell (r, cx + d) of a tile of runtime pitc
         __device__ __forceinline__ T operator()(int r, int cx, int d) const { return p[r * P + cx + d]; }
     };
 };
-
-template <typename T>
-__device__ __forceinline__ T bracket_by_kind(int kind, const ArakawaWin<T> &w, T base, T factor, T af1, T af2)
-{
-    if (kind == VV_BRACKET_J4) return arakawa_add<VV_BRACKET_J4>(w, base, factor, af1, af2);
-    if (kind == VV_BRACKET_J1) return arakawa_add<VV_BRACKET_J1>(w, base, factor, af1, af2);
-    return arakawa_add<VV_BRACKET_J2>(w, base, factor, af1, af2);
-}
 
 // the collision term at the window's centre, as collision_kernel adds it
 __device__ __forceinline__ double add_collision(double y, double fm, double f0, double fp, double vp, double vm,
@@ -199,19 +190,15 @@ __device__ __forceinline__ T residual_base(T ht_inv, T f, T fh)
     const T d = f - fh;
     return T(0) + ht_inv * d;
 }
-template <typename T>
-__device__ __forceinline__ T scaled(T f, T s)
-{
-    return f * s;
-}
-
 // One workgroup: RW rows.  Per strip the tile of the bracket's first argument
-// and of H_ave with a 2-cell halo is staged in LDS (every load of a thread
-// issued before the first store), thread t walks column t % W of row group
-// t / W down its R rows with the bracket kernel's register window (the same
-// values, bit for bit), and the results go to the packed lines.  hs: as in the
-// strip kernel.  Measured at 64 x 128: J u 5.1 + rFFT 4.1 + update 2.9 us and
-// their gaps before, one launch of 5-6 us; 201 x 401: 5.6 + 9.3 + 3.3 us.
+// with a 2-cell halo and the x-part of H_ave are staged in LDS (every load of a
+// thread issued before the first store), thread t walks column t % W of row group
+// t / W down its R rows (SepWin), and the results, times the Krylov vector's
+// scale (known one barrier later than the tile), go to the packed lines.  hs: as
+// in the strip kernel.  Measured at 64 x 128: J u 5.1 + rFFT 4.1 + update 2.9 us
+// and their gaps as launches of their own, 8.0 us here with the unfactored
+// stencil, 7.3 now; 201 x 401: 5.6 + 9.3 + 3.3, 11.4, 10.4; 16 x (128 x 256): 11.4,
+// 10.0.
 template <int MODE, int R, int FK, typename T>
 __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, RowFwd<T> p, HessArgs hs, DftPlan plan,
                                                      cx_t<T> *__restrict__ spec)
@@ -232,6 +219,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
     const size_t xo = (size_t)b * nx;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ double red[kGdNW + 1];
+    __shared__ __align__(16) T sA[16][4];      // the rows' coefficients of the bracket
     C *buf = reinterpret_cast<C *>(lds_raw + g.fft_off);
     C *stw = reinterpret_cast<C *>(lds_raw + g.tw_off);
     const int j0 = xcd_tile((int)blockIdx.x - extra, (int)gridDim.x - extra) * RW;
@@ -249,18 +237,15 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
         }
     } else {
         T *sF = reinterpret_cast<T *>(lds_raw);
-        T *sH = sF + RH * SP;
-        double *sX = reinterpret_cast<double *>(lds_raw + (((size_t)2 * RH * SP * sizeof(T) + 15) & ~(size_t)15));
-        double *sV = sX + 4 * SP;
-        // FP32: H_ave relative to h0 at the centre of the rows' 16-row band
-        const int jc = ((j0 >> 4) << 4) + 8;
-        const double href = (sizeof(T) == 4 && jc < nv) ? p.jr.h0[jc] : 0.0;
+        double *sP = reinterpret_cast<double *>(lds_raw + (((size_t)RH * SP * sizeof(T) + 15) & ~(size_t)15));
         double usd = MODE == F_JAC && p.jr.uscale != nullptr && !extra
                          ? *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p.jr.uscale) +
                                                              b * a.gstride)
                          : 1.0;
-        const T ht_inv = (T)p.jr.ht_inv, factor = (T)p.jr.factor;
-        const T af1 = (T)p.jr.inst[b].af1, af2 = (T)p.jr.inst[b].af2;
+        const T ht_inv = (T)p.jr.ht_inv;
+        double c1, c2;
+        sep_weights(p.kind, p.jr.factor, p.jr.inst[b].af1, p.jr.inst[b].af2, c1, c2);
+        const bool far = p.kind != VV_BRACKET_J1;
         const int grp = g.G > 1 ? div_by(t, g.mW) : 0, col = t - grp * W;
         T us = T(1);
         for (int s = 0; s < g.NS; ++s) {
@@ -283,7 +268,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                     fb[q] = gj >= 0 ? h : T(0);
                 }
             }
-            double xf[2][4], vf = 0.0;
+            double xf[2][4];
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int c = t + q * NT;
@@ -293,13 +278,10 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                 xf[q][2] = p.jr.h2p[gi];
                 xf[q][3] = p.jr.h2h[gi];
             }
-            if (t < RH) {
-                const int gj = jr_row(j0, t, nv);
-                vf = gj >= 0 ? p.jr.h0[gj] : 0.0;
-            }
+            if (s == 0 && t < RW) sep_row(p.jr.h0, j0 + t, nv, c1, c2, sA[t]);
             if (s == 0) {
                 if (dflag) return;         // uniform over the block, before any barrier
-                if (extra) {               // summed after the factors' barrier
+                if (extra) {               // summed after the tile's barrier
                     const double ws = wave_sum(nshare);
                     if ((t & 63) == 0) red[t >> 6] = ws;
                 }
@@ -309,12 +291,13 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int c = t + q * NT;
-                if (c < SP) {
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) sX[m * SP + c] = xf[q][m];
-                }
+                if (c < SP) sP[c] = phi_ave(xf[q][0], xf[q][1], xf[q][2], xf[q][3]);
             }
-            if (t < RH) sV[t] = vf;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const int idx = t + q * NT;
+                if (idx < RH * SP) sF[idx] = MODE == F_RES ? fave(fa[q], fb[q]) : fa[q];
+            }
             __syncthreads();
             if (s == 0) {
                 if (extra) {
@@ -324,23 +307,14 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                 }
                 us = (T)usd;
             }
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                const int idx = t + q * NT;
-                if (idx < RH * SP) {
-                    const int r = div_by(idx, g.mSP), c = idx - r * SP;
-                    sF[idx] = MODE == F_RES ? fave(fa[q], fb[q]) : scaled(fa[q], us);
-                    const double x4[4] = {sX[c], sX[SP + c], sX[2 * SP + c], sX[3 * SP + c]};
-                    sH[idx] = jr_row(j0, r, nv) >= 0 ? have_rel<T>(sV[r], x4, href) : T(0);
-                }
-            }
-            __syncthreads();
             const int i = cb + col;
             if (grp < g.G && col < W && i < nx) {
                 const int cx = col + 2, r0 = grp * R;
-                const PitchRd::Of<T> rF{sF, SP}, rH{sH, SP};
-                ArakawaWin<T> win;
-                win.load(rF, rH, r0 + 2, cx);
+                const PitchRd::Of<T> rF{sF, SP};
+                T B[4];
+                sep_coef(sP[cx - 2], sP[cx - 1], sP[cx], sP[cx + 1], sP[cx + 2], c1, c2, B);
+                SepWin<T> win;
+                win.load(rF, r0 + 2, cx);
                 double cn = 1.0, cU = 0.0, ca = 1.0;
                 const bool coll = MODE == F_JAC && sizeof(T) == 8 && p.cn != nullptr;
                 if (coll) {
@@ -349,7 +323,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                     ca = p.ca[i];
                 }
                 T *z = reinterpret_cast<T *>(buf + (r0 >> 1) * nx + i);
-#pragma unroll 1
+#pragma unroll
                 for (int q = 0; q < R; ++q) {
                     const int j = j0 + r0 + q;
                     T out = T(0);
@@ -359,15 +333,15 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                         else base = jacobian_base(ht_inv, win.f0[2]);
                         out = base;
                         if (j >= 2 && j < nv - 2) {
-                            out = bracket_by_kind(p.kind, win, base, factor, af1, af2);
+                            out = base + win.bracket(sA[r0 + q], B, far);
                             if (coll)
                                 out = (T)add_collision((double)out, (double)win.f0[1], (double)win.f0[2],
                                                        (double)win.f0[3], p.cv[j + 1], p.cv[j - 1], cn, cU, ca,
                                                        p.drag_fac, p.diff_fac, p.coll_e != 0);
                         }
                     }
-                    z[(q >> 1) * 2 * nx + (q & 1)] = out;
-                    if (q + 1 < R) win.advance(rF, rH, r0 + q + 3, cx);
+                    z[(q >> 1) * 2 * nx + (q & 1)] = MODE == F_JAC ? scaled(out, us) : out;
+                    if (q + 1 < R) win.advance(rF, r0 + q + 3, cx);
                 }
             }
         }
@@ -586,7 +560,7 @@ RowGeom geom_for(const vv_ctx *c, int mode, int R, size_t *lds)
     g.mW = 0xffffffffu / (uint32_t)g.W + 1;
     g.mSP = 0xffffffffu / (uint32_t)(g.W + 4) + 1;
     const int RH = g.RW + 4, SP = g.W + 4;
-    size_t strip = (((size_t)2 * RH * SP * sizeof(T) + 15) & ~(size_t)15) + (size_t)(4 * SP + RH) * sizeof(double);
+    size_t strip = (((size_t)RH * SP * sizeof(T) + 15) & ~(size_t)15) + (size_t)SP * sizeof(double);
     strip = (strip + 15) & ~(size_t)15;
     const bool dft = fft_kind(nx) == kDft;
     const size_t lines = (size_t)(g.RW >> 1) * nx * sizeof(cx_t<T>) * (dft ? 2 : 1);

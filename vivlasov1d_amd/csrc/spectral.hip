@@ -112,24 +112,25 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
 // Y = 0; Y += u/dt; Y += 0.5 {u, H_ave} on rows 2..nv-3) is formed in LDS row
 // block by row block and transformed there, so X never goes to HBM.
 // The workgroup's R rows are computed in strips of NT columns: the strip of
-// u (times the Krylov vector's scale) and of H_ave with a 2-cell halo,
-// (R+4) x (NT+4) cells each, is staged in LDS; thread t walks column t of
-// the strip down the R rows with the bracket kernel's stencil window
-// (arakawa.h), so every value is the bracket kernel's, bit for bit.  The next
-// strip's loads are in flight during the current strip's walk, and the
+// u with a 2-cell halo, (R+4) x (NT+4) cells, and the x-part of H_ave are
+// staged in LDS, two strips in turn (one barrier each); thread t walks column t
+// of the strip down the R rows (SepWin, arakawa.h; the result is multiplied by
+// the Krylov vector's scale), the values of bracket_sep_kernel bit for bit.  The
+// next strip's loads are in flight during the current strip's walk, and the
 // results stay in registers until the last walk is done, so the FFT buffer
 // reuses the strips' LDS.  nx = 4 NT: thread t's columns over the 4 strips,
 // t + m NT, are exactly the inputs of radix-4 butterfly t of the first FFT
 // stage, which then runs in registers as in rfft_kernel (the same
 // arithmetic, bit for bit).  nx = NT, 2 NT: the rows go to the FFT buffer and
 // the transform starts from LDS (its unit twiddles can change only the sign
-// of an exact zero).  R in 2, 4, 8.
+// of an exact zero).  R in 2, 4, 8.  1024 x 2048: 22.5 us with H staged beside u
+// and the unfactored stencil, 17.5 now (FP32 16.8, 14.3).
 template <int R, typename T>
 struct JacStrip {
     T u[R + 4];          // own column, rows j0-2 .. j0+R+1 (0 outside the grid)
     double x[4];         // own column's x-factors
     T eu;                // halo cell (threads t < 4 (R+4))
-    double ex[4], eh0;
+    double ex[4];
 };
 
 template <int R, typename T>
@@ -153,35 +154,38 @@ __device__ __forceinline__ void jac_strip_load(const T *__restrict__ u, const Ja
         jr_halo_cell(t, RH, &hr, &tc);
         const int gi = jr_col(cb, tc, nx);
         const int gj = jr_row(j0, hr, nv);
-        const bool in = gj >= 0;
-        g.eu = in ? u[(size_t)gj * nx + gi] : T(0);
-        g.eh0 = in ? jr.h0[gj] : 0.0;
-        g.ex[0] = jr.h1p[xo + gi];
-        g.ex[1] = jr.h1h[xo + gi];
-        g.ex[2] = jr.h2p[xo + gi];
-        g.ex[3] = jr.h2h[xo + gi];
+        g.eu = gj >= 0 ? u[(size_t)gj * nx + gi] : T(0);
+        if (hr == 0) {
+            g.ex[0] = jr.h1p[xo + gi];
+            g.ex[1] = jr.h1h[xo + gi];
+            g.ex[2] = jr.h2p[xo + gi];
+            g.ex[3] = jr.h2h[xo + gi];
+        }
     }
 }
 
 // Thread t's column of the staged strip down the R output rows (tile rows
 // 2 .. R+1): J u, or 0 on rows past nv (the rFFT's zero rows).
-template <int KIND, int R, typename T, typename RF, typename RH>
-__device__ __forceinline__ void jac_walk(const RF &rF, const RH &rH, int j0, int nv, T ht_inv, T factor, T af1,
-                                         T af2, T (&res)[R])
+template <bool FAR, int R, typename T, typename RF>
+__device__ __forceinline__ void jac_walk(const RF &rF, const T (*sA)[4], const double *sP, double c1, double c2,
+                                         int j0, int nv, T ht_inv, T us, T (&res)[R])
 {
     const int cx = threadIdx.x + 2;
-    ArakawaWin<T> win;
-    win.load(rF, rH, 2, cx);
+    T B[4];
+    sep_coef(sP[cx - 2], sP[cx - 1], sP[cx], sP[cx + 1], sP[cx + 2], c1, c2, B);
+    SepWin<T> win;
+    win.load(rF, 2, cx);
 #pragma unroll
     for (int q = 0; q < R; ++q) {
         const int j = j0 + q;
         T out = T(0);
         if (j < nv) {
-            const T base = jacobian_base(ht_inv, win.f0[2]);
-            out = (j >= 2 && j < nv - 2) ? arakawa_add<KIND>(win, base, factor, af1, af2) : base;
+            out = jacobian_base(ht_inv, win.f0[2]);
+            if (j >= 2 && j < nv - 2) out += win.bracket(sA[q], B, FAR);
+            out = scaled(out, us);                     // == J of the VecScale'd Krylov vector
         }
         res[q] = out;
-        if (q + 1 < R) win.advance(rF, rH, q + 3, cx);
+        if (q + 1 < R) win.advance(rF, q + 3, cx);
     }
 }
 
@@ -191,6 +195,12 @@ __device__ __forceinline__ void jac_walk(const RF &rF, const RH &rH, int j0, int
 // strip's loads).  A launch of its own took 4.9 us a step at 1024 x 2048 and
 // 3-4 us with its gap on small grids.  The step that follows an instance's
 // convergence then runs this kernel in vain (its later kernels return at once).
+template <typename T>
+constexpr size_t jac_strip_lds(int R, int NS)
+{
+    return (NS > 1 ? 2 : 1) * ((size_t)(R + 4) * (NT + 4) * sizeof(T) + (NT + 4) * sizeof(double));
+}
+
 template <int KIND, int R, int NS, typename T>
 __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs hs, const T *__restrict__ u,
                                               cx_t<T> *__restrict__ spec)
@@ -214,55 +224,59 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C *buf = reinterpret_cast<C *>(lds_raw);
     T *sF = reinterpret_cast<T *>(lds_raw);
-    T *sH = sF + RH * SP;
+    constexpr int NBUF = NS > 1 ? 2 : 1;               // strips in turn: one barrier each
+    constexpr size_t kStrip = jac_strip_lds<T>(R, NS), kLines = (size_t)(R >> 1) * nx * sizeof(C);
+    double *sP = reinterpret_cast<double *>(lds_raw + NBUF * (size_t)RH * SP * sizeof(T));
     const int nv = a.nv, t = threadIdx.x;
     const int j0 = xcd_tile((int)blockIdx.x - extra, (int)gridDim.x - extra) * R;
     // nx = NT, 2 NT: the twiddles' copy lies behind the strips and the FFT buffer
-    constexpr size_t kStrip = 2 * (size_t)RH * SP * sizeof(T), kLines = (size_t)(R >> 1) * nx * sizeof(C);
     const C *tw = tw_table<NS != 4>(a.tw, reinterpret_cast<C *>(lds_raw + (kStrip > kLines ? kStrip : kLines)), nx);
     __shared__ double red[kGdNW + 1];
+    __shared__ __align__(16) T sA[R][4];
     const double nshare = extra ? norm_share(hs.part + b * hs.pstride, hs.nb) : 0.0;
-    // FP32: H_ave - href, href = h0 at the centre row of the bracket kernel's
-    // 16-row band that holds the workgroup's rows (R divides 16), as the FP32
-    // bracket kernel stages it
-    const int jc = ((j0 >> 4) << 4) + 8;
-    const double href = (sizeof(T) == 4 && jc < nv) ? jr.h0[jc] : 0.0;
     double usd = jr.uscale != nullptr && !extra
                      ? *reinterpret_cast<const double *>(reinterpret_cast<const char *>(jr.uscale) + b * a.gstride)
                      : 1.0;
-    double h0r[RH];
-#pragma unroll
-    for (int r = 0; r < RH; ++r) {
-        const int gj = jr_row(j0, r, nv);
-        h0r[r] = gj >= 0 ? jr.h0[gj] : 0.0;
-    }
+    double c1, c2;
+    sep_weights(KIND, jr.factor, jr.inst[b].af1, jr.inst[b].af2, c1, c2);
     JacStrip<R, T> g;
     jac_strip_load<R>(u, jr, xo, nx, nv, j0, 0, g);
+    if (t < R) sep_row(jr.h0, j0 + t, nv, c1, c2, sA[t]);
     if (dflag) return;                 // uniform over the block, before any barrier
-    if (extra) usd = scale_of(block_sum_all(nshare, red));
-    const T us = (T)usd, ht_inv = (T)jr.ht_inv, factor = (T)jr.factor;
-    const T af1 = (T)jr.inst[b].af1, af2 = (T)jr.inst[b].af2;
+    if (extra) {
+        const double ws = wave_sum(nshare);            // summed after the first strip's barrier
+        if ((t & 63) == 0) red[t >> 6] = ws;
+    }
+    const T ht_inv = (T)jr.ht_inv;
+    T us = T(1);
     T res[NS][R];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        // stage the strip: u times its scale (== the VecScale'd Krylov
-        // vector) and H_ave (0 outside the grid), as the bracket kernel does
+        // stage the strip: u and the x-part of H_ave
+        T *cF = sF + (s & (NBUF - 1)) * RH * SP;
+        double *cP = sP + (s & (NBUF - 1)) * SP;
 #pragma unroll
-        for (int r = 0; r < RH; ++r) {
-            sF[r * SP + t + 2] = g.u[r] * us;
-            sH[r * SP + t + 2] = jr_row(j0, r, nv) >= 0 ? have_rel<T>(h0r[r], g.x, href) : T(0);
-        }
+        for (int r = 0; r < RH; ++r) cF[r * SP + t + 2] = g.u[r];
+        cP[t + 2] = phi_ave(g.x[0], g.x[1], g.x[2], g.x[3]);
         if (t < 4 * RH) {
             int hr, tc;
             jr_halo_cell(t, RH, &hr, &tc);
-            sF[hr * SP + tc] = g.eu * us;
-            sH[hr * SP + tc] = jr_row(j0, hr, nv) >= 0 ? have_rel<T>(g.eh0, g.ex, href) : T(0);
+            cF[hr * SP + tc] = g.eu;
+            if (hr == 0) cP[tc] = phi_ave(g.ex[0], g.ex[1], g.ex[2], g.ex[3]);
         }
         __syncthreads();
         if (s + 1 < NS) jac_strip_load<R>(u, jr, xo, nx, nv, j0, (s + 1) * NT, g);
-        jac_walk<KIND, R>(TileRd<T, SP>{sF}, TileRd<T, SP>{sH}, j0, nv, ht_inv, factor, af1, af2, res[s]);
-        __syncthreads();
+        if (s == 0) {
+            if (extra) {
+                double tot = 0.0;
+                for (int w = 0; w < kGdNW; ++w) tot += red[w];
+                usd = scale_of(tot);
+            }
+            us = (T)usd;
+        }
+        jac_walk<KIND != VV_BRACKET_J1, R>(TileRd<T, SP>{cF}, sA, cP, c1, c2, j0, nv, ht_inv, us, res[s]);
     }
+    __syncthreads();
     // twiddles in flight during the first stage (not held through the walks)
     FftTw<false, C> pt;
     if (NS == 4) pt.load(a.tw);
@@ -293,7 +307,7 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
     store_real_spectrum(buf, nx, R, j0, nv, spec);
 }
 
-// LDS max(R/2 nx 16, 2 (R+4)(NT+4) 8) bytes (33 KB at R = 4), so three
+// LDS max(R/2 nx 16, 2 (R+5)(NT+4) 8) bytes (37 KB at R = 4), so three
 // workgroups per CU fit when the registers do (R <= 4; four cost register
 // spills and were slower)
 template <int KIND, int R, int NS, typename T>
@@ -1408,7 +1422,7 @@ template <int KIND, int R, int NS, typename T>
 void jac_rfft_launch(vv_ctx *c, const FftArgs<T> &a, const JacRows &jr, const T *u, cx_t<T> *spec)
 {
     const size_t fft = (size_t)(R >> 1) * a.nx * sizeof(cx_t<T>);
-    const size_t strip = 2 * (size_t)(R + 4) * (NT + 4) * sizeof(T);
+    const size_t strip = jac_strip_lds<T>(R, NS);
     const HessArgs hs = take_update(c);
     const dim3 grid((a.nv + R - 1) / R + (hs.nb > 0 ? 1 : 0), c->B);
     const size_t tws = NS != 4 ? a.nx * sizeof(cx_t<T>) : 0;

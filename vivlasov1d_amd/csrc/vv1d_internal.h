@@ -223,6 +223,10 @@ namespace vv {
 // part: per-workgroup sums of y^2 (residual_blocks of them, instances part_stride apart) when not null
 hipError_t launch_residual(vv_ctx *c, const double *f, const double *fh, double *y, double *part = nullptr);
 int residual_blocks(const vv_ctx *c);
+hipError_t launch_jacobian_plain(vv_ctx *c, const double *u, double *y);
+// the solver's own F(f) and J u (H split into row and column coefficients; the
+// two above keep the reference's operation order)
+hipError_t launch_residual_sep(vv_ctx *c, const double *f, const double *fh, double *y);
 hipError_t launch_jacobian(vv_ctx *c, const double *u, const double *uscale, double *y);
 hipError_t launch_bracket_add(vv_ctx *c, const double *x, double *y, double factor);
 hipError_t launch_jacobian32(vv_ctx *c, const float *u, const double *uscale, float *y);
