@@ -1139,7 +1139,7 @@ int create_impl(const vv_params *p, int B, const double *hxs, void *stream, vv_c
     VV_CCHECK(dalloc(c, &c->vgrid, nv), "alloc v grid");
     VV_CCHECK(dalloc(c, &c->twiddle, c->fft_n), "alloc twiddle");
     VV_CCHECK(dalloc(c, &c->twiddle32, c->fft_n), "alloc twiddle32");
-    VV_CCHECK(dalloc(c, &c->spec, (size_t)c->nmodes * c->fft_rows * Bz), "alloc spectrum");
+    VV_CCHECK(dalloc(c, &c->spec, (size_t)spec_stride(c) * Bz), "alloc spectrum");
     if (p->precond == VV_PRECOND_TENSOR_KINETIC) {
         VV_CCHECK(dalloc(c, &c->lu64, (size_t)c->nmodes * lu_pivots_per_mode(c->fft_rows) * Bz), "alloc pivots");
         VV_CCHECK(dalloc(c, &c->lu_gm, lu_pivots_per_mode(c->fft_rows)), "alloc band factors");

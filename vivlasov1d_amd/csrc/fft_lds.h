@@ -10,6 +10,9 @@ namespace {
 
 constexpr int NT = 256;
 constexpr int MAXE = 4096;   // complex elements of one FFT workgroup (64 KiB of LDS)
+// threads of the long lines' kernels (64 KB of LDS, two workgroups a CU): with 256
+// rfft and irfft take 46.5 us at 2048 x 4096, with 512 and the swizzle below 44.6
+constexpr int NTL = 512;
 
 // complex arithmetic on double2 / float2
 template <typename C> __device__ __forceinline__ C cmk(typename C::value_type re, typename C::value_type im)
@@ -246,13 +249,26 @@ __device__ __forceinline__ void lds_fft1024(C *buf, int nb, const FftTw<INV, C> 
     __syncthreads();
 }
 
+// Place of element i of a long line (n >= 2048) in LDS.  The 16 lanes that a
+// 16-byte access serves together take i = 4j, 8j, 32 (j >> 2) + (j & 3) or
+// 64 (j >> 3) + (j & 7) in the stores of the first two stages, 2 to 4 of the 16
+// bank groups; bits 4, 5, 6 are folded into the low four so that each of these
+// (and 16 elements in a row) meets all 16.
+template <bool SWZ>
+__device__ __forceinline__ int swz(int i)
+{
+    if constexpr (!SWZ) return i;
+    const int a = (i >> 4) & 7;
+    return i ^ a ^ ((a & 6) << 1);
+}
+
 // One Stockham stage of radix RAD (4 or 8) on nb transforms of length 2^logn:
 // sub-transforms of length Ns = 2^l combined; butterfly j of a transform takes
 // elements j + r n/RAD, twiddled by W_n^(r k n/(RAD Ns)), k = j mod Ns, and
 // stores output m at RAD (j - k) + k + m Ns.  Every butterfly of the thread (Q
 // at most) is loaded before the barrier and stored after it, so one buffer
 // suffices; the final stage's outputs go to `last`.
-template <int RAD, bool INV, int Q, typename C, typename Sink>
+template <int RAD, bool INV, int Q, int NTH, bool SWZ, typename C, typename Sink>
 __device__ __forceinline__ void fft_stage(C *buf, int logn, int nb, int l, const C *tw, bool fin, const Sink &last)
 {
     constexpr int LR = RAD == 8 ? 3 : 2;
@@ -261,11 +277,11 @@ __device__ __forceinline__ void fft_stage(C *buf, int logn, int nb, int l, const
     int dst[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const int bq = threadIdx.x + q * NT;
+        const int bq = threadIdx.x + q * NTH;
         dst[q] = -1;
         if (bq < total) {
             const int b = bq >> lq, j = bq & (nq - 1), k = j & (Ns - 1);
-            const C *src = buf + (b << logn) + j;
+            const C *src = buf + swz<SWZ>((b << logn) + j);     // r << lq leaves the swizzle alone
 #pragma unroll
             for (int r = 0; r < RAD; ++r) v[q][r] = src[r << lq];
             if (l > 0) {
@@ -284,7 +300,7 @@ __device__ __forceinline__ void fft_stage(C *buf, int logn, int nb, int l, const
 #pragma unroll
             for (int m = 0; m < RAD; ++m) {
                 if (fin) last(dst[q] + (m << l), v[q][m]);
-                else buf[dst[q] + (m << l)] = v[q][m];
+                else buf[swz<SWZ>(dst[q] + (m << l))] = v[q][m];
             }
         }
     }
@@ -313,7 +329,9 @@ __host__ __device__ __forceinline__ int fft_first(int logn) { return fft_lead4(l
 // stays a few KB (unrolled by stage and butterfly it was 25-40 KB, and a small
 // grid's kernels, each on a few CUs for a few microseconds, fetched it all).
 // Inlined so that buf is known to be LDS (ds_read/ds_write, not flat accesses).
-template <bool INV, bool P8, int EB, typename C, typename Sink>
+// NTH: threads of the workgroup; SWZ: the elements lie at swz<true> (the
+// outputs to `last` have their natural index).
+template <bool INV, bool P8, int EB, int NTH = NT, bool SWZ = false, typename C, typename Sink>
 __device__ __forceinline__ void lds_fft(C *buf, int logn, int nb, const C *tw, const FftTw<INV, C> &pt, int l0,
                                         const Sink &last)
 {
@@ -322,8 +340,8 @@ __device__ __forceinline__ void lds_fft(C *buf, int logn, int nb, const C *tw, c
     } else {
         const int l4 = 2 * fft_lead4(logn);
         int l = l0;
-        for (; l < l4; l += 2) fft_stage<4, INV, EB, C>(buf, logn, nb, l, tw, l + 2 == logn, last);
-        for (; l < logn; l += 3) fft_stage<8, INV, (EB + 1) / 2, C>(buf, logn, nb, l, tw, l + 3 == logn, last);
+        for (; l < l4; l += 2) fft_stage<4, INV, (EB * NT + NTH - 1) / NTH, NTH, SWZ, C>(buf, logn, nb, l, tw, l + 2 == logn, last);
+        for (; l < logn; l += 3) fft_stage<8, INV, (EB * NT / 2 + NTH - 1) / NTH, NTH, SWZ, C>(buf, logn, nb, l, tw, l + 3 == logn, last);
     }
 }
 
@@ -342,7 +360,7 @@ __device__ __forceinline__ const C *tw_table(const C *__restrict__ tw, C *stw, i
 template <typename T>
 struct FftArgs {
     int nx, logn, nv, rows;     // rows: v-rows per workgroup (even)
-    int64_t N, S, gstride;
+    int64_t N, S, pitch, gstride;   // pitch: elements from mode to mode of a spectrum
     const cx_t<T> *tw;
     const int32_t *done;
     const T *add;               // rfft: x-only field added to every row, gamma add (null: none), nx per instance
@@ -357,14 +375,17 @@ __device__ __forceinline__ int32_t cycle_done(const int32_t *done, int64_t gstri
 
 // The R real rows' spectra from their packed transforms in buf (complex row
 // p = real rows 2p + i 2p+1), stored mode-major: S[k][j0 + r], k <= nx/2.
-template <typename C>
-__device__ __forceinline__ void store_real_spectrum(const C *buf, int nx, int R, int j0, int nv, C *__restrict__ spec)
+template <int NTH = NT, typename C>
+__device__ __forceinline__ void store_real_spectrum(const C *buf, int nx, int R, int j0, int nv, int64_t pitch,
+                                                    C *__restrict__ spec)
 {
     using T = typename C::value_type;
     const int nk = (nx >> 1) + 1;
     const T half = T(0.5);
-    for (int idx = threadIdx.x; idx < nk * R; idx += NT) {
-        const int k = idx / R;
+    const int lr = __ffs(R) - 1;
+    const bool p2 = (R & (R - 1)) == 0;
+    for (int idx = threadIdx.x; idx < nk * R; idx += NTH) {
+        const int k = p2 ? idx >> lr : idx / R;
         const int r = idx - k * R;
         if (j0 + r >= nv) continue;
         const C *z = buf + (r >> 1) * nx;
@@ -373,7 +394,7 @@ __device__ __forceinline__ void store_real_spectrum(const C *buf, int nx, int R,
         C out;
         if ((r & 1) == 0) out = cmk<C>((zk.x + zm.x) * half, (zk.y - zm.y) * half);
         else out = cmk<C>((zk.y + zm.y) * half, (zm.x - zk.x) * half);
-        spec[(size_t)k * nv + j0 + r] = out;
+        spec[(size_t)k * pitch + j0 + r] = out;
     }
 }
 

@@ -104,7 +104,8 @@ struct LineSink {
 
 // R real rows' spectra from their packed transforms, any length
 template <typename C>
-__device__ __forceinline__ void store_rows_spectrum(const C *buf, int n, int R, int j0, int nv, C *__restrict__ spec)
+__device__ __forceinline__ void store_rows_spectrum(const C *buf, int n, int R, int j0, int nv, int64_t pitch,
+                                                    C *__restrict__ spec)
 {
     using T = typename C::value_type;
     const int nk = n / 2 + 1;
@@ -120,7 +121,7 @@ __device__ __forceinline__ void store_rows_spectrum(const C *buf, int n, int R, 
         C out;
         if ((r & 1) == 0) out = cmk<C>((zk.x + zm.x) * half, (zk.y - zm.y) * half);
         else out = cmk<C>((zk.y + zm.y) * half, (zm.x - zk.x) * half);
-        spec[(size_t)k * nv + j0 + r] = out;
+        spec[(size_t)k * pitch + j0 + r] = out;
     }
 }
 
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
     } else {
         lds_fft<false, false, 1>(buf, a.logn, RW >> 1, (const C *)stw, FftTw<false, C>{}, 0, LdsSink<C>{buf});
     }
-    store_rows_spectrum(out, nx, RW, j0, nv, spec);
+    store_rows_spectrum(out, nx, RW, j0, nv, a.pitch, spec);
 }
 
 // ---- inverse ----------------------------------------------------------------
@@ -435,8 +436,8 @@ __global__ __launch_bounds__(NT) void row_inv_kernel(FftArgs<T> a, const cx_t<T>
         const int idx = t + q * NT;
         const int k = npair > 1 ? div_by(idx, mp) : idx;
         const int ja = j0 + 2 * (idx - k * npair);
-        va[q] = load_or_zero(spec, (int64_t)k * a.nv + ja, idx < total && ja < a.nv);
-        vb[q] = load_or_zero(spec, (int64_t)k * a.nv + ja + 1, idx < total && ja + 1 < a.nv);
+        va[q] = load_or_zero(spec, (int64_t)k * a.pitch + ja, idx < total && ja < a.nv);
+        vb[q] = load_or_zero(spec, (int64_t)k * a.pitch + ja + 1, idx < total && ja + 1 < a.nv);
     }
     const double sc = t < nvec ? (g.g + bi)->scale[t] : 0.0;
     C *stw = buf + (FK == kDft ? 2 : 1) * (size_t)npair * nx;
@@ -606,7 +607,7 @@ hipError_t row_fwd_t(vv_ctx *c, RowFwd<T> p, cx_t<T> *spec, const int32_t *done,
     int R;
     size_t lds;
     const RowGeom g = row_geom<T>(c, MODE, &R, &lds);
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, g.RW, c->N, spec_stride(c), (int64_t)sizeof(GmresState),
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, g.RW, c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState),
                  twiddles<T>(c), done, add, gamma};
     HessArgs hs{};
     if (MODE == F_JAC) hs = take_update(c);
@@ -642,7 +643,7 @@ template <typename T>
 hipError_t row_inv_t(vv_ctx *c, const T *basis, const cx_t<T> *spec, int col, T *y, double *part, const int32_t *done)
 {
     const int RI = inv_rows(c);
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, RI, c->N, spec_stride(c), (int64_t)sizeof(GmresState),
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, RI, c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState),
                  twiddles<T>(c), done};
     const int nb = (a.nv + RI - 1) / RI;
     const bool dft = fft_kind(a.nx) == kDft;

@@ -38,13 +38,15 @@ namespace {
 // with preloaded twiddles; VTWL shorter powers of two, twiddles copied to LDS;
 // VLONG longer ones, twiddles from the table.
 enum { VTWL = 0, VP8 = 1, VLONG = 2 };
+// threads of a variant's workgroup
+constexpr int vthreads(int V) { return V == VLONG ? NTL : NT; }
 
 // LF: log2 of the first stage's radix (fft_first), which runs in registers:
 // butterfly (p, j) of complex row p (real rows 2p, 2p+1) takes z_p[j + m nx/2^LF],
 // exactly the elements the thread loads (coalesced along j); its twiddles are
 // 1.  Every global load of the thread is issued before anything waits.
 template <typename T, int V, int LF>
-__global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restrict__ x, cx_t<T> *__restrict__ spec)
+__global__ __launch_bounds__(vthreads(V)) void rfft_kernel(FftArgs<T> a, const T *__restrict__ x, cx_t<T> *__restrict__ spec)
 {
     using C = cx_t<T>;
     const int32_t dflag = cycle_done(a.done, a.gstride);
@@ -57,13 +59,13 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
     // XCD-aware row-block order: the mode-major segments of neighbouring row
     // blocks share L2 lines, so they are kept on one XCD
     const int j0 = xcd_tile(blockIdx.x, gridDim.x) * R;
-    constexpr int RAD = 1 << LF, QB = MAXE / RAD / NT;    // butterflies per thread
+    constexpr int NTH = vthreads(V), RAD = 1 << LF, QB = MAXE / RAD / NTH;    // butterflies per thread
     const int lq = a.logn - LF, nq = 1 << lq;
     const int total = (R >> 1) * nq;
     T xr[QB][RAD], xi[QB][RAD];
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
-        const int bq = threadIdx.x + q * NT;
+        const int bq = threadIdx.x + q * NTH;
         const int p = bq >> lq, j = bq & (nq - 1);
         const bool ok = bq < total;
         const bool r0 = ok && j0 + 2 * p < a.nv, r1 = ok && j0 + 2 * p + 1 < a.nv;
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
     if (dflag) return;                 // uniform over the block, before any barrier
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
-        const int bq = threadIdx.x + q * NT;
+        const int bq = threadIdx.x + q * NTH;
         if (bq < total) {
             const int p = bq >> lq, j = bq & (nq - 1);
             C v[RAD];
@@ -97,14 +99,14 @@ __global__ __launch_bounds__(NT) void rfft_kernel(FftArgs<T> a, const T *__restr
             for (int m = 0; m < RAD; ++m) v[m] = cmk<C>(xr[q][m], xi[q][m]);
             if constexpr (LF == 3) dft8<false>(v);
             else dft4<false>(v[0], v[1], v[2], v[3]);
-            C *z = buf + (p << a.logn) + (j << LF);     // first stage's outputs: RAD j + m
+            const int z = (p << a.logn) + (j << LF);    // first stage's outputs: RAD j + m
 #pragma unroll
-            for (int m = 0; m < RAD; ++m) z[m] = v[m];
+            for (int m = 0; m < RAD; ++m) buf[swz<V == VLONG>(z + m)] = v[m];
         }
     }
     __syncthreads();
-    lds_fft<false, V == VP8, 4>(buf, a.logn, R >> 1, tw, pt, LF, LdsSink<C>{buf});
-    store_real_spectrum(buf, nx, R, j0, a.nv, spec);
+    lds_fft<false, V == VP8, 4, NTH, V == VLONG>(buf, a.logn, R >> 1, tw, pt, LF, LdsSink<C>{buf});
+    store_real_spectrum<NTH>(buf, nx, R, j0, a.nv, a.pitch, spec);
 }
 
 // Jacobian-vector product fused with the forward rFFT of its rows:
@@ -304,7 +306,7 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
     }
     __syncthreads();
     lds_fft<false, NS == 4, 4>(buf, a.logn, R >> 1, tw, pt, NS == 4 ? 2 : 0, LdsSink<C>{buf});
-    store_real_spectrum(buf, nx, R, j0, nv, spec);
+    store_real_spectrum(buf, nx, R, j0, nv, a.pitch, spec);
 }
 
 // LDS max(R/2 nx 16, 2 (R+5)(NT+4) 8) bytes (37 KB at R = 4), so three
@@ -361,7 +363,7 @@ __global__ __launch_bounds__(NT) void rfft_cols_kernel(FftArgs<T> a, const T *__
     }
     __syncthreads();
     lds_fft<false, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, LdsSink<C>{buf});
-    store_real_spectrum(buf, n, a.rows, i0, nc, spec);
+    store_real_spectrum(buf, n, a.rows, i0, nc, a.pitch, spec);
 }
 
 // the same columns back: line b of the workgroup to x = i0 + 2b, i0 + 2b + 1
@@ -394,7 +396,7 @@ struct IrfftSink {
 };
 
 template <typename T, int V, bool COLS>
-__global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *__restrict__ spec, T *__restrict__ y)
+__global__ __launch_bounds__(vthreads(V)) void irfft_kernel(FftArgs<T> a, const cx_t<T> *__restrict__ spec, T *__restrict__ y)
 {
     using C = cx_t<T>;
     const int32_t dflag = cycle_done(a.done, a.gstride);
@@ -409,15 +411,17 @@ __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *
     // Z_k = A_k + i B_k (k <= nx/2) and its Hermitian extension for k > nx/2;
     // every global load of the thread is issued before the LDS stores.
     const int total = (nh + 1) * npair;
-    constexpr int PER = (MAXE / 2 + 64 + NT - 1) / NT;   // (nx/2 + 1) R/2 <= MAXE/2 + 64
+    constexpr int NTH = vthreads(V), PER = (MAXE / 2 + 64 + NTH - 1) / NTH;   // (nx/2 + 1) R/2 <= MAXE/2 + 64
+    const bool p2 = (npair & (npair - 1)) == 0;
+    const int lp = __ffs(npair) - 1;
     C va[PER], vb[PER];
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
-        const int idx = threadIdx.x + q * NT;
-        const int k = idx / npair;
+        const int idx = threadIdx.x + q * NTH;
+        const int k = p2 ? idx >> lp : idx / npair;
         const int ja = j0 + 2 * (idx - k * npair);
-        va[q] = load_or_zero(spec, (int64_t)k * a.nv + ja, idx < total && ja < a.nv);
-        vb[q] = load_or_zero(spec, (int64_t)k * a.nv + ja + 1, idx < total && ja + 1 < a.nv);
+        va[q] = load_or_zero(spec, (int64_t)k * a.pitch + ja, idx < total && ja < a.nv);
+        vb[q] = load_or_zero(spec, (int64_t)k * a.pitch + ja + 1, idx < total && ja + 1 < a.nv);
     }
     FftTw<true, C> pt;
     if (V == VP8) pt.load(a.tw);
@@ -425,24 +429,24 @@ __global__ __launch_bounds__(NT) void irfft_kernel(FftArgs<T> a, const cx_t<T> *
     if (dflag) return;                 // uniform over the block, before any barrier
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
-        const int idx = threadIdx.x + q * NT;
+        const int idx = threadIdx.x + q * NTH;
         if (idx < total) {
-            const int k = idx / npair;
+            const int k = p2 ? idx >> lp : idx / npair;
             const int p = idx - k * npair;
             C A = va[q], B = vb[q];
             if (k == 0 || k == nh) {
                 A.y = T(0);
                 B.y = T(0);
             }
-            C *z = buf + p * nx;
-            z[k] = cmk<C>(A.x - B.y, A.y + B.x);
-            if (k != 0 && k != nh) z[nx - k] = cmk<C>(A.x + B.y, B.x - A.y);
+            const int z = p * nx;
+            buf[swz<V == VLONG>(z + k)] = cmk<C>(A.x - B.y, A.y + B.x);
+            if (k != 0 && k != nh) buf[swz<V == VLONG>(z + nx - k)] = cmk<C>(A.x + B.y, B.x - A.y);
         }
     }
     __syncthreads();
     // the last stage's outputs (natural order) go straight to the output rows
-    if constexpr (COLS) lds_fft<true, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, IrfftColSink<T>{y, j0, nx, a.logn, a.nv});
-    else lds_fft<true, V == VP8, 4>(buf, a.logn, npair, tw, pt, 0, IrfftSink<T>{y, j0, nx, a.logn, a.nv});
+    if constexpr (COLS) lds_fft<true, V == VP8, 4, NTH, V == VLONG>(buf, a.logn, npair, tw, pt, 0, IrfftColSink<T>{y, j0, nx, a.logn, a.nv});
+    else lds_fft<true, V == VP8, 4, NTH, V == VLONG>(buf, a.logn, npair, tw, pt, 0, IrfftSink<T>{y, j0, nx, a.logn, a.nv});
 }
 
 // Real rows of the irFFT left in the workgroup's LDS buffer itself, natural
@@ -505,8 +509,8 @@ __global__ __launch_bounds__(NT) void irfft_mdot_kernel(FftArgs<T> a, const cx_t
         const int idx = threadIdx.x + q * NT;
         const int k = idx / npair;
         const int ja = j0 + 2 * (idx - k * npair);
-        va[q] = load_or_zero(spec, (int64_t)k * a.nv + ja, idx < total);
-        vb[q] = load_or_zero(spec, (int64_t)k * a.nv + ja + 1, idx < total);
+        va[q] = load_or_zero(spec, (int64_t)k * a.pitch + ja, idx < total);
+        vb[q] = load_or_zero(spec, (int64_t)k * a.pitch + ja + 1, idx < total);
     }
     const double sc = (int)threadIdx.x < nvec ? gs->scale[threadIdx.x] : 0.0;
     FftTw<true, C> pt;
@@ -623,7 +627,7 @@ __global__ __launch_bounds__(NT) void rdft_kernel(FftArgs<T> a, const T *__restr
             t += k;
             if (t >= n) t -= n;
         }
-        spec[(size_t)k * a.nv + j0 + r] = cmk<C>(re, im);
+        spec[(size_t)k * a.pitch + j0 + r] = cmk<C>(re, im);
     }
 }
 
@@ -643,7 +647,7 @@ __global__ __launch_bounds__(NT) void irdft_kernel(FftArgs<T> a, const cx_t<T> *
     const int nr = a.nv - j0 < R ? a.nv - j0 : R;
     for (int e = threadIdx.x; e < nk * nr; e += NT) {
         const int k = e / nr, r = e - k * nr;
-        C v = spec[(size_t)k * a.nv + j0 + r];
+        C v = spec[(size_t)k * a.pitch + j0 + r];
         if (k == 0 || 2 * k == n) v.y = T(0);
         ss[r * nk + k] = v;
     }
@@ -671,7 +675,7 @@ __global__ __launch_bounds__(NT) void irdft_kernel(FftArgs<T> a, const cx_t<T> *
 struct TriArgs {
     int nv;           // system size
     int P;            // chunks (threads), power of two
-    int64_t S, gstride;
+    int64_t S, pitch, gstride;
     const double2 *eigen;
     const double *gm, *g0, *gp;
     int64_t cstride;         // instance stride of gm/g0/gp (0: shared)
@@ -745,7 +749,7 @@ __global__ __launch_bounds__(NT) void tridiag_kernel(TriArgs a, cx_t<T> *__restr
     const double2 e = a.eigen[k];
     const int P = a.P, n = P * M;
     const C zero = cmk<C>(T(0), T(0));
-    C *S = spec + (size_t)k * a.nv;
+    C *S = spec + (size_t)k * a.pitch;
     const int c = threadIdx.x;
     double clo[M], cmid[M], chi[M];   // per-row factors of the thread's chunk
     {
@@ -914,7 +918,7 @@ __global__ __launch_bounds__(NT) void tridiag_wave_kernel(TriArgs a, int nmodes,
     __shared__ C lds[NT / 64][64 * (M + 1)];
     C *sd = lds[wave];                    // chunk c at c (M + 1)
     const double2 e = a.eigen[k];
-    C *S = spec + blockIdx.y * a.S + (size_t)k * a.nv;
+    C *S = spec + blockIdx.y * a.S + (size_t)k * a.pitch;
     const C zero = cmk<C>(T(0), T(0));
     double lo[M], mid[M], hi[M];
     {
@@ -1132,7 +1136,7 @@ __global__ __launch_bounds__(TN) __attribute__((amdgpu_waves_per_eu(2))) void tr
     const int k = blockIdx.x;
     const double af = a.inst[blockIdx.y].afpc;
     const double2 e = a.eigen[k];
-    C *S = spec + blockIdx.y * a.S + (size_t)k * a.nv;
+    C *S = spec + blockIdx.y * a.S + (size_t)k * a.pitch;
     // pivots and band factors in chunk-interleaved order: thread t's rows
     // t M + q at q TN + t, loaded coalesced straight into registers
     const C *Rg = rp + ((size_t)blockIdx.y * gridDim.x + k) * (TN * M);
@@ -1352,7 +1356,7 @@ FftArgs<T> dft_args(vv_ctx *c, const cx_t<T> *tw, const int32_t *done, bool *twl
     if (R > cap) R = cap > 1 ? cap : 1;
     *twl = (size_t)n * sizeof(cx_t<T>) <= 32768;
     *lds = (*twl ? (size_t)n * sizeof(cx_t<T>) : 0) + (size_t)R * row_bytes;
-    return FftArgs<T>{n, 0, c->fft_rows, R, c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
+    return FftArgs<T>{n, 0, c->fft_rows, R, c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), tw, done};
 }
 
 // LDS of an FFT kernel: the packed rows, and the twiddles' copy below 1024
@@ -1404,7 +1408,7 @@ hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const
 {
     if (c->dft.n) return row_rfft(c, x, spec, done, add, gamma);
     if (c->fft_n & (c->fft_n - 1)) return add != nullptr ? hipErrorInvalidValue : rdft_t<T>(c, tw, x, spec, done);
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done, add, gamma};
     const int nb = (a.nv + a.rows - 1) / a.rows;
     const uint32_t lds = (uint32_t)fft_lds<T>(a);
@@ -1413,8 +1417,8 @@ hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const
     if (a.nx == N8) launch_timed(c, rfft_kernel<T, VP8, 2>, grid, block, lds, a, x, spec);
     else if (a.nx < N8 && first8) launch_timed(c, rfft_kernel<T, VTWL, 3>, grid, block, lds, a, x, spec);
     else if (a.nx < N8) launch_timed(c, rfft_kernel<T, VTWL, 2>, grid, block, lds, a, x, spec);
-    else if (first8) launch_timed(c, rfft_kernel<T, VLONG, 3>, grid, block, lds, a, x, spec);
-    else launch_timed(c, rfft_kernel<T, VLONG, 2>, grid, block, lds, a, x, spec);
+    else if (first8) launch_timed(c, rfft_kernel<T, VLONG, 3>, grid, dim3(NTL), lds, a, x, spec);
+    else launch_timed(c, rfft_kernel<T, VLONG, 2>, grid, dim3(NTL), lds, a, x, spec);
     return hipGetLastError();
 }
 
@@ -1453,7 +1457,7 @@ hipError_t jac_rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *u, const double *us
                       const int32_t *done)
 {
     const int R = jac_rfft_rows(c);
-    const FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, R, c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
+    const FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, R, c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), tw, done};
     const JacRows jr{uscale, c->h0, c->h1p, c->h1h, c->h2p, c->h2h, c->inst, c->ht_inv, 0.5};
     switch (R) {
     case 2: jac_rfft_kind<2>(c, a, jr, u, spec); break;
@@ -1470,14 +1474,14 @@ hipError_t irfft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, cons
     // the row blocks store pairs: a y that is not aligned for them takes the direct DFT
     if (c->dft.n && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0) return row_irfft(c, spec, y, done);
     if (c->fft_n & (c->fft_n - 1)) return irdft_t<T>(c, tw, spec, y, done);
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done};
     const int nb = (a.nv + a.rows - 1) / a.rows;
     const uint32_t lds = (uint32_t)fft_lds<T>(a);
     const dim3 grid(nb, c->B), block(NT);
     if (a.nx == N8) launch_timed(c, irfft_kernel<T, VP8, false>, grid, block, lds, a, spec, y);
     else if (a.nx < N8) launch_timed(c, irfft_kernel<T, VTWL, false>, grid, block, lds, a, spec, y);
-    else launch_timed(c, irfft_kernel<T, VLONG, false>, grid, block, lds, a, spec, y);
+    else launch_timed(c, irfft_kernel<T, VLONG, false>, grid, dim3(NTL), lds, a, spec, y);
     return hipGetLastError();
 }
 
@@ -1493,7 +1497,7 @@ bool cols_apply(const vv_ctx *c, const T *f)
 template <typename T>
 hipError_t rfft_cols_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done)
 {
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), tw, done};
     const uint32_t lds = (uint32_t)fft_lds<T>(a);
     const dim3 grid((a.nv + a.rows - 1) / a.rows, c->B), block(NT);
     if (a.nx == N8) launch_timed(c, rfft_cols_kernel<T, VP8>, grid, block, lds, a, x, spec);
@@ -1505,12 +1509,12 @@ hipError_t rfft_cols_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, 
 template <typename T>
 hipError_t irfft_cols_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, const int32_t *done)
 {
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), (int64_t)sizeof(GmresState), tw, done};
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), tw, done};
     const uint32_t lds = (uint32_t)fft_lds<T>(a);
     const dim3 grid((a.nv + a.rows - 1) / a.rows, c->B), block(NT);
     if (a.nx == N8) launch_timed(c, irfft_kernel<T, VP8, true>, grid, block, lds, a, spec, y);
     else if (a.nx < N8) launch_timed(c, irfft_kernel<T, VTWL, true>, grid, block, lds, a, spec, y);
-    else launch_timed(c, irfft_kernel<T, VLONG, true>, grid, block, lds, a, spec, y);
+    else launch_timed(c, irfft_kernel<T, VLONG, true>, grid, dim3(NTL), lds, a, spec, y);
     return hipGetLastError();
 }
 
@@ -1558,7 +1562,7 @@ hipError_t irfft_mdot_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, const
                         const int32_t *done)
 {
     const int ept = irfft_mdot_ept<T>(c);
-    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c),
+    FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done};
     const int nb = a.nv / a.rows;
     const size_t lds = fft_lds<T>(a);
@@ -1582,7 +1586,7 @@ template <> const float2 *lu_factors<float>(const vv_ctx *c) { return c->lu32; }
 template <typename T, bool TR>
 hipError_t tridiag_lu_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 {
-    TriArgs a{c->fft_rows, NT, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->lu_gm, nullptr, c->lu_gp,
+    TriArgs a{c->fft_rows, NT, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), c->eigen, c->lu_gm, nullptr, c->lu_gp,
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, done};
     const int TN = lu_threads(c->fft_rows), M = lu_rows(c->fft_rows);
     const size_t lds = (size_t)TN * (M + 1) * sizeof(cx_t<T>);
@@ -1607,7 +1611,7 @@ hipError_t tridiag_lu_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 template <typename T, bool TR>
 hipError_t tridiag_wave_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
 {
-    TriArgs a{c->fft_rows, 64, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
+    TriArgs a{c->fft_rows, 64, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, done};
     const dim3 grid((c->nmodes + NT / 64 - 1) / (NT / 64), c->B), block(NT);
     if (c->fft_rows <= 128) launch_timed(c, tridiag_wave_kernel<2, T, TR>, grid, block, 0, a, c->nmodes, spec);
@@ -1622,7 +1626,7 @@ hipError_t tridiag_t(vv_ctx *c, cx_t<T> *spec, const int32_t *done)
     if (lu_factors<T>(c) != nullptr) return tridiag_lu_t<T, TR>(c, spec, done);
     if (c->fft_rows <= 512) return tridiag_wave_t<T, TR>(c, spec, done);
     const int P = 256, m = (c->fft_rows + 255) / 256, M = m <= 4 ? 4 : (m <= 8 ? 8 : 16);
-    TriArgs a{c->fft_rows, P, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
+    TriArgs a{c->fft_rows, P, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, done};
     const size_t lds = (size_t)P * (M + 1) * sizeof(cx_t<T>);
     dim3 grid(c->nmodes, c->B), block(NT);
@@ -1745,7 +1749,7 @@ hipError_t launch_tridiag32(vv_ctx *c, float2 *spec, const int32_t *done)
 
 hipError_t launch_tridiag_factor(vv_ctx *c, double2 *rp64, float2 *rp32)
 {
-    TriArgs a{c->fft_rows, NT, spec_stride(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
+    TriArgs a{c->fft_rows, NT, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState), c->eigen, c->gm, c->g0, c->gp,
               c->coef_stride, c->cf_lo, c->cf_mid, c->cf_hi, c->inst, c->ht_inv, nullptr};
     dim3 grid((c->nmodes + NT - 1) / NT, c->B);
     const int M = lu_rows(c->fft_rows);
