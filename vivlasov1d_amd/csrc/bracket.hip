@@ -33,6 +33,8 @@ constexpr int HX = kBrHX;
 constexpr int HY = kBrHY;
 constexpr int NT = 256;
 constexpr int ROWS_PER_WAVE = TY / (NT / 64);
+constexpr int NQ = kBrCells;
+static_assert(ROWS_PER_WAVE == kBrOwn && TX == 64 && NT == 256, "br_cell's shape");
 
 // MODE_TRANSPOSED: y = alpha u + factor {u~, H} on every row, u~ = u with the
 // rows outside 2..nv-3 zeroed.  The Arakawa stencils are skew-symmetric in
@@ -114,18 +116,15 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<double> a)
         const int gj = br_halo_row(tile, (int)threadIdx.x - HX, nv);
         if (factors && gj >= 0) vf = a.h0[gj];
     }
-    constexpr int NQ = (HY * HX + NT - 1) / NT;
     double fa[NQ], fb[NQ];
     double hq[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int idx = threadIdx.x + q * NT;
+        int r, c;
         fa[q] = 0.0;
         fb[q] = 0.0;
         hq[q] = 0.0;
-        if (idx < HY * HX) {
-            const int r = idx / HX;
-            const int c = idx - r * HX;
+        if (br_cell(threadIdx.x, q, &r, &c)) {
             const int64_t o = br_halo_offset(tile, r, c, nx, nv);
             if (o >= 0) {
                 fa[q] = fin[o];
@@ -150,10 +149,8 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<double> a)
     const double us = usd;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int idx = threadIdx.x + q * NT;
-        if (idx < HY * HX) {
-            const int r = idx / HX;
-            const int c = idx - r * HX;
+        int r, c;
+        if (br_cell(threadIdx.x, q, &r, &c)) {
             const int gj = br_halo_row(tile, r, nv);
             const bool in = gj >= 0;
             double fv;
@@ -203,12 +200,12 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<double> a)
             const size_t o = (size_t)j * nx + i;
             double base;
             if (MODE == MODE_RESIDUAL) {
-                const double fder = fin[o] - fhin[o];                 // Fder = (0 + F) - Fh
+                const double fder = fa[q] - fb[q];                   // Fder = (0 + F) - Fh
                 base = 0.0 + ht_inv * fder;                     // Y = 0; Y += Fder/dt
             } else if (MODE == MODE_JACOBIAN) {
                 base = jacobian_base(ht_inv, win.f0[2]);         // Y = 0; Y += u/dt
             } else if (MODE == MODE_TRANSPOSED) {
-                base = a.alpha * (fin[o] * us);
+                base = a.alpha * (fa[q] * us);
             } else {
                 base = a.store ? 0.0 : yout[o];
             }
@@ -267,16 +264,14 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
                            : 1.0;
     double c1, c2;
     sep_weights(kind, a.factor, a.inst[b].af1, a.inst[b].af2, c1, c2);
-    constexpr int NQ = (HY * HX + NT - 1) / NT;
     T fa[NQ], fb[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int idx = t + q * NT;
+        int r, c;
         fa[q] = T(0);
         fb[q] = T(0);
-        if (idx < HY * HX) {
-            const int r = idx / HX;
-            const int64_t o = br_halo_offset(tile, r, idx - r * HX, nx, nv);
+        if (br_cell(t, q, &r, &c)) {
+            const int64_t o = br_halo_offset(tile, r, c, nx, nv);
             if (o >= 0) {
                 fa[q] = fin[o];
                 if (MODE == MODE_RESIDUAL) fb[q] = fhin[o];
@@ -295,8 +290,8 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
     const T us = (T)usd;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int idx = t + q * NT;
-        if (idx < HY * HX) (&sF[0][0])[idx] = MODE == MODE_RESIDUAL ? half * fb[q] + half * fa[q] : fa[q];
+        int r, c;
+        if (br_cell(t, q, &r, &c)) sF[r][c] = MODE == MODE_RESIDUAL ? half * fb[q] + half * fa[q] : fa[q];
     }
     if (t < HX) sP[t] = phi;
     if (krow) {
@@ -319,7 +314,7 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
         if (j < nv) {
             const size_t o = (size_t)j * nx + i;
             T out;
-            if (MODE == MODE_RESIDUAL) out = T(0) + ht_inv * (fin[o] - fhin[o]);
+            if (MODE == MODE_RESIDUAL) out = T(0) + ht_inv * (fa[q] - fb[q]);
             else out = jacobian_base(ht_inv, win.f0[2]);
             if (j >= 2 && j < nv - 2) out += win.bracket(sA[rr], B, FAR);
             if (MODE == MODE_JACOBIAN) out = scaled(out, us);      // J is linear
@@ -377,15 +372,13 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
         const int gj = br_halo_row(tile, (int)threadIdx.x - HX, nv);
         if (gj >= 0) vf = a.h0[gj];
     }
-    constexpr int NQ = (HY * HX + NT - 1) / NT;
     double fa[NQ], ga[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int idx = threadIdx.x + q * NT;
+        int r, c;
         fa[q] = ga[q] = 0.0;
-        if (idx < HY * HX) {
-            const int r = idx / HX;
-            const int64_t o = br_halo_offset(tile, r, idx - r * HX, nx, nv);
+        if (br_cell(threadIdx.x, q, &r, &c)) {
+            const int64_t o = br_halo_offset(tile, r, c, nx, nv);
             if (o >= 0) {
                 fa[q] = fin[o];
                 ga[q] = gin[o];
@@ -403,9 +396,8 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int idx = threadIdx.x + q * NT;
-        if (idx < HY * HX) {
-            const int r = idx / HX, c = idx - r * HX;
+        int r, c;
+        if (br_cell(threadIdx.x, q, &r, &c)) {
             const int gj = br_halo_row(tile, r, nv);
             sF[r][c] = (gj >= 2 && gj < nv - 2) ? fa[q] * us : 0.0;
             sH[r][c] = gj >= 0 ? compose_have(sV[r], sX[0][c], sX[1][c], sX[2][c], sX[3][c]) : 0.0;
@@ -427,7 +419,7 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
         const int j = tile.j0 + rr0 + q;
         if (j < nv && i < nx) {
             const size_t o = (size_t)j * nx + i;
-            yout[o] = arakawa_add<KIND>(wh, a.alpha * (fin[o] * us), a.factor, af1, af2);
+            yout[o] = arakawa_add<KIND>(wh, a.alpha * (fa[q] * us), a.factor, af1, af2);
             cs += arakawa_add<KIND>(wg, 0.0, 1.0, af1, af2);
         }
         if (q + 1 < ROWS_PER_WAVE) {

@@ -79,6 +79,32 @@ __host__ __device__ __forceinline__ int64_t br_halo_offset(const BrTile &t, int 
     return (int64_t)gj * nx + wrap_x(t.i0 - 2 + c, nx);
 }
 
+// Cell q (< kBrCells) of thread t of a bracket workgroup (256 threads): the
+// thread's own output cells first (rows 4 (t / 64) .. + 3 of the tile, column
+// t % 64: consecutive rows of one column, so the later ones cost an addition each, and
+// what a thread loaded for its outputs it keeps), then its share of the halo
+// (four rows of HX cells and four columns of TY).  False where it has none.
+constexpr int kBrOwn = 4, kBrCells = 6;
+__host__ __device__ __forceinline__ bool br_cell(int t, int q, int *r, int *c)
+{
+    if (q < kBrOwn) {
+        *r = (t >> 6) * kBrOwn + q + 2;
+        *c = (t & 63) + 2;
+        return true;
+    }
+    const int h = t + (q - kBrOwn) * 256;
+    if (h < 4 * kBrHX) {
+        const int k = h / kBrHX;
+        *r = k < 2 ? k : kBrTY + k;
+        *c = h - k * kBrHX;
+        return true;
+    }
+    const int k = h - 4 * kBrHX;
+    *r = 2 + (k >> 2);
+    *c = (k & 3) < 2 ? (k & 3) : kBrTX + (k & 3);
+    return k < 4 * kBrTY;
+}
+
 // x index of staged column c (the 1D x-factors of H), always in [0, nx).
 __host__ __device__ __forceinline__ int br_halo_column(const BrTile &t, int c, int nx)
 {
