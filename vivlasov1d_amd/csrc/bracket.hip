@@ -329,8 +329,10 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
 //   y = alpha u + factor {u~, H_ave} on all rows,  csum = sum_j {u~, g}_ij
 // by 16-row bands (tile row t at csum[t nx + i], instances cstride apart): the
 // coupling term needs only the column sums of its bracket (g = f_bar in a.h2d),
-// so that field is neither stored nor read back.  u~ is staged once for both;
-// three 20 x 68 tiles (33 KB of LDS).  hs: the previous step's Hessenberg
+// so that field is neither stored nor read back.  u~ is staged once for both, and
+// the bracket with H_ave is the factored one (SepWin: H is 0 outside the grid, where
+// its coefficients only meet rows of u~ that are 0): two 20 x 68 tiles (22 KB of
+// LDS).  hs: the previous step's Hessenberg
 // update or the cycle's start, as in the fused J u + rFFT.  At 256 x 512 it
 // replaces two bracket launches (5.2 us each), the density (3.7 us) and the
 // update (3.6 us).
@@ -344,8 +346,9 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
         return;
     }
     const int b = blockIdx.y;
-    __shared__ double sF[HY][HX], sH[HY][HX], sG[HY][HX];
-    __shared__ double sX[4][HX], sV[HY];
+    __shared__ double sF[HY][HX], sG[HY][HX];
+    __shared__ double sP[HX], sS[NT / 64][TX];
+    __shared__ __align__(16) double sA[TY][4];
     __shared__ double red[kGdNW + 1];
     const int nx = a.nx, nv = a.nv;
     const BrTile tile = br_tile((int)blockIdx.x - extra, nx, nv);
@@ -361,17 +364,16 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
     double us = a.uscale != nullptr && !extra
                     ? *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a.uscale) + b * a.gstride)
                     : 1.0;
-    double xf[4] = {0.0, 0.0, 0.0, 0.0}, vf = 0.0;
+    double c1, c2, phi = 0.0;
+    sep_weights(KIND, a.factor, a.inst[b].af1, a.inst[b].af2, c1, c2);
     if (threadIdx.x < HX) {
         const size_t gi = xo + br_halo_column(tile, (int)threadIdx.x, nx);
-        xf[0] = a.h1p[gi];
-        xf[1] = a.h1h[gi];
-        xf[2] = a.h2p[gi];
-        xf[3] = a.h2h[gi];
-    } else if (threadIdx.x < HX + HY) {
-        const int gj = br_halo_row(tile, (int)threadIdx.x - HX, nv);
-        if (gj >= 0) vf = a.h0[gj];
+        phi = phi_ave(a.h1p[gi], a.h1h[gi], a.h2p[gi], a.h2h[gi]);
     }
+    const int kr = (int)threadIdx.x - 128;
+    const bool krow = kr >= 0 && kr < TY;
+    double kc[4];
+    if (krow) sep_row(a.h0, tile.j0 + kr, nv, c1, c2, kc);
     double fa[NQ], ga[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -387,20 +389,17 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
     }
     if (dflag) return;                 // uniform over the block, before any barrier
     if (extra) us = scale_of(block_sum_all(nshare, red));
-    if (threadIdx.x < HX) {
+    if (threadIdx.x < HX) sP[threadIdx.x] = phi;
+    if (krow) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) sX[m][threadIdx.x] = xf[m];
-    } else if (threadIdx.x < HX + HY) {
-        sV[threadIdx.x - HX] = vf;
+        for (int q = 0; q < 4; ++q) sA[kr][q] = kc[q];
     }
-    __syncthreads();
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         int r, c;
         if (br_cell(threadIdx.x, q, &r, &c)) {
             const int gj = br_halo_row(tile, r, nv);
             sF[r][c] = (gj >= 2 && gj < nv - 2) ? fa[q] * us : 0.0;
-            sH[r][c] = gj >= 0 ? compose_have(sV[r], sX[0][c], sX[1][c], sX[2][c], sX[3][c]) : 0.0;
             sG[r][c] = ga[q];
         }
     }
@@ -408,30 +407,32 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = tile.i0 + lane, cx = lane + 2, rr0 = wave * ROWS_PER_WAVE;
     const double af1 = a.inst[b].af1, af2 = a.inst[b].af2;
-    const TileRd<double, HX> rF{&sF[0][0]}, rH{&sH[0][0]}, rG{&sG[0][0]};
+    const TileRd<double, HX> rF{&sF[0][0]}, rG{&sG[0][0]};
     double *__restrict__ yout = a.y + fo;
     double cs = 0.0;
-    ArakawaWin<double> wh, wg;
-    wh.load(rF, rH, rr0 + 2, cx);
+    double B[4];
+    sep_coef(sP[cx - 2], sP[cx - 1], sP[cx], sP[cx + 1], sP[cx + 2], c1, c2, B);
+    SepWin<double> wh;
+    ArakawaWin<double> wg;
+    wh.load(rF, rr0 + 2, cx);
     wg.load(rF, rG, rr0 + 2, cx);
 #pragma unroll
     for (int q = 0; q < ROWS_PER_WAVE; ++q) {
         const int j = tile.j0 + rr0 + q;
         if (j < nv && i < nx) {
             const size_t o = (size_t)j * nx + i;
-            yout[o] = arakawa_add<KIND>(wh, a.alpha * (fa[q] * us), a.factor, af1, af2);
+            yout[o] = a.alpha * (fa[q] * us) + wh.bracket(sA[rr0 + q], B, KIND != VV_BRACKET_J1);
             cs += arakawa_add<KIND>(wg, 0.0, 1.0, af1, af2);
         }
         if (q + 1 < ROWS_PER_WAVE) {
-            wh.advance(rF, rH, rr0 + q + 3, cx);
+            wh.advance(rF, rr0 + q + 3, cx);
             wg.advance(rF, rG, rr0 + q + 3, cx);
         }
     }
-    __syncthreads();                   // the tiles are read: sX takes the waves' sums
-    sX[wave][lane] = cs;
+    sS[wave][lane] = cs;
     __syncthreads();
     if (wave == 0 && i < nx)
-        csum[b * cstride + (size_t)(tile.j0 / TY) * nx + i] = ((sX[0][lane] + sX[1][lane]) + sX[2][lane]) + sX[3][lane];
+        csum[b * cstride + (size_t)(tile.j0 / TY) * nx + i] = ((sS[0][lane] + sS[1][lane]) + sS[2][lane]) + sS[3][lane];
 }
 
 template <int MODE>
