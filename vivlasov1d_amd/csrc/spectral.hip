@@ -1675,8 +1675,8 @@ hipError_t launch_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t 
 // layout does not depend on it): the largest of 8, 4, 2 that still leaves
 // >= 6 workgroups per CU (fewer halo rows per output row; batched contexts),
 // else the FFT kernels' rows when those are 2, 4 or 8, else 2.  Measured at
-// 512x1024 with 22 instances: 108 / 82 / 80 us at 2 / 4 / 8 rows; a single
-// 1024x2048 instance: 23.4 / 23.2 / 28.9 us.
+// 512x1024 with 22 instances: 108 / 82 / 80 us at 2 / 4 / 8 rows (unfactored
+// stencil); a single 1024x2048 instance: 21.0 / 17.2 us at 2 / 4 rows.
 int jac_rfft_rows(const vv_ctx *c)
 {
     const int nx = c->fft_n;
