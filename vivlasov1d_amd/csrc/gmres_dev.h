@@ -38,16 +38,16 @@ __device__ __forceinline__ double norm_share(const double *part, int nb)
 }
 
 // the scale of the Krylov vector whose squared norm is tot (VecNormalize)
-__device__ __forceinline__ double scale_of(double tot)
+__host__ __device__ __forceinline__ double scale_of(double tot)
 {
     const double tt = sqrt(tot);
     return tt != 0.0 ? 1.0 / tt : 1.0;
 }
 
-__device__ __forceinline__ int ksp_test(const GmresState *g, double res)
+__host__ __device__ __forceinline__ int ksp_test(const GmresState *g, double res)
 {
 #pragma clang fp contract(off)
-    if (!isfinite(res)) return VV_KSP_DIVERGED_NANORINF;
+    if (!__builtin_isfinite(res)) return VV_KSP_DIVERGED_NANORINF;
     if (res <= g->ttol) return res < g->atol ? VV_KSP_CONVERGED_ATOL : VV_KSP_CONVERGED_RTOL;
     if (res >= g->dtol * g->st.rnorm0) return VV_KSP_DIVERGED_DTOL;
     return 0;
@@ -61,13 +61,32 @@ __device__ __forceinline__ void report(uint32_t *hout, uint32_t seq, bool done)
     __hip_atomic_store(hout, 2 * seq + (done ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Start of a cycle on V_0 with ||V_0||^2 = tot (KSPGMRESCycle entry:
-// VecNormalize(VV(0)), zero-residual and convergence tests), by one thread.
-__device__ __forceinline__ void cycle_start(const HessArgs &a, GmresState *g, double tot)
+// The end of the cycle as the launch that carries update it + 1 takes it (it = -1:
+// after the cycle's start); st.done is for every other launch.
+__host__ __device__ __forceinline__ void set_skip(GmresState *g, int it, bool end) { g->skip[(it + 1) & 1] = end; }
+
+// Whether a launch that carries the update or start `a` has nothing to do for
+// instance b besides it: done as of the update before; at a start, not taking part.
+// The launch's other workgroups ask while hess_update runs in its first one, so
+// nothing that hess_update writes is read here: skip by the parity of the step
+// (it writes the other one), at a restart what the solution update of the cycle
+// before left, at a first start the instance mask.
+__host__ __device__ __forceinline__ bool carried_skip(const HessArgs &a, const GmresState *g, int b)
+{
+    if (a.start == 2) return a.init.active != nullptr && a.init.active[b] == 0;
+    if (a.start == 1) return g->over != 0;
+    return g->skip[a.it & 1] != 0;
+}
+
+__device__ __forceinline__ bool hess_skip(const HessArgs &a) { return carried_skip(a, a.g + blockIdx.y, blockIdx.y); }
+
+// Start of a cycle on V_0 of instance b with ||V_0||^2 = tot (KSPGMRESCycle
+// entry: VecNormalize(VV(0)), zero-residual and convergence tests), by one thread.
+__host__ __device__ __forceinline__ void cycle_start(const HessArgs &a, GmresState *g, int b, double tot)
 {
 #pragma clang fp contract(off)
     if (a.start == 2) {
-        const int32_t act = a.init.active != nullptr ? a.init.active[blockIdx.y] : 1;
+        const int32_t act = a.init.active != nullptr ? a.init.active[b] : 1;
         g->st.its = 0;
         g->st.reason = 0;
         g->st.active = act;
@@ -84,16 +103,19 @@ __device__ __forceinline__ void cycle_start(const HessArgs &a, GmresState *g, do
     // an instance that is not solving, or whose solve has ended, stays done
     if (!g->st.active || g->st.reason != 0) {
         g->st.done = 1;
+        set_skip(g, -1, true);
         return;
     }
     const double nrm = sqrt(tot);
     g->st.done = 0;
+    set_skip(g, -1, false);
     g->scale[0] = scale_of(tot);
     g->grs[0] = nrm;
     g->st.res = nrm;
     if (nrm == 0.0) {
         g->st.reason = VV_KSP_CONVERGED_ATOL;
         g->st.done = 1;
+        set_skip(g, -1, true);
         return;
     }
     if (a.start == 2) {
@@ -104,18 +126,8 @@ __device__ __forceinline__ void cycle_start(const HessArgs &a, GmresState *g, do
     if (rsn != 0) {
         g->st.reason = rsn;
         g->st.done = 1;
+        set_skip(g, -1, true);
     }
-}
-
-// Whether a kernel that carries the update or start `a` has nothing to do for
-// its instance: done as of the step before; at a start the flag is stale, and
-// the instances that take part count.
-__device__ __forceinline__ bool hess_skip(const HessArgs &a)
-{
-    const GmresState *g = a.g + blockIdx.y;
-    if (a.start == 2) return a.init.active != nullptr && a.init.active[blockIdx.y] == 0;
-    if (a.start == 1) return !g->st.active || g->st.reason != 0;
-    return g->st.done != 0;
 }
 
 // VecNormalize of V_{it+1} from the maxpy partials, then
@@ -134,7 +146,7 @@ __device__ __forceinline__ void hess_update(const HessArgs &a)
     if (a.start) {
         __shared__ double sred[kGdNW + 1];
         const double tot = block_sum_all(norm_share(part, a.nb), sred);
-        if (threadIdx.x == 0) cycle_start(a, g, tot);
+        if (threadIdx.x == 0) cycle_start(a, g, blockIdx.y, tot);
         return;
     }
     const int it = a.it;
@@ -151,6 +163,7 @@ __device__ __forceinline__ void hess_update(const HessArgs &a)
     const double grs_it = g->grs[it];
     const double acc = norm_share(part, a.nb);
     if (done) {                        // uniform over the block, before any barrier
+        if (t == 0) set_skip(g, it, true);
         if (hout && t == 0) report(hout, a.seq, true);
         return;
     }
@@ -203,6 +216,7 @@ __device__ __forceinline__ void hess_update(const HessArgs &a)
     g->st.reason = reason;
     const bool end = reason != 0 || g->st.it >= g->max_k || g->st.its >= g->max_it;
     if (end) g->st.done = 1;
+    set_skip(g, it, end);
     if (hout) report(hout, a.seq, end);
 }
 

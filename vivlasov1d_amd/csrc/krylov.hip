@@ -350,6 +350,7 @@ __global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, doub
         reason = VV_KSP_DIVERGED_BREAKDOWN;
         if (blockIdx.x == 0 && t == 0) g->st.reason = reason;
     }
+    if (blockIdx.x == 0 && t == 0) g->over = !g->st.active || reason != 0;
     if (hout != nullptr && blockIdx.x == 0 && t == 0) {
         // per-field stores by one lane
         GmresStatus *ho = hout + blockIdx.y;

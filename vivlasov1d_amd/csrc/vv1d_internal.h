@@ -56,6 +56,9 @@ struct GmresState {
     double ttol, rtol, atol, dtol, haptol;
     int32_t max_it;
     int32_t max_k;
+    int32_t skip[2];                 // done as of update it - 1, at it & 1: for the launch that carries update it
+    int32_t over;                    // the solve has ended, as of the last solution update: for a restart's launch
+    int32_t pad;
 };
 
 // Tolerances and limits a solve starts with, and which instances take part
