@@ -663,6 +663,21 @@ int arnoldi_step32(vv_ctx *c, int it)
     return VV_OK;
 }
 
+// What a solve leaves due goes with it: one that ended well leaves nothing, but an
+// error can come between the launch of an update's (or a start's) partials and
+// the launch that takes it, and the next call on the context must not find it.
+struct DueScope {
+    vv_ctx *c;
+    explicit DueScope(vv_ctx *ctx) : c(ctx) {}
+    DueScope(const DueScope &) = delete;
+    ~DueScope()
+    {
+        c->pend_it = -1;
+        c->pend_start = 0;
+        c->report_out = nullptr;
+    }
+};
+
 int max_it_of(const GmresStatus *s, int B)
 {
     int m = 0;
@@ -779,6 +794,7 @@ int restart_cycles(vv_ctx *c, const double *b, double *x)
 
 int ksp_solve_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_params *kp, vv_ksp_result *res)
 {
+    const DueScope due(c);
     set_start(c, kp->rtol, kp->atol, kp->dtol, kp->max_it);
     VV_CHECK(launch_start(c, b, true), "cycle start");
     if (int r = run_cycle(c, false, x, true)) return r;
@@ -886,6 +902,7 @@ int snes_graph(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp)
 
 int snes_impl(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp, vv_ksp_result *res)
 {
+    const DueScope due(c);
     if (c->use_graph) {
         if (int r = no_diss(c, "graph replay")) return r;
         if (int r = snes_graph(c, f, fh, kp)) return r;
@@ -937,6 +954,7 @@ int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_par
 {
     if (c->B != 1) return fail(c, VV_ERR_UNSUPPORTED, "the mixed-precision solve takes one instance");
     if (int r = ensure_mixed(c)) return r;
+    const DueScope due(c);
     const int64_t N = c->N;
     double rnorm0 = 0.0, rnorm = 0.0;
     const double *rsrc = b;
@@ -1402,6 +1420,7 @@ int vv_autotune(vv_ctx *c, int32_t *fft_rows, int32_t *cgs_ept)
     if (c->p.precond == VV_PRECOND_NONE)
         return fail(c, VV_ERR_UNSUPPORTED, "autotune needs a tensor-product preconditioner");
     drop_graph(c);
+    const DueScope due(c);
     const int prof = c->prof;
     c->prof = 0;
     hipEvent_t e0, e1;

@@ -610,7 +610,7 @@ hipError_t row_fwd_t(vv_ctx *c, RowFwd<T> p, cx_t<T> *spec, const int32_t *done,
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, g.RW, c->N, spec_stride(c), spec_pitch(c), (int64_t)sizeof(GmresState),
                  twiddles<T>(c), done, add, gamma};
     HessArgs hs{};
-    if (MODE == F_JAC) hs = take_update(c);
+    if (MODE == F_JAC && p.jr.uscale != nullptr) hs = take_update(c);    // a Krylov vector: its scale is due
     const dim3 grid((a.nv + g.RW - 1) / g.RW + (hs.nb > 0 ? 1 : 0), c->B);
     if (R == 4) fwd_launch<MODE, 4, T>(c, a, g, p, hs, grid, lds, spec);
     else fwd_launch<MODE, 2, T>(c, a, g, p, hs, grid, lds, spec);

@@ -1427,7 +1427,8 @@ void jac_rfft_launch(vv_ctx *c, const FftArgs<T> &a, const JacRows &jr, const T 
 {
     const size_t fft = (size_t)(R >> 1) * a.nx * sizeof(cx_t<T>);
     const size_t strip = jac_strip_lds<T>(R, NS);
-    const HessArgs hs = take_update(c);
+    HessArgs hs{};
+    if (jr.uscale != nullptr) hs = take_update(c);     // a Krylov vector: its scale is due
     const dim3 grid((a.nv + R - 1) / R + (hs.nb > 0 ? 1 : 0), c->B);
     const size_t tws = NS != 4 ? a.nx * sizeof(cx_t<T>) : 0;
     launch_timed(c, jac_rfft_kernel<KIND, R, NS, T>, grid, dim3(NT), (uint32_t)((fft > strip ? fft : strip) + tws), a,
