@@ -411,12 +411,14 @@ __global__ __launch_bounds__(vthreads(V)) void irfft_kernel(FftArgs<T> a, const 
     // Z_k = A_k + i B_k (k <= nx/2) and its Hermitian extension for k > nx/2;
     // every global load of the thread is issued before the LDS stores.
     const int total = (nh + 1) * npair;
-    constexpr int NTH = vthreads(V), PER = (MAXE / 2 + 64 + NTH - 1) / NTH;   // (nx/2 + 1) R/2 <= MAXE/2 + 64
+    // (nx/2 + 1) R/2 <= MAXE/2 + MAXE/nx: nx >= 8 for the short lines, else >= 1024
+    constexpr int NTH = vthreads(V), PER = (MAXE / 2 + (V == VTWL ? MAXE / 8 : MAXE / N8) + NTH - 1) / NTH;
     const bool p2 = (npair & (npair - 1)) == 0;
     const int lp = __ffs(npair) - 1;
     C va[PER], vb[PER];
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
+        if (V == VTWL && q * NTH >= total) break;   // uniform: short blocks skip the rest
         const int idx = threadIdx.x + q * NTH;
         const int k = p2 ? idx >> lp : idx / npair;
         const int ja = j0 + 2 * (idx - k * npair);
