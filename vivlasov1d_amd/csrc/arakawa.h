@@ -166,16 +166,19 @@ __device__ __forceinline__ void sep_weights(int kind, double factor, double af1,
     c2 = kind == VV_BRACKET_J1 ? 0.0 : kind == VV_BRACKET_J4 ? -(factor * af2) : factor * af2;
 }
 
-// A (or B) from the five values of h0 (or phi) around the centre h
+// A (or B) from the five values of h0 (or phi) around the centre h.  J1 has no
+// terms at distance 2: those values are left out, not multiplied by 0 (an
+// infinity or NaN there would spread to points whose stencil does not hold it).
 template <typename T>
 __device__ __forceinline__ void sep_coef(double hmm, double hm, double h, double hp, double hpp, double c1, double c2,
                                          T (&k)[4])
 {
 #pragma clang fp contract(off)
     const double W = hp - hm;
-    k[0] = (T)(c1 * (hp - h) + c2 * (W + (hpp - h)));
+    const bool far = c2 != 0.0;
+    k[0] = (T)(c1 * (hp - h) + (far ? c2 * (W + (hpp - h)) : 0.0));
     k[1] = (T)(2.0 * (c1 * W));
-    k[2] = (T)(c1 * (h - hm) + c2 * (W + (h - hmm)));
+    k[2] = (T)(c1 * (h - hm) + (far ? c2 * (W + (h - hmm)) : 0.0));
     k[3] = (T)(c2 * W);
 }
 
@@ -232,17 +235,20 @@ struct SepWin {
         fp2 = F(cn, cx, 2);
     }
 
-    // the weighted bracket at the centre; far: the kind has J2 terms (their
-    // points at distance 2 are not read into a J1 result)
-    __device__ __forceinline__ T bracket(const T *A, const T (&B)[4], bool far) const
+    // the weighted bracket at the centre, of the points that the kind's stencil
+    // holds: J1 none at distance 2, J2 no nearest neighbours (coefficients that
+    // are 0, but an infinity or NaN would come through them)
+    __device__ __forceinline__ T bracket(const T *A, const T (&B)[4], int kind) const
     {
 #pragma clang fp contract(off)
         T s = A[0] * (fp[2] - fm[2]), t = B[0] * (fp[2] - fp[0]);
-        s = fma_t(A[1], fp[1] - fm[1], s);
-        t = fma_t(B[1], f0[3] - f0[1], t);
+        if (kind != VV_BRACKET_J2) {
+            s = fma_t(A[1], fp[1] - fm[1], s);
+            t = fma_t(B[1], f0[3] - f0[1], t);
+        }
         s = fma_t(A[2], fp[0] - fm[0], s);
         t = fma_t(B[2], fm[2] - fm[0], t);
-        if (far) {
+        if (kind != VV_BRACKET_J1) {
             s = fma_t(A[3], fp2 - fm2, s);
             t = fma_t(B[3], f0[4] - f0[0], t);
         }

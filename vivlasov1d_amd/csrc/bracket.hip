@@ -240,8 +240,8 @@ __global__ __launch_bounds__(NT) void bracket_kernel(BrArgs<double> a)
 // many wavefronts a CU as there are slots for, against 24 with H beside it) and
 // a quarter of the arithmetic.  F(f) at 1024 x 2048 18.6 us unfactored, 13.9 here;
 // J u at 2048 x 1024 13.7, 9.6.  T is double, or float for the FP32 cycle.
-template <bool FAR, int MODE, typename T>
-__global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
+template <int KIND, int MODE, typename T>
+__global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a)
 {
     const int b = blockIdx.y;
     __shared__ T sF[HY][HX];
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
                            ? *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a.uscale) + b * a.gstride)
                            : 1.0;
     double c1, c2;
-    sep_weights(kind, a.factor, a.inst[b].af1, a.inst[b].af2, c1, c2);
+    sep_weights(KIND, a.factor, a.inst[b].af1, a.inst[b].af2, c1, c2);
     T fa[NQ], fb[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a, int kind)
             T out;
             if (MODE == MODE_RESIDUAL) out = T(0) + ht_inv * (fa[q] - fb[q]);
             else out = jacobian_base(ht_inv, win.f0[2]);
-            if (j >= 2 && j < nv - 2) out += win.bracket(sA[rr], B, FAR);
+            if (j >= 2 && j < nv - 2) out += win.bracket(sA[rr], B, KIND);
             if (MODE == MODE_JACOBIAN) out = scaled(out, us);      // J is linear
             yout[o] = out;
         }
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
         const int j = tile.j0 + rr0 + q;
         if (j < nv && i < nx) {
             const size_t o = (size_t)j * nx + i;
-            yout[o] = a.alpha * (fa[q] * us) + wh.bracket(sA[rr0 + q], B, KIND != VV_BRACKET_J1);
+            yout[o] = a.alpha * (fa[q] * us) + wh.bracket(sA[rr0 + q], B, KIND);
             cs += arakawa_add<KIND>(wg, 0.0, 1.0, af1, af2);
         }
         if (q + 1 < ROWS_PER_WAVE) {
@@ -460,9 +460,11 @@ template <int MODE, typename T>
 hipError_t launch_sep(vv_ctx *c, BrArgs<T> a)
 {
     const dim3 grid(br_tiles(c->p.nx, c->p.nv), c->B), block(NT);
-    const int kind = c->p.bracket;
-    if (kind == VV_BRACKET_J1) launch_timed(c, bracket_sep_kernel<false, MODE, T>, grid, block, 0, a, kind);
-    else launch_timed(c, bracket_sep_kernel<true, MODE, T>, grid, block, 0, a, kind);
+    switch (c->p.bracket) {
+    case VV_BRACKET_J1: launch_timed(c, bracket_sep_kernel<VV_BRACKET_J1, MODE, T>, grid, block, 0, a); break;
+    case VV_BRACKET_J2: launch_timed(c, bracket_sep_kernel<VV_BRACKET_J2, MODE, T>, grid, block, 0, a); break;
+    default: launch_timed(c, bracket_sep_kernel<VV_BRACKET_J4, MODE, T>, grid, block, 0, a); break;
+    }
     return hipGetLastError();
 }
 

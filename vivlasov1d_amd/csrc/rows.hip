@@ -246,7 +246,6 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
         const T ht_inv = (T)p.jr.ht_inv;
         double c1, c2;
         sep_weights(p.kind, p.jr.factor, p.jr.inst[b].af1, p.jr.inst[b].af2, c1, c2);
-        const bool far = p.kind != VV_BRACKET_J1;
         const int grp = g.G > 1 ? div_by(t, g.mW) : 0, col = t - grp * W;
         T us = T(1);
         for (int s = 0; s < g.NS; ++s) {
@@ -334,7 +333,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                         else base = jacobian_base(ht_inv, win.f0[2]);
                         out = base;
                         if (j >= 2 && j < nv - 2) {
-                            out = base + win.bracket(sA[r0 + q], B, far);
+                            out = base + win.bracket(sA[r0 + q], B, p.kind);
                             if (coll)
                                 out = (T)add_collision((double)out, (double)win.f0[1], (double)win.f0[2],
                                                        (double)win.f0[3], p.cv[j + 1], p.cv[j - 1], cn, cU, ca,

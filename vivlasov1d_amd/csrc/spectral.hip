@@ -168,7 +168,7 @@ __device__ __forceinline__ void jac_strip_load(const T *__restrict__ u, const Ja
 
 // Thread t's column of the staged strip down the R output rows (tile rows
 // 2 .. R+1): J u, or 0 on rows past nv (the rFFT's zero rows).
-template <bool FAR, int R, typename T, typename RF>
+template <int KIND, int R, typename T, typename RF>
 __device__ __forceinline__ void jac_walk(const RF &rF, const T (*sA)[4], const double *sP, double c1, double c2,
                                          int j0, int nv, T ht_inv, T us, T (&res)[R])
 {
@@ -183,7 +183,7 @@ __device__ __forceinline__ void jac_walk(const RF &rF, const T (*sA)[4], const d
         T out = T(0);
         if (j < nv) {
             out = jacobian_base(ht_inv, win.f0[2]);
-            if (j >= 2 && j < nv - 2) out += win.bracket(sA[q], B, FAR);
+            if (j >= 2 && j < nv - 2) out += win.bracket(sA[q], B, KIND);
             out = scaled(out, us);                     // == J of the VecScale'd Krylov vector
         }
         res[q] = out;
@@ -276,7 +276,7 @@ __device__ __forceinline__ void jac_rfft_body(FftArgs<T> a, JacRows jr, HessArgs
             }
             us = (T)usd;
         }
-        jac_walk<KIND != VV_BRACKET_J1, R>(TileRd<T, SP>{cF}, sA, cP, c1, c2, j0, nv, ht_inv, us, res[s]);
+        jac_walk<KIND, R>(TileRd<T, SP>{cF}, sA, cP, c1, c2, j0, nv, ht_inv, us, res[s]);
     }
     __syncthreads();
     // twiddles in flight during the first stage (not held through the walks)
