@@ -1550,14 +1550,22 @@ int vv_function(vv_ctx *c, const double *f, const double *fh, double *y)
 {
     if (int r = check_ctx(c)) return r;
     if (!f || !fh || !y) return fail(c, VV_ERR_INVALID, "null field");
-    return pc_residual(c, f, fh, y);
+    if (c->p.precond != VV_PRECOND_NONE) return pc_residual(c, f, fh, y);
+    // F itself, in the reference's operation order (through X: y may be f or fh)
+    VV_PLAUNCH(P_RES, 3 * b_field(c), -1, launch_residual(c, f, fh, c->X), "residual");
+    if (int r = diss_function(c, f, fh, c->X)) return r;
+    return precond(c, c->X, y, nullptr);
 }
 
 int vv_jacobian(vv_ctx *c, const double *u, double *y)
 {
     if (int r = check_ctx(c)) return r;
     if (!u || !y) return fail(c, VV_ERR_INVALID, "null field");
-    return pc_jacobian(c, u, y);
+    if (c->p.precond != VV_PRECOND_NONE) return pc_jacobian(c, u, y);
+    // J u itself, as above
+    VV_PLAUNCH(P_JAC, 2 * b_field(c), -1, launch_jacobian_plain(c, u, c->X), "jacobian");
+    if (int r = diss_jacobian(c, u, nullptr, c->X, nullptr)) return r;
+    return precond(c, c->X, y, nullptr);
 }
 
 namespace {
@@ -1980,7 +1988,7 @@ int vv_snes_ksponly_mixed(vv_ctx *c, double *f, const double *fh, const vv_ksp_p
     if (!(mp->inner_rtol > 0.0 && mp->inner_rtol < 1.0) || mp->max_cycles < 1)
         return fail(c, VV_ERR_INVALID, "inner_rtol must be in (0, 1) and max_cycles >= 1");
     if (c->B != 1) return fail(c, VV_ERR_UNSUPPORTED, "the mixed-precision solve takes one instance");
-    if (int r = vv_function(c, f, fh, c->rhs)) return r;
+    if (int r = pc_residual(c, f, fh, c->rhs)) return r;
     vv_ksp_result kr{};
     // SNESSolve_KSPONLY takes the step unless the linear solve diverged
     if (int r = ksp_solve_mixed_impl(c, c->rhs, c->D, kp, mp, &kr, cycles, f)) return r;
