@@ -397,8 +397,8 @@ int no_diss(vv_ctx *c, const char *what)
 }
 
 // The spectrum of J u (u times its optional device scale) in one launch: the
-// strip kernel (nx = 256, 512, 1024), or the row blocks for every other length
-// up to kRowsNx and for a collision term.  fwd_fused: whether there is such a
+// strip kernel (nx = 256, 512, 1024), or the row blocks for other lengths
+// (rows_apply) and for a collision term.  fwd_fused: whether there is such a
 // launch for the context.
 bool fwd_fused(const vv_ctx *c)
 {
@@ -496,7 +496,7 @@ int apply_pc(vv_ctx *c, const double *x, double *y, const int32_t *done)
 // whether the rFFT takes an x-only field along (not the direct DFT of long odd lengths)
 bool add_fused(const vv_ctx *c)
 {
-    return c->tb == nullptr && ((c->fft_n & (c->fft_n - 1)) == 0 || c->dft.n > 0);
+    return c->tb == nullptr && ((c->fft_n & (c->fft_n - 1)) == 0 || dft_rows(c));
 }
 
 // one Arnoldi step of GMRES on P^-1 J: V_{it+1} from V_it (every instance)

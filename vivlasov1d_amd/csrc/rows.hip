@@ -1,5 +1,5 @@
 // Row blocks of the kinetic preconditioner for short x-lengths (powers of two
-// up to 512) and for any other up to 2048: a
+// up to 512) and for composite ones up to 2048 (primes: see rows_apply): a
 // workgroup owns RW consecutive v-rows (all of x), forms what is to be
 // transformed in LDS (J u, the residual F(f), or rows as they are), transforms
 // it there and stores the spectrum mode-major; and back: spectrum -> rows,
@@ -9,8 +9,10 @@
 // Stockham FFT of fft_lds.h; any other length through a mixed-radix one of the
 // same shape whose stages sum their r inputs directly (radices up to 64, or
 // the prime where it is larger), twiddles from an LDS copy of the table of
-// exp(-2 pi i m/n) at exact indices m: n sum(r) complex products a line
-// instead of the n^2 / 2 of a direct DFT (201 = 3 x 67: 70 a point).
+// exp(-2 pi i m/n) at exact indices m: n sum(r) complex products a line, so of
+// two real rows (201 = 3 x 67: 70 a point of the line), where a direct real DFT
+// takes n^2 real by complex ones for the two.  A prime's single stage does twice
+// the direct one's arithmetic.
 //
 // The strip kernel of spectral.hip keeps nx = 256, 512, 1024 (compile-time
 // width, the first FFT stage in registers) for J u; this one serves the rest:
@@ -572,7 +574,7 @@ RowGeom geom_for(const vv_ctx *c, int mode, int R, size_t *lds)
 }
 
 // rows per thread of the forward kernel: 4 (fewer halo rows) where that still
-// leaves two workgroups a CU, in number and in LDS, else 2 (at most 132 KB, at
+// leaves two workgroups a CU, in number and in LDS, else 2 (at most 113 KB, at
 // nx = 2047)
 template <typename T>
 RowGeom row_geom(const vv_ctx *c, int mode, int *R, size_t *lds)
@@ -664,9 +666,18 @@ hipError_t row_inv_t(vv_ctx *c, const T *basis, const cx_t<T> *spec, int col, T 
 // strips, 25 KB beside 32 KB and more of lines, leave one or two workgroups a
 // CU (F(f) + rFFT at 1024 x 2048: 44.8 us against 18.6 + 13.0; J u + rFFT at
 // 2048 x 1024: 41 against 12.8 + 13.2).
+// Lengths of a single stage (primes, 9, 10, 12, 14, 15) are transformed by the
+// direct real DFT (dft_rows), half the arithmetic; fusing J u and the dots with the
+// line sum still saves more launches than that costs on grids of one strip and
+// up to 2^25 products.  A solve of 8 iterations, fused and separate: 211 x 512
+// 345 and 391 us, 101 x 2048 306 and 345, but 101 x 4096 460 and 447, 151 x 2048
+// 537 and 512, 257 x 128 577 and 502, 1999 x 2048 39.2 ms and 25.6.
 bool rows_apply(const vv_ctx *c)
 {
-    return c->fuse && c->p.precond == VV_PRECOND_TENSOR_KINETIC && (c->p.nx <= 512 || c->dft.n > 0);
+    if (!c->fuse || c->p.precond != VV_PRECOND_TENSOR_KINETIC) return false;
+    const int nx = c->p.nx;
+    if (pow2(nx)) return nx <= 512;
+    return dft_rows(c) || (c->dft.n > 0 && nx <= NT && (int64_t)nx * nx * c->fft_rows * c->B <= 1 << 25);
 }
 
 int row_inv_blocks(const vv_ctx *c)
@@ -713,7 +724,7 @@ hipError_t launch_row_res(vv_ctx *c, const double *f, const double *fh, double2 
     return row_fwd_t<F_RES, double>(c, p, spec, nullptr);
 }
 
-// rows as they are (lengths with a DFT plan); y of the inverse 16-byte aligned
+// rows as they are (dft_rows); y of the inverse 16-byte aligned
 hipError_t launch_row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add,
                            double gamma)
 {

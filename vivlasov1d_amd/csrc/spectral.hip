@@ -1408,7 +1408,7 @@ template <typename T>
 hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done,
                   const T *add = nullptr, T gamma = T(0))
 {
-    if (c->dft.n) return row_rfft(c, x, spec, done, add, gamma);
+    if (dft_rows(c)) return row_rfft(c, x, spec, done, add, gamma);
     if (c->fft_n & (c->fft_n - 1)) return add != nullptr ? hipErrorInvalidValue : rdft_t<T>(c, tw, x, spec, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done, add, gamma};
@@ -1475,7 +1475,7 @@ template <typename T>
 hipError_t irfft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, const int32_t *done)
 {
     // the row blocks store pairs: a y that is not aligned for them takes the direct DFT
-    if (c->dft.n && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0) return row_irfft(c, spec, y, done);
+    if (dft_rows(c) && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0) return row_irfft(c, spec, y, done);
     if (c->fft_n & (c->fft_n - 1)) return irdft_t<T>(c, tw, spec, y, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done};

@@ -125,7 +125,7 @@ struct vv_ctx {
     int nmodes;         // fft_n/2 + 1
     int logn;           // log2(fft_n) when fft_n is a power of two (FFT kernels); else a direct DFT
     int fft_n, fft_rows;
-    vv::DftPlan dft;    // fft_n no power of two and <= kRowsNx: the line transform's plan (else n = 0)
+    vv::DftPlan dft;    // fft_n no power of two and <= kRowsNx: the line transform's plan (else n = 0); see dft_rows
     int64_t coef_stride;        // instance stride of gm/g0/gp (0: shared)
     double cf_lo, cf_mid, cf_hi;  // band constants: kinetic 0.5/1.0/0.5, potential 1.0/2.0/1.0
     double *tb;                 // potential: the transposed field (B N doubles)
@@ -266,11 +266,15 @@ hipError_t launch_rk18_stage4(vv_ctx *c, const double *x, const double *t1, cons
 hipError_t launch_rk4_end(vv_ctx *c, bool three_eighths, double *x, const double *t1, const double *t2,
                           const double *t3, const double *t4, double s);
 bool collision_term(vv_ctx *c, const double *n, const double *U, const double *a, double factor, CollTerm *t);
-// rows.hip: row blocks of the kinetic form for any nx <= kRowsNx (rows_apply);
+// rows.hip: row blocks of the kinetic form (where: rows_apply);
 // J u (with the previous step's Hessenberg update, and the collision term when
 // given) or F(f) formed and transformed in one launch, and the irFFT into
 // basis[col+1] with its CGS dots in row_inv_blocks partial rows
 DftPlan make_dft_plan(int n);
+// whether rows of an fft_n that is no power of two go through the plan: more than
+// one stage (of one the direct real DFT takes half the arithmetic: P^-1 at 1999 x
+// 2048 4.4 ms with the stage, 3.1 without; 211 x 2048 67.6 us, 59.2)
+inline bool dft_rows(const vv_ctx *c) { return c->dft.stages > 1; }
 bool rows_apply(const vv_ctx *c);
 int row_inv_blocks(const vv_ctx *c);
 hipError_t launch_row_jac(vv_ctx *c, const double *u, const double *uscale, const CollTerm *coll, double2 *spec,
