@@ -439,13 +439,16 @@ int pc_residual(vv_ctx *c, const double *f, const double *fh, double *y)
     return VV_OK;
 }
 
-// V_0 = P^-1 F(f) and its norm partials, a solve's start: the irFFT writes V_0
-// where a fused form applies, else it is copied from rhs
+// Whether residual_start's irFFT writes V_0 itself: a slice of it, or row blocks
+// (else P^-1 F is in rhs, and copied).
+bool start_slices(const vv_ctx *c) { return c->p.precond != VV_PRECOND_NONE && irfft_mdot_rows(c, false) > 0; }
+bool start_fused(const vv_ctx *c) { return start_slices(c) || (rows_apply(c) && !jac_rfft_rows(c)); }
+
+// V_0 = P^-1 F(f) and its norm partials, a solve's start
 int residual_start(vv_ctx *c, const double *f, const double *fh)
 {
-    const int slices = c->p.precond != VV_PRECOND_NONE ? irfft_mdot_rows(c, false) : 0;
-    const bool blocks = !slices && rows_apply(c) && !jac_rfft_rows(c);
-    if (!slices && !blocks) {
+    const int slices = start_slices(c) ? irfft_mdot_rows(c, false) : 0;
+    if (!start_fused(c)) {
         if (int r = pc_residual(c, f, fh, c->rhs)) return r;
         VV_CHECK(launch_start(c, c->rhs, true), "cycle start");
         return VV_OK;
@@ -917,9 +920,9 @@ int snes_impl(vv_ctx *c, double *f, const double *fh, const vv_ksp_params *kp, v
             return VV_OK;
         }
     }
-    // the right-hand side of the restarts, formed again (the first cycle's V_0
-    // was it, and f is still as it was)
-    if (more_cycles(c))
+    // the right-hand side of the restarts, formed again where only the first
+    // cycle's V_0 was it (f is still as it was)
+    if (more_cycles(c) && start_fused(c))
         if (int r = pc_residual(c, f, fh, c->rhs)) return r;
     if (int r = restart_cycles(c, c->rhs, c->D)) return r;
     // SNESSolve_KSPONLY takes the step unless the linear solve diverged
