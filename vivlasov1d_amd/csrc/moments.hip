@@ -235,8 +235,11 @@ struct ReX {                             // real parts of a complex line
 // first row of the circulant inverse, dealt to PT / span threads an output.
 // Latency-bound (barriers, LDS passes); what it saves is two dependent
 // launches and the pass over `work`: prep + conv + post took 13.0 + 11.2 +
-// 4.3 us at nx = 1024 and 6.1 + 2.7 + 3.3 us at nx = 64.
-constexpr int kPoissonOne = 320;
+// 4.3 us at nx = 1024 and 6.1 + 2.7 + 3.3 us at nx = 64.  The convolution up to 256
+// points, four threads an output; with two (257 .. 512) its chain of sums takes
+// longer than the three launches: 12.9 us at 260 and 13.9 at 300, where they take
+// 10.3 and 10.5.
+constexpr int kPoissonOne = 256;
 constexpr int kPoissonTw = 2048;
 template <bool FFT>
 __global__ __launch_bounds__(PT) void poisson_kernel(PoiArgs a)
