@@ -1368,6 +1368,21 @@ size_t fft_lds(const FftArgs<T> &a)
     return ((size_t)(a.rows >> 1) * a.nx + (a.nx < N8 ? a.nx : 0)) * sizeof(cx_t<T>);
 }
 
+// Lines that the direct real DFT transforms at least as fast as the row blocks:
+// those of a single stage, and short ones on small grids, where a pass over LDS
+// between two barriers costs more than a sum of n terms.  rFFT up to 64 points
+// (direct and row blocks, us: 50 x 128 4.2 and 5.0, 50 x 4096 5.5 and 6.0, 63 x 128
+// 4.6 and 5.0; 72 x 128 5.0 and 4.9, 80 x 1024 6.3 and 5.3), irFFT up to 96 (36 x 4096
+// 4.1 and 5.4, 80 x 1024 5.1 and 6.4, 96 x 128 4.9 and 5.1; 99 x 1024 5.9 and 5.1), both
+// up to 2^23 products (irFFT 63 x 2048 4.6 and 4.9; 50 x 4096 5.2 and 4.6, 80 x 2048 6.7
+// and 6.2).
+constexpr int kDirectFwd = 64, kDirectInv = 96;
+bool direct_lines(const vv_ctx *c, int longest)
+{
+    const int64_t n = c->fft_n;
+    return !dft_rows(c) || (n <= longest && n * n * c->fft_rows * c->B <= 1 << 23);
+}
+
 // the row-block transforms of lengths with a plan
 hipError_t row_rfft(vv_ctx *c, const double *x, double2 *spec, const int32_t *done, const double *add, double gamma)
 {
@@ -1408,7 +1423,7 @@ template <typename T>
 hipError_t rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *x, cx_t<T> *spec, const int32_t *done,
                   const T *add = nullptr, T gamma = T(0))
 {
-    if (dft_rows(c)) return row_rfft(c, x, spec, done, add, gamma);
+    if (dft_rows(c) && (add != nullptr || !direct_lines(c, kDirectFwd))) return row_rfft(c, x, spec, done, add, gamma);
     if (c->fft_n & (c->fft_n - 1)) return add != nullptr ? hipErrorInvalidValue : rdft_t<T>(c, tw, x, spec, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done, add, gamma};
@@ -1474,8 +1489,9 @@ hipError_t jac_rfft_t(vv_ctx *c, const cx_t<T> *tw, const T *u, const double *us
 template <typename T>
 hipError_t irfft_t(vv_ctx *c, const cx_t<T> *tw, const cx_t<T> *spec, T *y, const int32_t *done)
 {
-    // the row blocks store pairs: a y that is not aligned for them takes the direct DFT
-    if (dft_rows(c) && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0) return row_irfft(c, spec, y, done);
+    // the row blocks store pairs: a y that is not aligned for them takes the direct DFT too
+    if (!direct_lines(c, kDirectInv) && (reinterpret_cast<uintptr_t>(y) & (2 * sizeof(T) - 1)) == 0)
+        return row_irfft(c, spec, y, done);
     if (c->fft_n & (c->fft_n - 1)) return irdft_t<T>(c, tw, spec, y, done);
     FftArgs<T> a{c->fft_n, c->logn, c->fft_rows, fft_rows(c), c->N, spec_stride(c), spec_pitch(c),
                  (int64_t)sizeof(GmresState), tw, done};

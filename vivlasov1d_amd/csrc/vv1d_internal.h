@@ -271,7 +271,7 @@ bool collision_term(vv_ctx *c, const double *n, const double *U, const double *a
 // given) or F(f) formed and transformed in one launch, and the irFFT into
 // basis[col+1] with its CGS dots in row_inv_blocks partial rows
 DftPlan make_dft_plan(int n);
-// whether rows of an fft_n that is no power of two go through the plan: more than
+// whether rows of an fft_n that is no power of two can gain by the plan: more than
 // one stage (of one the direct real DFT takes half the arithmetic: P^-1 at 1999 x
 // 2048 4.4 ms with the stage, 3.1 without; 211 x 2048 67.6 us, 59.2)
 inline bool dft_rows(const vv_ctx *c) { return c->dft.stages > 1; }
