@@ -2,9 +2,9 @@
 
 Each translation unit is compiled separately so that the bracket kernels can
 use ``-ffp-contract=off`` (bit-faithful to the reference's unfused double
-arithmetic) while the spectral kernels keep FMA contraction; the spectral
-unit honours ``#pragma clang fp contract(off)``, which the stencil code it
-shares with the bracket kernels (arakawa.h) carries.
+arithmetic) while the spectral and row kernels keep FMA contraction; those
+units honour ``#pragma clang fp contract(off)``, which the stencil code they
+share with the bracket kernels (arakawa.h) carries.
 Usage: ``python -m vivlasov1d_amd.build`` or ``build()``.
 """
 

@@ -1037,7 +1037,7 @@ int ksp_solve_mixed_impl(vv_ctx *c, const double *b, double *x, const vv_ksp_par
 int check_params(const vv_params *p)
 {
     if (p->nx < 8 || p->nx > kMaxNx) return fail(nullptr, VV_ERR_INVALID, "nx must be in [8, 4096]");
-    if (p->nv < 8 || p->nv > 4096) return fail(nullptr, VV_ERR_INVALID, "nv must be in [8, 4096]");
+    if (p->nv < 8 || p->nv > kMaxNv) return fail(nullptr, VV_ERR_INVALID, "nv must be in [8, 4096]");
     if (p->bracket != VV_BRACKET_J1 && p->bracket != VV_BRACKET_J2 && p->bracket != VV_BRACKET_J4)
         return fail(nullptr, VV_ERR_UNSUPPORTED, "bracket must be arakawaj1, arakawaj2 or arakawaj4");
     if (p->precond != VV_PRECOND_NONE && p->precond != VV_PRECOND_TENSOR_KINETIC &&

@@ -18,10 +18,11 @@
 //
 // All reductions have a fixed grid and a fixed summation tree, so results
 // are reproducible run to run.  Each reduction kernel writes one partial per
-// workgroup; a one-workgroup "finish" kernel sums them (and, for GMRES, does
-// the Hessenberg / Givens bookkeeping).  The kernel boundary orders the
-// partials before the finish, so no device-scope fence (an L2 write-back on
-// this GPU) is needed inside the streaming kernels.
+// workgroup; one workgroup of a later launch sums them (for GMRES with the
+// Hessenberg / Givens bookkeeping, mostly inside the next step's fused J u,
+// gmres_dev.h).  The kernel boundary orders the partials before their sum, so no
+// device-scope fence (an L2 write-back on this GPU) is needed inside the
+// streaming kernels.
 #include "cgs_vec.h"
 #include "gmres_dev.h"
 
@@ -234,10 +235,7 @@ __global__ __launch_bounds__(NT) void maxpy_norm_kernel(CgsArgs<S> a, int it)
     if (threadIdx.x < nvec) {
         const double h = s_h[threadIdx.x];
         s_coef[threadIdx.x] = -h;            // VecMAXPY coefficients lhh = -HH(:, it)
-        if (blockIdx.x == 0) {
-            g->hh[it * (kMaxRestart + 1) + threadIdx.x] = h;
-            g->coef[threadIdx.x] = -h;
-        }
+        if (blockIdx.x == 0) g->hh[it * (kMaxRestart + 1) + threadIdx.x] = h;
     }
     __syncthreads();
     double w[EPT][L];

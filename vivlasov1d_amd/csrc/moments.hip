@@ -12,7 +12,8 @@
 //                    ||A phi + (n - mean n) q|| of run_base.py:631-637.
 //  poisson_prep / conv / post_kernel
 //                    the same in three launches, the convolution spread over
-//                    the chip, for long x-grids that are no power of two.
+//                    the chip, for x-grids of more than 256 points that are no
+//                    power of two.
 //  invariants_kernel mass, L2, kinetic / potential energy over f, plus the
 //                    field energy over phi (distribution_function.pyx:130-199,
 //                    hamiltonian.pyx:67-100, potential.pyx:48-59).

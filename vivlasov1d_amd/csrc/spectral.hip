@@ -3,26 +3,29 @@
 //
 //  rfft_kernel    real rows x[j][0..nx) -> spectrum S[k][j], k = 0..nx/2.
 //                 Two real rows are packed as one complex row and transformed
-//                 by an in-LDS Stockham FFT (radix-4/2; length 1024 as
-//                 4 x 8 x 8 x 4); the output is written
+//                 by an in-LDS Stockham FFT (radix 8 after up to two stages of
+//                 radix 4; length 1024 as 4 x 8 x 8 x 4); the output is written
 //                 mode-major (the transpose the reference does with a
 //                 VecScatter is folded into the store).
-//  tridiag_kernel one workgroup per mode k solves T_k c = S[k][.] along v:
-//                 partitioned Thomas (one chunk of M rows per thread) whose
-//                 reduced system (one unknown per chunk) is solved by parallel
-//                 cyclic reduction in LDS.  T_k's coefficients are rebuilt
-//                 from the mode's eigenvalue and three per-row factors, so
-//                 no factor arrays are streamed from HBM.
+//  tridiag_lu_kernel  one workgroup per mode k solves T_k c = S[k][.] along v
+//                 from reciprocal LU pivots formed once per context, which are
+//                 streamed (16 bytes a row, FP64); the bands are rebuilt from the
+//                 mode's eigenvalue and two per-row factors.
+//  tridiag_wave_kernel, tridiag_kernel  the same without pivots, for the
+//                 potential form, whose bands change every step: a wavefront or
+//                 a workgroup per mode, partitioned Thomas (one chunk of M rows
+//                 per lane or thread) whose reduced system is solved by parallel
+//                 cyclic reduction on shuffles or in LDS.
 //  irfft_kernel   spectrum -> real rows, backward-normalised like
 //                 numpy.fft.irfft / pyFFTW (imaginary parts of the k = 0 and
 //                 k = nx/2 coefficients are ignored, as in a c2r transform).
 //
-// The potential form (TensorProductPotential.pyx:157-173) runs the same three
-// kernels with the roles of x and v exchanged: the field is transposed
-// (transpose_kernel), rFFT along v, one tridiagonal system along x per
-// v-mode with bands from phi differences (potential_bands_kernel), irFFT,
-// transposed back.  The transform geometry (length, rows, modes, band
-// constants) comes from the context.
+// The potential form (TensorProductPotential.pyx:157-173) has the roles of x and
+// v exchanged: rFFT along v down the field's columns (rfft_cols_kernel; where that
+// does not apply the field is transposed, transpose_kernel, and back), one
+// tridiagonal system along x per v-mode with bands from phi differences
+// (potential_bands_kernel), irFFT.  The transform geometry (length, rows, modes,
+// band constants) comes from the context.
 //
 // Every kernel is a template on the real type: double for the FP64 path,
 // float for the FP32 preconditioner inside the mixed-precision GMRES cycle

@@ -17,7 +17,7 @@ constexpr int kMaxRestart = 64;     // GMRES restart limit (basis of restart+1 v
 constexpr int kGraphSteps = 6;      // Arnoldi steps of a part of the captured cycle
 constexpr int kGraphParts = (kMaxRestart + kGraphSteps - 1) / kGraphSteps;
 constexpr int kMaxNx = 4096;        // largest x size
-constexpr int kMaxNv = 8192;
+constexpr int kMaxNv = 4096;
 constexpr int kReduceBlocks = 512;  // fixed block count of N-sized reductions
 constexpr int kDensityChunks = 64;  // rows of nx partial sums kept per instance for the column sums
 
@@ -42,9 +42,11 @@ struct InstConst {
     double afpc;       // preconditioner band factor 0.5 hx^-1 hv^-1 / 12
 };
 
-// Device-resident GMRES state.  Written only by the one-workgroup control
-// kernels (cycle start, mdot finish, Hessenberg update, back substitution);
-// read by every Krylov kernel.
+// Device-resident GMRES state, read by every Krylov kernel.  Written by one
+// workgroup a launch and instance: the Hessenberg update or cycle start
+// (gmres_dev.h; in a launch of its own or the first workgroup of the launch that
+// carries it), the CGS update (its column of hh) and the solution update (a
+// singular triangle's reason, over).
 struct GmresState {
     GmresStatus st;
     double hh[(kMaxRestart + 1) * kMaxRestart];  // rotated Hessenberg, column it at hh[it*(kMaxRestart+1)]
@@ -52,7 +54,6 @@ struct GmresState {
     double ss[kMaxRestart];
     double grs[kMaxRestart + 1];
     double scale[kMaxRestart + 1];   // v_j = scale[j] * V_j (V_j stored unnormalised)
-    double coef[kMaxRestart + 1];    // coefficients of the pending maxpy
     double ttol, rtol, atol, dtol, haptol;
     int32_t max_it;
     int32_t max_k;
