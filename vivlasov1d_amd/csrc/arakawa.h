@@ -199,6 +199,11 @@ __device__ __forceinline__ void sep_row(const double *__restrict__ h0, int j, in
     for (int q = 0; q < 4; ++q) k[q] = a[q];
 }
 
+// the points of a kind's stencil besides the diagonal ones: the nearest
+// neighbours, and those at distance 2
+constexpr bool sep_near(int kind) { return kind != VV_BRACKET_J2; }
+constexpr bool sep_far(int kind) { return kind != VV_BRACKET_J1; }
+
 // The first argument's window alone.
 template <typename T>
 struct SepWin {
@@ -238,17 +243,17 @@ struct SepWin {
     // the weighted bracket at the centre, of the points that the kind's stencil
     // holds: J1 none at distance 2, J2 no nearest neighbours (coefficients that
     // are 0, but an infinity or NaN would come through them)
-    __device__ __forceinline__ T bracket(const T *A, const T (&B)[4], int kind) const
+    __device__ __forceinline__ T bracket(const T *A, const T (&B)[4], bool near, bool far) const
     {
 #pragma clang fp contract(off)
         T s = A[0] * (fp[2] - fm[2]), t = B[0] * (fp[2] - fp[0]);
-        if (kind != VV_BRACKET_J2) {
+        if (near) {
             s = fma_t(A[1], fp[1] - fm[1], s);
             t = fma_t(B[1], f0[3] - f0[1], t);
         }
         s = fma_t(A[2], fp[0] - fm[0], s);
         t = fma_t(B[2], fm[2] - fm[0], t);
-        if (kind != VV_BRACKET_J1) {
+        if (far) {
             s = fma_t(A[3], fp2 - fm2, s);
             t = fma_t(B[3], f0[4] - f0[0], t);
         }

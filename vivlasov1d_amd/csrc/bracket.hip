@@ -319,7 +319,7 @@ __global__ __launch_bounds__(NT) void bracket_sep_kernel(BrArgs<T> a)
             T out;
             if (MODE == MODE_RESIDUAL) out = T(0) + ht_inv * (fa[q] - fb[q]);
             else out = jacobian_base(ht_inv, win.f0[2]);
-            if (j >= 2 && j < nv - 2) out += win.bracket(sA[rr], B, KIND);
+            if (j >= 2 && j < nv - 2) out += win.bracket(sA[rr], B, sep_near(KIND), sep_far(KIND));
             if (MODE == MODE_JACOBIAN) out = scaled(out, us);      // J is linear
             yout[o] = out;
         }
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(NT) void bracket_pair_kernel(BrArgs<double> a, Hess
         const int j = tile.j0 + rr0 + q;
         if (j < nv && i < nx) {
             const size_t o = (size_t)j * nx + i;
-            yout[o] = a.alpha * (fa[q] * us) + wh.bracket(sA[rr0 + q], B, KIND);
+            yout[o] = a.alpha * (fa[q] * us) + wh.bracket(sA[rr0 + q], B, sep_near(KIND), sep_far(KIND));
             cs += arakawa_add<KIND>(wg, 0.0, 1.0, af1, af2);
         }
         if (q + 1 < ROWS_PER_WAVE) {

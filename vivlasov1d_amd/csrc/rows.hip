@@ -202,7 +202,9 @@ __device__ __forceinline__ T residual_base(T ht_inv, T f, T fh)
 // and their gaps as launches of their own, 8.0 us here with the unfactored
 // stencil, 7.3 now; 201 x 401: 5.6 + 9.3 + 3.3, 11.4, 10.4; 16 x (128 x 256): 11.4,
 // 10.0.
-template <int MODE, int R, int FK, typename T>
+// NEAR: the kind has nearest neighbours (not J2; as a branch a point 10.4 -> 10.8 us
+// at 201 x 401).
+template <int MODE, int R, int FK, bool NEAR, typename T>
 __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, RowFwd<T> p, HessArgs hs, DftPlan plan,
                                                      cx_t<T> *__restrict__ spec)
 {
@@ -248,6 +250,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
         const T ht_inv = (T)p.jr.ht_inv;
         double c1, c2;
         sep_weights(p.kind, p.jr.factor, p.jr.inst[b].af1, p.jr.inst[b].af2, c1, c2);
+        const bool far = sep_far(p.kind);
         const int grp = g.G > 1 ? div_by(t, g.mW) : 0, col = t - grp * W;
         T us = T(1);
         for (int s = 0; s < g.NS; ++s) {
@@ -335,7 +338,7 @@ __global__ __launch_bounds__(NT) void row_fwd_kernel(FftArgs<T> a, RowGeom g, Ro
                         else base = jacobian_base(ht_inv, win.f0[2]);
                         out = base;
                         if (j >= 2 && j < nv - 2) {
-                            out = base + win.bracket(sA[r0 + q], B, p.kind);
+                            out = base + win.bracket(sA[r0 + q], B, NEAR, far);
                             if (coll)
                                 out = (T)add_collision((double)out, (double)win.f0[1], (double)win.f0[2],
                                                        (double)win.f0[3], p.cv[j + 1], p.cv[j - 1], cn, cU, ca,
@@ -591,14 +594,21 @@ void fwd_launch(vv_ctx *c, const FftArgs<T> &a, const RowGeom &g, const RowFwd<T
                 size_t lds, cx_t<T> *spec)
 {
     const dim3 block(NT);
+#define VV_FWD(FK_, NEAR_) \
+    launch_timed(c, row_fwd_kernel<MODE, R, FK_, NEAR_, T>, grid, block, (uint32_t)lds, a, g, p, hs, c->dft, spec)
     if constexpr (MODE == F_PLAIN) {      // powers of two have kernels of their own
-        launch_timed(c, row_fwd_kernel<MODE, R, kDft, T>, grid, block, (uint32_t)lds, a, g, p, hs, c->dft, spec);
-        return;
-    } else
-    switch (fft_kind(a.nx)) {
-    case kFftPre: launch_timed(c, row_fwd_kernel<MODE, R, kFftPre, T>, grid, block, (uint32_t)lds, a, g, p, hs, c->dft, spec); break;
-    default: launch_timed(c, row_fwd_kernel<MODE, R, kDft, T>, grid, block, (uint32_t)lds, a, g, p, hs, c->dft, spec); break;
+        VV_FWD(kDft, true);
+    } else {
+        const bool near = sep_near(p.kind);
+        if (fft_kind(a.nx) == kFftPre) {
+            if (near) VV_FWD(kFftPre, true);
+            else VV_FWD(kFftPre, false);
+        } else {
+            if (near) VV_FWD(kDft, true);
+            else VV_FWD(kDft, false);
+        }
     }
+#undef VV_FWD
 }
 
 template <int MODE, typename T>

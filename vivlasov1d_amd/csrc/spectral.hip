@@ -186,7 +186,7 @@ __device__ __forceinline__ void jac_walk(const RF &rF, const T (*sA)[4], const d
         T out = T(0);
         if (j < nv) {
             out = jacobian_base(ht_inv, win.f0[2]);
-            if (j >= 2 && j < nv - 2) out += win.bracket(sA[q], B, KIND);
+            if (j >= 2 && j < nv - 2) out += win.bracket(sA[q], B, sep_near(KIND), sep_far(KIND));
             out = scaled(out, us);                     // == J of the VecScale'd Krylov vector
         }
         res[q] = out;
