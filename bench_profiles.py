@@ -44,16 +44,19 @@ import sys
 
 # library kernel name -> substring of the HIP kernel symbol
 SYMBOLS = {
-    "mdot": "::mdot_kernel<", "maxpy_norm": "::maxpy_norm_kernel<", "jacobian": "bracket_kernel<4, 1, double>",
-    "residual": "bracket_kernel<4, 0, double>", "rfft": "::rfft_kernel<double", "irfft": "::irfft_kernel<double",
-    "tridiag": "tridiag_lu_kernel<8, double>", "mdot32": "::mdot_kernel<", "maxpy_norm32": "::maxpy_norm_kernel<",
-    "jacobian32": "bracket_kernel<4, 1, float>", "irfft_mdot": "::irfft_mdot_kernel<double",
-    "irfft_mdot32": "::irfft_mdot_kernel<float", "jac_rfft": "::jac_rfft_kernel<4, 4, 4, double>",
-    "jac_rfft32": "::jac_rfft_kernel<4, 4, 4, float>",
+    "mdot": "::mdot_kernel<", "maxpy_norm": "::maxpy_norm_kernel<", "jacobian": "bracket_sep_kernel<4, 1, double>",
+    "residual": "bracket_kernel<4, 0>", "rfft": "::rfft_kernel<double", "irfft": "::irfft_kernel<double",
+    "tridiag": "tridiag_lu_kernel<256, 8, double, false>", "mdot32": "::mdot_kernel<",
+    "maxpy_norm32": "::maxpy_norm_kernel<", "jacobian32": "bracket_sep_kernel<4, 1, float>",
+    "irfft_mdot": "::irfft_mdot_kernel<double", "irfft_mdot32": "::irfft_mdot_kernel<float",
+    "jac_rfft": "::jac_rfft_kernel<4, 4, 4, double>", "jac_rfft32": "::jac_rfft_kernel<4, 4, 4, float>",
 }
+# the solve's start has an instance of its own of this kernel (last template argument)
+NOT = {"irfft_mdot": ", true>("}
 # kernels that return at once when enqueued past a cycle's convergence
-EARLY = ("mdot_kernel", "maxpy_norm_kernel", "bracket_kernel<4, 1", "rfft_kernel", "tridiag_kernel",
-         "tridiag_lu_kernel", "irfft_kernel", "irfft_mdot_kernel", "jac_rfft_kernel")
+EARLY = ("mdot_kernel", "maxpy_norm_kernel", "bracket_sep_kernel<4, 1", "rfft_kernel", "tridiag_lu_kernel",
+         "irfft_kernel", "irfft_mdot_kernel", "jac_rfft_kernel", "row_fwd_kernel", "row_inv_kernel",
+         "bracket_pair_kernel")
 
 
 def _short(name):
@@ -66,8 +69,10 @@ def _dur_us(r):
     return (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1000.0
 
 
-def _is_double(name, kernel):
-    # FP64 and FP32 instances share a symbol prefix; the template argument decides
+def _is_instance(name, kernel):
+    # FP64 and FP32 instances share a symbol prefix; the template arguments decide
+    if kernel in NOT and NOT[kernel] in name:
+        return False
     if kernel.endswith("32"):
         return "float" in name
     return "float" not in name
@@ -90,7 +95,7 @@ def trace_table(trace_csv, idle_us=8.0):
 def kernel_launches(rows, kernel, idle_us=8.0):
     """Durations (us) of the working launches of one library kernel, in launch order."""
     sym = SYMBOLS[kernel]
-    sel = sorted((r for r in rows if sym in r["Kernel_Name"] and _is_double(r["Kernel_Name"], kernel)),
+    sel = sorted((r for r in rows if sym in r["Kernel_Name"] and _is_instance(r["Kernel_Name"], kernel)),
                  key=lambda r: int(r["Start_Timestamp"]))
     return [d for d in (_dur_us(r) for r in sel) if d > idle_us]
 
@@ -105,7 +110,7 @@ def pmc_kib(counter_dir, counter, sym, kernel=None, idle_us=8.0, big_only=False,
     for r in csv.DictReader(open(path)):
         if r["Counter_Name"] != counter or sym not in r["Kernel_Name"]:
             continue
-        if kernel is not None and not _is_double(r["Kernel_Name"], kernel):
+        if kernel is not None and not _is_instance(r["Kernel_Name"], kernel):
             continue
         if kernel is not None and _dur_us(r) <= idle_us:
             continue

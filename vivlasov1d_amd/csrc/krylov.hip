@@ -344,7 +344,7 @@ __global__ __launch_bounds__(NT) void update_kernel(double *__restrict__ x, doub
         if (t < n) s_coef[t] = coef;
     }
     __syncthreads();
-    if (s_sing) {
+    if (s_sing) {                      // alike in every workgroup, whatever `reason` was read as
         reason = VV_KSP_DIVERGED_BREAKDOWN;
         if (blockIdx.x == 0 && t == 0) g->st.reason = reason;
     }
